@@ -2,11 +2,21 @@
 // (duplicates accumulate), fp32 / fp16 / bf16.
 //
 // Counterpart of ke_scatter_nd and its host launcher (src/kernels/scatter_nd.cu:10-95).  What
-// differs: one thread per (index row, slice element) so that a slice is read and written with
-// consecutive lanes (the reference walks a slice serially in one thread); the strides travel
-// as kernel arguments (the reference cudaMallocs them per call and never frees them); index
-// rows that point outside `data` are skipped instead of written out of bounds.
-#include <hip/hip_bf16.h>
+// differs: a slice is read and written with consecutive lanes (the reference walks it serially in
+// one thread); duplicates inside a workgroup are added up in fp32 registers before they touch
+// memory; the strides travel as kernel arguments (the reference cudaMallocs them per call and never
+// frees them); index rows that point outside `data` are skipped instead of written out of bounds.
+//
+// What bounds it: atomics on one 128-byte line are served one after another, ~20 ns each (the eight
+// L2s are not coherent with each other, so a device-wide atomic is done on the memory side).  With
+// indices that repeat as word frequencies do, the most frequent row of 8192 updates is hit ~550
+// times.  So a workgroup takes kRows updates, sorts their rows in LDS and issues ONE hardware atomic
+// per word and distinct row (16-bit types: packed pairs; a compare-and-swap loop per element, tried
+// first, retries for as long as others win).  8192 bf16 updates of 1024 into 32000 rows, log-uniform
+// indices: 2620 us with compare-and-swap, 41 with a packed atomic per update and word, 20 as here.
+// What is left is the rate of the atomics themselves, ~0.9 TB/s with distinct rows as well.
+#include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -19,56 +29,259 @@ struct Strides {
   long long dim[kMaxRank];     // their extents
 };
 
-TFK_DEVICE void atomic_add(float* p, float v) { atomicAdd(p, v); }
+constexpr int kScatterThreads = 256;
 
-// 16-bit types: compare-and-swap on the aligned 32-bit word that holds the element
+// One 32-bit word of a slice: an fp32 element or an aligned pair of 16-bit ones.
 template <typename T>
-TFK_DEVICE void atomic_add_16(T* p, T v) {
-  const size_t addr = reinterpret_cast<size_t>(p);
-  unsigned* word = reinterpret_cast<unsigned*>(addr & ~size_t(3));
-  const bool high = addr & 2;
-  unsigned old = *word, assumed;
-  do {
-    assumed = old;
-    const unsigned short cur = high ? (assumed >> 16) : (assumed & 0xffffu);
-    T x = __builtin_bit_cast(T, cur);
-    x = (T)((float)x + (float)v);
-    const unsigned short nxt = __builtin_bit_cast(unsigned short, x);
-    const unsigned repl = high ? ((assumed & 0xffffu) | ((unsigned)nxt << 16)) : ((assumed & 0xffff0000u) | nxt);
-    old = atomicCAS(word, assumed, repl);
-  } while (old != assumed);
-}
-TFK_DEVICE void atomic_add(half_t* p, half_t v) { atomic_add_16(p, v); }
-TFK_DEVICE void atomic_add(__bf16* p, __bf16 v) { atomic_add_16(p, v); }
+struct Word {
+  static constexpr int kElems = 4 / (int)sizeof(T);
+  float v[kElems];
+};
 
+// Adds `w` to the aligned word at `p` with one hardware atomic.  A 16-bit half that has nothing to
+// add passes -0.0, which changes no value.
 template <typename T>
-__global__ __launch_bounds__(256) void scatter_nd_kernel(const T* __restrict__ updates, T* __restrict__ data,
-                                                         const long long* __restrict__ indices, Strides s,
-                                                         long long n, int k, long long slice) {
-  const long long total = n * slice;
-  for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < total;
-       t += (long long)gridDim.x * blockDim.x) {
-    const long long row = t / slice, off = t - row * slice;
-    long long base = 0;
-    bool inside = true;
-    for (int j = 0; j < k; ++j) {
-      const long long ix = indices[row * k + j];
-      inside &= ix >= 0 && ix < s.dim[j];
-      base += ix * s.stride[j];
-    }
-    if (inside) atomic_add(data + base + off, updates[t]);
+TFK_DEVICE void atomic_add_word(T* p, const Word<T>& w) {
+  if constexpr (sizeof(T) == 4) {
+    unsafeAtomicAdd(p, w.v[0]);
+  } else {
+    typedef T t2 __attribute__((ext_vector_type(2)));
+    typedef short s2 __attribute__((ext_vector_type(2)));
+    const t2 x = {(T)w.v[0], (T)w.v[1]};
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (std::is_same_v<T, bf16_t>)
+      (void)__builtin_amdgcn_global_atomic_fadd_v2bf16((__attribute__((address_space(1))) s2*)p, __builtin_bit_cast(s2, x));
+    else
+      (void)__builtin_amdgcn_global_atomic_fadd_v2f16((__attribute__((address_space(1))) half2_t*)p, x);
+#endif
   }
+}
+
+// The words of one slice's sum that a lane holds: loads and adds, and the atomics.
+template <typename T, bool kSplitPairs>
+TFK_DEVICE void add_word_of_slice(Word<T>& sum, const T* src, long long e0, long long slice) {
+  constexpr int kElems = Word<T>::kElems;
+  if constexpr (kElems == 2 && !kSplitPairs) {
+    typedef T t2 __attribute__((ext_vector_type(2)));
+    if (e0 < slice) {
+      const t2 x = *reinterpret_cast<const t2*>(src + e0);
+      sum.v[0] += (float)x[0];
+      sum.v[1] += (float)x[1];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < kElems; ++e)
+      if (e0 + e >= 0 && e0 + e < slice) sum.v[e] += (float)src[e0 + e];
+  }
+}
+// with kSplitPairs a slice may start in the upper half of its first word
+template <typename T, bool kSplitPairs>
+TFK_DEVICE int first_word_shift(const T* dst) {
+  return kSplitPairs ? (int)((reinterpret_cast<size_t>(dst) / sizeof(T)) % Word<T>::kElems) : 0;
+}
+
+// Few updates: a group of `lanes` adjacent lanes (a power of two up to 64) per update, one word per
+// lane, no sort.  The call is then the latency of a load of the index, one of the update and an atomic.
+template <typename T, bool kSplitPairs>
+__global__ __launch_bounds__(kScatterThreads) void scatter_nd_direct_kernel(
+    const T* __restrict__ updates, T* __restrict__ data, const long long* __restrict__ indices, Strides s, long long n,
+    int k, long long slice, int lanes) {
+  constexpr int kElems = Word<T>::kElems;
+  const int lane = threadIdx.x & (lanes - 1);
+  const long long row = blockIdx.x * (long long)(kScatterThreads / lanes) + threadIdx.x / lanes;
+  if (row >= n) return;
+  bool inside = true;
+  long long at = 0;
+  for (int j = 0; j < k; ++j) {
+    const long long ix = indices[row * k + j];
+    inside &= ix >= 0 && ix < s.dim[j];
+    at += ix * s.stride[j];
+  }
+  if (!inside) return;
+  T* const dst = data + at;
+  const int shift = first_word_shift<T, kSplitPairs>(dst);
+  const long long step = (long long)gridDim.y * lanes * kElems;
+  for (long long e0 = ((long long)blockIdx.y * lanes + lane) * kElems - shift; e0 < slice; e0 += step) {
+    Word<T> w;
+#pragma unroll
+    for (int e = 0; e < kElems; ++e) w.v[e] = -0.f;
+    add_word_of_slice<T, kSplitPairs>(w, updates + row * slice, e0, slice);
+    atomic_add_word(dst + e0, w);
+  }
+}
+
+// Many updates: kRows per workgroup; a group of `lanes` adjacent lanes (a power of two up to 64) takes one
+// distinct row at a time, kWords words per lane.  kSplitPairs: 16-bit slices whose words are not
+// pairs of the slice (an odd slice length or an odd start); their halves are loaded one by one.
+template <typename T, int kThreads, int kRows, int kWords, bool kSplitPairs>
+__global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
+    const T* __restrict__ updates, T* __restrict__ data, const long long* __restrict__ indices, Strides s, long long n,
+    int k, long long slice, int lanes) {
+  static_assert((kRows % kWaveSize == 0 || kRows < kWaveSize) && kRows <= kThreads,
+                "part of one wavefront or whole wavefronts sort the workgroup's rows");
+  constexpr int kElems = Word<T>::kElems;
+  constexpr int kSortWaves = (kRows + kWaveSize - 1) / kWaveSize;
+  constexpr unsigned long long kOutside = ~0ull;
+  __shared__ unsigned long long s_base[kRows];   // element offset of an update's slice in data
+  __shared__ unsigned long long s_sorted[kRows];
+  __shared__ int s_order[kRows];                 // update numbers in the order of their slices
+  __shared__ int s_first[kRows + 1];             // first position of every distinct slice
+  __shared__ unsigned long long s_firsts[kSortWaves], s_valid[kSortWaves];
+  const int tid = threadIdx.x;
+  for (long long row0 = blockIdx.x * (long long)kRows; row0 < n; row0 += gridDim.x * (long long)kRows) {
+    unsigned long long base = kOutside;
+    if (tid < kRows) {
+      if (row0 + tid < n) {
+        bool inside = true;
+        unsigned long long at = 0;
+        for (int j = 0; j < k; ++j) {
+          const long long ix = indices[(row0 + tid) * k + j];
+          inside &= ix >= 0 && ix < s.dim[j];
+          at += (unsigned long long)(ix * s.stride[j]);
+        }
+        if (inside) base = at;
+      }
+      s_base[tid] = base;
+    }
+    __syncthreads();
+    if (tid < kRows) {
+      int rank = 0;
+#pragma unroll 16
+      for (int j = 0; j < kRows; ++j) {
+        const unsigned long long other = s_base[j];
+        rank += other < base || (other == base && j < tid);
+      }
+      s_order[rank] = tid;
+      s_sorted[rank] = base;
+    }
+    __syncthreads();
+    const unsigned long long mine = tid < kRows ? s_sorted[tid] : kOutside;
+    const bool first = mine != kOutside && (tid == 0 || s_sorted[tid - 1] != mine);
+    if (tid < kRows) {
+      const unsigned long long f = __ballot(first), v = __ballot(mine != kOutside);
+      if (tid % kWaveSize == 0) {
+        s_firsts[tid / kWaveSize] = f;
+        s_valid[tid / kWaveSize] = v;
+      }
+    }
+    __syncthreads();
+    int count = 0, valid = 0, before = 0;
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w) {
+      if (w == tid / kWaveSize) before = count + __popcll(s_firsts[w] & ((1ull << (tid % kWaveSize)) - 1));
+      count += __popcll(s_firsts[w]);
+      valid += __popcll(s_valid[w]);
+    }
+    if (first) s_first[before] = tid;
+    if (tid == 0) s_first[count] = valid;
+    __syncthreads();
+
+    const int groups = kThreads / lanes, lane = tid & (lanes - 1);
+    const long long words = (slice + kElems - 1 + (kSplitPairs ? 1 : 0)) / kElems;
+    for (long long word0 = (long long)blockIdx.y * lanes * kWords + lane; word0 - lane < words;
+         word0 += (long long)gridDim.y * lanes * kWords) {
+      for (int g = tid / lanes; g < count; g += groups) {
+        const int begin = s_first[g], end = s_first[g + 1];
+        T* const dst = data + s_sorted[begin];
+        const int shift = first_word_shift<T, kSplitPairs>(dst);
+        Word<T> sum[kWords];
+#pragma unroll
+        for (int v = 0; v < kWords; ++v)
+#pragma unroll
+          for (int e = 0; e < kElems; ++e) sum[v].v[e] = -0.f;
+#pragma unroll 2
+        for (int p = begin; p < end; ++p) {
+          const T* src = updates + (row0 + s_order[p]) * slice;
+#pragma unroll
+          for (int v = 0; v < kWords; ++v) {
+            const long long e0 = (word0 + (long long)v * lanes) * kElems - shift;
+            add_word_of_slice<T, kSplitPairs>(sum[v], src, e0, slice);
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < kWords; ++v) {
+          const long long e0 = (word0 + (long long)v * lanes) * kElems - shift;
+          if (e0 >= slice) continue;
+          if constexpr (std::is_same_v<T, half_t>) {
+            // a finite sum beyond fp16's largest number is added in pieces, as the single updates would be
+            constexpr float kMax = 65504.f;
+            auto beyond = [](float x) { return __builtin_fabsf(x) > kMax && __builtin_isfinite(x); };
+            while (beyond(sum[v].v[0]) || beyond(sum[v].v[1])) {
+              Word<T> part;
+#pragma unroll
+              for (int e = 0; e < 2; ++e) {
+                part.v[e] = beyond(sum[v].v[e]) ? __builtin_copysignf(kMax, sum[v].v[e]) : -0.f;
+                sum[v].v[e] -= part.v[e];
+              }
+              atomic_add_word(dst + e0, part);
+            }
+          }
+          atomic_add_word(dst + e0, sum[v]);
+        }
+      }
+    }
+    __syncthreads();   // the next updates are sorted into the same arrays
+  }
+}
+
+template <typename T, int kThreads, int kRows, int kWords, bool kSplitPairs>
+int launch_shape(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
+                 long long slice, int lanes, long long words, hipStream_t st) {
+  const long long per = (long long)lanes * kWords;
+  const dim3 grid((unsigned)std::min<long long>((n + kRows - 1) / kRows, 1 << 20),
+                  (unsigned)std::min<long long>((words + per - 1) / per, 1024));
+  hipLaunchKernelGGL((scatter_nd_kernel<T, kThreads, kRows, kWords, kSplitPairs>), grid, dim3(kThreads), 0, st,
+                     static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, lanes);
+  TFK_HIP_TRY(hipGetLastError());
+  return TF_OK;
+}
+
+template <typename T, bool kSplitPairs>
+int launch_direct(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
+                  long long slice, int lanes, long long words, hipStream_t st) {
+  const int per = kScatterThreads / lanes;
+  const dim3 grid((unsigned)((n + per - 1) / per), (unsigned)std::min<long long>((words + lanes - 1) / lanes, 1024));
+  hipLaunchKernelGGL((scatter_nd_direct_kernel<T, kSplitPairs>), grid, dim3(kScatterThreads), 0, st,
+                     static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, lanes);
+  TFK_HIP_TRY(hipGetLastError());
+  return TF_OK;
+}
+
+template <typename T, bool kSplitPairs>
+int launch_rows(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
+                long long slice, long long targets, int lanes, long long words, hipStream_t st) {
+  // Times in us with log-uniform indices (threads / updates a workgroup).  Few updates: no sort (806 of
+  // 34 fp32: direct 3.3, 256/16 5.6).  From 1024 on contention shows (2048 of 64 bf16 into 64 rows:
+  // direct 10.8, 256/16 6.3, 512/64 8.2), beyond 2048 more updates per sort pay (4096 of 1024 bf16
+  // into 1000 rows: direct 26, 256/16 17.6, 512/64 12.9).
+  if (n <= 1024) return launch_direct<T, kSplitPairs>(updates, data, indices, s, n, k, slice, lanes, words, st);
+  if (n <= 2048)
+    return launch_shape<T, 256, 16, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, lanes, words, st);
+  // Every target hit at least eight times on average: the deeper sort (59764 of 21 fp32 into 219 rows:
+  // 512/64 43, 1024/128 31; 49954 of 622 fp32 into 77: 175 and 143).
+  if (n / 8 >= targets)
+    return launch_shape<T, 1024, 128, 2, kSplitPairs>(updates, data, indices, s, n, k, slice, lanes, words, st);
+  // A workgroup of eight wavefronts hides its own latencies where there are few of them (16384 of 64
+  // bf16: 256/64 13.8, 512/64 12.5); enough of four do it better (8192 of 1024 fp32: 31.9 and 40.1).
+  if ((n / 64) * ((words + lanes - 1) / lanes) < 1024)
+    return launch_shape<T, 512, 64, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, lanes, words, st);
+  return launch_shape<T, 256, 64, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, lanes, words, st);
 }
 
 template <typename T>
 int launch(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
-           long long slice, hipStream_t st) {
-  const long long total = n * slice;
-  const int grid = (int)std::min<long long>((total + 255) / 256, 256 * 32);
-  hipLaunchKernelGGL(scatter_nd_kernel<T>, dim3(grid), dim3(256), 0, st, static_cast<const T*>(updates),
-                     static_cast<T*>(data), indices, s, n, k, slice);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+           long long slice, long long targets, hipStream_t st) {
+  constexpr int kElems = Word<T>::kElems;
+  // slices whose words are pairs of one slice in both arrays; otherwise a slice may take one word more
+  const bool pairs = kElems == 1 || (slice % 2 == 0 && reinterpret_cast<size_t>(updates) % 4 == 0 &&
+                                     reinterpret_cast<size_t>(data) % 4 == 0);
+  const long long words = (slice + kElems - 1 + (pairs ? 0 : 1)) / kElems;
+  int lanes = 1;
+  while (lanes < kWaveSize && lanes < words) lanes *= 2;
+  if constexpr (kElems == 2) {
+    if (!pairs) return launch_rows<T, true>(updates, data, indices, s, n, k, slice, targets, lanes, words, st);
+  }
+  return launch_rows<T, false>(updates, data, indices, s, n, k, slice, targets, lanes, words, st);
 }
 
 }  // namespace
@@ -85,12 +298,13 @@ extern "C" int tf_scatter_nd(const void* updates, void* data, const int64_t* ind
   TFK_REQUIRE(num_index_rows >= 0, TF_ERR_INVALID_ARG, "tf_scatter_nd: negative number of index rows");
   TFK_REQUIRE(dtype >= 0 && dtype <= 2, TF_ERR_UNSUPPORTED, "tf_scatter_nd: dtype %d (0 f32, 1 f16, 2 bf16)", dtype);
   Strides s{};
-  long long stride = 1;
+  long long stride = 1, targets = 1;
   for (int i = rank - 1; i >= 0; --i) {
     TFK_REQUIRE(data_dims[i] > 0, TF_ERR_INVALID_ARG, "tf_scatter_nd: data dimension %d is not positive", i);
     if (i < index_depth) {
       s.stride[i] = stride;
       s.dim[i] = data_dims[i];
+      targets *= data_dims[i];
     }
     stride *= data_dims[i];
   }
@@ -99,7 +313,7 @@ extern "C" int tf_scatter_nd(const void* updates, void* data, const int64_t* ind
   if (num_index_rows == 0) return TF_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const long long* idx = reinterpret_cast<const long long*>(indices);
-  if (dtype == 0) return launch<float>(updates, data, idx, s, num_index_rows, index_depth, slice, st);
-  if (dtype == 1) return launch<half_t>(updates, data, idx, s, num_index_rows, index_depth, slice, st);
-  return launch<__bf16>(updates, data, idx, s, num_index_rows, index_depth, slice, st);
+  if (dtype == 0) return launch<float>(updates, data, idx, s, num_index_rows, index_depth, slice, targets, st);
+  if (dtype == 1) return launch<half_t>(updates, data, idx, s, num_index_rows, index_depth, slice, targets, st);
+  return launch<bf16_t>(updates, data, idx, s, num_index_rows, index_depth, slice, targets, st);
 }
