@@ -13,12 +13,14 @@
 //   * the main kernel (gemm_ring64_kernel) uses 64-deep k-tiles so that every request fetches
 //     whole 128-byte lines, keeps the ring in units of one operand, and issues its MFMAs from
 //     assembly with a hand-placed instruction order (a lone wavefront issues one instruction
-//     per 4 cycles: at most three others fit behind a 16-cycle MFMA); it comes with 256 x 256
-//     tiles and, for grids that those would leave most CUs idle on, with 128 x 128 tiles;
-//     K % 64 != 0 falls back to the 32-deep direct-to-LDS kernel, other shapes to a
-//     bounds-checked one;
+//     per 4 cycles: at most three others fit behind a 16-cycle MFMA); it comes with tiles from
+//     128 x 128 to 256 x 256, for any M and N from one tile on and any K % 8 == 0 from 64 on;
+//   * problems of few rows, columns or tiles run gemm_split_k_kernel, whose wavefronts share one small
+//     tile and split K; a measured cost model picks the kernel and the tile;
 //   * workgroup -> tile map keeps the workgroups of one XCD (one L2) on a compact block of
 //     output tiles.
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "common.hpp"
@@ -53,12 +55,16 @@ struct GemmShape {
   }
 };
 
-// XCD-aware tile order.  Workgroup ids are dealt round-robin to the 8 XCDs, so ids that are
-// equal mod 8 share an L2.  Give each XCD a run of consecutive positions in a grouped
-// (4 tile-rows at a time) walk of the output so its workgroups re-use A and B panels.
+// Workgroup ids are dealt round-robin to the 8 XCDs, so ids that are equal mod 8 share an L2.  This
+// gives each XCD a run of consecutive positions out of 0 .. nblocks-1.
+TFK_DEVICE int xcd_major(int bid, int nblocks) {
+  const int xcd = bid & 7;
+  return xcd * (nblocks >> 3) + min(xcd, nblocks & 7) + (bid >> 3);
+}
+// XCD-aware tile order: a grouped (4 tile-rows at a time) walk of the output, so that the workgroups
+// of an XCD re-use A and B panels.
 TFK_DEVICE void tile_of_block(int bid, int nblocks, int tiles_m, int tiles_n, int& tm, int& tn) {
-  int pid = bid;
-  if ((nblocks & 7) == 0) pid = (bid & 7) * (nblocks >> 3) + (bid >> 3);
+  const int pid = xcd_major(bid, nblocks);
   constexpr int kGroup = 4;
   const int group_size = kGroup * tiles_n;
   const int gid = pid / group_size;
@@ -92,248 +98,6 @@ TFK_DEVICE float16_t mfma32_t(in8_t<InT> a, in8_t<InT> b, float16_t c) {
 }
 
 // ------------------------------------------------------------------------------------------
-// Fast path: M % BM == 0, N % BN == 0, K % 32 == 0.  Direct global->LDS ring, 16x16x32 MFMA.
-// ------------------------------------------------------------------------------------------
-// Tile shape of the fast path.  BK is fixed at 32: one v_mfma_f32_16x16x32_f16 consumes a whole
-// k-tile, a 16-row operand fragment is one contiguous 1 KiB of LDS, and a tile is 32 KiB at
-// 256 x 256 so that four of them are in the ring.  (Under realistic operand data the MFMA
-// rate on MI355X is set by power, and the 16x16x32 shape sustains ~17% more flop/s than
-// 32x32x16 for the same 128 x 128 wavefront tile.)
-template <int BM_, int BN_, int BK_, int WAVES_M_, int WAVES_N_, int STAGES_>
-struct DirectShape {
-  static constexpr int BM = BM_, BN = BN_, BK = BK_;
-  static constexpr int kKSteps = BK / 32;                     // MFMA k-steps per tile
-  static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_;
-  static constexpr int kStages = STAGES_;
-  static constexpr int kWaves = WAVES_M * WAVES_N;
-  static constexpr int kThreads = kWaves * kWaveSize;
-  static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;  // tile of one wavefront
-  static constexpr int TM = WM / 16, TN = WN / 16;            // 16x16 MFMA tiles per wavefront
-  static constexpr int kChunks = BK / 8;                      // 16-byte chunks per tile row
-  static constexpr int kRowsPer256B = 16 / kChunks;           // rows sharing one pass over the banks
-  static constexpr int kRowsPerInstr = 64 / kChunks;          // rows one wavefront load covers
-  static constexpr int kABytes = BM * BK * 2;
-  static constexpr int kBBytes = BN * BK * 2;
-  static constexpr int kStageBytes = kABytes + kBBytes;
-  static constexpr int kAInstr = BM * kChunks / 64 / kWaves;  // 1 KiB loads per wavefront
-  static constexpr int kBInstr = BN * kChunks / 64 / kWaves;
-  static_assert(WM % 16 == 0 && WN % 16 == 0, "wavefront tile must be MFMA-sized");
-  static_assert((BM * kChunks) % (64 * kWaves) == 0 && (BN * kChunks) % (64 * kWaves) == 0,
-                "tile rows must split evenly over the wavefronts' 1 KiB loads");
-  // XOR swizzle of the 16-byte chunk index against LDS bank conflicts of the fragment reads
-  // (lane l reads row l % 16 of a 16-row block, logical chunk l / 16 of the k-step).
-  // ds_read_b128 serves a wavefront in four passes of 16 lanes, and the passes are NOT runs of
-  // consecutive lanes: measured on gfx950 they are {0-3, 12-15, 20-23, 24-27},
-  // {4-7, 8-11, 16-19, 28-31} and the same two sets + 32.  Each pass must touch 16 different
-  // 16-byte bank groups (address mod 256).
-  //   128-byte rows and wider: chunk ^ (row / kRowsPer256B) % kChunks does that.
-  //   64-byte rows: a row supplies address bits 6-7 itself (row % 4), the chunk the bits 4-5;
-  //   a pass mixes row quads t = (row / 4) % 4 of two different chunk indices, {0, 3} of one
-  //   with {1, 2} of the next, so the XOR mask per row quad has to be 0, 2, 3, 1 (a plain
-  //   chunk ^ t leaves every pass with a two-way conflict).
-  __host__ __device__ static constexpr int swizzle(int row, int c) {
-    if constexpr (kChunks == 4) return c ^ ((0x78 >> (2 * ((row / 4) % 4))) & 3);
-    return c ^ ((row / kRowsPer256B) % kChunks);
-  }
-};
-
-template <typename S, typename OutT, typename InT>
-__global__ __launch_bounds__(S::kThreads) void gemm_direct_lds_kernel(
-    const InT* __restrict__ A, const InT* __restrict__ B, OutT* __restrict__ C, int M,
-    int N, int K, int tiles_m, int tiles_n) {
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int tile_m, tile_n;
-  tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, tile_m, tile_n);
-  const int m0 = tile_m * S::BM, n0 = tile_n * S::BN;
-  const int wm = wave / S::WAVES_N, wn = wave % S::WAVES_N;
-
-  // --- global -> LDS plan -----------------------------------------------------------------
-  // Wavefront instruction i of a tile covers 16 rows; lane l fills physical chunk l % 4 of
-  // row 16*i + l / 4 and fetches the logical chunk that the swizzle maps there.
-  constexpr int kAInstr = S::kAInstr, kBInstr = S::kBInstr;
-  const int ld_row = lane / S::kChunks;
-  const int ld_pc = lane % S::kChunks;
-  const char* a_tile = reinterpret_cast<const char*>(A + (size_t)m0 * K);
-  const char* b_tile = reinterpret_cast<const char*>(B + (size_t)n0 * K);
-  unsigned a_goff[kAInstr], b_goff[kBInstr];
-#pragma unroll
-  for (int t = 0; t < kAInstr; ++t) {
-    const int row = (wave + S::kWaves * t) * S::kRowsPerInstr + ld_row;
-    a_goff[t] = (unsigned)row * (unsigned)K * 2u + (unsigned)S::swizzle(row, ld_pc) * 16u;
-  }
-#pragma unroll
-  for (int t = 0; t < kBInstr; ++t) {
-    const int row = (wave + S::kWaves * t) * S::kRowsPerInstr + ld_row;
-    b_goff[t] = (unsigned)row * (unsigned)K * 2u + (unsigned)S::swizzle(row, ld_pc) * 16u;
-  }
-
-  // --- LDS -> register plan ---------------------------------------------------------------
-  // Fragment i of A at k-step ks: lane l reads row wm*WM + 16*i + l%16, logical chunk
-  // 4*ks + l/16 (8 halves of k).
-  const int fr = lane & 15, fg = lane >> 4;
-  const int ra = wm * S::WM + fr, rb = wn * S::WN + fr;
-  unsigned a_rd[S::kKSteps], b_rd[S::kKSteps];
-#pragma unroll
-  for (int ks = 0; ks < S::kKSteps; ++ks) {
-    a_rd[ks] = ra * S::BK * 2 + S::swizzle(ra, 4 * ks + fg) * 16;
-    b_rd[ks] = rb * S::BK * 2 + S::swizzle(rb, 4 * ks + fg) * 16;
-  }
-
-  // acc[i][j][r] = C[m0 + wm*WM + 16*i + l%16][n0 + wn*WN + 16*j + 4*(l/16) + r]: the MFMA is
-  // issued with the B fragment as its row operand, so a lane owns 4 consecutive columns of
-  // one row of C and stores them with one 8- or 16-byte instruction.
-  float4_t acc[S::TM][S::TN];
-#pragma unroll
-  for (int i = 0; i < S::TM; ++i)
-#pragma unroll
-    for (int j = 0; j < S::TN; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-  // --- main loop --------------------------------------------------------------------------
-  // kStages LDS stages, two sets of fragment registers, and an explicit issue schedule.
-  // A loaded MI355X needs the better part of a microsecond from issuing a tile's global->LDS
-  // loads to having it in LDS - about the MFMA time of a k-tile - so tile kt+kStages-1 is
-  // requested while tile kt is multiplied.  A k-tile is TM "slots" of TN MFMAs.  Per slot the
-  // wavefront also issues its share of the 1 KiB global->LDS loads of the far tile and the
-  // LDS reads that fetch one A and one B fragment of the NEXT tile, so neither the LDS pipe
-  // nor the texture-address path ever sees a burst (a burst of loads blocks the wavefront's
-  // MFMA issue while the address FIFO drains).  One workgroup barrier per k-tile, at its
-  // start: by then tile kt+1 has landed (s_waitcnt vmcnt leaves only the younger tiles'
-  // loads outstanding) and every wavefront has read all of tile kt into registers, so stage
-  // kt is free for the next iteration's loads.
-  constexpr int kLoadsPerTile = kAInstr + kBInstr;
-  constexpr int NS = S::kStages;
-  constexpr int KS = S::kKSteps;
-  constexpr int kSlots = KS * S::TM;
-  constexpr int kBarrierSlot = (KS - 1) * S::TM;  // in front of the tile's last k-step
-  static_assert(S::TN <= S::TM && (NS >= 3 || (NS == 2 && KS == 2)),
-                "issue schedule: TN <= TM; >= 3 stages, or 2 stages of 2 k-steps");
-  // NS >= 3: every slot of iteration kt requests a piece of tile kt+NS-1 (stage of tile kt-1,
-  // free since the previous barrier).  NS == 2: the slots in front of the barrier request the
-  // second half of tile kt+1, the slots behind it the first half of tile kt+2 (into the stage
-  // this barrier frees).
-  auto first_load = [](int slot) constexpr {
-    if (NS >= 3) return slot * kLoadsPerTile / kSlots;
-    return slot < kBarrierSlot ? kLoadsPerTile / 2 + slot * (kLoadsPerTile / 2) / kBarrierSlot
-                               : (slot - kBarrierSlot) * (kLoadsPerTile / 2) / (kSlots - kBarrierSlot);
-  };
-  auto end_load = [&](int slot) constexpr {
-    if (NS >= 3) return (slot + 1) * kLoadsPerTile / kSlots;
-    return slot < kBarrierSlot ? kLoadsPerTile / 2 + (slot + 1) * (kLoadsPerTile / 2) / kBarrierSlot
-                               : (slot + 1 - kBarrierSlot) * (kLoadsPerTile / 2) / (kSlots - kBarrierSlot);
-  };
-  // loads that may still be in flight when tile kt+1 is needed
-  constexpr int kInFlightAtBarrier =
-      NS >= 3 ? (NS - 3) * kLoadsPerTile + kBarrierSlot * kLoadsPerTile / kSlots : 0;
-  const int num_k_tiles = K / S::BK;
-  in8_t<InT> af[2][S::TM], bf[2][S::TN];
-
-  auto issue_load = [&](int stage, int k0, int n) __attribute__((always_inline)) {
-    char* sa = smem + stage * S::kStageBytes;
-    if (n < kAInstr) {
-      load_global_to_lds_16B(a_tile + (size_t)k0 * 2 + a_goff[n], sa + (wave + S::kWaves * n) * 1024);
-    } else {
-      const int t = n - kAInstr;
-      load_global_to_lds_16B(b_tile + (size_t)k0 * 2 + b_goff[t],
-                             sa + S::kABytes + (wave + S::kWaves * t) * 1024);
-    }
-  };
-  // Slot i of a k-step fetches its share of the NEXT k-step's fragments.  Every slot of that
-  // next step multiplies ALL B fragments with one A fragment, so B goes first (slots 0 ..
-  // TM/2-1, two fragments each) and the A fragments follow in the order they are used: when
-  // the next step starts, everything its first slots touch was requested at least TM/2 slots
-  // earlier and no MFMA ever waits on a fragment read issued just in front of it.
-  auto load_frags = [&](int stage, int ks, int buf, int i) __attribute__((always_inline)) {
-    const char* sa = smem + stage * S::kStageBytes;
-    const char* sb = sa + S::kABytes;
-    constexpr int kTotal = S::TM + S::TN;               // fragments per k-step
-    constexpr int kPerSlot = (kTotal + S::TM - 1) / S::TM;
-#pragma unroll
-    for (int f = i * kPerSlot; f < (i + 1) * kPerSlot && f < kTotal; ++f) {
-      if (f < S::TN) bf[buf][f] = *reinterpret_cast<const in8_t<InT>*>(sb + b_rd[ks] + f * 16 * S::BK * 2);
-      else af[buf][f - S::TN] = *reinterpret_cast<const in8_t<InT>*>(sa + a_rd[ks] + (f - S::TN) * 16 * S::BK * 2);
-    }
-  };
-  // Past the end the schedule keeps running on a clamped tile index: the extra loads land in
-  // a stage nobody reads again, which is cheaper than a branch per slot.
-  auto tile_k = [&](int t) __attribute__((always_inline)) { return min(t, num_k_tiles - 1) * S::BK; };
-
-  if constexpr (NS >= 3) {
-#pragma unroll
-    for (int t = 0; t < NS - 1; ++t)
-#pragma unroll
-      for (int n = 0; n < kLoadsPerTile; ++n) issue_load(t, tile_k(t), n);
-    barrier_keep_vmem<(NS - 2) * kLoadsPerTile>();
-  } else {
-#pragma unroll
-    for (int n = 0; n < kLoadsPerTile; ++n) issue_load(0, tile_k(0), n);
-#pragma unroll
-    for (int n = 0; n < kLoadsPerTile / 2; ++n) issue_load(1, tile_k(1), n);
-    barrier_keep_vmem<kLoadsPerTile / 2>();
-  }
-#pragma unroll
-  for (int i = 0; i < S::TM; ++i) load_frags(0, 0, 0, i);
-
-  // (No branch may sit inside this loop: at every control-flow join the compiler drains the
-  // LDS-direct loads with vmcnt(0), which serialises the whole pipeline.)
-  auto iteration = [&](int kt, auto parity_c) __attribute__((always_inline)) {
-    // fragment set used by k-step ks of this tile (steps alternate sets across tiles)
-    constexpr int base = (KS % 2) ? decltype(parity_c)::value : 0;
-    const int stage = kt % NS;
-    const int stage_next = (kt + 1) % NS;
-#pragma unroll
-    for (int slot = 0; slot < kSlots; ++slot) {
-      const int ks = slot / S::TM, i = slot % S::TM;
-      const int cur = base ^ (ks & 1);
-      __builtin_amdgcn_sched_barrier(0);
-      if (slot == kBarrierSlot) barrier_keep_vmem<kInFlightAtBarrier>();
-#pragma unroll
-      for (int n = first_load(slot); n < end_load(slot); ++n) {
-        if constexpr (NS >= 3) {
-          issue_load((kt + NS - 1) % NS, tile_k(kt + NS - 1), n);
-        } else {
-          if (slot < kBarrierSlot) issue_load(stage_next, tile_k(kt + 1), n);
-          else issue_load(stage, tile_k(kt + 2), n);
-        }
-      }
-      if (ks + 1 < KS) load_frags(stage, ks + 1, cur ^ 1, i);
-      else load_frags(stage_next, 0, cur ^ 1, i);
-#pragma unroll
-      for (int j = 0; j < S::TN; ++j) acc[i][j] = mfma16_t<InT>(bf[cur][j], af[cur][i], acc[i][j]);
-    }
-  };
-  int kt = 0;
-  for (; kt + 1 < num_k_tiles; kt += 2) {
-    iteration(kt, std::integral_constant<int, 0>{});
-    iteration(kt + 1, std::integral_constant<int, 1>{});
-  }
-  if (kt < num_k_tiles) iteration(kt, std::integral_constant<int, 0>{});
-  __builtin_amdgcn_sched_barrier(0);
-  wait_vmem_all();  // the clamped tail loads must not outlive the workgroup's LDS
-
-  // --- epilogue ---------------------------------------------------------------------------
-  const int c_row0 = m0 + wm * S::WM + fr;
-  const int c_col0 = n0 + wn * S::WN + 4 * fg;
-#pragma unroll
-  for (int i = 0; i < S::TM; ++i)
-#pragma unroll
-    for (int j = 0; j < S::TN; ++j) {
-      OutT* dst = C + (size_t)(c_row0 + 16 * i) * N + c_col0 + 16 * j;
-      if constexpr (sizeof(OutT) == 2) {
-        typedef OutT out4_t __attribute__((ext_vector_type(4)));
-        out4_t v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = (OutT)acc[i][j][r];
-        *reinterpret_cast<out4_t*>(dst) = v;
-      } else {
-        *reinterpret_cast<float4_t*>(dst) = acc[i][j];
-      }
-    }
-}
-
-// ------------------------------------------------------------------------------------------
 // 256 x 256 x 64 path: same 2 x 2 wavefronts of 128 x 128, but k-tiles of 64 so that every
 // global->LDS instruction fetches whole 128-byte lines (8 rows x 128 bytes).  The vector L1
 // moves full lines, so the 64-byte row segments of a 32-deep tile spend half of the L2->L1
@@ -351,21 +115,25 @@ __global__ __launch_bounds__(S::kThreads) void gemm_direct_lds_kernel(
 // Every request has at least 8 MFMA slots (1024 MFMA cycles) to land.
 // ------------------------------------------------------------------------------------------
 //
-// The same kernel serves 128 x 128 tiles (2 x 2 wavefronts of 64 x 64, units of 16 KiB) for
-// grids that 256 x 256 tiles would leave most CUs idle on.  Its k-steps are four times
-// shorter, so requests run kAhead = 4 tiles ahead (a ring of 2 * kAhead + 1 = 9 units).
-template <int BM_, int WAVES_N_, int AHEAD_>
+// The same kernel serves smaller tiles (2 x 2 wavefronts of half a tile each way), for grids that 256 x 256
+// tiles would leave CUs idle on: 3333 x 2288 x 1944 takes 45.5 us with 126 tiles of 256 x 256 and 36.7 with
+// 216 of 192 x 192; 2999 x 1544 x 1032 27.6 and, with 192 x 128, 18.7 (the bounds-checked kernel that ran
+// these shapes before: 37.8).  Units then have the size of the larger operand.  128 x 128 tiles have k-steps
+// four times shorter; where a workgroup has its CU to itself their requests run kAhead = 4 tiles
+// ahead (a ring of 2 * kAhead + 1 = 9 units).
+template <int BM_, int BN_, int AHEAD_>
 struct Ring64Shape {
-  static constexpr int BM = BM_, BN = BM_, BK = 64;
-  static constexpr int WAVES_M = 2, WAVES_N = WAVES_N_;
+  static constexpr int BM = BM_, BN = BN_, BK = 64;
+  static constexpr int WAVES_M = 2, WAVES_N = 2;
   static constexpr int kWaves = WAVES_M * WAVES_N, kThreads = kWaves * kWaveSize;
   static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
   static constexpr int TM = WM / 16, TN = WN / 16;          // 16x16 MFMA tiles per wavefront
   static constexpr int kRowBytes = BK * 2;                  // 128
-  static constexpr int kUnitBytes = BM * kRowBytes;         // one operand of one tile
+  static constexpr int kUnitBytes = (BM > BN ? BM : BN) * kRowBytes;   // one operand of one tile
   static constexpr int kAhead = AHEAD_;                     // tiles between a request and its use
   static constexpr int kUnits = 2 * kAhead + 1;
-  static constexpr int kLoads = BM / 8 / kWaves;            // 1 KiB requests per wavefront and unit
+  static constexpr int kLoadsA = BM / 8 / kWaves, kLoadsB = BN / 8 / kWaves;   // 1 KiB requests per wavefront and unit
+  static constexpr int kLoadsMax = kLoadsA > kLoadsB ? kLoadsA : kLoadsB;
   // slot schedule of a k-step (TM slots of TN MFMAs): the TM + TN fragment reads of the next
   // k-step are dealt to the first kReadSlots slots; the scalar bookkeeping runs in the gaps
   // without a read from slot kPrepSlot on
@@ -403,16 +171,22 @@ struct Ring64Shape {
     }
     return true;
   }
-  static_assert((TM == 8 || TM == 4) && (TN == 8 || TN == 4) && TM % kLoads == 0 && kLoads % 4 == 0,
-                "slot schedule: a request every TM / kLoads slots, M0 shared by four requests");
+  static_assert(BM % 64 == 0 && BN % 64 == 0, "whole MFMA tile pairs; even request counts (see the swizzle of g_off)");
   static_assert(reads_fit() && free_gaps() >= 7,
                 "slot schedule: every read and bookkeeping piece needs its own gap");
-  static_assert((2 * kAhead - 3) * kLoads < 64, "vmcnt is a 6-bit counter");
+  // requests in flight behind the barrier in the middle of a tile: A of tile t+kAhead, all of the
+  // tiles t+2 .. t+kAhead-1
+  static constexpr int kInFlight = kLoadsA + (kAhead - 2) * (kLoadsA + kLoadsB);
+  static_assert((kAhead - 1) * (kLoadsA + kLoadsB) < 64, "vmcnt is a 6-bit counter");
   // 128-byte rows: two rows per pass over the banks; chunk ^ (row / 2) % 8 keeps every
   // ds_read_b128 lane pass on 16 different bank groups
   __host__ __device__ static constexpr int swizzle(int row, int c) { return c ^ ((row / 2) % 8); }
 };
 
+__device__ const uint4_t kZeros[1] = {};   // what the chunks in front of a row are fetched from
+
+// M >= BM, N >= BN, and K >= BK: requests past the last k-tile ask for that tile again, which must not
+// be the one completed with zeros.
 // InT is half_t or bf16_t: the two differ in the MFMA mnemonic and in the conversion of the
 // result, everything else moves 16-bit elements without looking at them.
 template <typename S, typename InT, typename OutT>
@@ -426,7 +200,10 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int tile_m, tile_n;
   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, tile_m, tile_n);
-  const int m0 = tile_m * S::BM, n0 = tile_n * S::BN;
+  // The last tile of a row or column of tiles ends where C ends: it overlaps its neighbour, and the rows
+  // and columns both compute are written twice with the same bits.  No request, product or store has
+  // to know about edges.
+  const int m0 = min(tile_m * S::BM, M - S::BM), n0 = min(tile_n * S::BN, N - S::BN);
   const int wm = wave / S::WAVES_N, wn = wave % S::WAVES_N;
 
   // global -> LDS plan: request n of a wavefront covers rows (wave * kLoads + n) * 8 .. +7 of a
@@ -435,12 +212,17 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
   // swizzle maps there.  A and B share the per-lane offsets (same row stride K); the address
   // is a scalar base (tile origin + k offset) plus this 32-bit per-lane offset, so a request
   // needs no vector arithmetic.
-  const int ld_row = wave * 8 * S::kLoads + lane / 8, ld_c = lane % 8;
-  const char* a_tile = reinterpret_cast<const char*>(A + (size_t)m0 * K);
-  const char* b_tile = reinterpret_cast<const char*>(B + (size_t)n0 * K);
-  unsigned g_off[S::kLoads];
+  const int ld_row = lane / 8, ld_c = lane % 8;
+  // K is completed to whole k-tiles at its FRONT: k-tile t starts at element 64 * t - k_pad of a row, and
+  // the chunks of tile 0 that lie in front of the row are fetched from a block of zeros.  Only the
+  // prologue knows about it.
+  const int num_k_tiles = (K + S::BK - 1) / S::BK;
+  const int k_pad = num_k_tiles * S::BK - K;
+  const char* a_tile = reinterpret_cast<const char*>(A + (size_t)(m0 + wave * 8 * S::kLoadsA) * K) - 2 * k_pad;
+  const char* b_tile = reinterpret_cast<const char*>(B + (size_t)(n0 + wave * 8 * S::kLoadsB) * K) - 2 * k_pad;
+  unsigned g_off[S::kLoadsMax];
 #pragma unroll
-  for (int n = 0; n < S::kLoads; ++n)
+  for (int n = 0; n < S::kLoadsMax; ++n)
     g_off[n] = (unsigned)(ld_row + 8 * n) * (unsigned)K * 2u + (unsigned)S::swizzle(ld_row + 8 * n, ld_c) * 16u -
                1024u * (n % 4);   // the instruction's immediate offset (added to both addresses) gives it back
   // LDS -> fragment plan: fragment i of k-step ks: row 16*i + l%16 of the wavefront's rows,
@@ -459,7 +241,6 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
 #pragma unroll
     for (int j = 0; j < S::TN; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-  const int num_k_tiles = K / S::BK;
   const unsigned smem_addr = lds_address(smem);
   // Slot i of a k-step multiplies A fragment i with all B fragments; both operands have two
   // register sets (this k-step's and the next one's).
@@ -483,7 +264,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
   auto k_src = [&](const char* tile, int t) __attribute__((always_inline)) {
     return tile + (size_t)min(t, num_k_tiles - 1) * S::BK * 2;   // clamped past the end
   };
-  const unsigned lds_wave = smem_addr + wave * S::kLoads * 1024;
+  const unsigned lds_wave_a = smem_addr + wave * S::kLoadsA * 1024, lds_wave_b = smem_addr + wave * S::kLoadsB * 1024;
   // Slot with the MFMAs issued from inline assembly, accumulators pinned to AGPRs, and the
   // slot's fragment reads placed by hand between them.  (With compiler-issued MFMAs the
   // register allocator, at exactly 256 live accumulators, shuffles accumulators through VGPRs
@@ -522,24 +303,40 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
   // Workgroup barrier in the middle of tile t: tile t+1 must have landed, the requests of
   // tiles t+2 .. t+kAhead-1 and of this tile's k-step 0 stay in flight.  The LDS wait and the
   // barrier are builtins so that the compiler knows every earlier fragment read has returned.
-  constexpr int kInFlight = (2 * S::kAhead - 3) * S::kLoads;
+  constexpr int kInFlight = S::kInFlight;
   auto ring_barrier = [&]() __attribute__((always_inline)) {
     // one s_waitcnt: vmcnt(kInFlight) lgkmcnt(0); a builtin, so the compiler knows the LDS part
     __builtin_amdgcn_s_waitcnt((kInFlight & 15) | 0x70 | ((kInFlight >> 4) << 14));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  constexpr int kSlotsPerLoad = S::TM / S::kLoads;   // a request every so many slots
+  // the requests of a k-step sit at the heads of its slots, evenly spread
+  auto request_slot = [&](int i, const char* src, unsigned lds_unit, auto loads_c) __attribute__((always_inline)) {
+    constexpr int kLoads = decltype(loads_c)::value;
+#pragma unroll
+    for (int n = 0; n < kLoads; ++n)
+      if ((n * S::TM) / kLoads == i) request(src, lds_unit, n);
+  };
+  constexpr std::integral_constant<int, S::kLoadsA> kOfA{};
+  constexpr std::integral_constant<int, S::kLoadsB> kOfB{};
 
   // prologue: tiles 0 .. kAhead-1 into the first 2 * kAhead units; fragments (0, 0) once
   // tile 0 is there
 #pragma unroll
   for (int u = 0; u < 2 * S::kAhead; ++u)
 #pragma unroll
-    for (int n = 0; n < S::kLoads; ++n) {
-      request(k_src(u % 2 ? b_tile : a_tile, u / 2), lds_wave + u * S::kUnitBytes, n);
+    for (int n = 0; n < (u % 2 ? S::kLoadsB : S::kLoadsA); ++n) {
+      const char* tile = u % 2 ? b_tile : a_tile;
+      const unsigned unit = (u % 2 ? lds_wave_b : lds_wave_a) + u * S::kUnitBytes;
+      if (u < 2 && k_pad != 0) {
+        const bool in_front = S::swizzle(ld_row + 8 * n, ld_c) * 8 < k_pad;
+        const char* src = tile + (g_off[n] + 1024u * (n % 4));
+        lds_dma_16B(in_front ? reinterpret_cast<const char*>(kZeros) : src, unit + n * 1024);
+      } else {
+        request(k_src(tile, u / 2), unit, n);
+      }
     }
-  wait_vmem<2 * (S::kAhead - 1) * S::kLoads>();
+  wait_vmem<(S::kAhead - 1) * (S::kLoadsA + S::kLoadsB)>();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 #pragma unroll
@@ -568,7 +365,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
   unsigned oa = 0;                                             // A of tile t
   unsigned oa1 = 2 * S::kUnitBytes, ob1 = 3 * S::kUnitBytes;   // A, B of tile t+1
   unsigned rd_a1 = rdbase_a1, rd_b1 = rdbase_b1 + S::kUnitBytes;   // reads of (t, k-step 1)
-  unsigned req_a = lds_wave + 2 * S::kAhead * S::kUnitBytes;       // A of t+kAhead
+  unsigned req_a = lds_wave_a + 2 * S::kAhead * S::kUnitBytes;       // A of t+kAhead
   const char* src_a = k_src(a_tile, S::kAhead);
   unsigned rd_a0 = 0, rd_b0 = 0, req_b = 0;                        // set during k-step 0
   const char* src_b = b_tile;
@@ -583,7 +380,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
       case 1: ob1 = ring(oa1 + S::kUnitBytes); TFK_PIN_S(ob1); break;
       case 2: rd_a0 = rdbase_a0 + oa1; TFK_PIN_V(rd_a0); break;
       case 3: rd_b0 = rdbase_b0 + ob1; TFK_PIN_V(rd_b0); break;
-      case 4: req_b = lds_wave + oa; TFK_PIN_S(req_b); break;
+      case 4: req_b = lds_wave_b + oa; TFK_PIN_S(req_b); break;
       case 5: kt = t; TFK_PIN_S(kt); kt = min(kt + S::kAhead, last_tile); TFK_PIN_S(kt); break;
       case 6: src_b = b_tile + (size_t)(unsigned)(kt * (S::BK * 2)); TFK_PIN_S(src_b); break;
       default: break;
@@ -596,19 +393,18 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
       case 0: oa = oa1; TFK_PIN_S(oa); rd_a1 = rdbase_a1 + oa; TFK_PIN_V(rd_a1); break;
       case 1: rd_b1 = rdbase_b1 + ob1; TFK_PIN_V(rd_b1); break;
       case 2: req_a = ring(oa + 2 * S::kAhead * S::kUnitBytes); TFK_PIN_S(req_a); break;
-      case 3: req_a += lds_wave; TFK_PIN_S(req_a); break;
+      case 3: req_a += lds_wave_a; TFK_PIN_S(req_a); break;
       case 4: kt = t; TFK_PIN_S(kt); kt = min(kt + S::kAhead + 1, last_tile); TFK_PIN_S(kt); break;
       case 5: src_a = a_tile + (size_t)(unsigned)(kt * (S::BK * 2)); TFK_PIN_S(src_a); break;
       default: break;
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  // request n of a k-step goes at the head of slot n * kSlotsPerLoad
   for (int t = 0; t < num_k_tiles; ++t) {
 #pragma unroll
     for (int i = 0; i < S::TM; ++i) {
       __builtin_amdgcn_sched_barrier(0);
-      if (i % kSlotsPerLoad == 0) request(src_a, req_a, i / kSlotsPerLoad);
+      request_slot(i, src_a, req_a, kOfA);
       slot_pinned(0, i, rd_a1, rd_b1, [&](int j) __attribute__((always_inline)) {
         prep0(S::kPrep.piece[i * S::TN + j], t);
       });
@@ -618,7 +414,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
 #pragma unroll
     for (int i = 0; i < S::TM; ++i) {
       __builtin_amdgcn_sched_barrier(0);
-      if (i % kSlotsPerLoad == 0) request(src_b, req_b, i / kSlotsPerLoad);
+      request_slot(i, src_b, req_b, kOfB);
       slot_pinned(1, i, rd_a0, rd_b0, [&](int j) __attribute__((always_inline)) {
         prep1(S::kPrep.piece[i * S::TN + j], t);
       });
@@ -644,6 +440,9 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
   // of a pair of tiles (v_permlane16_swap), after which group 0/2 holds columns 0-7 / 8-15 of
   // tile j and group 1/3 the same of tile j+1, 16 bytes per lane.  Step 2: ds_bpermute moves
   // the 16 bytes of (row r, segment s) to lane 4*r + s.
+  // (An odd N leaves the rows of C, and then the vectors of a store, without alignment.)
+  typedef uint4_t out16B_t __attribute__((aligned(2)));
+  typedef float4_t out4f_t __attribute__((aligned(4)));
   const int c_row0 = m0 + wm * S::WM;
   if constexpr (sizeof(OutT) == 2) {
     const int st_row = lane >> 2, st_seg = lane & 3;
@@ -674,7 +473,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
         v[1] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)x[1]);
         v[2] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)y[0]);
         v[3] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)y[1]);
-        *reinterpret_cast<uint4_t*>(c_lane + (size_t)(16 * i) * N + 16 * j) = v;
+        *reinterpret_cast<out16B_t*>(c_lane + (size_t)(16 * i) * N + 16 * j) = v;
       }
   } else {
     const int c_col0 = n0 + wn * S::WN + 4 * fg;
@@ -682,21 +481,17 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
     for (int i = 0; i < S::TM; ++i)
 #pragma unroll
       for (int j = 0; j < S::TN; ++j)
-        *reinterpret_cast<float4_t*>(C + (size_t)(c_row0 + fr + 16 * i) * N + c_col0 + 16 * j) = acc[i][j];
+        *reinterpret_cast<out4f_t*>(C + (size_t)(c_row0 + fr + 16 * i) * N + c_col0 + 16 * j) = acc[i][j];
   }
 }
 
-using RingBig = Ring64Shape<256, 2, 2>;   // 5 units of 32 KiB
-using RingMid = Ring64Shape<128, 2, 4>;   // 9 units of 16 KiB: one workgroup per CU, requests 4 tiles ahead
-using RingMid2 = Ring64Shape<128, 2, 2>;  // 5 units of 16 KiB: two workgroups per CU cover each other's stalls
-
-template <typename S, typename OutT, typename InT = half_t>
+template <typename S, typename OutT, typename InT>
 int launch_ring64(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st) {
   auto kern = gemm_ring64_kernel<S, InT, OutT>;
   constexpr int lds = S::kUnits * S::kUnitBytes;
   static_assert(lds <= kMaxLdsBytes, "ring does not fit in LDS");
   TFK_LDS_OPT_IN(kern, lds);
-  const int tiles_m = M / S::BM, tiles_n = N / S::BN;
+  const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
   hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(S::kThreads), lds, st,
                      static_cast<const InT*>(A), static_cast<const InT*>(B),
                      static_cast<OutT*>(C), M, N, K, tiles_m, tiles_n);
@@ -705,7 +500,192 @@ int launch_ring64(const void* A, const void* B, void* C, int M, int N, int K, hi
 }
 
 // ------------------------------------------------------------------------------------------
-// General path: any M, N; K % 8 == 0.  Register-staged, bounds-checked, one LDS stage.
+// Few rows, few columns or few tiles: the wavefronts of a workgroup share ONE output tile of
+// 16*TM x 16*TN and split K among themselves (k-tile t goes to wavefront t % kWaves), each streaming
+// its own part of both operands through an LDS ring of its own: no barrier until the partial tiles
+// are added up in LDS at the end.
+//
+// Such problems are bound by how fast a CU takes in its operands: a tile of 32 x 16 does 21 flops per
+// byte.  Operand fragments read straight from memory into registers run into the address unit, which
+// merges only ADJACENT lanes - the sixteen rows of a fragment lie 16 lanes apart, 64 accesses per
+// KiB, a quarter of the L1's rate (32 x 4096 x 4096: 12.7 us).  LDS-direct requests of 8 rows x 128 bytes
+// are whole lines: 7.8 us, 4.4 TB/s (the 64 x 64 bounds-checked kernel that ran before: 68.6).
+// ------------------------------------------------------------------------------------------
+template <int TM_, int TN_, int WAVES_, int STAGES_>
+struct SplitKShape {
+  static constexpr int TM = TM_, TN = TN_, kWaves = WAVES_, kStages = STAGES_;
+  static constexpr int BM = 16 * TM, BN = 16 * TN, BK = 64;
+  static constexpr int kThreads = kWaves * kWaveSize;
+  static constexpr int kFrags = TM + TN;                      // 16-row operand fragments per 32-deep step
+  static constexpr int kLoads = 2 * kFrags;                   // 1 KiB requests (8 rows x 128 bytes) per k-tile
+  static constexpr int kStageBytes = kLoads * 1024;
+  static constexpr int kPitch = BN + 4;                       // floats per row of a partial tile in LDS
+  static constexpr int kRingBytes = kWaves * kStages * kStageBytes;
+  static constexpr int kPartBytes = kWaves * BM * kPitch * 4;
+  static constexpr int kLdsBytes = kRingBytes > kPartBytes ? kRingBytes : kPartBytes;
+  static_assert(kStages >= 2 && kStages <= 4 && (kStages - 1) * kLoads < 64, "vmcnt is a 6-bit counter");
+  // the same swizzle as the big kernel's: conflict-free fragment reads of 128-byte rows
+  __host__ __device__ static constexpr int swizzle(int row, int c) { return c ^ ((row / 2) % 8); }
+};
+
+template <typename S, typename InT, typename OutT>
+__global__ __launch_bounds__(S::kThreads) void gemm_split_k_kernel(
+    const InT* __restrict__ A, const InT* __restrict__ B, OutT* __restrict__ C, int M, int N, int K, int tiles_m,
+    int tiles_n) {
+  using V8 = in8_t<InT>;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  // consecutive tiles of one XCD share columns of B (m runs fastest)
+  const int pid = xcd_major(blockIdx.x, tiles_m * tiles_n);
+  const int m0 = pid % tiles_m * S::BM, n0 = pid / tiles_m * S::BN;
+
+  // Request n of a k-tile: rows 8n .. 8n+7 of A (n < 2 TM) or B, lane l fills physical chunk l % 8 of
+  // row l / 8.  Rows past the edge re-fetch the last one.  The chunks of the last k-tile that lie
+  // behind K fetch that tile's first chunk instead; their products are masked below.
+  const char* a_tile = reinterpret_cast<const char*>(A + (size_t)m0 * K);
+  const char* b_tile = reinterpret_cast<const char*>(B + (size_t)n0 * K);
+  const int num_k_tiles = (K + S::BK - 1) / S::BK, last_tile = num_k_tiles - 1;
+  unsigned off[S::kLoads], off_last[S::kLoads];
+#pragma unroll
+  for (int n = 0; n < S::kLoads; ++n) {
+    const bool of_a = n < 2 * S::TM;
+    const int row = (of_a ? n : n - 2 * S::TM) * 8 + lane / 8;
+    const int c = S::swizzle(row, lane % 8);
+    const unsigned base = (unsigned)min(row, (of_a ? M - m0 : N - n0) - 1) * (unsigned)K * 2u;
+    off[n] = base + 16u * c;
+    off_last[n] = last_tile * S::BK + 8 * c < K ? off[n] : base;
+  }
+  const unsigned ring = lds_address(smem) + wave * S::kStages * S::kStageBytes;
+  auto request = [&](int stage, int kt) __attribute__((always_inline)) {
+    const bool last = kt == last_tile;
+#pragma unroll
+    for (int n = 0; n < S::kLoads; ++n) {
+      const char* src = (n < 2 * S::TM ? a_tile : b_tile) + (size_t)kt * (S::BK * 2);
+      // (the LDS destination is an M0 input of the statement, the s_nop the wait state behind an M0 write)
+      asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                   :
+                   : "v"(last ? off_last[n] : off[n]), "s"(src), "{m0}"(ring + stage * S::kStageBytes + n * 1024)
+                   : "memory");
+    }
+  };
+  unsigned rd[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) rd[ks] = ring + lr * 128 + S::swizzle(lr, 4 * ks + lg) * 16;
+
+  float4_t acc[S::TM][S::TN];
+#pragma unroll
+  for (int i = 0; i < S::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < S::TN; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+  V8 fr[2][2][S::kFrags];   // [set][32-deep step][fragments of A, then of B]
+  auto read = [&](int set, int stage) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int f = 0; f < S::kFrags; ++f)
+        fr[set][ks][f] =
+            *(__attribute__((address_space(3))) const V8*)(size_t)(rd[ks] + stage * S::kStageBytes + f * 2048);
+  };
+  auto mask_behind_k = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      if (last_tile * S::BK + (4 * ks + lg) * 8 >= K) {
+#pragma unroll
+        for (int f = 0; f < S::kFrags; ++f)
+#pragma unroll
+          for (int t = 0; t < 8; ++t) fr[set][ks][f][t] = (InT)0.f;
+      }
+  };
+  // waits until only this wavefront's `tiles` youngest k-tiles are still in flight
+  auto wait_behind = [&](int tiles) __attribute__((always_inline)) {
+    if (S::kStages > 3 && tiles >= 3) wait_vmem<3 * (S::kStages > 3 ? S::kLoads : 0)>();
+    else if (S::kStages > 2 && tiles >= 2) wait_vmem<2 * (S::kStages > 2 ? S::kLoads : 0)>();
+    else if (tiles >= 1) wait_vmem<S::kLoads>();
+    else wait_vmem<0>();
+  };
+  const int mine = wave < num_k_tiles ? (last_tile - wave) / S::kWaves + 1 : 0;   // k-tiles of this wavefront
+  auto tile_of = [&](int t) __attribute__((always_inline)) { return wave + t * S::kWaves; };
+#pragma unroll
+  for (int t = 0; t < S::kStages; ++t)
+    if (t < mine) request(t, tile_of(t));
+  if (mine > 0) {
+    wait_behind(min(mine, S::kStages) - 1);
+    read(0, 0);
+  }
+  int stage = 0;   // of tile t
+  // Tile t: its fragments are on their way into set t % 2; once they have arrived its stage takes tile
+  // t + kStages, and the fragments of tile t + 1 are requested under the products of tile t.
+  auto step = [&](int t, auto set_c) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_c)::value;
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + S::kStages < mine) request(stage, tile_of(t + S::kStages));
+    stage = stage + 1 == S::kStages ? 0 : stage + 1;
+    if (t + 1 < mine) {
+      wait_behind(min(mine - 2 - t, S::kStages - 1));
+      read(set ^ 1, stage);
+    }
+    if (K % S::BK != 0 && tile_of(t) == last_tile) mask_behind_k(set);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < S::TM; ++i)
+#pragma unroll
+        for (int j = 0; j < S::TN; ++j) acc[i][j] = mfma16_t<InT>(fr[set][ks][S::TM + j], fr[set][ks][i], acc[i][j]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (int t = 0; t < mine; t += 2) {
+    step(t, std::integral_constant<int, 0>{});
+    if (t + 1 < mine) step(t + 1, std::integral_constant<int, 1>{});
+  }
+  __syncthreads();   // every ring has been read: the partial tiles take their place
+
+  float* s_part = reinterpret_cast<float*>(smem);
+  float* own = s_part + wave * S::BM * S::kPitch;
+#pragma unroll
+  for (int i = 0; i < S::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < S::TN; ++j)
+      *reinterpret_cast<float4_t*>(own + (16 * i + lr) * S::kPitch + 16 * j + 4 * lg) = acc[i][j];
+  __syncthreads();
+  for (int f = tid; f < S::BM * S::BN / 4; f += S::kThreads) {
+    const int row = f / (S::BN / 4), col = f % (S::BN / 4) * 4;
+    float4_t sum = *reinterpret_cast<const float4_t*>(s_part + row * S::kPitch + col);
+#pragma unroll
+    for (int w = 1; w < S::kWaves; ++w)
+      sum += *reinterpret_cast<const float4_t*>(s_part + (w * S::BM + row) * S::kPitch + col);
+    if (m0 + row >= M) continue;
+    OutT* dst = C + (size_t)(m0 + row) * N + n0 + col;
+    if (n0 + col + 4 <= N) {
+      typedef OutT out4_t __attribute__((ext_vector_type(4)));
+      typedef out4_t out4_any_t __attribute__((aligned(sizeof(OutT))));   // rows of an odd N have no alignment
+      *reinterpret_cast<out4_any_t*>(dst) = out4_t{(OutT)sum[0], (OutT)sum[1], (OutT)sum[2], (OutT)sum[3]};
+    } else {
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+        if (n0 + col + r < N) dst[r] = (OutT)sum[r];
+    }
+  }
+}
+
+template <typename S, typename OutT, typename InT>
+int launch_split_k(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st) {
+  auto kern = gemm_split_k_kernel<S, InT, OutT>;
+  static_assert(S::kLdsBytes <= kMaxLdsBytes, "rings do not fit in LDS");
+  if constexpr (S::kLdsBytes > 64 * 1024) TFK_LDS_OPT_IN(kern, S::kLdsBytes);
+  const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
+  hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(S::kThreads), S::kLdsBytes, st, static_cast<const InT*>(A),
+                     static_cast<const InT*>(B), static_cast<OutT*>(C), M, N, K, tiles_m, tiles_n);
+  TFK_HIP_TRY(hipGetLastError());
+  return TF_OK;
+}
+
+// ------------------------------------------------------------------------------------------
+// Operands that do not start at a 16-byte boundary: any M, N; K % 8 == 0.  Register-staged,
+// bounds-checked, one LDS stage.
 // ------------------------------------------------------------------------------------------
 template <typename S, typename OutT, typename InT>
 __global__ __launch_bounds__(S::kThreads) void gemm_guarded_kernel(
@@ -777,23 +757,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_guarded_kernel(
       }
 }
 
-using ShapeBig = DirectShape<256, 256, 32, 2, 2, 4>;         // 4 x 32 KiB of LDS, 128x128 per wavefront
-using ShapeMid = DirectShape<128, 128, 32, 2, 2, 4>;      // 4 x 16 KiB, 64x64 per wavefront
 using ShapeSmall = GemmShape<64, 64, 32, 2, 2, 1>;    // bounds-checked path
-
-template <typename S, typename OutT, typename InT>
-int launch_direct(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st) {
-  auto kern = gemm_direct_lds_kernel<S, OutT, InT>;
-  constexpr int lds = S::kStages * S::kStageBytes;
-  static_assert(lds <= kMaxLdsBytes, "tile does not fit in LDS");
-  TFK_LDS_OPT_IN(kern, lds);
-  const int tiles_m = M / S::BM, tiles_n = N / S::BN;
-  hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(S::kThreads), lds, st,
-                     static_cast<const InT*>(A), static_cast<const InT*>(B),
-                     static_cast<OutT*>(C), M, N, K, tiles_m, tiles_n);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
-}
 
 template <typename S, typename OutT, typename InT>
 int launch_guarded(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st) {
@@ -805,33 +769,99 @@ int launch_guarded(const void* A, const void* B, void* C, int M, int N, int K, h
   return TF_OK;
 }
 
-bool ring64_fits(int M, int N, int K) { return M % 128 == 0 && N % 128 == 0 && K % 64 == 0; }
+// ------------------------------------------------------------------------------------------
+// Which kernel: the one that a cost model expects to be done first.
+//
+// The tiles of a problem, the rounds in which 256 CUs do them and the k-tiles of each are known; what
+// a k-tile costs is measured.  Microseconds, fitted to 264 problems (M 1-8192, N and K 64-8192, bf16, three
+// to eight rotating operand sets; root mean square error 8-16% a kernel).  Taking the expected best is
+// 3.5% behind taking the measured best of all kernels on average, and never 2x.
+//   ring kernels:    start + rounds * (round + ktiles * (step + shared * fill + unaligned))
+//     `shared` is what a CU pays for the others' requests, times how much of the chip a round fills: a
+//     128 x 128 tile's k-tile takes 0.30 us with few workgroups, 0.56 with one on every CU (its
+//     32 KiB a k-tile then ask 15 TB/s of the L2s), a 256 x 256 tile's 0.85 and 1.6 for four times the work.
+//   split-K kernels: start + max(rounds * ktiles of one wavefront * step,
+//                                tiles per CU * ktiles * (shared + unaligned)) + tiles per CU * round
+//     the latency of one workgroup's chain, or the rate at which a CU takes in all of its workgroups.
+// `unaligned` applies where K is no multiple of 64: rows then start anywhere in a 128-byte line.
+// ------------------------------------------------------------------------------------------
+struct GemmKernel {
+  int bm, bn, waves;        // output tile; wavefronts that share its K (ring kernels: 1)
+  int per_cu;               // workgroups that a CU holds
+  bool ring;
+  float start, round, step, shared, unaligned;
+  int64_t min_tiles = 0, max_tiles = INT64_MAX;   // where the figures apply
+};
+constexpr GemmKernel kGemmKernels[] = {
+    {16, 16, 4, 4, false, 2.25f, 0.18f, 0.208f, 0.056f, 0.005f},
+    {16, 16, 8, 2, false, 2.32f, 0.42f, 0.279f, 0.057f, 0.005f},
+    {32, 16, 4, 3, false, 2.36f, 0.28f, 0.259f, 0.089f, 0.009f},
+    {32, 32, 1, 8, false, 2.41f, 0.13f, 0.294f, 0.100f, 0.050f},
+    {32, 32, 4, 2, false, 2.30f, 0.50f, 0.342f, 0.128f, 0.012f},
+    {64, 32, 4, 1, false, 2.42f, 1.44f, 0.527f, 0.235f, 0.042f},
+    {64, 64, 4, 1, false, 2.87f, 2.12f, 0.785f, 0.324f, 0.092f},
+    {128, 128, 1, 1, true, 0.58f, 3.23f, 0.298f, 0.260f, 0.205f},              // requests 4 tiles ahead
+    {128, 128, 1, 1, true, 0.92f, 2.29f, 0.386f, 0.284f, 0.129f, 0, 256},      // 2 tiles ahead: starts sooner
+    {128, 128, 1, 2, true, 2.30f, 1.51f, 0.160f, 0.349f, 0.176f, 257},         // ... and shares a CU in pairs
+    {192, 128, 1, 1, true, 0.21f, 3.75f, 0.426f, 0.331f, 0.212f},
+    {192, 192, 1, 1, true, 0.00f, 4.93f, 0.529f, 0.509f, 0.233f},
+    {256, 128, 1, 1, true, 0.00f, 4.60f, 0.496f, 0.447f, 0.266f},
+    {256, 192, 1, 1, true, 0.00f, 5.84f, 0.670f, 0.583f, 0.240f},
+    {256, 256, 1, 1, true, 0.00f, 6.63f, 0.851f, 0.729f, 0.216f},
+};
+constexpr int kNumGemmKernels = sizeof(kGemmKernels) / sizeof(kGemmKernels[0]);
 
-template <typename OutT, typename InT>
-int dispatch_ring64(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st) {
-  // 256 x 256 tiles do ~1.5x the work per cycle of 128 x 128 tiles (measured: 96 vs 146 us at
-  // 4096^3) but come in quarters as many: compare the rounds of tiles the 256 CUs need, a round
-  // of big tiles costing 4 units and a round of mid tiles 1.6.
-  constexpr int64_t kCUs = 256;
-  const bool big_fits = M % 256 == 0 && N % 256 == 0;
-  const int64_t big_rounds = ((M / 256) * (N / 256) + kCUs - 1) / kCUs;
-  const int64_t mid_rounds = ((M / 128) * (N / 128) + kCUs - 1) / kCUs;
-  if (big_fits && 5 * big_rounds <= 2 * mid_rounds)
-    return launch_ring64<RingBig, OutT, InT>(A, B, C, M, N, K, st);
-  // more 128 x 128 tiles than CUs: the 80 KiB variant, so that two workgroups share a CU
-  // (2048 x 4096 x 2048: 33.3 -> 30.5 us); otherwise the deep ring
-  if ((M / 128) * (N / 128) > kCUs) return launch_ring64<RingMid2, OutT, InT>(A, B, C, M, N, K, st);
-  return launch_ring64<RingMid, OutT, InT>(A, B, C, M, N, K, st);
+float expected_us(const GemmKernel& g, int64_t tiles, int ktiles, bool unaligned_rows) {
+  const int64_t rounds = (tiles + 256 * g.per_cu - 1) / (256 * g.per_cu);
+  const float unaligned = unaligned_rows ? g.unaligned : 0.f;
+  const float per_cu = tiles / 256.f;
+  if (g.ring) {
+    const float fill = std::min(1.f, per_cu / (rounds * g.per_cu));
+    return g.start + rounds * g.per_cu * (g.round + ktiles * (g.step + g.shared * fill + unaligned));
+  }
+  const int chain = (ktiles + g.waves - 1) / g.waves;
+  return g.start + std::max(rounds * chain * g.step, per_cu * ktiles * (g.shared + unaligned)) + per_cu * g.round;
+}
+
+int pick_gemm_kernel(int M, int N, int K) {
+  int best = 0;
+  float best_us = INFINITY;
+  const int ktiles = (K + 63) / 64;
+#pragma unroll   // the divisions are by constants then
+  for (int i = 0; i < kNumGemmKernels; ++i) {
+    const GemmKernel& g = kGemmKernels[i];
+    if (g.ring && (M < g.bm || N < g.bn || K < 64)) continue;   // (what gemm_ring64_kernel asks for)
+    const int64_t tiles = (int64_t)((M + g.bm - 1) / g.bm) * ((N + g.bn - 1) / g.bn);
+    if (tiles < g.min_tiles || tiles > g.max_tiles) continue;
+    const float us = expected_us(g, tiles, ktiles, K % 64 != 0);
+    if (us < best_us) {
+      best = i;
+      best_us = us;
+    }
+  }
+  return best;
 }
 
 template <typename OutT, typename InT>
 int dispatch(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st) {
-  if (ring64_fits(M, N, K)) return dispatch_ring64<OutT, InT>(A, B, C, M, N, K, st);
-  if (M % 256 == 0 && N % 256 == 0 && K % ShapeBig::BK == 0 && (int64_t)(M / 256) * (N / 256) >= 128)
-    return launch_direct<ShapeBig, OutT, InT>(A, B, C, M, N, K, st);
-  if (M % 128 == 0 && N % 128 == 0 && K % 32 == 0)
-    return launch_direct<ShapeMid, OutT, InT>(A, B, C, M, N, K, st);
-  return launch_guarded<ShapeSmall, OutT, InT>(A, B, C, M, N, K, st);
+  using Launcher = int (*)(const void*, const void*, void*, int, int, int, hipStream_t);
+  static constexpr Launcher kLaunchers[] = {
+      launch_split_k<SplitKShape<1, 1, 4, 2>, OutT, InT>, launch_split_k<SplitKShape<1, 1, 8, 2>, OutT, InT>,
+      launch_split_k<SplitKShape<2, 1, 4, 2>, OutT, InT>, launch_split_k<SplitKShape<2, 2, 1, 2>, OutT, InT>,
+      launch_split_k<SplitKShape<2, 2, 4, 2>, OutT, InT>, launch_split_k<SplitKShape<4, 2, 4, 2>, OutT, InT>,
+      launch_split_k<SplitKShape<4, 4, 4, 2>, OutT, InT>,
+      launch_ring64<Ring64Shape<128, 128, 4>, OutT, InT>, launch_ring64<Ring64Shape<128, 128, 2>, OutT, InT>,
+      launch_ring64<Ring64Shape<128, 128, 2>, OutT, InT>, launch_ring64<Ring64Shape<192, 128, 2>, OutT, InT>,
+      launch_ring64<Ring64Shape<192, 192, 2>, OutT, InT>, launch_ring64<Ring64Shape<256, 128, 2>, OutT, InT>,
+      launch_ring64<Ring64Shape<256, 192, 2>, OutT, InT>, launch_ring64<Ring64Shape<256, 256, 2>, OutT, InT>,
+  };
+  static_assert(sizeof(kLaunchers) / sizeof(kLaunchers[0]) == kNumGemmKernels, "one launcher per row of kGemmKernels");
+  // LDS-direct requests take 16 bytes at a 16-byte boundary.  (2^35 elements of C with a K below the ring
+  // kernels' are more threads than a launch of the split-K kernels may have.)
+  if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) % 16 != 0 ||
+      (K < 64 && (int64_t)M * N >= (int64_t)1 << 35))
+    return launch_guarded<ShapeSmall, OutT, InT>(A, B, C, M, N, K, st);
+  return kLaunchers[pick_gemm_kernel(M, N, K)](A, B, C, M, N, K, st);
 }
 
 }  // namespace
