@@ -103,3 +103,21 @@ def test_c5_full_size():
         assert ok, f"slice {i}: rel_l2={r:.3e} max_abs={m:.3e}"
     o16 = c_decode(q, k, v, 16)
     assert (o.float() - o16.float()).abs().max() < 1e-3
+
+
+# The cut is the library's: one workgroup of 8 or (from 512 slices on) 4 wavefronts per slice and no
+# partials, or up to num_splits ranges reduced by workgroups of 8 (fewer than 1024 of them) or 4
+# wavefronts.  Lengths around the rows of a load step (32 or 64) and of the two batches in flight.
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, (1e-3, 2e-2)), (torch.bfloat16, (4e-3, 4e-2))])
+@pytest.mark.parametrize("bh,lkv,d,splits", [(3, 31, 128, 64), (3, 65, 64, 64), (513, 33, 128, 64), (520, 63, 64, 3),
+                                             (600, 300, 64, 64), (4, 2047, 128, 64), (5, 4097, 64, 64),
+                                             (2, 9000, 128, 2), (40, 6000, 64, 64), (270, 2100, 128, 9), (1, 1, 64, 2)])
+def test_every_way_to_cut(bh, lkv, d, splits, dtype, tol):
+    g = torch.Generator(device=DEV).manual_seed(bh + lkv)
+    q = torch.randn(bh, d, device=DEV, generator=g).to(dtype)
+    k = torch.randn(bh, lkv, d, device=DEV, generator=g).to(dtype)
+    v = torch.randn(bh, lkv, d, device=DEV, generator=g).to(dtype)
+    scores = (k.float() * q.float()[:, None]).sum(-1) / math.sqrt(d)
+    ref = (torch.softmax(scores, -1)[..., None] * v.float()).sum(1)
+    o = c_decode(q, k, v, splits)
+    assert o.dtype == dtype and N.rel_l2(o, ref) <= tol[0] and N.max_abs(o, ref) <= tol[1]

@@ -1,22 +1,25 @@
 // Split-KV flash-decoding for gfx950: single-query attention per (batch x head) slice with the
-// key/value range cut into `num_splits` chunks, followed by a log-sum-exp combine.
+// key/value range cut into up to `num_splits` chunks, followed by a log-sum-exp combine (or, where one
+// workgroup per slice is done sooner, not cut and finished in one kernel).
 //
 // No counterpart in the reference (it has no decoding kernel); the per-chunk algebra is the
 // online softmax of include/kernels/flash_attention_device.cuh:257-301 with one query row.
 // Both kernels are HBM-bound streaming kernels, MFMA is irrelevant (1 flop per byte):
-//   * split kernel: grid (num_splits, batch_heads), 4 wavefronts.  One key row of 128 16-bit
+//   * split kernel: grid (splits, batch_heads), 4 or 8 wavefronts.  One key row of 128 16-bit
 //     elements is 256 bytes = 16 lanes x 16 bytes (head dimension 64: 8 lanes), so a wavefront
 //     load instruction fetches 4 (8) whole rows fully coalesced; every group of 16 (8) lanes keeps
-//     its own running (max, sum, o[D]) over the rows it sees and only the final merge of the 16
-//     (32) groups of a workgroup goes through LDS.  The dot product is v_dot2 (fp16 or bf16) +
+//     its own running (max, sum, o[D]) over the rows it sees; the groups of a wavefront are merged with
+//     lane swaps, the wavefronts through LDS.  The dot product is v_dot2 (fp16 or bf16) +
 //     a DPP reduction inside the lane group;
-//     two batches of 8 rows per group are in flight (32 KiB per wavefront), the next one
+//     two batches of 4 rows per group are in flight (16 KiB per wavefront), the next one
 //     requested before the current one is consumed; the partials leave through streaming
 //     stores (ordinary stores in the middle of the read stream cost 7% of its bandwidth);
-//   * combine kernel: grid batch_heads, 128 threads, merges the fp32 partials.
+//   * combine kernel: grid batch_heads, merges the fp32 partials.
 // The kernels are templates of the element type (fp16 / bf16, the reference's 16-bit types,
 // include/kernels/dispatch_macros.hpp:6-23) and of the head dimension (128 / 64).
 // All offsets are 64-bit.
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -25,10 +28,12 @@
 namespace tfk {
 namespace {
 
+// Rows per lane group in one batch of loads; two batches are in flight.  Eight instead of four took 214
+// registers and two wavefronts per SIMD (802 slices of 2574 x 128 in 4 splits: 171 us, with four 165).
+constexpr int kBatchRows = 4;
+using float2_t = float __attribute__((ext_vector_type(2)));
+
 constexpr int kD = 128;   // head dimension of the benchmark configuration (and of the static entry point)
-constexpr int kDecWaves = 4;
-constexpr int kDecThreads = kDecWaves * kWaveSize;
-constexpr int kBatchRows = 8;                // rows per lane group in one batch of loads (two batches in flight)
 
 template <int CTRL>
 TFK_DEVICE float dpp_f32(float x) {
@@ -52,6 +57,31 @@ TFK_DEVICE float group_sum(float x) {
   return x;
 }
 
+// op(x of this lane, x of the lane kXor away), kXor = 8, 16 or 32
+template <int kXor, typename Op>
+TFK_DEVICE float xor_combine(float x, Op op) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (kXor == 8) {
+    return op(x, dpp_f32<0x128>(x));  // row_ror:8
+  } else {
+    const unsigned u = __builtin_bit_cast(unsigned, x);
+    // with both operands x, the swap leaves the even rows (halves) in one and the odd ones in the other
+    const auto sw = kXor == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false)
+                               : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const unsigned a = sw[0], b = sw[1];
+    return op(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+  }
+#else
+  return x;
+#endif
+}
+// op over the lanes that hold the same vector of different rows; every lane ends up with the result
+template <int kLanesPerRow, typename Op>
+TFK_DEVICE float across_rows(float x, Op op) {
+  if constexpr (kLanesPerRow == 8) x = xor_combine<8>(x, op);
+  return xor_combine<32>(xor_combine<16>(x, op), op);
+}
+
 template <typename T>
 struct Vec8 {
   using type = T __attribute__((ext_vector_type(8)));
@@ -69,19 +99,21 @@ TFK_DEVICE float dot8(typename Vec8<T>::type k, typename Vec8<T>::type q) {
   return acc;
 }
 
-// workspace: o_part [batch_heads][num_splits][D] fp32, then ml_part [batch_heads][num_splits][2]
-template <typename T, int D>
-__global__ __launch_bounds__(kDecThreads) void flash_decode_split_kernel(
-    const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
+// workspace: o_part [batch_heads][num_splits][D] fp32, then ml_part [batch_heads][num_splits][2].
+// kWhole: one workgroup per slice, which writes O itself (num_splits == 1, chunk == Lkv).
+// `chunk` is a multiple of the rows of one load step.
+// kDecWaves wavefronts per workgroup.
+template <typename T, int D, int kDecWaves, bool kWhole>
+__global__ __launch_bounds__(kDecWaves * kWaveSize) void flash_decode_split_kernel(
+    const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, T* __restrict__ O,
     float* __restrict__ o_part, float* __restrict__ ml_part, int64_t Lkv, int num_splits,
     int64_t chunk, float scale_log2) {
   using V8 = typename Vec8<T>::type;
   constexpr int kLanesPerRow = D / 8;                   // 16-byte vectors per row
   constexpr int kRowsPerWave = kWaveSize / kLanesPerRow;  // rows one wavefront load instruction covers
   constexpr int kRowsPerStep = kDecWaves * kRowsPerWave;  // ... and one workgroup load step
-  constexpr int kGroups = kDecThreads / kLanesPerRow;
-  __shared__ float s_o[kGroups][D];
-  __shared__ float s_m[kGroups], s_l[kGroups];
+  __shared__ float s_o[kDecWaves][D];
+  __shared__ float s_m[kDecWaves], s_l[kDecWaves];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lv = lane % kLanesPerRow, gw = lane / kLanesPerRow;   // vector of the row, row of the wavefront's load
@@ -122,15 +154,21 @@ __global__ __launch_bounds__(kDecThreads) void flash_decode_split_kernel(
       for (int u = 0; u < kBatchRows; ++u)
         vd[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(vb + lane_off + u * (kRowsPerStep * D * 2)));
     } else {
+      // the steps behind the end of the chunk are left out (workgroup-uniform); their V is zero because
+      // their weights are
 #pragma unroll
       for (int u = 0; u < kBatchRows; ++u) {
         const int64_t row = min(base + lane_row + (int64_t)u * kRowsPerStep, Lkv - 1);
-        kd[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(kbase + row * D));
+        if (base + (int64_t)u * kRowsPerStep < row_end)
+          kd[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(kbase + row * D));
       }
 #pragma unroll
       for (int u = 0; u < kBatchRows; ++u) {
         const int64_t row = min(base + lane_row + (int64_t)u * kRowsPerStep, Lkv - 1);
-        vd[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(vbase + row * D));
+        if (base + (int64_t)u * kRowsPerStep < row_end)
+          vd[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(vbase + row * D));
+        else
+          vd[u] = V8{};
       }
     }
     __builtin_amdgcn_sched_barrier(0);   // the requests leave before the other batch is consumed
@@ -172,26 +210,37 @@ __global__ __launch_bounds__(kDecThreads) void flash_decode_split_kernel(
     consume(k_b, v_b, base + kBatchSpan);
   }
 
-  // merge the lane groups of the workgroup
-  const int grp = tid / kLanesPerRow;
+  // merge the lane groups of the wavefront, then the wavefronts
+  const auto add = [](float a, float b) { return a + b; };
+  float big = across_rows<kLanesPerRow>(m_run, [](float a, float b) { return fmaxf(a, b); });
+  const float scale = __builtin_amdgcn_exp2f(m_run - ((big == -INFINITY) ? 0.f : big));
+  l_run = across_rows<kLanesPerRow>(l_run * scale, add);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) s_o[grp][8 * lv + i] = o[i];
-  if (lv == 0) {
-    s_m[grp] = m_run;
-    s_l[grp] = l_run;
+  for (int i = 0; i < 8; ++i) o[i] = across_rows<kLanesPerRow>(o[i] * scale, add);
+  if (gw == 0) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s_o[wave][8 * lv + i] = o[i];
+  }
+  if (lane == 0) {
+    s_m[wave] = big;
+    s_l[wave] = l_run;
   }
   __syncthreads();
   if (tid < D) {
-    float big = -INFINITY;
+    big = -INFINITY;
 #pragma unroll
-    for (int g = 0; g < kGroups; ++g) big = fmaxf(big, s_m[g]);
+    for (int w = 0; w < kDecWaves; ++w) big = fmaxf(big, s_m[w]);
     const float big_safe = (big == -INFINITY) ? 0.f : big;
     float acc = 0.f, l = 0.f;
 #pragma unroll
-    for (int g = 0; g < kGroups; ++g) {
-      const float w = __builtin_amdgcn_exp2f(s_m[g] - big_safe);
-      acc += w * s_o[g][tid];
-      l += w * s_l[g];
+    for (int w = 0; w < kDecWaves; ++w) {
+      const float f = __builtin_amdgcn_exp2f(s_m[w] - big_safe);
+      acc += f * s_o[w][tid];
+      l += f * s_l[w];
+    }
+    if constexpr (kWhole) {
+      O[bh * D + tid] = (T)(acc / l);
+      return;
     }
     const int64_t idx = bh * num_splits + split;
     // Streaming stores: an ordinary store of these few hundred bytes per workgroup, issued in
@@ -205,24 +254,59 @@ __global__ __launch_bounds__(kDecThreads) void flash_decode_split_kernel(
   }
 }
 
+// One workgroup per slice: groups of D / 4 lanes take every kGroups-th split with its loads in flight at
+// once, then the groups are added up in LDS.  (One thread per column that walks the splits one after
+// another is a chain of loads: 9.5 us for 64 splits of 32 slices, 2.4 as here.)
+constexpr int kCombThreads = 256;
 template <typename T, int D>
-__global__ __launch_bounds__(D) void flash_decode_combine_kernel(
+__global__ __launch_bounds__(kCombThreads) void flash_decode_combine_kernel(
     const float* __restrict__ o_part, const float* __restrict__ ml_part, T* __restrict__ O,
     int num_splits) {
+  constexpr int kLanes = D / 4, kGroups = kCombThreads / kLanes, kUnroll = 8;
+  __shared__ float4_t s_o[kGroups][kLanes];
+  __shared__ float s_l[kGroups];
   const int64_t bh = blockIdx.x;
-  const int d = threadIdx.x;
-  const float* ml = ml_part + bh * num_splits * 2;
-  const float* op = o_part + bh * num_splits * D + d;
+  const int lane = threadIdx.x % kLanes, grp = threadIdx.x / kLanes;
+  const float2_t* ml = reinterpret_cast<const float2_t*>(ml_part) + bh * num_splits;
+  const float4_t* op = reinterpret_cast<const float4_t*>(o_part + bh * num_splits * D) + lane;
+  float4_t o[kUnroll];
+  float2_t m[kUnroll];
+  auto load = [&](int s0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int s = min(s0 + u * kGroups, num_splits - 1);
+      o[u] = op[(int64_t)s * kLanes];
+      m[u] = ml[s];
+    }
+  };
+  load(grp);   // in flight while the maximum is found
   float big = -INFINITY;
-  for (int s = 0; s < num_splits; ++s) big = fmaxf(big, ml[2 * s]);
-  float acc = 0.f, l = 0.f;
-#pragma unroll 8
-  for (int s = 0; s < num_splits; ++s) {
-    const float w = __builtin_amdgcn_exp2f(ml[2 * s] - big);
-    acc += w * op[(int64_t)s * D];
-    l += w * ml[2 * s + 1];
+  for (int s = threadIdx.x % kWaveSize; s < num_splits; s += kWaveSize) big = fmaxf(big, ml[s][0]);
+#pragma unroll
+  for (int x = 1; x < kWaveSize; x *= 2) big = fmaxf(big, __shfl_xor(big, x));
+  float4_t acc = {0.f, 0.f, 0.f, 0.f};
+  float l = 0.f;
+  for (int s0 = grp; s0 < num_splits; s0 += kGroups * kUnroll) {
+    if (s0 != grp) load(s0);
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const float w = s0 + u * kGroups < num_splits ? __builtin_amdgcn_exp2f(m[u][0] - big) : 0.f;
+      acc += w * o[u];
+      l += w * m[u][1];
+    }
   }
-  O[bh * D + d] = (T)(acc / l);
+  s_o[grp][lane] = acc;
+  if (lane == 0) s_l[grp] = l;
+  __syncthreads();
+  if (threadIdx.x < D) {
+    float sum = 0.f, total = 0.f;
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+      sum += s_o[g][threadIdx.x / 4][threadIdx.x % 4];
+      total += s_l[g];
+    }
+    O[bh * D + threadIdx.x] = (T)(sum / total);
+  }
 }
 
 }  // namespace
@@ -251,21 +335,82 @@ int check_decode_args(const char* who, const void* Q, const void* K, const void*
   return TF_OK;
 }
 
-// Split kernel + combine kernel on `st`; `partials` holds o_part then ml_part.
+template <typename T, int D, int kDecWaves, int kBatchRows, bool kWhole>
+int launch_split(const void* Q, const void* K, const void* V, void* O, float* o_part, float* ml_part,
+                 int64_t batch_heads, int64_t Lkv, int splits, int64_t chunk, double softmax_scale, hipStream_t st) {
+  const float scale_log2 = (float)(softmax_scale * 1.4426950408889634);
+  hipLaunchKernelGGL((flash_decode_split_kernel<T, D, kDecWaves, kBatchRows, kWhole>), dim3(splits, (unsigned)batch_heads),
+                     dim3(kDecWaves * kWaveSize), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K),
+                     static_cast<const T*>(V), static_cast<T*>(O), o_part, ml_part, Lkv, splits, chunk, scale_log2);
+  TFK_HIP_TRY(hipGetLastError());
+  return TF_OK;
+}
+
+// How a problem is cut.  `splits` ranges of `chunk` keys per slice; 1: one workgroup per slice, no partials
+// and no second kernel.
+struct DecodePlan {
+  int splits;
+  int64_t chunk;
+};
+// One workgroup takes in ~45 GB/s when few run, all of them together 6.7 TB/s; the second kernel and its
+// launch cost ~4 us.  Measured (fp16, us, one workgroup per slice / best split): 33 slices of 662 x 64
+// 6.5 / 8.1, 964 of 913 x 128 68 / 73, 11 of 825 x 128 10.4 / 8.5, 64 of 8192 x 128 85 / 44.  Slices that the
+// CUs cannot share evenly cost about a third of the unevenness (802 of 2574 x 128: 180 / 165).
+// Otherwise the cut aims at 1024 workgroups, and at no more than 256 KiB of keys and values in each: they
+// come in rounds, and the last one fills the chip badly (584 of 16256 x 64: 4 splits 411, 16 364; 136 of
+// 36053 x 64: 8 splits 201, 32 192), but at 32 KiB at least (32 of 1999 x 64: 16 splits 10.2, 64 12.8),
+// all within the caller's num_splits.
+template <int D>
+DecodePlan plan_decode(int64_t batch_heads, int64_t Lkv, int num_splits) {
+  const double slice_bytes = 4.0 * D * Lkv, stream_us = slice_bytes * batch_heads / 6.7e6, alone_us = slice_bytes / 45e3;
+  const double per_cu = batch_heads / 256.0;
+  const double uneven = per_cu > 1.0 ? 1.0 + 0.35 * (std::ceil(per_cu) / per_cu - 1.0) : 1.0;
+  const DecodePlan whole = {1, Lkv};
+  if (num_splits == 1 || 2.5 + std::max(alone_us, stream_us * uneven) <= 6.5 + stream_us) return whole;
+  constexpr int64_t kStep = 8 * (kWaveSize / (D / 8));   // rows of one load step of the larger workgroup
+  const int64_t fill = (1024 + batch_heads - 1) / batch_heads;
+  const int64_t least = (int64_t)(slice_bytes / 262144.0) + 1, most = (int64_t)(slice_bytes / 32768.0) + 1;
+  const int64_t want = std::min<int64_t>(num_splits, std::min(std::max(fill, least), most));
+  const int64_t chunk = ((Lkv + want - 1) / want + kStep - 1) / kStep * kStep;
+  const int64_t splits = (Lkv + chunk - 1) / chunk;
+  return splits > 1 ? DecodePlan{(int)splits, chunk} : whole;
+}
+
+template <typename T, int D, int kDecWaves, bool kWhole>
+int launch_split(const void* Q, const void* K, const void* V, void* O, float* o_part, float* ml_part,
+                 int64_t batch_heads, int64_t Lkv, DecodePlan plan, double softmax_scale, hipStream_t st) {
+  const float scale_log2 = (float)(softmax_scale * 1.4426950408889634);
+  hipLaunchKernelGGL((flash_decode_split_kernel<T, D, kDecWaves, kWhole>), dim3(plan.splits, (unsigned)batch_heads),
+                     dim3(kDecWaves * kWaveSize), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K),
+                     static_cast<const T*>(V), static_cast<T*>(O), o_part, ml_part, Lkv, plan.splits, plan.chunk,
+                     scale_log2);
+  TFK_HIP_TRY(hipGetLastError());
+  return TF_OK;
+}
+
+// Split kernel and, if the plan cuts, combine kernel on `st`; `partials` holds o_part then ml_part.
 template <typename T, int D>
 int launch_decode_t(const void* Q, const void* K, const void* V, void* O, float* partials,
                     int64_t batch_heads, int64_t Lkv, int num_splits, double softmax_scale,
                     hipStream_t st) {
+  const DecodePlan plan = plan_decode<D>(batch_heads, Lkv, num_splits);
+  if (plan.splits == 1) {
+    // eight wavefronts take in a slice faster, four share a full chip better (512 slices of 32768 x 128:
+    // 1254 and 1203 us; 33 of 662 x 64: 6.5 and 8.1)
+    if (batch_heads >= 512)
+      return launch_split<T, D, 4, true>(Q, K, V, O, nullptr, nullptr, batch_heads, Lkv, plan, softmax_scale, st);
+    return launch_split<T, D, 8, true>(Q, K, V, O, nullptr, nullptr, batch_heads, Lkv, plan, softmax_scale, st);
+  }
   float* o_part = partials;
-  float* ml_part = o_part + (size_t)batch_heads * num_splits * D;
-  const int64_t chunk = (Lkv + num_splits - 1) / num_splits;
-  const float scale_log2 = (float)(softmax_scale * 1.4426950408889634);
-  hipLaunchKernelGGL((flash_decode_split_kernel<T, D>), dim3(num_splits, (unsigned)batch_heads),
-                     dim3(kDecThreads), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K),
-                     static_cast<const T*>(V), o_part, ml_part, Lkv, num_splits, chunk, scale_log2);
-  TFK_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL((flash_decode_combine_kernel<T, D>), dim3((unsigned)batch_heads), dim3(D), 0, st,
-                     o_part, ml_part, static_cast<T*>(O), num_splits);
+  float* ml_part = o_part + (size_t)batch_heads * plan.splits * D;
+  // few workgroups: eight wavefronts each (8 slices of 65536 x 128 in 16 splits: 76 us with four, 54 with
+  // eight; 802 of 2574 x 128 in 4: 165 and 173)
+  const int rc = batch_heads * plan.splits < 1024
+      ? launch_split<T, D, 8, false>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st)
+      : launch_split<T, D, 4, false>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st);
+  if (rc != TF_OK) return rc;
+  hipLaunchKernelGGL((flash_decode_combine_kernel<T, D>), dim3((unsigned)batch_heads), dim3(kCombThreads), 0, st,
+                     o_part, ml_part, static_cast<T*>(O), plan.splits);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
