@@ -120,6 +120,13 @@ TF_API int tf_flash_attention_fwd(const void* Q, const void* K, const void* V, v
                                   int tile_hidden_qk, int tile_hidden_v, double softmax_scale,
                                   int causal, void* stream);
 
+/* Head dimensions 160, 192 and 256 (D == Dv) with V in its natural [batch, Lkv, Dv] layout: tuned kernels, any Lq,
+ * Lkv % 32 == 0, operands at 16-byte boundaries, else TF_ERR_UNSUPPORTED.  Q is not rescaled: the
+ * softmax scale is applied to the fp32 scores. */
+TF_API int tf_flash_attention_fwd_wide(const void* Q, const void* K, const void* V, void* O, int dtype, int64_t batch,
+                                       int64_t Lq, int64_t Lkv, int64_t D, double softmax_scale, int causal,
+                                       void* stream);
+
 /* Single-query (decoding) attention with the KV range split into `num_splits` chunks:
  * kernel 1 writes per-split partial (o, max, sum) in fp32 into `workspace`, kernel 2 merges
  * them with a log-sum-exp weighted sum into O.

@@ -183,6 +183,40 @@ def test_flash_attention_ops_shrink_tiles_that_do_not_fit_the_lds(d, dv, lq, lkv
     assert ok, (r, m)
 
 
+# Both workgroup sizes (64 queries; 128 where that saves a round of the 256 CUs), one key tile, fewer than
+# the ring holds and more, rows that no tile divides, the paired and the one-tile causal orders.
+# Bounds: four times what the kernel shows against 64-bit sums (2.8e-4 fp16, 2.3e-3 bf16: the 16-bit weights
+# and result).
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 1.2e-3), (torch.bfloat16, 1e-2)])
+@pytest.mark.parametrize("d", [160, 192, 256])
+@pytest.mark.parametrize("bh,lq,lkv,causal", [(1, 1, 32, False), (2, 65, 96, False), (2, 130, 160, True), (2, 512, 512, True),
+                                              (150, 129, 64, False), (80, 500, 512, True), (150, 384, 384, True)])
+def test_flash_attention_wide_heads(bh, lq, lkv, causal, d, dtype, tol):
+    g = torch.Generator().manual_seed(d + lq + lkv)
+    q, k, v = (torch.randn(bh, n, d, generator=g).to(dtype) for n in (lq, lkv, lkv))
+    scale = 1.0 / math.sqrt(d)
+    o = torch.full((bh, lq, d), float("nan"), dtype=dtype, device=DEV)
+    torch.ops.tilefusion.flash_attention_fwd(q.to(DEV), k.to(DEV), v.to(DEV), o, scale, causal)
+    s = q.to(DEV).float() @ k.to(DEV).float().transpose(-1, -2).contiguous() * scale
+    if causal:
+        s.masked_fill_(torch.ones(lq, lkv, dtype=torch.bool, device=DEV).triu(1), -math.inf)
+    ref = torch.softmax(s, -1) @ v.to(DEV).float()
+    assert ((o.float() - ref).norm() / ref.norm()).item() < tol
+
+
+def test_flash_attention_wide_heads_keep_rows_whose_first_scores_are_minus_infinity():
+    # the first two key tiles score -inf: their weights are zero and the row's reference comes from the third
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(1, n, 256, generator=g).half() for n in (40, 128, 128))
+    q[..., 0] = 1.0
+    k[:, :64, 0] = -math.inf
+    scale = 4.0
+    o = torch.empty(1, 40, 256, dtype=torch.float16, device=DEV)
+    torch.ops.tilefusion.flash_attention_fwd(q.to(DEV), k.to(DEV), v.to(DEV), o, scale, False)
+    ref = torch.softmax(q.float() @ k.float().transpose(1, 2) * scale, -1) @ v.float()
+    assert ((o.float().cpu() - ref).norm() / ref.norm()).item() < 1.2e-3
+
+
 def test_flash_attention_key_length_that_cannot_be_padded_is_a_clear_error():
     # above 128 the header kernel is what runs, and its key tiles are 32 wide
     q = torch.randn(16, 160, dtype=torch.float16, device=DEV)

@@ -27,21 +27,25 @@
 namespace tfk {
 namespace {
 
-constexpr int kBN = 64;   // keys per tile
+// Keys per tile.  Above a head dimension of 128 a tile of 64 keys is 64 KiB, of which the LDS holds two;
+// 32 keys leave room for a ring of four.
+__host__ __device__ constexpr int key_tile(int d) { return d <= 128 ? 64 : 32; }
 // LDS ring depth: the 8-wavefront kernel keeps two tiles live (its two wavefront sets are half a
 // tile apart) and three in flight; the 4-wavefront kernel one live and three in flight.
 __host__ __device__ constexpr int ring_stages(int waves) { return waves == 8 ? 5 : 4; }
 // Row pitch (in elements) of a [key][dim] tile in LDS: the next power of two.  The swizzles XOR
 // chunk indices, which needs a power-of-two chunk count, and a 1 KiB request must cover whole
-// rows.  A head dimension of 96 is kept in 128-element rows whose last quarter is never read.
-__host__ __device__ constexpr int lds_pitch(int d) { return d <= 64 ? 64 : 128; }
+// rows.  A head dimension of 96 is kept in 128-element rows whose last quarter is never read (160 and
+// 192 likewise in 256-element rows).
+__host__ __device__ constexpr int lds_pitch(int d) { return d <= 64 ? 64 : d <= 128 ? 128 : 256; }
 
 // K tile [kBN][D] (and a transposed V tile [DV][kBN]): 16 consecutive rows reading one logical
-// 16-byte chunk hit 16 different bank groups.
+// 16-byte chunk hit 16 different bank groups.  The pattern repeats every 16 rows at the latest, so that
+// the fragments of different 16-row blocks differ by a constant.
 template <int CH>
 __host__ __device__ constexpr int swz_k(int row, int c) {
   constexpr int kRowsPer256B = CH >= 16 ? 1 : 16 / CH;
-  return c ^ ((row / kRowsPer256B) % CH);
+  return c ^ ((row / kRowsPer256B) % (CH > 16 ? 16 : CH));
 }
 // V tile [kBN][DV] read by transposing 4-row x 16-column blocks: a half wavefront touches 8
 // rows x 32 bytes at the same column, which must land in 8 different 32-byte bank windows.
@@ -106,14 +110,24 @@ TFK_DEVICE float quad_max(float x) {
 
 // kWavesT wavefronts x 32 queries per workgroup.  8 wavefronts (256 queries) halve the
 // K/V traffic per query and put two wavefronts on every SIMD, so one wavefront's softmax
-// (VALU) overlaps the other's MFMAs; 4 wavefronts serve short query ranges.
+// (VALU) overlaps the other's MFMAs; 4 wavefronts serve short query ranges and, with 32 or 16
+// queries each (kQB), head dimensions above 128.
+//
+// Above 128 (kWide) the output accumulators and Q fragments of 32 queries take 192 registers, which two
+// wavefronts on a SIMD do not have.  What bounds these instances: the four wavefronts read the whole
+// K and V tile for 32 queries each, 128 KiB of LDS reads a key tile for 64 MFMAs on each SIMD (1024 cycles of
+// either), and one wavefront per SIMD puts the softmax behind them instead of beside them.
+// The scale is applied to the fp32 scores there: Q stays as it came, a second rounding of Q
+// would make a 16-bit result measurably worse.
 template <typename T, int D, int DV, bool kVT, bool kCausal, int kWavesT, int kQB>
 __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
-    T* __restrict__ O, int Lq, int Lkv, float scale_log2, int q_tiles, int total_items) {
+    T* __restrict__ O, int Lq, int Lkv, float scale_log2, int q_tiles, int total_items, int paired) {
   using V2 = typename Vec<T>::v2;
   using V4 = typename Vec<T>::v4;
   using V8 = typename Vec<T>::v8;
+  constexpr bool kWide = D > 128;
+  constexpr int kBN = key_tile(D);
   constexpr int kStages = ring_stages(kWavesT);
   constexpr int kRowsPerWave = 16 * kQB;  // kQB 16-query blocks per wavefront
   constexpr int kBMq = kWavesT * kRowsPerWave;
@@ -145,12 +159,13 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   //   causal:     work per query tile grows with its position, so a workgroup takes query
   //               tile q_tiles-1-p and then tile p of the same slice: every workgroup does the
   //               same amount of work, no sorting by weight is needed and the slice-major
-  //               order (with its L2 locality) is kept.  An odd number of query tiles falls
-  //               back to one tile per workgroup, heaviest tiles first over all slices.
+  //               order (with its L2 locality) is kept.  An odd number of query tiles, or fewer
+  //               tiles than CUs (see launch_w), runs one tile per workgroup, heaviest first
+  //               over all slices.
   int qt_of_pass[2] = {0, 0};
   int num_passes = 1;
   size_t bh;
-  if (!kCausal || q_tiles % 2 == 0) {
+  if (!kCausal || paired) {
     const int per_slice = kCausal ? q_tiles / 2 : q_tiles;
     const int per_xcd = (total_items + 7) / 8;
     const int item = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
@@ -192,8 +207,12 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
 #pragma unroll
     for (int kk = 0; kk < kKK; ++kk) {
       const V8 raw = *reinterpret_cast<const V8*>(Q + (size_t)m_ld * D + kk * 32 + lg * 8);
+      if constexpr (kWide) {
+        qf[kk][qb] = raw;
+      } else {
 #pragma unroll
-      for (int t = 0; t < 8; ++t) qf[kk][qb][t] = to_elem_saturating<T>((float)raw[t] * scale_log2);
+        for (int t = 0; t < 8; ++t) qf[kk][qb][t] = to_elem_saturating<T>((float)raw[t] * scale_log2);
+      }
     }
   }
 
@@ -333,8 +352,10 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   // another wavefront of the SIMD streams MFMAs - against 8 for an ordinary VALU instruction.)
   float neg_m[kQB];
   float4_t l_acc[kQB];
+  bool unset[kQB];    // kWide: no finite score seen yet (the row's reference is not set)
 #pragma unroll
   for (int qb = 0; qb < kQB; ++qb) {
+    unset[qb] = true;
     neg_m[qb] = 0.f;  // reference 0 until the first tile raises it
     l_acc[qb] = float4_t{0.f, 0.f, 0.f, 0.f};
   }
@@ -386,7 +407,10 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
 #pragma unroll
     for (int kb = 0; kb < kKB; ++kb)
 #pragma unroll
-      for (int qb = 0; qb < kQB; ++qb) s[kb][qb] = float4_t{neg_m[qb], neg_m[qb], neg_m[qb], neg_m[qb]};
+      for (int qb = 0; qb < kQB; ++qb) {
+        const float start = kWide ? 0.f : neg_m[qb];
+        s[kb][qb] = float4_t{start, start, start, start};
+      }
 #pragma unroll
     for (int kk = 0; kk < kKK; ++kk) {
       const unsigned ka = kk + 1 < kKK ? opaque(smem_base + (it % kStages) * kStageBytes + k_off[kk + 1]) : 0u;
@@ -415,6 +439,14 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     const int n0 = it * kBN;
     v_reads(0, it, 0);
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kWide) {
+#pragma unroll
+      for (int kb = 0; kb < kKB; ++kb)
+#pragma unroll
+        for (int qb = 0; qb < kQB; ++qb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) s[kb][qb][r] = fmaf(s[kb][qb][r], scale_log2, neg_m[qb]);
+    }
     // ---- mask -------------------------------------------------------------------------
     if constexpr (kMask) {
 #pragma unroll
@@ -446,16 +478,23 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) mx[qb] = fmaxf(mx[qb], s[kb][qb][r]);
       grow |= mx[qb] > kLazy;
+      if constexpr (kWide) grow |= unset[qb];
     }
     // The first tile sets the reference to the row's true maximum, whichever way that is from
     // the initial 0 (every row has at least key 0 unmasked there; nothing is accumulated yet).
-    const bool first = it == 0;
+    // kWide: a row whose scores were all -inf so far takes its reference from the first tile that has another.
+    const bool first = !kWide && it == 0;
     if (first || __builtin_amdgcn_ballot_w64(grow) != 0) {
 #pragma unroll
       for (int qb = 0; qb < kQB; ++qb) {
         const float qmax = quad_max(mx[qb]);
-        const float shift = first ? qmax : fmaxf(0.f, qmax);  // afterwards the reference only rises
-        const float alpha = first ? 1.f : __builtin_amdgcn_exp2f(-shift);
+        const bool set = kWide ? unset[qb] : first;
+        float shift = set ? qmax : fmaxf(0.f, qmax);  // afterwards the reference only rises
+        const float alpha = set ? 1.f : __builtin_amdgcn_exp2f(-shift);
+        if constexpr (kWide) {
+          if (set && qmax == -INFINITY) shift = 0.f;
+          unset[qb] = set && qmax == -INFINITY;
+        }
         l_acc[qb] *= alpha;
 #pragma unroll
         for (int db = 0; db < kDB; ++db) o_acc[db][qb] *= alpha;
@@ -651,18 +690,23 @@ template <typename T, int D, int DV, bool kVT, bool kCausal, int kWavesT, int kQ
 int launch_w(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv,
              float scale_log2, hipStream_t st) {
   auto kern = flash_attention_fwd_kernel<T, D, DV, kVT, kCausal, kWavesT, kQB>;
+  constexpr int kBN = key_tile(D);
   constexpr int lds = ring_stages(kWavesT) * (kBN * lds_pitch(D) * 2 + (kVT ? DV * kBN * 2 : kBN * lds_pitch(DV) * 2));
   static_assert(lds <= kMaxLdsBytes, "tiles do not fit in LDS");
   TFK_LDS_OPT_IN(kern, lds);
   constexpr int bm = kWavesT * 16 * kQB;
   const int q_tiles = (Lq + bm - 1) / bm;
-  // causal with an even tile count: one workgroup per PAIR of query tiles (see the kernel)
-  const int total_items = (kCausal && q_tiles % 2 == 0) ? (q_tiles / 2) * batch : q_tiles * batch;
+  // Causal with an even tile count: one workgroup per PAIR of query tiles (see the kernel), unless every
+  // tile can have a CU to itself (a workgroup takes most of a CU's LDS): the heaviest tile alone is then
+  // done before a pair is (bf16, D = 128: 8 slices of 1024 x 1024 29 us against 40, 64 of them 33 against 42,
+  // 32 of 2048 x 2048 52 against 61).
+  const bool paired = kCausal && q_tiles % 2 == 0 && (int64_t)q_tiles * batch > 256;
+  const int total_items = paired ? (q_tiles / 2) * batch : q_tiles * batch;
   const dim3 grid(8 * ((total_items + 7) / 8));
   hipLaunchKernelGGL(kern, grid, dim3(kWavesT * 64), lds, st,
                      static_cast<const T*>(Q), static_cast<const T*>(K),
                      static_cast<const T*>(V), static_cast<T*>(O), Lq, Lkv, scale_log2,
-                     q_tiles, total_items);
+                     q_tiles, total_items, paired ? 1 : 0);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
@@ -672,6 +716,36 @@ int launch(const void* Q, const void* K, const void* V, void* O, int batch, int 
            float scale_log2, hipStream_t st) {
   if (Lq > 128) return launch_w<T, D, DV, kVT, kCausal, 8, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
   return launch_w<T, D, DV, kVT, kCausal, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+}
+
+// Head dimensions above 128 (V as it comes, whole key tiles): 64 or 128 queries a workgroup.  A key tile
+// takes a workgroup of 64 queries 1.4 us (the LDS reads of K and V, which both sizes have in common)
+// and one of 128 queries 1.7 us, one workgroup a CU: the larger one where it saves a round.  bf16, D = 256,
+// 64 / 128 queries: 8 slices of 2048 x 2048 85 / 100 us, 32 of 1024 x 1024 88 / 55, 100 of 384 x 384 56 / 49;
+// causal, 32 of 1024 x 1024 52 / 56 (193 by the kernel compiled at run time, with its transposed copy of V),
+// 64 of them 132 / 87.
+template <typename T, int D>
+int launch_wide(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv, float scale_log2,
+                bool causal, hipStream_t st) {
+  auto rounds = [&](int rows) {
+    const int64_t items = (int64_t)((Lq + rows - 1) / rows) * batch;
+    return causal && items > 256 ? (items + 511) / 512 : (items + 255) / 256;   // (a causal pair counts as one)
+  };
+  const bool wide_tile = 1.3 * rounds(128) < rounds(64);
+  if (causal) {
+    if (wide_tile) return launch_w<T, D, D, false, true, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+    return launch_w<T, D, D, false, true, 4, 1>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+  }
+  if (wide_tile) return launch_w<T, D, D, false, false, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+  return launch_w<T, D, D, false, false, 4, 1>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+}
+
+template <typename T>
+int pick_wide(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv, int D,
+              float scale_log2, bool causal, hipStream_t st) {
+  if (D == 160) return launch_wide<T, 160>(Q, K, V, O, batch, Lq, Lkv, scale_log2, causal, st);
+  if (D == 192) return launch_wide<T, 192>(Q, K, V, O, batch, Lq, Lkv, scale_log2, causal, st);
+  return launch_wide<T, 256>(Q, K, V, O, batch, Lq, Lkv, scale_log2, causal, st);
 }
 
 template <typename T, int D, int DV>
@@ -781,4 +855,26 @@ extern "C" int tf_flash_attention_fwd(const void* Q, const void* K, const void* 
                                 v_is_transposed != 0, causal != 0, st);
   return pick<bf16_t, 64, 64>(Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, scale_log2,
                               v_is_transposed != 0, causal != 0, st);
+}
+
+extern "C" int tf_flash_attention_fwd_wide(const void* Q, const void* K, const void* V, void* O, int dtype,
+                                           int64_t batch, int64_t Lq, int64_t Lkv, int64_t D, double softmax_scale,
+                                           int causal, void* stream) {
+  using namespace tfk;
+  if (int rc = check_attention_args("tf_flash_attention_fwd_wide", Q, K, V, O, batch, Lq, Lkv, D, D, 1, 1, 1, 1,
+                                    softmax_scale))
+    return rc;
+  TFK_REQUIRE(dtype == TF_DTYPE_F16 || dtype == TF_DTYPE_BF16, TF_ERR_UNSUPPORTED,
+              "tf_flash_attention_fwd_wide: dtype must be TF_DTYPE_F16 or TF_DTYPE_BF16");
+  TFK_REQUIRE((D == 160 || D == 192 || D == 256) && Lkv % 32 == 0, TF_ERR_UNSUPPORTED,
+              "tf_flash_attention_fwd_wide: needs a head dimension of 160, 192 or 256 and Lkv %% 32 == 0 "
+              "(got D=%lld Lkv=%lld)", (long long)D, (long long)Lkv);
+  TFK_REQUIRE((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V) |
+               reinterpret_cast<uintptr_t>(O)) % 16 == 0, TF_ERR_UNSUPPORTED,
+              "tf_flash_attention_fwd_wide: operands must start at a 16-byte boundary");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const float scale_log2 = (float)(softmax_scale * 1.4426950408889634);
+  if (dtype == TF_DTYPE_BF16)
+    return pick_wide<bf16_t>(Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, scale_log2, causal != 0, st);
+  return pick_wide<half_t>(Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, scale_log2, causal != 0, st);
 }

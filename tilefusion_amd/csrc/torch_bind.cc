@@ -202,6 +202,17 @@ void attention_impl(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& 
     if (dv != hp) O.copy_(Op.narrow(-1, 0, dv));
     return;
   }
+  // Wide heads with V as it comes: no transposed copy of V, no compilation at the first call.  (Key lengths
+  // and operands that the kernel does not take go on to the general path.)
+  if (!v_transposed && d == dv && (d == 160 || d == 192 || d == 256)) {
+    const int status = tf_flash_attention_fwd_wide(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dtype,
+                                                   batch, lq, lkv, d, softmax_scale, causal ? 1 : 0,
+                                                   current_stream());
+    if (status != TF_ERR_UNSUPPORTED) {
+      check_status(status, op);
+      return;
+    }
+  }
   const int status = tf_flash_attention_fwd(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dtype,
                                             batch, lq, lkv, d, dv, v_transposed ? 1 : 0, (int)tq,
                                             (int)tkv, (int)thqk, (int)thv, softmax_scale,
