@@ -19,6 +19,7 @@
 //     V is kept [key][dim] in LDS and transposed on the way to registers with
 //     ds_read_b64_tr_b16; both tiles are XOR-swizzled against bank conflicts;
 //   * causal: tiles right of the diagonal are skipped, only tiles crossing it are masked.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -159,13 +160,13 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   //   causal:     work per query tile grows with its position, so a workgroup takes query
   //               tile q_tiles-1-p and then tile p of the same slice: every workgroup does the
   //               same amount of work, no sorting by weight is needed and the slice-major
-  //               order (with its L2 locality) is kept.  An odd number of query tiles, or fewer
-  //               tiles than CUs (see launch_w), runs one tile per workgroup, heaviest first
-  //               over all slices.
+  //               order (with its L2 locality) is kept.  Where that is done sooner (see
+  //               pair_query_tiles) and with an odd number of query tiles, one tile per workgroup,
+  //               heaviest first over all slices.
   int qt_of_pass[2] = {0, 0};
   int num_passes = 1;
   size_t bh;
-  if (!kCausal || paired) {
+  if (!kCausal || (D <= 128 && paired)) {
     const int per_slice = kCausal ? q_tiles / 2 : q_tiles;
     const int per_xcd = (total_items + 7) / 8;
     const int item = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
@@ -686,6 +687,23 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   }  // pass
 }
 
+// Causal: one workgroup per PAIR of query tiles (see the kernel), or per tile, heaviest first?  In units of the
+// lightest tile, one workgroup a CU: pairs take q_tiles + 1 a round, and a last round that is nearly empty
+// costs as much as a full one; single tiles take what the heaviest does, or the mean over the CUs and a
+// tenth (a slice's key tiles are then spread over time and leave the L2).  1.04 is what pairs are ahead by at equal
+// counts.  bf16, D = 128, pairs / single tiles: 64 slices of 1024 x 1024 42 / 33 us (no more tiles than
+// CUs: half of the chip had nothing to do), 80 of 1024 44 / 36, 100 of 1500 107 / 80, 33 of 4096 213 / 137,
+// 128 of 1024 48 / 51, 77 of 1500 55 / 60, 128 of 2048 142 / 156.
+// Above a head dimension of 128 single tiles won everywhere (64 of 2048, whole rounds of pairs: 308 / 271; 80 of
+// 1024 169 / 107): a second pass starts with nothing beside it to cover its Q and first key tiles.
+inline bool pair_query_tiles(int64_t q_tiles, int64_t batch) {
+  const int64_t pairs = q_tiles / 2 * batch;
+  if (q_tiles % 2 != 0 || 2 * pairs <= 256) return false;
+  const double paired = (double)((pairs + 255) / 256 * (q_tiles + 1));
+  const double single = std::max((double)q_tiles, 1.1 * (double)pairs * (double)(q_tiles + 1) / 256.0);
+  return paired <= 1.04 * single;
+}
+
 template <typename T, int D, int DV, bool kVT, bool kCausal, int kWavesT, int kQB>
 int launch_w(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv,
              float scale_log2, hipStream_t st) {
@@ -696,11 +714,7 @@ int launch_w(const void* Q, const void* K, const void* V, void* O, int batch, in
   TFK_LDS_OPT_IN(kern, lds);
   constexpr int bm = kWavesT * 16 * kQB;
   const int q_tiles = (Lq + bm - 1) / bm;
-  // Causal with an even tile count: one workgroup per PAIR of query tiles (see the kernel), unless every
-  // tile can have a CU to itself (a workgroup takes most of a CU's LDS): the heaviest tile alone is then
-  // done before a pair is (bf16, D = 128: 8 slices of 1024 x 1024 29 us against 40, 64 of them 33 against 42,
-  // 32 of 2048 x 2048 52 against 61).
-  const bool paired = kCausal && q_tiles % 2 == 0 && (int64_t)q_tiles * batch > 256;
+  const bool paired = kCausal && D <= 128 && pair_query_tiles(q_tiles, batch);
   const int total_items = paired ? (q_tiles / 2) * batch : q_tiles * batch;
   const dim3 grid(8 * ((total_items + 7) / 8));
   hipLaunchKernelGGL(kern, grid, dim3(kWavesT * 64), lds, st,
@@ -722,16 +736,17 @@ int launch(const void* Q, const void* K, const void* V, void* O, int batch, int 
 // takes a workgroup of 64 queries 1.4 us (the LDS reads of K and V, which both sizes have in common)
 // and one of 128 queries 1.7 us, one workgroup a CU: the larger one where it saves a round.  bf16, D = 256,
 // 64 / 128 queries: 8 slices of 2048 x 2048 85 / 100 us, 32 of 1024 x 1024 88 / 55, 100 of 384 x 384 56 / 49;
-// causal, 32 of 1024 x 1024 52 / 56 (193 by the kernel compiled at run time, with its transposed copy of V),
-// 64 of them 132 / 87.
+// causal, 32 of 1024 x 1024 53 / 58 (193 by the kernel compiled at run time, with its transposed copy of V),
+// 40 of them 69 / 58, 64 of them 95 / 72.
 template <typename T, int D>
 int launch_wide(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv, float scale_log2,
                 bool causal, hipStream_t st) {
-  auto rounds = [&](int rows) {
+  auto rounds = [&](int rows) -> double {
     const int64_t items = (int64_t)((Lq + rows - 1) / rows) * batch;
-    return causal && items > 256 ? (items + 511) / 512 : (items + 255) / 256;   // (a causal pair counts as one)
+    if (causal) return std::max(1.0, (double)items / 512.0);   // a tile is half of the heaviest on average
+    return (double)((items + 255) / 256);
   };
-  const bool wide_tile = 1.3 * rounds(128) < rounds(64);
+  const bool wide_tile = 1.1 * rounds(128) < rounds(64);
   if (causal) {
     if (wide_tile) return launch_w<T, D, D, false, true, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
     return launch_w<T, D, D, false, true, 4, 1>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
