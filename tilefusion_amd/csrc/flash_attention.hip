@@ -368,17 +368,24 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   // Operand fragments are requested from LDS one step ahead of the MFMAs that use them, into
   // ping-pong registers, so that LDS latency is covered by the previous step's MFMAs (or by
   // the softmax arithmetic) instead of stalling the wavefront in front of every MFMA group.
-  V8 kf[2][kKB];   // K fragments of reduction step kk (buffer kk & 1)
+  // kWide: one wavefront a SIMD and few MFMAs a step, so K fragments are requested two steps ahead, and the V
+  // fragments during the QK product, behind whose MFMAs they arrive (causal, D = 256: 32 slices of 1024 x 1024
+  // 52.5 -> 47.0 us, 8 of 4096 173 -> 157, 50 of 2048 215 -> 206; D = 160: 46.2 -> 44.8).
+  constexpr int kKAhead = kWide ? 2 : 1;
+  V8 kf[kKAhead + 1][kKB];   // K fragments of reduction step kk (buffer kk % (kKAhead + 1))
   V8 vf[2][kDB];   // V fragments of reduction step j (buffer j & 1)
   auto k_reads = [&](int buf, int it, int kk) __attribute__((always_inline)) {
     const unsigned ka = opaque(smem_base + (it % kStages) * kStageBytes + k_off[kk]);
 #pragma unroll
     for (int kb = 0; kb < kKB; ++kb) kf[buf][kb] = lds_read_b128<V8>(ka + kb * 16 * DP * 2);
   };
-  auto v_reads = [&](int buf, int it, int j) __attribute__((always_inline)) {
-    const unsigned stage_base = smem_base + (it % kStages) * kStageBytes;
+  auto first_k_reads = [&](int it) __attribute__((always_inline)) {
 #pragma unroll
-    for (int db = 0; db < kDB; ++db) {
+    for (int kk = 0; kk < kKAhead; ++kk) k_reads(kk, it, kk);
+  };
+  auto v_read = [&](int buf, int it, int j, int db) __attribute__((always_inline)) {
+    const unsigned stage_base = smem_base + (it % kStages) * kStageBytes;
+    {
       V4 lo, hi;
       if constexpr (!kVT) {
         const unsigned va = opaque(stage_base + v_off[db]) + kKBytes;
@@ -394,6 +401,10 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
         vf[buf][db][4 + t] = hi[t];
       }
     }
+  };
+  auto v_reads = [&](int buf, int it, int j) __attribute__((always_inline)) {
+#pragma unroll
+    for (int db = 0; db < kDB; ++db) v_read(buf, it, j, db);
   };
   // ---- S^T = K Q'^T - m: s[kb][qb][r] = log2-scaled score of key 64*it + 16*kb + 4*lg + r
   //      against row lr of query block qb, minus that row's reference maximum.  Expects the
@@ -414,13 +425,19 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
       }
 #pragma unroll
     for (int kk = 0; kk < kKK; ++kk) {
-      const unsigned ka = kk + 1 < kKK ? opaque(smem_base + (it % kStages) * kStageBytes + k_off[kk + 1]) : 0u;
+      const int next = kk + kKAhead;
+      const unsigned ka = next < kKK ? opaque(smem_base + (it % kStages) * kStageBytes + k_off[next < kKK ? next : 0]) : 0u;
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int kb = 0; kb < kKB; ++kb) {
 #pragma unroll
-        for (int qb = 0; qb < kQB; ++qb) s[kb][qb] = mfma_t<T>(kf[kk & 1][kb], qf[kk][qb], s[kb][qb]);
-        if (kk + 1 < kKK) kf[(kk + 1) & 1][kb] = lds_read_b128<V8>(ka + kb * 16 * DP * 2);
+        for (int qb = 0; qb < kQB; ++qb) s[kb][qb] = mfma_t<T>(kf[kk % (kKAhead + 1)][kb], qf[kk][qb], s[kb][qb]);
+        if (next < kKK) kf[next % (kKAhead + 1)][kb] = lds_read_b128<V8>(ka + kb * 16 * DP * 2);
+        if constexpr (kWide) {
+#pragma unroll
+          for (int db = 0; db < kDB; ++db)
+            if ((db * kKK * kKB) / kDB == kk * kKB + kb) v_read(0, it, 0, db);
+        }
         if (req_tile >= 0) {
 #pragma unroll
           for (int r = 0; r < kLoadsPerTile; ++r)
@@ -434,11 +451,11 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     }
   };
   V8 pb[kJ][kQB];  // 16-bit weights, B operand of the second product
-  // ---- mask, online softmax, fp16 weights.  Requests the V fragments of step j = 0. -------
+  // ---- mask, online softmax, fp16 weights.  Requests the V fragments of step j = 0 (unless kWide). -------
   auto softmax_tile = [&](int it, auto mask_c) __attribute__((always_inline)) {
     constexpr bool kMask = decltype(mask_c)::value;
     const int n0 = it * kBN;
-    v_reads(0, it, 0);
+    if constexpr (!kWide) v_reads(0, it, 0);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (kWide) {
 #pragma unroll
@@ -529,7 +546,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
 #pragma unroll
     for (int j = 0; j < kJ; ++j) {
       if (j + 1 < kJ) v_reads((j + 1) & 1, it, j + 1);
-      else k_reads(0, it_next, 0);
+      else first_k_reads(it_next);
 #pragma unroll
       for (int db = 0; db < kDB; ++db)
 #pragma unroll
@@ -573,7 +590,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     barrier_keep_vmem<2 * kLoadsPerTile>();  // tile 0 has landed
     const bool second_set = wave >= 4;
     if (second_set) barrier_only();  // slot 0: set 0 alone
-    k_reads(0, 0, 0);
+    first_k_reads(0);
     if (n_compute > 0) qk_tile(0, 3, std::false_type{});
     else issue_tile_loads(3);
     auto tile_step = [&](int t, auto mask_c, auto lean_c) __attribute__((always_inline)) {
@@ -613,7 +630,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     };
     const int n_lean = min(n_plain, n_fast - (kStages - 1));
     int it = 0;
-    k_reads(0, 0, 0);
+    first_k_reads(0);
     for (; it < n_lean; ++it) {
       ring_barrier();
       qk_tile(it, it + kStages - 1, std::true_type{});
@@ -733,11 +750,11 @@ int launch(const void* Q, const void* K, const void* V, void* O, int batch, int 
 }
 
 // Head dimensions above 128 (V as it comes, whole key tiles): 64 or 128 queries a workgroup.  A key tile
-// takes a workgroup of 64 queries 1.4 us (the LDS reads of K and V, which both sizes have in common)
-// and one of 128 queries 1.7 us, one workgroup a CU: the larger one where it saves a round.  bf16, D = 256,
+// takes a workgroup of 64 queries 1.3 us (0.74 with few workgroups: its 32 KiB then come sooner from the L2)
+// and one of 128 queries 1.6 us, one workgroup a CU: the larger one where it saves a round.  bf16, D = 256,
 // 64 / 128 queries: 8 slices of 2048 x 2048 85 / 100 us, 32 of 1024 x 1024 88 / 55, 100 of 384 x 384 56 / 49;
-// causal, 32 of 1024 x 1024 53 / 58 (193 by the kernel compiled at run time, with its transposed copy of V),
-// 40 of them 69 / 58, 64 of them 95 / 72.
+// causal, 32 of 1024 x 1024 47 / 55 (193 by the kernel compiled at run time, with its transposed copy of V),
+// 40 of them 63 / 55, 64 of them 91 / 71.
 template <typename T, int D>
 int launch_wide(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv, float scale_log2,
                 bool causal, hipStream_t st) {
