@@ -72,6 +72,20 @@ def test_causal_pass_orders(lq, d):
     assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
 
 
+# Whole rounds of pairs (256 and 512 of them), a ragged last query tile, and a nearly empty last round that
+# runs single tiles instead: every slice against the same slice alone, which is never paired (bit for bit).
+@pytest.mark.parametrize("bh,lq", [(256, 512), (256, 500), (512, 300), (264, 512)])
+@pytest.mark.parametrize("d", [64, 128])
+def test_causal_pairs_and_single_tiles_agree(bh, lq, d):
+    q, k, v = (x.to(DEV) for x in _inputs(bh, lq, lq, d, bh + lq + d))
+    o = c_attention(q, k, v, True)
+    for i in (0, 1, 7, 8, bh // 2, bh - 1):
+        alone = c_attention(q[i:i + 1].contiguous(), k[i:i + 1].contiguous(), v[i:i + 1].contiguous(), True)
+        assert torch.equal(o[i:i + 1], alone), i
+    ok, r, m = N.check_close(o[-1:].cpu(), N.attention_ref(q[-1:].cpu(), k[-1:].cpu(), v[-1:].cpu(), causal=True))
+    assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
+
+
 def test_scale_and_large_logits():
     # scale enters the logits; big logits need the running max (exp would overflow otherwise)
     q, k, v = _inputs(2, 128, 256, 128, 77)

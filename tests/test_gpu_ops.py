@@ -184,7 +184,7 @@ def test_flash_attention_ops_shrink_tiles_that_do_not_fit_the_lds(d, dv, lq, lkv
 
 
 # Both workgroup sizes (64 queries; 128 where that saves a round of the 256 CUs), one key tile, fewer than
-# the ring holds and more, rows that no tile divides, the paired and the one-tile causal orders.
+# the ring holds and more, rows that no tile divides, causal tiles heaviest first.
 # Bounds: four times what the kernel shows against 64-bit sums (2.8e-4 fp16, 2.3e-3 bf16: the 16-bit weights
 # and result).
 @pytest.mark.parametrize("dtype,tol", [(torch.float16, 1.2e-3), (torch.bfloat16, 1e-2)])
