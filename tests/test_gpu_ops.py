@@ -204,6 +204,48 @@ def test_flash_attention_wide_heads(bh, lq, lkv, causal, d, dtype, tol):
     assert ((o.float() - ref).norm() / ref.norm()).item() < tol
 
 
+@pytest.mark.parametrize("dtype,half_ulp", [(torch.float16, 2.0 ** -11), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("d", [160, 192, 256])
+@pytest.mark.parametrize("bh", [1, 300])
+def test_flash_attention_wide_heads_round_no_error_into_the_largest_weight(bh, d, dtype, half_ulp):
+    # Two keys count: one in the first key tile, and far behind it one whose weight is 1.5 + half_ulp times
+    # as large, halfway between two 16-bit numbers.  Relative to the row's largest score the second weight
+    # is 1 and the first one is never rounded in 16 bits other than as 1: what is left is the fp32 arithmetic,
+    # which the values -1.5 and 1 let show as half_ulp / 2.5.  A weight of 1.5 + half_ulp kept against the
+    # first score would be rounded to 1.5 or 1.5 + 2 half_ulp and give 0 or twice that.
+    import tilefusion_amd.ops  # noqa: F401
+    lq, lkv, far = 70, 512, 400
+    q = torch.zeros(bh, lq, d); q[..., :3] = 1.0
+    k = torch.zeros(bh, lkv, d); k[..., 0] = -60.0
+    k[:, 3, 0] = 0.0
+    score = torch.tensor(math.log(1.5 + half_ulp), dtype=torch.float64)
+    for i in range(3):                                   # as a sum of three 16-bit numbers
+        k[:, far, i] = score.to(dtype)
+        score -= k[0, far, i].double()
+    v = torch.zeros(bh, lkv, d); v[:, 3] = -1.5; v[:, far] = 1.0
+    o = torch.full((bh, lq, d), float("nan"), dtype=dtype, device=DEV)
+    torch.ops.tilefusion.flash_attention_fwd(*(x.to(dtype).to(DEV) for x in (q, k, v)), o, 1.0, False)
+    want = half_ulp / (2.5 + half_ulp)
+    # exp2, the score and the sums in fp32: a few 2^-23 of the two terms of 1.5 / 2.5; the result's own rounding
+    assert (o.double() - want).abs().max().item() <= 16 * 2.0 ** -23 + half_ulp * want
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [160, 192, 256])
+def test_flash_attention_wide_heads_pass_infinite_values_on(d, dtype):
+    # every weight is positive (key 90's is exact in 16 bits), so an infinite value makes its column that infinity
+    import tilefusion_amd.ops  # noqa: F401
+    g = torch.Generator().manual_seed(d)
+    q, k, v = (torch.randn(3, n, d, generator=g).to(dtype) for n in (130, 160, 160))
+    k[:, 90] = 0.0
+    v[:, 5, 1], v[:, 90, 2], v[:, 150, d - 1] = math.inf, -math.inf, math.inf
+    o = torch.full((3, 130, d), float("nan"), dtype=dtype, device=DEV)
+    torch.ops.tilefusion.flash_attention_fwd(q.to(DEV), k.to(DEV), v.to(DEV), o, 0.1, False)
+    ref = torch.softmax(q.float() @ k.float().transpose(1, 2) * 0.1, -1) @ v.float()
+    assert torch.equal(o.isinf().cpu(), ref.isinf()) and not o.isnan().any()
+    assert (o[..., 1] > 0).all() and (o[..., 2] < 0).all() and (o[..., d - 1] > 0).all()
+
+
 def test_flash_attention_wide_heads_keep_rows_whose_first_scores_are_minus_infinity():
     # the first two key tiles score -inf: their weights are zero and the row's reference comes from the third
     g = torch.Generator().manual_seed(5)

@@ -109,6 +109,30 @@ TFK_DEVICE float quad_max(float x) {
   return fmaxf(x, __shfl_xor(x, 32));
 }
 
+// A weight p >= 0 as a 16-bit number cut off behind its last bit and a 16-bit remainder.  The remainder of a
+// weight that the 16-bit number holds exactly is the smallest number instead of zero, so that
+// both have the weight's sign and an infinite value stays that infinity (zero or a negative remainder
+// would make it NaN).
+template <typename T>
+struct SplitWeight {
+  T whole, rest;
+};
+template <typename T>
+TFK_DEVICE SplitWeight<T> split_weight(float p) {
+  SplitWeight<T> w;
+  float smallest;
+  if constexpr (std::is_same_v<T, bf16_t>) {
+    w.whole = __builtin_bit_cast(T, (unsigned short)(__builtin_bit_cast(unsigned, p) >> 16));
+    smallest = 0x1p-126f;
+  } else {
+    w.whole = __builtin_bit_cast(T, (unsigned short)__builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(p, 0.f)));
+    smallest = 0x1p-24f;
+  }
+  // p where p is below `smallest` (0 for 0), else the remainder, `smallest` at least
+  w.rest = (T)__builtin_amdgcn_fmed3f(p, p - (float)w.whole, smallest);
+  return w;
+}
+
 // kWavesT wavefronts x 32 queries per workgroup.  8 wavefronts (256 queries) halve the
 // K/V traffic per query and put two wavefronts on every SIMD, so one wavefront's softmax
 // (VALU) overlaps the other's MFMAs; 4 wavefronts serve short query ranges and, with 32 or 16
@@ -116,8 +140,15 @@ TFK_DEVICE float quad_max(float x) {
 //
 // Above 128 (kWide) the output accumulators and Q fragments of 32 queries take 192 registers, which two
 // wavefronts on a SIMD do not have.  What bounds these instances: the four wavefronts read the whole
-// K and V tile for 32 queries each, 128 KiB of LDS reads a key tile for 64 MFMAs on each SIMD (1024 cycles of
-// either), and one wavefront per SIMD puts the softmax behind them instead of beside them.
+// K and V tile each, 128 KiB of LDS reads a key tile (1024 cycles) for 100 MFMAs (1600 cycles) on each SIMD with 32
+// queries a wavefront and 50 (800) with 16, and one wavefront per SIMD puts the softmax behind them
+// instead of beside them.
+// The weights enter the second product as a 16-bit number and a 16-bit remainder (pb_rest): rounded to 16
+// bits once, against a reference that is raised lazily, they made the result 5% worse (relative error of
+// 4 slices of 1024 x 1024 x 256, bf16, against 64 bits: 2.33e-3, against the true running maximum, whose
+// weight of 1 has no error, 2.22e-3, with the remainder 1.66e-3).  Raising the reference to every larger
+// score instead, which gives 2.22e-3, multiplies all accumulators in most tiles and is slower: causal, 32 slices
+// of 1024 x 1024 x 256: 45 us without either, 51 with the remainder, 57 with the true maximum.
 // The scale is applied to the fp32 scores there: Q stays as it came, a second rounding of Q
 // would make a 16-bit result measurably worse.
 template <typename T, int D, int DV, bool kVT, bool kCausal, int kWavesT, int kQB>
@@ -369,8 +400,8 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   // ping-pong registers, so that LDS latency is covered by the previous step's MFMAs (or by
   // the softmax arithmetic) instead of stalling the wavefront in front of every MFMA group.
   // kWide: one wavefront a SIMD and few MFMAs a step, so K fragments are requested two steps ahead, and the V
-  // fragments during the QK product, behind whose MFMAs they arrive (causal, D = 256: 32 slices of 1024 x 1024
-  // 52.5 -> 47.0 us, 8 of 4096 173 -> 157, 50 of 2048 215 -> 206; D = 160: 46.2 -> 44.8).
+  // fragments during the QK product, behind whose MFMAs they arrive (causal, D = 256, before the
+  // weights had a remainder: 32 slices of 1024 x 1024 52.5 -> 47.0 us, 8 of 4096 173 -> 157; D = 160: 46.2 -> 44.8).
   constexpr int kKAhead = kWide ? 2 : 1;
   V8 kf[kKAhead + 1][kKB];   // K fragments of reduction step kk (buffer kk % (kKAhead + 1))
   V8 vf[2][kDB];   // V fragments of reduction step j (buffer j & 1)
@@ -406,7 +437,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
 #pragma unroll
     for (int db = 0; db < kDB; ++db) v_read(buf, it, j, db);
   };
-  // ---- S^T = K Q'^T - m: s[kb][qb][r] = log2-scaled score of key 64*it + 16*kb + 4*lg + r
+  // ---- S^T = K Q'^T - m: s[kb][qb][r] = log2-scaled score of key kBN*it + 16*kb + 4*lg + r
   //      against row lr of query block qb, minus that row's reference maximum.  Expects the
   //      fragments of step kk = 0 to be on their way into kf[0]. ---------------------------
   //      req_tile >= 0: that tile's requests are issued between the reduction steps.
@@ -451,6 +482,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     }
   };
   V8 pb[kJ][kQB];  // 16-bit weights, B operand of the second product
+  V8 pb_rest[kJ][kQB];   // kWide: what their rounding left out, rounded in turn
   // ---- mask, online softmax, fp16 weights.  Requests the V fragments of step j = 0 (unless kWide). -------
   auto softmax_tile = [&](int it, auto mask_c) __attribute__((always_inline)) {
     constexpr bool kMask = decltype(mask_c)::value;
@@ -485,7 +517,10 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     // reference.  The check needs no cross-lane traffic: it looks at each lane's own 16 keys;
     // only when it fires are the 4 lanes that share a query reduced, every O accumulator
     // multiplied and this tile's scores re-based.
-    constexpr float kLazy = 8.f;
+    // kWide, fp16: weights are taken 2^7 times as large (up to 2^15), which leaves the smallest remainder
+    // at 2^-31 of the largest weight.
+    constexpr float kUp = kWide && !std::is_same_v<T, bf16_t> ? 7.f : 0.f;
+    constexpr float kLazy = kUp + 8.f;
     float mx[kQB];
     bool grow = false;
 #pragma unroll
@@ -505,7 +540,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     if (first || __builtin_amdgcn_ballot_w64(grow) != 0) {
 #pragma unroll
       for (int qb = 0; qb < kQB; ++qb) {
-        const float qmax = quad_max(mx[qb]);
+        const float qmax = quad_max(mx[qb]) - kUp;
         const bool set = kWide ? unset[qb] : first;
         float shift = set ? qmax : fmaxf(0.f, qmax);  // afterwards the reference only rises
         const float alpha = set ? 1.f : __builtin_amdgcn_exp2f(-shift);
@@ -534,8 +569,16 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
       for (int qb = 0; qb < kQB; ++qb) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          pb[j][qb][t] = (T)s[2 * j][qb][t];
-          pb[j][qb][4 + t] = (T)s[2 * j + 1][qb][t];
+          if constexpr (kWide) {
+            const SplitWeight<T> lo = split_weight<T>(s[2 * j][qb][t]), hi = split_weight<T>(s[2 * j + 1][qb][t]);
+            pb[j][qb][t] = lo.whole;
+            pb_rest[j][qb][t] = lo.rest;
+            pb[j][qb][4 + t] = hi.whole;
+            pb_rest[j][qb][4 + t] = hi.rest;
+          } else {
+            pb[j][qb][t] = (T)s[2 * j][qb][t];
+            pb[j][qb][4 + t] = (T)s[2 * j + 1][qb][t];
+          }
         }
       }
     __builtin_amdgcn_sched_barrier(0);
@@ -553,6 +596,14 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
         for (int qb = 0; qb < kQB; ++qb) o_acc[db][qb] = mfma_t<T>(vf[j & 1][db], pb[j][qb], o_acc[db][qb]);
 #pragma unroll
       for (int qb = 0; qb < kQB; ++qb) l_acc[qb] = mfma_t<T>(ones_frag, pb[j][qb], l_acc[qb]);
+      if constexpr (kWide) {
+#pragma unroll
+        for (int db = 0; db < kDB; ++db)
+#pragma unroll
+          for (int qb = 0; qb < kQB; ++qb) o_acc[db][qb] = mfma_t<T>(vf[j & 1][db], pb_rest[j][qb], o_acc[db][qb]);
+#pragma unroll
+        for (int qb = 0; qb < kQB; ++qb) l_acc[qb] = mfma_t<T>(ones_frag, pb_rest[j][qb], l_acc[qb]);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -749,12 +800,10 @@ int launch(const void* Q, const void* K, const void* V, void* O, int batch, int 
   return launch_w<T, D, DV, kVT, kCausal, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
 }
 
-// Head dimensions above 128 (V as it comes, whole key tiles): 64 or 128 queries a workgroup.  A key tile
-// takes a workgroup of 64 queries 1.3 us (0.74 with few workgroups: its 32 KiB then come sooner from the L2)
-// and one of 128 queries 1.6 us, one workgroup a CU: the larger one where it saves a round.  bf16, D = 256,
-// 64 / 128 queries: 8 slices of 2048 x 2048 85 / 100 us, 32 of 1024 x 1024 88 / 55, 100 of 384 x 384 56 / 49;
-// causal, 32 of 1024 x 1024 47 / 55 (193 by the kernel compiled at run time, with its transposed copy of V),
-// 40 of them 63 / 55, 64 of them 91 / 71.
+// Head dimensions above 128 (V as it comes, whole key tiles): 64 or 128 queries a workgroup, the larger one
+// where it saves a round of the CUs.  bf16, D = 256, 64 / 128 queries: 8 slices of 2048 x 2048 69 / 95 us, 32 of
+// 1024 x 1024 89 / 64, 100 of 384 x 384 58 / 56; causal, 32 of 1024 x 1024 49 / 64 (193 by the kernel compiled
+// at run time, with its transposed copy of V), 40 of them 67 / 63, 64 of them 100 / 81.
 template <typename T, int D>
 int launch_wide(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv, float scale_log2,
                 bool causal, hipStream_t st) {
