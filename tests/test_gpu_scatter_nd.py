@@ -75,3 +75,43 @@ def test_scatter_nd_fp16_sum_of_duplicates_beyond_its_range():
     upd = torch.full((2, 2), 60000.0, dtype=torch.float16, device=DEV)
     scatter_nd(data, torch.tensor([[1], [1]], device=DEV), upd)
     assert data[1].tolist() == [60000.0, 60000.0] and data[0].tolist() == [-60000.0, -60000.0]
+
+
+# Of a word of two 16-bit elements a slice may hold one: the other one, of a neighbouring row, keeps its value
+# (the smallest subnormal number here), and memory outside the tensor its bits, also those of a signalling NaN.
+@pytest.mark.parametrize("dtype,bits", [(torch.float16, 0x7D01), (torch.bfloat16, 0x7F81), (torch.float32, 0x7F800001)],
+                         ids=["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("start", [0, 1, 2, 3])
+@pytest.mark.parametrize("slice_", [1, 3, 66, 131])
+@pytest.mark.parametrize("n", [2, 1500])
+@pytest.mark.parametrize("first,second", [(0, 4), (1, 3)])
+def test_scatter_nd_leaves_what_lies_next_to_a_slice_alone(dtype, bits, start, slice_, n, first, second):
+    from tilefusion_amd.ops import scatter_nd
+    ints = torch.int32 if dtype == torch.float32 else torch.int16
+    buf = torch.full((start + 5 * slice_ + 3,), bits, dtype=ints, device=DEV)
+    inside = buf[start:start + 5 * slice_]
+    inside.fill_(1)
+    data = inside.view(dtype).view(5, slice_)
+    data[first], data[second] = 1.0, 2.0
+    want = buf.clone()
+    rows = want.view(dtype)[start:start + 5 * slice_].view(5, slice_)
+    rows[first], rows[second] = 4.0, 6.0
+    upd = torch.zeros(n, slice_, dtype=dtype, device=DEV)
+    upd[0], upd[1] = 3.0, 4.0
+    scatter_nd(data, (torch.arange(n, device=DEV) % 2 * (second - first) + first).unsqueeze(1), upd)
+    assert torch.equal(buf, want)
+
+
+@pytest.mark.parametrize("dtype,tiny", [(torch.float16, 2.0 ** -24), (torch.bfloat16, 2.0 ** -133), (torch.float32, 2.0 ** -149)],
+                         ids=["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("slice_", [8, 7])
+@pytest.mark.parametrize("n", [3, 1500, 3000])
+def test_scatter_nd_adds_subnormal_numbers_exactly(dtype, tiny, slice_, n):
+    from tilefusion_amd.ops import scatter_nd
+    data = ((torch.arange(64 * slice_) % 7).double() * tiny).to(dtype).view(64, slice_)
+    idx = torch.arange(n) % 64
+    upd = ((torch.arange(n * slice_) % 5 - 2).double() * tiny).to(dtype).view(n, slice_)
+    want = data.double().index_add(0, idx, upd.double())
+    dev = data.to(DEV)
+    scatter_nd(dev, idx.unsqueeze(1).to(DEV), upd.to(DEV))
+    assert torch.equal(dev.double().cpu(), want)

@@ -38,8 +38,24 @@ struct Word {
   float v[kElems];
 };
 
+// Adds to one element by compare-and-swap on the aligned word that holds it; the other half of
+// the word keeps its bits.
+template <typename T>
+TFK_DEVICE void atomic_add_element(T* p, float v) {
+  const size_t at = reinterpret_cast<size_t>(p);
+  unsigned* const word = reinterpret_cast<unsigned*>(at & ~size_t(3));
+  const int shift = at & 2 ? 16 : 0;
+  unsigned old = *word, seen;
+  do {
+    seen = old;
+    const float sum = (float)__builtin_bit_cast(T, (unsigned short)(seen >> shift)) + (float)(T)v;
+    const unsigned half = __builtin_bit_cast(unsigned short, (T)sum);
+    old = atomicCAS(word, seen, (seen & ~(0xffffu << shift)) | (half << shift));
+  } while (old != seen);
+}
+
 // Adds `w` to the aligned word at `p` with one hardware atomic.  A 16-bit half that has nothing to
-// add passes -0.0, which changes no value.
+// add passes -0.0, which changes no number; a NaN stays one, but loses its signalling bit.
 template <typename T>
 TFK_DEVICE void atomic_add_word(T* p, const Word<T>& w) {
   if constexpr (sizeof(T) == 4) {
@@ -74,6 +90,22 @@ TFK_DEVICE void add_word_of_slice(Word<T>& sum, const T* src, long long e0, long
       if (e0 + e >= 0 && e0 + e < slice) sum.v[e] += (float)src[e0 + e];
   }
 }
+// Adds word `w` at elements e0 .. of the slice at `dst`.  Of a word that the slice shares with memory outside the `total`
+// elements of `data` the other half keeps its bits, whatever they stand for: compare-and-swap.  Only the first
+// and the last word of `data` can be such; for every word that two slices share it would cost far too
+// much (2048 bf16 updates of 33 into 64 rows 8 us and 40, 30000 of 77 into 131072 rows 25 and 1260).
+template <typename T, bool kSplitPairs>
+TFK_DEVICE void add_to_slice(T* dst, const Word<T>& w, long long e0, long long slice, const T* data, long long total) {
+  T* const word = dst + e0;
+  if constexpr (kSplitPairs) {
+    const int outside = word < data ? 0 : word + 1 >= data + total ? 1 : -1;   // element of the word that is not data's
+    if (outside >= 0) {
+      atomic_add_element(word + (1 - outside), outside ? w.v[0] : w.v[1]);
+      return;
+    }
+  }
+  atomic_add_word(word, w);
+}
 // with kSplitPairs a slice may start in the upper half of its first word
 template <typename T, bool kSplitPairs>
 TFK_DEVICE int first_word_shift(const T* dst) {
@@ -85,7 +117,7 @@ TFK_DEVICE int first_word_shift(const T* dst) {
 template <typename T, bool kSplitPairs>
 __global__ __launch_bounds__(kScatterThreads) void scatter_nd_direct_kernel(
     const T* __restrict__ updates, T* __restrict__ data, const long long* __restrict__ indices, Strides s, long long n,
-    int k, long long slice, int lanes) {
+    int k, long long slice, long long total, int lanes) {
   constexpr int kElems = Word<T>::kElems;
   const int lane = threadIdx.x & (lanes - 1);
   const long long row = blockIdx.x * (long long)(kScatterThreads / lanes) + threadIdx.x / lanes;
@@ -106,7 +138,7 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_nd_direct_kernel(
 #pragma unroll
     for (int e = 0; e < kElems; ++e) w.v[e] = -0.f;
     add_word_of_slice<T, kSplitPairs>(w, updates + row * slice, e0, slice);
-    atomic_add_word(dst + e0, w);
+    add_to_slice<T, kSplitPairs>(dst, w, e0, slice, data, total);
   }
 }
 
@@ -116,7 +148,7 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_nd_direct_kernel(
 template <typename T, int kThreads, int kRows, int kWords, bool kSplitPairs>
 __global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
     const T* __restrict__ updates, T* __restrict__ data, const long long* __restrict__ indices, Strides s, long long n,
-    int k, long long slice, int lanes) {
+    int k, long long slice, long long total, int lanes) {
   static_assert((kRows % kWaveSize == 0 || kRows < kWaveSize) && kRows <= kThreads,
                 "part of one wavefront or whole wavefronts sort the workgroup's rows");
   constexpr int kElems = Word<T>::kElems;
@@ -213,10 +245,10 @@ __global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
                 part.v[e] = beyond(sum[v].v[e]) ? __builtin_copysignf(kMax, sum[v].v[e]) : -0.f;
                 sum[v].v[e] -= part.v[e];
               }
-              atomic_add_word(dst + e0, part);
+              add_to_slice<T, kSplitPairs>(dst, part, e0, slice, data, total);
             }
           }
-          atomic_add_word(dst + e0, sum[v]);
+          add_to_slice<T, kSplitPairs>(dst, sum[v], e0, slice, data, total);
         }
       }
     }
@@ -226,23 +258,23 @@ __global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
 
 template <typename T, int kThreads, int kRows, int kWords, bool kSplitPairs>
 int launch_shape(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
-                 long long slice, int lanes, long long words, hipStream_t st) {
+                 long long slice, long long total, int lanes, long long words, hipStream_t st) {
   const long long per = (long long)lanes * kWords;
   const dim3 grid((unsigned)std::min<long long>((n + kRows - 1) / kRows, 1 << 20),
                   (unsigned)std::min<long long>((words + per - 1) / per, 1024));
   hipLaunchKernelGGL((scatter_nd_kernel<T, kThreads, kRows, kWords, kSplitPairs>), grid, dim3(kThreads), 0, st,
-                     static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, lanes);
+                     static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
 
 template <typename T, bool kSplitPairs>
 int launch_direct(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
-                  long long slice, int lanes, long long words, hipStream_t st) {
+                  long long slice, long long total, int lanes, long long words, hipStream_t st) {
   const int per = kScatterThreads / lanes;
   const dim3 grid((unsigned)((n + per - 1) / per), (unsigned)std::min<long long>((words + lanes - 1) / lanes, 1024));
   hipLaunchKernelGGL((scatter_nd_direct_kernel<T, kSplitPairs>), grid, dim3(kScatterThreads), 0, st,
-                     static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, lanes);
+                     static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
@@ -254,18 +286,18 @@ int launch_rows(const void* updates, void* data, const long long* indices, const
   // 34 fp32: direct 3.3, 256/16 5.6).  From 1024 on contention shows (2048 of 64 bf16 into 64 rows:
   // direct 10.8, 256/16 6.3, 512/64 8.2), beyond 2048 more updates per sort pay (4096 of 1024 bf16
   // into 1000 rows: direct 26, 256/16 17.6, 512/64 12.9).
-  if (n <= 1024) return launch_direct<T, kSplitPairs>(updates, data, indices, s, n, k, slice, lanes, words, st);
+  if (n <= 1024) return launch_direct<T, kSplitPairs>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   if (n <= 2048)
-    return launch_shape<T, 256, 16, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, lanes, words, st);
+    return launch_shape<T, 256, 16, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   // Every target hit at least eight times on average: the deeper sort (59764 of 21 fp32 into 219 rows:
   // 512/64 43, 1024/128 31; 49954 of 622 fp32 into 77: 175 and 143).
   if (n / 8 >= targets)
-    return launch_shape<T, 1024, 128, 2, kSplitPairs>(updates, data, indices, s, n, k, slice, lanes, words, st);
+    return launch_shape<T, 1024, 128, 2, kSplitPairs>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   // A workgroup of eight wavefronts hides its own latencies where there are few of them (16384 of 64
   // bf16: 256/64 13.8, 512/64 12.5); enough of four do it better (8192 of 1024 fp32: 31.9 and 40.1).
   if ((n / 64) * ((words + lanes - 1) / lanes) < 1024)
-    return launch_shape<T, 512, 64, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, lanes, words, st);
-  return launch_shape<T, 256, 64, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, lanes, words, st);
+    return launch_shape<T, 512, 64, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+  return launch_shape<T, 256, 64, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
 }
 
 template <typename T>
