@@ -172,7 +172,10 @@ TF_API int tf_flash_decode_static_f16(const void* Q, const void* K, const void* 
  * `rank` dimensions data_dims (host array, row-major, contiguous); indices is a device
  * [num_index_rows, index_depth] int64 array; updates is [num_index_rows, prod(data_dims[
  * index_depth..])].  dtype: 0 fp32, 1 fp16, 2 bf16.  Nothing is allocated (the reference
- * cudaMallocs the strides on every call and leaks them).
+ * cudaMallocs the strides on every call and leaks them).  `data` in ordinary memory of the
+ * current device takes hardware floating-point atomics; elsewhere (host, managed, fine-grained or
+ * another device's memory, as hipPointerGetAttributes reports it), where those may lose updates,
+ * every element is added by compare-and-swap, which is many times slower where rows repeat.
  * Replaces: tilefusion::kernels::scatter_nd, src/kernels/scatter_nd.cu:36-95
  * (schema include/kernels/kernel_list.hpp:11-13). */
 TF_API int tf_scatter_nd(const void* updates, void* data, const int64_t* indices,

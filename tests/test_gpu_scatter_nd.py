@@ -115,3 +115,59 @@ def test_scatter_nd_adds_subnormal_numbers_exactly(dtype, tiny, slice_, n):
     dev = data.to(DEV)
     scatter_nd(dev, idx.unsqueeze(1).to(DEV), upd.to(DEV))
     assert torch.equal(dev.double().cpu(), want)
+
+
+# Hardware floating-point atomics are defined for a device's ordinary memory only.  Elsewhere every element
+# is added by compare-and-swap, which shows in the rows next to an odd slice: a signalling NaN keeps its bits.
+@pytest.mark.parametrize("dtype,bits", [(torch.float16, 0x7D01), (torch.bfloat16, 0x7F81), (torch.float32, 0x7F800001)],
+                         ids=["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("slice_,n", [(5, 3), (64, 3000), (77, 5000)])
+def test_scatter_nd_into_fine_grained_memory_adds_by_compare_and_swap(dtype, bits, slice_, n):
+    import ctypes
+
+    from tilefusion_amd import _capi
+    hip = ctypes.CDLL("libamdhip64.so")
+    rows, size = 9, torch.empty(0, dtype=dtype).element_size()
+    ints = torch.int32 if size == 4 else torch.int16
+    g = torch.Generator().manual_seed(n)
+    host = torch.randint(-2, 3, (rows, slice_), generator=g).to(dtype)
+    idx = torch.randint(0, rows, (n, 1), generator=g)
+    idx[idx == 4] = 3                                             # row 4 is not hit
+    host[4].view(ints).fill_(bits)
+    upd = torch.randint(-1, 2, (n, slice_), generator=g).to(dtype)
+    for i in range(rows):                                         # sums of hundreds of them stay exact: 0 for most
+        upd[(idx[:, 0] == i).nonzero()[32:, 0]] = 0.0
+    want = N.scatter_nd_ref(host, idx, upd)
+    p, flags_fine_grained = ctypes.c_void_p(), 1
+    assert hip.hipExtMallocWithFlags(ctypes.byref(p), ctypes.c_size_t(host.numel() * size), flags_fine_grained) == 0
+    to_device, to_host = 1, 2
+    assert hip.hipMemcpy(p, ctypes.c_void_p(host.data_ptr()), ctypes.c_size_t(host.numel() * size), to_device) == 0
+    upd_d, idx_d = upd.to(DEV), idx.to(DEV)
+    dims = (ctypes.c_int64 * 2)(rows, slice_)
+    _capi.check(_capi.load().tf_scatter_nd(upd_d.data_ptr(), p, idx_d.data_ptr(), dims, 2, n, 1,
+                                           {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dtype],
+                                           torch.cuda.current_stream().cuda_stream), "tf_scatter_nd")
+    torch.cuda.synchronize()
+    got = torch.empty_like(host)
+    assert hip.hipMemcpy(ctypes.c_void_p(got.data_ptr()), p, ctypes.c_size_t(host.numel() * size), to_host) == 0
+    assert hip.hipFree(p) == 0
+    assert (got[4].view(ints) == torch.tensor(bits, dtype=torch.int64).to(ints)).all()
+    keep = [i for i in range(rows) if i != 4]
+    assert torch.equal(got[keep].float(), want[keep])
+
+
+def test_scatter_nd_in_a_graph():
+    from tilefusion_amd.ops import scatter_nd
+    g = torch.Generator().manual_seed(3)
+    idx = torch.randint(0, 50, (1500, 1), generator=g).to(DEV)
+    upd = torch.randint(-1, 2, (1500, 33), generator=g).to(torch.bfloat16).to(DEV)
+    data, other = torch.zeros(50, 33, dtype=torch.bfloat16, device=DEV), torch.zeros(50, 33, dtype=torch.bfloat16, device=DEV)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        scatter_nd(data, idx, upd)
+    for _ in range(3):
+        data.zero_(), other.zero_()
+        graph.replay()
+        scatter_nd(other, idx, upd)
+        torch.cuda.synchronize()
+        assert torch.equal(data, other)

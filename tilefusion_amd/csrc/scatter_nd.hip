@@ -6,6 +6,7 @@
 // one thread); duplicates inside a workgroup are added up in fp32 registers before they touch
 // memory; the strides travel as kernel arguments (the reference cudaMallocs them per call and never
 // frees them); index rows that point outside `data` are skipped instead of written out of bounds.
+// `data` outside the device's ordinary memory is added to by compare-and-swap.
 //
 // What bounds it: atomics on one 128-byte line are served one after another, ~20 ns each (the eight
 // L2s are not coherent with each other, so a device-wide atomic is done on the memory side).  With
@@ -38,8 +39,16 @@ struct Word {
   float v[kElems];
 };
 
-// Adds to one element by compare-and-swap on the aligned word that holds it; the other half of
-// the word keeps its bits.
+// Adds to one element by compare-and-swap on the aligned word that holds it: in any memory that the device can
+// reach, and the other half of the word keeps its bits.
+TFK_DEVICE void atomic_add_element(float* p, float v) {
+  unsigned* const word = reinterpret_cast<unsigned*>(p);
+  unsigned old = *word, seen;
+  do {
+    seen = old;
+    old = atomicCAS(word, seen, __builtin_bit_cast(unsigned, __builtin_bit_cast(float, seen) + v));
+  } while (old != seen);
+}
 template <typename T>
 TFK_DEVICE void atomic_add_element(T* p, float v) {
   const size_t at = reinterpret_cast<size_t>(p);
@@ -94,9 +103,16 @@ TFK_DEVICE void add_word_of_slice(Word<T>& sum, const T* src, long long e0, long
 // elements of `data` the other half keeps its bits, whatever they stand for: compare-and-swap.  Only the first
 // and the last word of `data` can be such; for every word that two slices share it would cost far too
 // much (2048 bf16 updates of 33 into 64 rows 8 us and 40, 30000 of 77 into 131072 rows 25 and 1260).
-template <typename T, bool kSplitPairs>
+// kAnyMemory: every element by compare-and-swap.
+template <typename T, bool kSplitPairs, bool kAnyMemory>
 TFK_DEVICE void add_to_slice(T* dst, const Word<T>& w, long long e0, long long slice, const T* data, long long total) {
   T* const word = dst + e0;
+  if constexpr (kAnyMemory) {
+#pragma unroll
+    for (int e = 0; e < Word<T>::kElems; ++e)
+      if (e0 + e >= 0 && e0 + e < slice) atomic_add_element(word + e, w.v[e]);
+    return;
+  }
   if constexpr (kSplitPairs) {
     const int outside = word < data ? 0 : word + 1 >= data + total ? 1 : -1;   // element of the word that is not data's
     if (outside >= 0) {
@@ -114,31 +130,33 @@ TFK_DEVICE int first_word_shift(const T* dst) {
 
 // Few updates: a group of `lanes` adjacent lanes (a power of two up to 64) per update, one word per
 // lane, no sort.  The call is then the latency of a load of the index, one of the update and an atomic.
-template <typename T, bool kSplitPairs>
+// kAnyMemory: `data` is not known to be ordinary memory of this device; any number of updates.
+template <typename T, bool kSplitPairs, bool kAnyMemory>
 __global__ __launch_bounds__(kScatterThreads) void scatter_nd_direct_kernel(
     const T* __restrict__ updates, T* __restrict__ data, const long long* __restrict__ indices, Strides s, long long n,
     int k, long long slice, long long total, int lanes) {
   constexpr int kElems = Word<T>::kElems;
   const int lane = threadIdx.x & (lanes - 1);
-  const long long row = blockIdx.x * (long long)(kScatterThreads / lanes) + threadIdx.x / lanes;
-  if (row >= n) return;
-  bool inside = true;
-  long long at = 0;
-  for (int j = 0; j < k; ++j) {
-    const long long ix = indices[row * k + j];
-    inside &= ix >= 0 && ix < s.dim[j];
-    at += ix * s.stride[j];
-  }
-  if (!inside) return;
-  T* const dst = data + at;
-  const int shift = first_word_shift<T, kSplitPairs>(dst);
-  const long long step = (long long)gridDim.y * lanes * kElems;
-  for (long long e0 = ((long long)blockIdx.y * lanes + lane) * kElems - shift; e0 < slice; e0 += step) {
-    Word<T> w;
+  const long long rows_step = gridDim.x * (long long)(kScatterThreads / lanes);
+  for (long long row = blockIdx.x * (long long)(kScatterThreads / lanes) + threadIdx.x / lanes; row < n; row += rows_step) {
+    bool inside = true;
+    unsigned long long at = 0;
+    for (int j = 0; j < k; ++j) {
+      const long long ix = indices[row * k + j];
+      inside &= ix >= 0 && ix < s.dim[j];
+      at += (unsigned long long)ix * (unsigned long long)s.stride[j];
+    }
+    if (!inside) continue;
+    T* const dst = data + at;
+    const int shift = first_word_shift<T, kSplitPairs>(dst);
+    const long long step = (long long)gridDim.y * lanes * kElems;
+    for (long long e0 = ((long long)blockIdx.y * lanes + lane) * kElems - shift; e0 < slice; e0 += step) {
+      Word<T> w;
 #pragma unroll
-    for (int e = 0; e < kElems; ++e) w.v[e] = -0.f;
-    add_word_of_slice<T, kSplitPairs>(w, updates + row * slice, e0, slice);
-    add_to_slice<T, kSplitPairs>(dst, w, e0, slice, data, total);
+      for (int e = 0; e < kElems; ++e) w.v[e] = -0.f;
+      add_word_of_slice<T, kSplitPairs>(w, updates + row * slice, e0, slice);
+      add_to_slice<T, kSplitPairs, kAnyMemory>(dst, w, e0, slice, data, total);
+    }
   }
 }
 
@@ -169,7 +187,7 @@ __global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
         for (int j = 0; j < k; ++j) {
           const long long ix = indices[(row0 + tid) * k + j];
           inside &= ix >= 0 && ix < s.dim[j];
-          at += (unsigned long long)(ix * s.stride[j]);
+          at += (unsigned long long)ix * (unsigned long long)s.stride[j];
         }
         if (inside) base = at;
       }
@@ -245,10 +263,10 @@ __global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
                 part.v[e] = beyond(sum[v].v[e]) ? __builtin_copysignf(kMax, sum[v].v[e]) : -0.f;
                 sum[v].v[e] -= part.v[e];
               }
-              add_to_slice<T, kSplitPairs>(dst, part, e0, slice, data, total);
+              add_to_slice<T, kSplitPairs, false>(dst, part, e0, slice, data, total);
             }
           }
-          add_to_slice<T, kSplitPairs>(dst, sum[v], e0, slice, data, total);
+          add_to_slice<T, kSplitPairs, false>(dst, sum[v], e0, slice, data, total);
         }
       }
     }
@@ -268,25 +286,41 @@ int launch_shape(const void* updates, void* data, const long long* indices, cons
   return TF_OK;
 }
 
-template <typename T, bool kSplitPairs>
+template <typename T, bool kSplitPairs, bool kAnyMemory>
 int launch_direct(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
                   long long slice, long long total, int lanes, long long words, hipStream_t st) {
   const int per = kScatterThreads / lanes;
-  const dim3 grid((unsigned)((n + per - 1) / per), (unsigned)std::min<long long>((words + lanes - 1) / lanes, 1024));
-  hipLaunchKernelGGL((scatter_nd_direct_kernel<T, kSplitPairs>), grid, dim3(kScatterThreads), 0, st,
+  const dim3 grid((unsigned)std::min<long long>((n + per - 1) / per, 1 << 20),
+                  (unsigned)std::min<long long>((words + lanes - 1) / lanes, 1024));
+  hipLaunchKernelGGL((scatter_nd_direct_kernel<T, kSplitPairs, kAnyMemory>), grid, dim3(kScatterThreads), 0, st,
                      static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
 
+// Hardware floating-point atomics are defined for ordinary (coarse-grained) memory of the device that runs the kernel:
+// on host, managed or fine-grained memory an update may be lost.
+bool is_ordinary_device_memory(const void* p) {
+  int device = -1;
+  hipPointerAttribute_t a{};
+  if (hipGetDevice(&device) != hipSuccess || hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();   // not an error of this call
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && !a.isManaged && a.device == device && a.allocationFlags == hipDeviceMallocDefault;
+}
+
 template <typename T, bool kSplitPairs>
 int launch_rows(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
                 long long slice, long long targets, int lanes, long long words, hipStream_t st) {
+  if (!is_ordinary_device_memory(data))
+    return launch_direct<T, kSplitPairs, true>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   // Times in us with log-uniform indices (threads / updates a workgroup).  Few updates: no sort (806 of
   // 34 fp32: direct 3.3, 256/16 5.6).  From 1024 on contention shows (2048 of 64 bf16 into 64 rows:
   // direct 10.8, 256/16 6.3, 512/64 8.2), beyond 2048 more updates per sort pay (4096 of 1024 bf16
   // into 1000 rows: direct 26, 256/16 17.6, 512/64 12.9).
-  if (n <= 1024) return launch_direct<T, kSplitPairs>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+  if (n <= 1024)
+    return launch_direct<T, kSplitPairs, false>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   if (n <= 2048)
     return launch_shape<T, 256, 16, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   // Every target hit at least eight times on average: the deeper sort (59764 of 21 fp32 into 219 rows:
