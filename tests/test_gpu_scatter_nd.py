@@ -77,6 +77,25 @@ def test_scatter_nd_fp16_sum_of_duplicates_beyond_its_range():
     assert data[1].tolist() == [60000.0, 60000.0] and data[0].tolist() == [-60000.0, -60000.0]
 
 
+@pytest.mark.parametrize("dtype,big", [(torch.float32, 3e38), (torch.float16, 60000.0), (torch.bfloat16, 3e38)],
+                         ids=["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("slice_", [4, 5])
+@pytest.mark.parametrize("n", [1500, 2500])
+def test_scatter_nd_sums_beyond_the_range_of_the_type(dtype, big, slice_, n):
+    # the sum of the two updates is beyond the type's range, the result is not; sums with infinities stay theirs
+    from tilefusion_amd.ops import scatter_nd
+    data = torch.zeros(1000, slice_, dtype=dtype, device=DEV)
+    data[7] = -big
+    upd = torch.zeros(n, slice_, dtype=dtype, device=DEV)
+    idx = 8 + torch.arange(n, device=DEV) % 900
+    idx[[3, 9, 5, 6]] = torch.tensor([7, 7, 950, 950], device=DEV)
+    upd[[3, 9]], upd[5], upd[6] = big, float("inf"), 1.0
+    want = data.clone()
+    want[7], want[950] = upd[3], float("inf")
+    scatter_nd(data, idx.unsqueeze(1), upd)
+    assert torch.equal(data, want)
+
+
 # Of a word of two 16-bit elements a slice may hold one: the other one, of a neighbouring row, keeps its value
 # (the smallest subnormal number here), and memory outside the tensor its bits, also those of a signalling NaN.
 @pytest.mark.parametrize("dtype,bits", [(torch.float16, 0x7D01), (torch.bfloat16, 0x7F81), (torch.float32, 0x7F800001)],

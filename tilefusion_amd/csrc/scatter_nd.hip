@@ -172,6 +172,7 @@ __global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
   constexpr int kElems = Word<T>::kElems;
   constexpr int kSortWaves = (kRows + kWaveSize - 1) / kWaveSize;
   constexpr unsigned long long kOutside = ~0ull;
+  constexpr float kLargest = std::is_same_v<T, half_t> ? 65504.f : std::is_same_v<T, bf16_t> ? 0x1.FEp127f : 0x1.FFFFFEp127f;
   __shared__ unsigned long long s_base[kRows];   // element offset of an update's slice in data
   __shared__ unsigned long long s_sorted[kRows];
   __shared__ int s_order[kRows];                 // update numbers in the order of their slices
@@ -252,19 +253,19 @@ __global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
         for (int v = 0; v < kWords; ++v) {
           const long long e0 = (word0 + (long long)v * lanes) * kElems - shift;
           if (e0 >= slice) continue;
-          if constexpr (std::is_same_v<T, half_t>) {
-            // a finite sum beyond fp16's largest number is added in pieces, as the single updates would be
-            constexpr float kMax = 65504.f;
-            auto beyond = [](float x) { return __builtin_fabsf(x) > kMax && __builtin_isfinite(x); };
-            while (beyond(sum[v].v[0]) || beyond(sum[v].v[1])) {
-              Word<T> part;
+          // A sum that T does not hold is added as its single updates, which `data` may bring back into range.
+          bool held = true;
 #pragma unroll
-              for (int e = 0; e < 2; ++e) {
-                part.v[e] = beyond(sum[v].v[e]) ? __builtin_copysignf(kMax, sum[v].v[e]) : -0.f;
-                sum[v].v[e] -= part.v[e];
-              }
-              add_to_slice<T, kSplitPairs, false>(dst, part, e0, slice, data, total);
+          for (int e = 0; e < kElems; ++e) held &= __builtin_fabsf(sum[v].v[e]) <= kLargest;
+          if (!held) {
+            for (int p = begin; p < end; ++p) {
+              Word<T> w;
+#pragma unroll
+              for (int e = 0; e < kElems; ++e) w.v[e] = -0.f;
+              add_word_of_slice<T, kSplitPairs>(w, updates + (row0 + s_order[p]) * slice, e0, slice);
+              add_to_slice<T, kSplitPairs, false>(dst, w, e0, slice, data, total);
             }
+            continue;
           }
           add_to_slice<T, kSplitPairs, false>(dst, sum[v], e0, slice, data, total);
         }
