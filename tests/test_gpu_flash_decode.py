@@ -121,3 +121,17 @@ def test_every_way_to_cut(bh, lkv, d, splits, dtype, tol):
     ref = (torch.softmax(scores, -1)[..., None] * v.float()).sum(1)
     o = c_decode(q, k, v, splits)
     assert o.dtype == dtype and N.rel_l2(o, ref) <= tol[0] and N.max_abs(o, ref) <= tol[1]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bh,lkv,d,splits", [(8, 4096, 128, 64), (8, 4096, 64, 64), (4, 8192, 128, 5), (300, 8192, 64, 64),
+                                             (3, 1001, 128, 1), (3, 4099, 64, 7), (520, 1003, 128, 64), (4, 9, 64, 3)])
+def test_infinite_values_in_any_split_stay_infinite(bh, lkv, d, splits, dtype):
+    # every weight is positive: an infinite value makes its column that infinity, whichever split holds it
+    g = torch.Generator(device=DEV).manual_seed(lkv + d)
+    q, k, v = (torch.randn(*shape, device=DEV, generator=g).to(dtype) for shape in ((bh, d), (bh, lkv, d), (bh, lkv, d)))
+    v[:, 0, 1], v[:, lkv // 2, 2], v[:, lkv - 1, 3] = math.inf, -math.inf, math.inf
+    o = c_decode(q, k, v, splits)
+    want = torch.zeros(d, device=DEV)
+    want[1], want[2], want[3] = math.inf, -math.inf, math.inf
+    assert torch.equal(torch.where(o.isfinite(), torch.zeros_like(o), o).float(), want.expand(bh, d))

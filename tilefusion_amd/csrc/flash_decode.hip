@@ -99,6 +99,18 @@ TFK_DEVICE float dot8(typename Vec8<T>::type k, typename Vec8<T>::type q) {
   return acc;
 }
 
+// 16 bytes at base + offset, zeros where that is not within `bytes`; `base` and `bytes` are wavefront-uniform.
+template <typename V>
+TFK_DEVICE V load_below(const char* base, unsigned bytes, unsigned offset) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int kRaw32Bit = 0x00020000, kStreaming = 2;
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, bytes, kRaw32Bit);
+  return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset, 0, kStreaming));
+#else
+  return V{};
+#endif
+}
+
 // workspace: o_part [batch_heads][num_splits][D] fp32, then ml_part [batch_heads][num_splits][2].
 // kWhole: one workgroup per slice, which writes O itself (num_splits == 1, chunk == Lkv).
 // `chunk` is a multiple of the rows of one load step.
@@ -122,8 +134,6 @@ __global__ __launch_bounds__(kDecWaves * kWaveSize) void flash_decode_split_kern
   const int64_t row_begin = (int64_t)split * chunk;
   const int64_t row_end = min(row_begin + chunk, Lkv);
 
-  const T* kbase = K + bh * Lkv * D + 8 * lv;
-  const T* vbase = V + bh * Lkv * D + 8 * lv;
   const V8 q8 = *reinterpret_cast<const V8*>(Q + bh * D + 8 * lv);
 
   float m_run = -INFINITY, l_run = 0.f;
@@ -154,22 +164,13 @@ __global__ __launch_bounds__(kDecWaves * kWaveSize) void flash_decode_split_kern
       for (int u = 0; u < kBatchRows; ++u)
         vd[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(vb + lane_off + u * (kRowsPerStep * D * 2)));
     } else {
-      // the steps behind the end of the chunk are left out (workgroup-uniform); their V is zero because
-      // their weights are
+      // rows behind the end of the chunk come as zeros from the bounds check of a buffer load: their weight is
+      // zero, and zero times another row's infinity would be NaN
+      const unsigned left = (unsigned)((row_end - base) * (D * 2));
 #pragma unroll
-      for (int u = 0; u < kBatchRows; ++u) {
-        const int64_t row = min(base + lane_row + (int64_t)u * kRowsPerStep, Lkv - 1);
-        if (base + (int64_t)u * kRowsPerStep < row_end)
-          kd[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(kbase + row * D));
-      }
+      for (int u = 0; u < kBatchRows; ++u) kd[u] = load_below<V8>(k_slice + base * (D * 2), left, lane_off + u * (kRowsPerStep * D * 2));
 #pragma unroll
-      for (int u = 0; u < kBatchRows; ++u) {
-        const int64_t row = min(base + lane_row + (int64_t)u * kRowsPerStep, Lkv - 1);
-        if (base + (int64_t)u * kRowsPerStep < row_end)
-          vd[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(vbase + row * D));
-        else
-          vd[u] = V8{};
-      }
+      for (int u = 0; u < kBatchRows; ++u) vd[u] = load_below<V8>(v_slice + base * (D * 2), left, lane_off + u * (kRowsPerStep * D * 2));
     }
     __builtin_amdgcn_sched_barrier(0);   // the requests leave before the other batch is consumed
   };
@@ -290,7 +291,8 @@ __global__ __launch_bounds__(kCombThreads) void flash_decode_combine_kernel(
     if (s0 != grp) load(s0);
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
-      const float w = s0 + u * kGroups < num_splits ? __builtin_amdgcn_exp2f(m[u][0] - big) : 0.f;
+      if (s0 + u * kGroups >= num_splits) break;   // (the last split again, which may hold infinities)
+      const float w = __builtin_amdgcn_exp2f(m[u][0] - big);
       acc += w * o[u];
       l += w * m[u][1];
     }
