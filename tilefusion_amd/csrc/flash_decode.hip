@@ -337,17 +337,6 @@ int check_decode_args(const char* who, const void* Q, const void* K, const void*
   return TF_OK;
 }
 
-template <typename T, int D, int kDecWaves, int kBatchRows, bool kWhole>
-int launch_split(const void* Q, const void* K, const void* V, void* O, float* o_part, float* ml_part,
-                 int64_t batch_heads, int64_t Lkv, int splits, int64_t chunk, double softmax_scale, hipStream_t st) {
-  const float scale_log2 = (float)(softmax_scale * 1.4426950408889634);
-  hipLaunchKernelGGL((flash_decode_split_kernel<T, D, kDecWaves, kBatchRows, kWhole>), dim3(splits, (unsigned)batch_heads),
-                     dim3(kDecWaves * kWaveSize), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K),
-                     static_cast<const T*>(V), static_cast<T*>(O), o_part, ml_part, Lkv, splits, chunk, scale_log2);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
-}
-
 // How a problem is cut.  `splits` ranges of `chunk` keys per slice; 1: one workgroup per slice, no partials
 // and no second kernel.
 struct DecodePlan {
