@@ -347,6 +347,11 @@ struct DecodePlan {
 // launch cost ~4 us.  Measured (fp16, us, one workgroup per slice / best split): 33 slices of 662 x 64
 // 6.5 / 8.1, 964 of 913 x 128 68 / 73, 11 of 825 x 128 10.4 / 8.5, 64 of 8192 x 128 85 / 44.  Slices that the
 // CUs cannot share evenly cost about a third of the unevenness (802 of 2574 x 128: 180 / 165).
+// Of a slice beyond 4 MiB one workgroup never gets far while all the others do the same: hundreds of streams,
+// megabytes apart, and a first pass over memory whose translations no cache holds yet pays for each (512 of
+// 32768 x 128: 1460-1500 us, in 8 ranges 1320-1370; 155 of 36332 x 128 636 / 569, 180 of 50000 x 128 886 / 807).
+// Passes after that take as long as with one workgroup per slice (1237 / 1235; over ten caches in turn too).
+// So such slices come in ranges of at most 2 MiB.  (512 of 8192 x 128, 4 MiB: first pass 375 whole and 384 cut.)
 // Otherwise the cut aims at 1024 workgroups, and at no more than 256 KiB of keys and values in each: they
 // come in rounds, and the last one fills the chip badly (584 of 16256 x 64: 4 splits 411, 16 364; 136 of
 // 36053 x 64: 8 splits 201, 32 192), but at 32 KiB at least (32 of 1999 x 64: 16 splits 10.2, 64 12.8),
@@ -357,10 +362,12 @@ DecodePlan plan_decode(int64_t batch_heads, int64_t Lkv, int num_splits) {
   const double per_cu = batch_heads / 256.0;
   const double uneven = per_cu > 1.0 ? 1.0 + 0.35 * (std::ceil(per_cu) / per_cu - 1.0) : 1.0;
   const DecodePlan whole = {1, Lkv};
-  if (num_splits == 1 || 2.5 + std::max(alone_us, stream_us * uneven) <= 6.5 + stream_us) return whole;
+  const bool shared_evenly = 2.5 + std::max(alone_us, stream_us * uneven) <= 6.5 + stream_us;
+  if (num_splits == 1 || (shared_evenly && slice_bytes <= 4194304.0)) return whole;
   constexpr int64_t kStep = 8 * (kWaveSize / (D / 8));   // rows of one load step of the larger workgroup
   const int64_t fill = (1024 + batch_heads - 1) / batch_heads;
-  const int64_t least = (int64_t)(slice_bytes / 262144.0) + 1, most = (int64_t)(slice_bytes / 32768.0) + 1;
+  const int64_t least = shared_evenly ? (int64_t)std::ceil(slice_bytes / 2097152.0) : (int64_t)(slice_bytes / 262144.0) + 1;
+  const int64_t most = (int64_t)(slice_bytes / 32768.0) + 1;
   const int64_t want = std::min<int64_t>(num_splits, std::min(std::max(fill, least), most));
   const int64_t chunk = ((Lkv + want - 1) / want + kStep - 1) / kStep * kStep;
   const int64_t splits = (Lkv + chunk - 1) / chunk;
