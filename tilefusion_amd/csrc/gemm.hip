@@ -28,10 +28,9 @@
 namespace tfk {
 namespace {
 
-template <int BM_, int BN_, int BK_, int WAVES_M_, int WAVES_N_, int STAGES_>
+template <int BM_, int BN_, int BK_, int WAVES_M_, int WAVES_N_>
 struct GemmShape {
   static constexpr int BM = BM_, BN = BN_, BK = BK_;
-  static constexpr int kStages = STAGES_;  // LDS stages of the direct-load pipeline
   static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_;
   static constexpr int kWaves = WAVES_M * WAVES_N;
   static constexpr int kThreads = kWaves * kWaveSize;
@@ -40,13 +39,9 @@ struct GemmShape {
   static constexpr int kKSteps = BK / 16;
   static constexpr int kChunks = BK / 8;              // 16-byte chunks per tile row
   static constexpr int kRowsPer256B = 16 / kChunks;   // rows that share one pass over all banks
-  static constexpr int kRowsPerInstr = 64 / kChunks;  // rows one wavefront load covers
   static constexpr int kABytes = BM * BK * 2;
   static constexpr int kBBytes = BN * BK * 2;
-  static constexpr int kStageBytes = kABytes + kBBytes;
   static_assert(WM % 32 == 0 && WN % 32 == 0 && BK % 16 == 0, "wavefront tile must be MFMA-sized");
-  static_assert((BM * kChunks) % (64 * kWaves) == 0 && (BN * kChunks) % (64 * kWaves) == 0,
-                "tile rows must split evenly over the wavefronts' 1 KiB loads");
 
   // Physical 16-byte chunk of logical chunk `c` in tile row `row`.  Sixteen consecutive rows
   // reading the same logical chunk land in sixteen different 16-byte bank groups.
@@ -511,9 +506,10 @@ int launch_ring64(const void* A, const void* B, void* C, int M, int N, int K, hi
 // KiB, a quarter of the L1's rate (32 x 4096 x 4096: 12.7 us).  LDS-direct requests of 8 rows x 128 bytes
 // are whole lines: 7.8 us, 4.4 TB/s (the 64 x 64 bounds-checked kernel that ran before: 68.6).
 // ------------------------------------------------------------------------------------------
-template <int TM_, int TN_, int WAVES_, int STAGES_>
+template <int TM_, int TN_, int WAVES_>
 struct SplitKShape {
-  static constexpr int TM = TM_, TN = TN_, kWaves = WAVES_, kStages = STAGES_;
+  static constexpr int TM = TM_, TN = TN_, kWaves = WAVES_;
+  static constexpr int kStages = 2;                           // k-tiles in a wavefront's ring
   static constexpr int BM = 16 * TM, BN = 16 * TN, BK = 64;
   static constexpr int kThreads = kWaves * kWaveSize;
   static constexpr int kFrags = TM + TN;                      // 16-row operand fragments per 32-deep step
@@ -523,7 +519,7 @@ struct SplitKShape {
   static constexpr int kRingBytes = kWaves * kStages * kStageBytes;
   static constexpr int kPartBytes = kWaves * BM * kPitch * 4;
   static constexpr int kLdsBytes = kRingBytes > kPartBytes ? kRingBytes : kPartBytes;
-  static_assert(kStages >= 2 && kStages <= 4 && (kStages - 1) * kLoads < 64, "vmcnt is a 6-bit counter");
+  static_assert(kLoads < 64, "vmcnt is a 6-bit counter");
   // the same swizzle as the big kernel's: conflict-free fragment reads of 128-byte rows
   __host__ __device__ static constexpr int swizzle(int row, int c) { return c ^ ((row / 2) % 8); }
 };
@@ -599,11 +595,9 @@ __global__ __launch_bounds__(S::kThreads) void gemm_split_k_kernel(
           for (int t = 0; t < 8; ++t) fr[set][ks][f][t] = (InT)0.f;
       }
   };
-  // waits until only this wavefront's `tiles` youngest k-tiles are still in flight
-  auto wait_behind = [&](int tiles) __attribute__((always_inline)) {
-    if (S::kStages > 3 && tiles >= 3) wait_vmem<3 * (S::kStages > 3 ? S::kLoads : 0)>();
-    else if (S::kStages > 2 && tiles >= 2) wait_vmem<2 * (S::kStages > 2 ? S::kLoads : 0)>();
-    else if (tiles >= 1) wait_vmem<S::kLoads>();
+  // waits until at most this wavefront's youngest k-tile, if there is one behind the awaited, is still in flight
+  auto wait_for_tile = [&](bool one_behind) __attribute__((always_inline)) {
+    if (one_behind) wait_vmem<S::kLoads>();
     else wait_vmem<0>();
   };
   const int mine = wave < num_k_tiles ? (last_tile - wave) / S::kWaves + 1 : 0;   // k-tiles of this wavefront
@@ -612,7 +606,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_split_k_kernel(
   for (int t = 0; t < S::kStages; ++t)
     if (t < mine) request(t, tile_of(t));
   if (mine > 0) {
-    wait_behind(min(mine, S::kStages) - 1);
+    wait_for_tile(mine > 1);
     read(0, 0);
   }
   int stage = 0;   // of tile t
@@ -625,7 +619,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_split_k_kernel(
     if (t + S::kStages < mine) request(stage, tile_of(t + S::kStages));
     stage = stage + 1 == S::kStages ? 0 : stage + 1;
     if (t + 1 < mine) {
-      wait_behind(min(mine - 2 - t, S::kStages - 1));
+      wait_for_tile(t + 2 < mine);
       read(set ^ 1, stage);
     }
     if (K % S::BK != 0 && tile_of(t) == last_tile) mask_behind_k(set);
@@ -757,7 +751,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_guarded_kernel(
       }
 }
 
-using ShapeSmall = GemmShape<64, 64, 32, 2, 2, 1>;    // bounds-checked path
+using ShapeSmall = GemmShape<64, 64, 32, 2, 2>;    // bounds-checked path
 
 template <typename S, typename OutT, typename InT>
 int launch_guarded(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st) {
@@ -846,10 +840,10 @@ template <typename OutT, typename InT>
 int dispatch(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st) {
   using Launcher = int (*)(const void*, const void*, void*, int, int, int, hipStream_t);
   static constexpr Launcher kLaunchers[] = {
-      launch_split_k<SplitKShape<1, 1, 4, 2>, OutT, InT>, launch_split_k<SplitKShape<1, 1, 8, 2>, OutT, InT>,
-      launch_split_k<SplitKShape<2, 1, 4, 2>, OutT, InT>, launch_split_k<SplitKShape<2, 2, 1, 2>, OutT, InT>,
-      launch_split_k<SplitKShape<2, 2, 4, 2>, OutT, InT>, launch_split_k<SplitKShape<4, 2, 4, 2>, OutT, InT>,
-      launch_split_k<SplitKShape<4, 4, 4, 2>, OutT, InT>,
+      launch_split_k<SplitKShape<1, 1, 4>, OutT, InT>, launch_split_k<SplitKShape<1, 1, 8>, OutT, InT>,
+      launch_split_k<SplitKShape<2, 1, 4>, OutT, InT>, launch_split_k<SplitKShape<2, 2, 1>, OutT, InT>,
+      launch_split_k<SplitKShape<2, 2, 4>, OutT, InT>, launch_split_k<SplitKShape<4, 2, 4>, OutT, InT>,
+      launch_split_k<SplitKShape<4, 4, 4>, OutT, InT>,
       launch_ring64<Ring64Shape<128, 128, 4>, OutT, InT>, launch_ring64<Ring64Shape<128, 128, 2>, OutT, InT>,
       launch_ring64<Ring64Shape<128, 128, 2>, OutT, InT>, launch_ring64<Ring64Shape<192, 128, 2>, OutT, InT>,
       launch_ring64<Ring64Shape<192, 192, 2>, OutT, InT>, launch_ring64<Ring64Shape<256, 128, 2>, OutT, InT>,
