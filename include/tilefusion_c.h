@@ -182,6 +182,15 @@ TF_API int tf_scatter_nd(const void* updates, void* data, const int64_t* indices
                          const int64_t* data_dims, int rank, int64_t num_index_rows,
                          int index_depth, int dtype, void* stream);
 
+/* What a call would run, decided on the host from the sizes alone; nothing is launched.
+ * tf_gemm_kernel_index: position of the kernel in the table in front of pick_gemm_kernel (csrc/gemm.hip), for operands at
+ * 16-byte boundaries; -1 for sizes that tf_gemm rejects.  tf_flash_decode_plan: ranges per slice (1: not cut), and in
+ * *wavefronts those of a workgroup; 0 for arguments that tf_flash_decode rejects.  tf_flash_attention_wide_rows:
+ * query rows per workgroup of tf_flash_attention_fwd_wide. */
+TF_API int tf_gemm_kernel_index(int64_t M, int64_t N, int64_t K);
+TF_API int tf_flash_decode_plan(int64_t batch_heads, int64_t Lkv, int64_t D, int num_splits, int* wavefronts);
+TF_API int tf_flash_attention_wide_rows(int64_t batch, int64_t Lq, int causal);
+
 /* Run-time compilation of kernels written against the tile headers (tilefusion_amd/include),
  * for shapes that are template parameters there.  tf_jit_compile builds `source` with
  * `hipcc --genco` for gfx950 (the tile headers are on the include path; include_paths and

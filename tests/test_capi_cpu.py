@@ -81,6 +81,50 @@ def test_decode_argument_validation_and_workspace():
     assert f(p, p, p, p, p, 1 << 20, 4, 0, 128, 4, 0.1, None) == _capi.TF_ERR_INVALID_ARG
 
 
+# ---- what a call runs, decided on the host ------------------------------------------------------------
+def test_gemm_edge_cases_reach_every_kernel_of_the_table():
+    from tests.test_gpu_gemm import EDGES
+    lib = _capi.load()
+    for kernel, problems in EDGES.items():
+        assert [lib.tf_gemm_kernel_index(*mnk) for mnk in problems] == [kernel] * len(problems)
+    text = open(os.path.join(ROOT, "tilefusion_amd", "csrc", "gemm.hip")).read()
+    table = re.search(r"constexpr GemmKernel kGemmKernels\[\] = \{\n(.*?)\n\};", text, re.S).group(1)
+    assert sorted(EDGES) == list(range(len(table.splitlines())))
+    assert lib.tf_gemm_kernel_index(0, 64, 64) == -1 and lib.tf_gemm_kernel_index(64, 64, 1 << 22) == -1
+
+
+def _plan(bh, lkv, d, splits):
+    waves = ctypes.c_int(0)
+    return _capi.load().tf_flash_decode_plan(bh, lkv, d, splits, ctypes.byref(waves)), waves.value
+
+
+def test_decode_cases_reach_every_way_to_cut():
+    from tests.test_gpu_flash_decode import CUTS
+    ways = {(_plan(*c)[0] > 1, _plan(*c)[1], c[2]) for c in CUTS}
+    assert ways == {(cut, waves, d) for cut in (False, True) for waves in (4, 8) for d in (64, 128)}
+
+
+def test_decode_plan():
+    assert _plan(512, 32768, 128, 64) == (8, 4)      # ranges of 2 MiB
+    assert _plan(512, 32768, 128, 3) == (3, 4)       # the caller's limit
+    assert _plan(512, 32768, 128, 1) == (1, 4)
+    assert _plan(512, 8192, 128, 64) == (1, 4)       # 4 MiB a slice: not cut
+    assert _plan(256, 8193, 128, 64)[0] > 1          # beyond
+    assert _plan(0, 64, 128, 4)[0] == 0 and _plan(4, 64, 96, 4)[0] == 0
+    for bh, lkv, d, splits in [(1, 1, 64, 64), (3, 100000, 128, 5), (65535, 7, 64, 9), (40, 40000, 128, 65536)]:
+        n, waves = _plan(bh, lkv, d, splits)
+        assert 1 <= n <= splits and waves in (4, 8)  # the workspace holds `splits` partials a slice
+
+
+def test_wide_attention_cases_reach_both_workgroup_sizes():
+    import tests.test_gpu_ops as t
+    marks = t.test_flash_attention_wide_heads.pytestmark
+    cases = next(m.args[1] for m in marks if m.args[0] == "bh,lq,lkv,causal")
+    lib = _capi.load()
+    assert {(lib.tf_flash_attention_wide_rows(bh, lq, int(causal)), causal) for bh, lq, _, causal in cases} == {
+        (rows, causal) for rows in (64, 128) for causal in (False, True)}
+
+
 def test_python_wrappers_validate_like_the_reference():
     # python/ops/fused_two_gemms.py:33-38: ValueError for a CPU tensor, TypeError for dtype
     import torch

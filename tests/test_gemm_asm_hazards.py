@@ -88,7 +88,7 @@ def test_ring_kernel_has_no_unprotected_mfma_hazards():
                                "-S", "-x", "hip", src, "-o", out], stderr=subprocess.DEVNULL)
         text = open(out).read()
     kernels = re.findall(r"^(_ZN3tfk\S*gemm_ring64_kernel\S*):[^\n]*\n(.*?)s_endpgm", text, flags=re.S | re.M)
-    assert len(kernels) >= 6, "ring kernel instantiations (three shapes, fp16 and fp32 output) not found"
+    assert len(kernels) >= 28, "ring kernel instantiations (seven shapes, two operand types, 16-bit and fp32 output) not found"
     for name, body in kernels:
         n_mfma = _check(name, body)
         assert n_mfma >= 32, f"{name}: expected the unrolled MFMA loop, found {n_mfma} MFMAs"

@@ -132,42 +132,46 @@ def test_identity_operand():
     assert torch.equal(c, b.T)
 
 
-# One ragged problem for every kernel and tile that the dispatch can pick, at the edges where each can go
-# wrong: fewer rows or columns than a tile, a last tile that overlaps its neighbour by all but one row,
-# K that completes its first (ring kernels) or last (split-K kernels) 64-deep k-tile with 8 to 56 zeros,
-# fewer k-tiles than wavefronts.  Small integers: exact in fp32, whatever the order of the sums.
-@pytest.mark.parametrize("m,n,k", [
-    (1, 1, 8), (72, 1, 72), (17, 33, 8), (3, 577, 200),                  # 16 x 16, four wavefronts
-    (1, 264, 264), (15, 72, 4264), (33, 31, 1000),                       # 16 x 16, eight
-    (5390, 1, 200), (44, 650, 1160),                                     # 32 x 16
-    (33, 4449, 72), (131, 1433, 64), (925, 768, 64),                     # 32 x 32, one
-    (17, 4561, 72), (257, 513, 328),                                     # 32 x 32, four
-    (50, 6432, 5688),                                                    # 64 x 32
-    (3578, 101, 1000), (1088, 577, 1032),                                # 64 x 64
-    (205, 5613, 1904), (2048, 2048, 136),                                # 128 x 128, deep ring
-    (4794, 235, 72), (129, 4095, 120), (128, 6400, 64),                  # 128 x 128
-    (4939, 3091, 80), (5216, 6236, 256),                                 # 128 x 128, two per CU
-    (812, 4675, 72), (2999, 1544, 1032),                                 # 192 x 128
-    (1398, 5437, 72), (3333, 2288, 1944),                                # 192 x 192
-    (982, 5472, 72),                                                     # 256 x 128
-    (4929, 1741, 72),                                                    # 256 x 192
-    (4882, 2468, 72), (4097, 2305, 264)])                                # 256 x 256
-def test_every_kernel_at_its_edges_is_exact(m, n, k):
-    g = torch.Generator().manual_seed(m + n + k)
-    a = torch.randint(-2, 3, (m, k), generator=g).half()
-    b = torch.randint(-2, 3, (n, k), generator=g).half()
-    ref = (a.to(DEV).float() @ b.to(DEV).float().t())                    # exact: |sum| <= 4 k < 2^24
-    assert torch.equal(c_gemm(a.to(DEV), b.to(DEV), torch.float32), ref)
-    c16 = c_gemm(a.to(DEV), b.to(DEV), torch.float16)
-    assert torch.equal(c16, ref.half())
-    # and nothing behind C is written
-    buf = torch.full((m * n + 64,), 7.0, device=DEV, dtype=torch.float16)
+# Ragged problems for every kernel and tile that the dispatch can pick (position in its table: m, n, k), at the
+# edges where each can go wrong: fewer rows or columns than a tile, a last tile that overlaps its neighbour
+# by all but one row, K that completes its first (ring kernels) or last (split-K kernels) 64-deep k-tile
+# with 8 to 56 zeros, fewer k-tiles than wavefronts.  Small integers: exact in fp32, whatever the order of the sums.
+EDGES = {
+    0: [(1, 1, 8), (72, 1, 72), (17, 33, 8), (3, 577, 200)],                # 16 x 16, four wavefronts
+    1: [(1, 264, 264), (15, 72, 4264), (33, 31, 1000), (44, 650, 1160)],    # 16 x 16, eight
+    2: [(5390, 1, 200)],                                                    # 32 x 16
+    3: [(33, 4449, 72), (131, 1433, 64), (925, 768, 64), (129, 4095, 120), (128, 6400, 64)],   # 32 x 32, one
+    4: [(17, 4561, 72), (257, 513, 328)],                                   # 32 x 32, four
+    5: [(6426, 54, 4480), (165, 1765, 7616)],                               # 64 x 32
+    6: [(3578, 101, 1000), (1088, 577, 1032), (50, 6432, 5688)],            # 64 x 64
+    7: [(205, 5613, 1904)],                                                 # 128 x 128, requests four tiles ahead
+    8: [(4794, 235, 72), (2048, 2048, 136)],                                # 128 x 128, two ahead
+    9: [(4939, 3091, 80), (5216, 6236, 256)],                               # 128 x 128, two per CU
+    10: [(812, 4675, 72), (2999, 1544, 1032)],                              # 192 x 128
+    11: [(1398, 5437, 72)],                                                 # 192 x 192
+    12: [(982, 5472, 72), (3333, 2288, 1944)],                              # 256 x 128
+    13: [(4929, 1741, 72), (4097, 2305, 264)],                              # 256 x 192
+    14: [(4882, 2468, 72)],                                                 # 256 x 256
+}
+
+
+@pytest.mark.parametrize("kernel,m,n,k", [(kernel, *mnk) for kernel, problems in EDGES.items() for mnk in problems])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_every_kernel_at_its_edges_is_exact(kernel, m, n, k, dtype):
     from tilefusion_amd import _capi
     lib = _capi.load()
-    ad, bd = a.to(DEV), b.to(DEV)
-    _capi.check(lib.tf_gemm_f16(ad.data_ptr(), bd.data_ptr(), buf.data_ptr(), 1, m, n, k, m, n, k, 1, 0,
-                                torch.cuda.current_stream().cuda_stream), "tf_gemm_f16")
-    assert torch.equal(buf[:m * n].view(m, n), ref.half()) and bool((buf[m * n:] == 7.0).all())
+    assert lib.tf_gemm_kernel_index(m, n, k) == kernel
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randint(-2, 3, (m, k), generator=g).to(dtype).to(DEV)
+    b = torch.randint(-2, 3, (n, k), generator=g).to(dtype).to(DEV)
+    ref = a.float() @ b.float().t()                                      # exact: |sum| <= 4 k < 2^24
+    for out_dtype in (torch.float32, dtype):
+        buf = torch.full((m * n + 64,), 7.0, device=DEV, dtype=out_dtype)
+        _capi.check(lib.tf_gemm(a.data_ptr(), b.data_ptr(), buf.data_ptr(), 2 if dtype == torch.bfloat16 else 1,
+                                int(out_dtype == torch.float32), m, n, k, m, n, k, 1, 0,
+                                torch.cuda.current_stream().cuda_stream), "tf_gemm")
+        assert torch.equal(buf[:m * n].view(m, n), ref.to(out_dtype))
+        assert bool((buf[m * n:] == 7.0).all())                          # nothing behind C is written
 
 
 def test_operands_without_16_byte_alignment():

@@ -149,8 +149,9 @@ def test_flash_attention_ops_for_head_dims_without_a_tuned_kernel(d, dv, lq, lkv
 
 @pytest.mark.parametrize("d,dv,lq,lkv", [(160, 160, 48, 64), (192, 128, 40, 96)])
 def test_flash_attention_ops_for_head_dims_above_128_run_the_header_kernel(d, dv, lq, lkv):
-    # no tuned kernel and nothing to pad to: compiled at run time from the header kernel (query rows
-    # padded to whole MFMA tiles by the op)
+    # nothing to pad to, and no tuned kernel unless D == Dv and V is in its natural layout: compiled at run time
+    # from the header kernel (query rows padded to whole MFMA tiles by the op).  Both layouts of V: with the
+    # transposed one it is always the header kernel.
     g = torch.Generator().manual_seed(d + dv)
     q = torch.randn(1, lq, d, generator=g).half()
     k = torch.randn(1, lkv, d, generator=g).half()
@@ -158,6 +159,10 @@ def test_flash_attention_ops_for_head_dims_above_128_run_the_header_kernel(d, dv
     scale = 1.0 / math.sqrt(d)
     o = torch.full((1, lq, dv), float("nan"), dtype=torch.float16, device=DEV)
     torch.ops.tilefusion.flash_attention_fwd(q.to(DEV), k.to(DEV), v.to(DEV), o, scale, False)
+    ok, r, m = N.check_close(o, N.attention_ref(q, k, v, scale, False))
+    assert ok, (r, m)
+    o.fill_(float("nan"))
+    torch.ops.tilefusion.flash_attention(q.to(DEV), k.to(DEV), v.transpose(1, 2).contiguous().to(DEV), o, 8, 32, d, dv, scale, False)
     ok, r, m = N.check_close(o, N.attention_ref(q, k, v, scale, False))
     assert ok, (r, m)
 
@@ -181,6 +186,11 @@ def test_flash_attention_ops_shrink_tiles_that_do_not_fit_the_lds(d, dv, lq, lkv
     assert o.shape == (2, lq, dv)
     ok, r, m = N.check_close(o, ref)
     assert ok, (r, m)
+    # V transposed: the header kernel also where natural V has a tuned one (256)
+    o = torch.full((2, lq, dv), float("nan"), dtype=torch.float16, device=DEV)
+    torch.ops.tilefusion.flash_attention(q.to(DEV), k.to(DEV), v.transpose(1, 2).contiguous().to(DEV), o, tq, tkv, d, dv, scale, causal)
+    ok, r, m = N.check_close(o, ref)
+    assert ok, (r, m)
 
 
 # Both workgroup sizes (64 queries; 128 where that saves a round of the 256 CUs), one key tile, fewer than
@@ -190,7 +200,8 @@ def test_flash_attention_ops_shrink_tiles_that_do_not_fit_the_lds(d, dv, lq, lkv
 @pytest.mark.parametrize("dtype,tol", [(torch.float16, 1.2e-3), (torch.bfloat16, 1e-2)])
 @pytest.mark.parametrize("d", [160, 192, 256])
 @pytest.mark.parametrize("bh,lq,lkv,causal", [(1, 1, 32, False), (2, 65, 96, False), (2, 130, 160, True), (2, 512, 512, True),
-                                              (150, 129, 64, False), (80, 500, 512, True), (150, 384, 384, True)])
+                                              (150, 129, 64, False), (80, 500, 512, True), (150, 384, 384, True),
+                                              (100, 129, 64, False), (32, 1000, 1024, False)])
 def test_flash_attention_wide_heads(bh, lq, lkv, causal, d, dtype, tol):
     g = torch.Generator().manual_seed(d + lq + lkv)
     q, k, v = (torch.randn(bh, n, d, generator=g).to(dtype) for n in (lq, lkv, lkv))
@@ -260,7 +271,7 @@ def test_flash_attention_wide_heads_keep_rows_whose_first_scores_are_minus_infin
 
 
 def test_flash_attention_key_length_that_cannot_be_padded_is_a_clear_error():
-    # above 128 the header kernel is what runs, and its key tiles are 32 wide
+    # above 128 the key tiles are 32 wide, in the tuned kernels as in the header kernel
     q = torch.randn(16, 160, dtype=torch.float16, device=DEV)
     k = torch.randn(48, 160, dtype=torch.float16, device=DEV)
     v = torch.randn(48, 160, dtype=torch.float16, device=DEV)
@@ -283,9 +294,8 @@ def test_fused_two_gemms_op_pads_what_the_kernels_cannot_tile(m, n, k, p):
 @pytest.mark.parametrize("m,n,k", [(256, 256, 128), (4096, 512, 256), (96, 160, 64), (128, 128, 96),
                                    (4096, 2048, 96), (32, 32, 32)])
 def test_gemm_op_bf16(m, n, k):
-    # every kernel of the GEMM is a template of the operand type: the ring kernel (first two shapes),
-    # the bounds-checked kernel (96 x 160), the 32-deep direct-to-LDS kernels with 128- and 256-wide
-    # tiles (K = 96)
+    # every kernel of the GEMM is a template of the operand type; what runs here are split-K kernels and, at
+    # 4096 x 2048 x 96, a ring kernel whose first k-tile is completed with zeros
     from tilefusion_amd.ops import gemm
     a, b = oracle.make_c1_gemm_inputs(m, n, k, seed=77)
     a, b = a.bfloat16(), b.bfloat16()

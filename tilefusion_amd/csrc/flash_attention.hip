@@ -804,15 +804,19 @@ int launch(const void* Q, const void* K, const void* V, void* O, int batch, int 
 // where it saves a round of the CUs.  bf16, D = 256, 64 / 128 queries: 8 slices of 2048 x 2048 69 / 95 us, 32 of
 // 1024 x 1024 89 / 64, 100 of 384 x 384 58 / 56; causal, 32 of 1024 x 1024 49 / 64 (193 by the kernel compiled
 // at run time, with its transposed copy of V), 40 of them 67 / 63, 64 of them 100 / 81.
-template <typename T, int D>
-int launch_wide(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv, float scale_log2,
-                bool causal, hipStream_t st) {
+inline bool wide_takes_128_queries(int64_t batch, int64_t Lq, bool causal) {
   auto rounds = [&](int rows) -> double {
-    const int64_t items = (int64_t)((Lq + rows - 1) / rows) * batch;
+    const int64_t items = (Lq + rows - 1) / rows * batch;
     if (causal) return std::max(1.0, (double)items / 512.0);   // a tile is half of the heaviest on average
     return (double)((items + 255) / 256);
   };
-  const bool wide_tile = 1.1 * rounds(128) < rounds(64);
+  return 1.1 * rounds(128) < rounds(64);
+}
+
+template <typename T, int D>
+int launch_wide(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv, float scale_log2,
+                bool causal, hipStream_t st) {
+  const bool wide_tile = wide_takes_128_queries(batch, Lq, causal);
   if (causal) {
     if (wide_tile) return launch_w<T, D, D, false, true, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
     return launch_w<T, D, D, false, true, 4, 1>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
@@ -958,4 +962,8 @@ extern "C" int tf_flash_attention_fwd_wide(const void* Q, const void* K, const v
   if (dtype == TF_DTYPE_BF16)
     return pick_wide<bf16_t>(Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, scale_log2, causal != 0, st);
   return pick_wide<half_t>(Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, scale_log2, causal != 0, st);
+}
+
+extern "C" int tf_flash_attention_wide_rows(int64_t batch, int64_t Lq, int causal) {
+  return tfk::wide_takes_128_queries(batch, Lq, causal != 0) ? 128 : 64;
 }

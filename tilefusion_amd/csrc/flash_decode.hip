@@ -338,10 +338,11 @@ int check_decode_args(const char* who, const void* Q, const void* K, const void*
 }
 
 // How a problem is cut.  `splits` ranges of `chunk` keys per slice; 1: one workgroup per slice, no partials
-// and no second kernel.
+// and no second kernel.  `waves` wavefronts per workgroup.
 struct DecodePlan {
   int splits;
   int64_t chunk;
+  int waves;
 };
 // One workgroup takes in ~45 GB/s when few run, all of them together 6.7 TB/s; the second kernel and its
 // launch cost ~4 us.  Measured (fp16, us, one workgroup per slice / best split): 33 slices of 662 x 64
@@ -361,7 +362,9 @@ DecodePlan plan_decode(int64_t batch_heads, int64_t Lkv, int num_splits) {
   const double slice_bytes = 4.0 * D * Lkv, stream_us = slice_bytes * batch_heads / 6.7e6, alone_us = slice_bytes / 45e3;
   const double per_cu = batch_heads / 256.0;
   const double uneven = per_cu > 1.0 ? 1.0 + 0.35 * (std::ceil(per_cu) / per_cu - 1.0) : 1.0;
-  const DecodePlan whole = {1, Lkv};
+  // one workgroup per slice: eight wavefronts take it in faster, four share a full chip better (512 slices of
+  // 32768 x 128: 1254 and 1203 us; 33 of 662 x 64: 6.5 and 8.1)
+  const DecodePlan whole = {1, Lkv, batch_heads >= 512 ? 4 : 8};
   const bool shared_evenly = 2.5 + std::max(alone_us, stream_us * uneven) <= 6.5 + stream_us;
   if (num_splits == 1 || (shared_evenly && slice_bytes <= 4194304.0)) return whole;
   constexpr int64_t kStep = 8 * (kWaveSize / (D / 8));   // rows of one load step of the larger workgroup
@@ -371,7 +374,9 @@ DecodePlan plan_decode(int64_t batch_heads, int64_t Lkv, int num_splits) {
   const int64_t want = std::min<int64_t>(num_splits, std::min(std::max(fill, least), most));
   const int64_t chunk = ((Lkv + want - 1) / want + kStep - 1) / kStep * kStep;
   const int64_t splits = (Lkv + chunk - 1) / chunk;
-  return splits > 1 ? DecodePlan{(int)splits, chunk} : whole;
+  // few workgroups: eight wavefronts each (8 slices of 65536 x 128 in 16 splits: 76 us with four, 54 with
+  // eight; 802 of 2574 x 128 in 4: 165 and 173)
+  return splits > 1 ? DecodePlan{(int)splits, chunk, batch_heads * splits < 1024 ? 8 : 4} : whole;
 }
 
 template <typename T, int D, int kDecWaves, bool kWhole>
@@ -393,17 +398,13 @@ int launch_decode_t(const void* Q, const void* K, const void* V, void* O, float*
                     hipStream_t st) {
   const DecodePlan plan = plan_decode<D>(batch_heads, Lkv, num_splits);
   if (plan.splits == 1) {
-    // eight wavefronts take in a slice faster, four share a full chip better (512 slices of 32768 x 128:
-    // 1254 and 1203 us; 33 of 662 x 64: 6.5 and 8.1)
-    if (batch_heads >= 512)
+    if (plan.waves == 4)
       return launch_split<T, D, 4, true>(Q, K, V, O, nullptr, nullptr, batch_heads, Lkv, plan, softmax_scale, st);
     return launch_split<T, D, 8, true>(Q, K, V, O, nullptr, nullptr, batch_heads, Lkv, plan, softmax_scale, st);
   }
   float* o_part = partials;
   float* ml_part = o_part + (size_t)batch_heads * plan.splits * D;
-  // few workgroups: eight wavefronts each (8 slices of 65536 x 128 in 16 splits: 76 us with four, 54 with
-  // eight; 802 of 2574 x 128 in 4: 165 and 173)
-  const int rc = batch_heads * plan.splits < 1024
+  const int rc = plan.waves == 8
       ? launch_split<T, D, 8, false>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st)
       : launch_split<T, D, 4, false>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st);
   if (rc != TF_OK) return rc;
@@ -438,6 +439,14 @@ int decode_with_workspace(const char* who, const void* Q, const void* K, const v
 
 }  // namespace
 }  // namespace tfk
+
+extern "C" int tf_flash_decode_plan(int64_t batch_heads, int64_t Lkv, int64_t D, int num_splits, int* wavefronts) {
+  using namespace tfk;
+  if (batch_heads <= 0 || Lkv <= 0 || num_splits <= 0 || !wavefronts || (D != 128 && D != 64)) return 0;
+  const DecodePlan plan = D == 128 ? plan_decode<128>(batch_heads, Lkv, num_splits) : plan_decode<64>(batch_heads, Lkv, num_splits);
+  *wavefronts = plan.waves;
+  return plan.splits;
+}
 
 extern "C" int tf_flash_decode_f16(const void* Q, const void* K, const void* V, void* O,
                                    void* workspace, size_t workspace_bytes, int64_t batch_heads,

@@ -906,3 +906,8 @@ extern "C" int tf_gemm(const void* A, const void* B, void* C, int dtype, int c_i
   if (c_is_f32) return dispatch<float, bf16_t>(A, B, C, (int)M, (int)N, (int)K, st);
   return dispatch<bf16_t, bf16_t>(A, B, C, (int)M, (int)N, (int)K, st);
 }
+
+extern "C" int tf_gemm_kernel_index(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0 || M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 22)) return -1;
+  return tfk::pick_gemm_kernel((int)M, (int)N, (int)K);
+}
