@@ -103,17 +103,17 @@ def test_scatter_nd_sums_beyond_the_range_of_the_type(dtype, big, slice_, n):
 @pytest.mark.parametrize("start", [0, 1, 2, 3])
 @pytest.mark.parametrize("slice_", [1, 3, 66, 131])
 @pytest.mark.parametrize("n", [2, 1500])
-@pytest.mark.parametrize("first,second", [(0, 4), (1, 3)])
-def test_scatter_nd_leaves_what_lies_next_to_a_slice_alone(dtype, bits, start, slice_, n, first, second):
+@pytest.mark.parametrize("rows_,first,second", [(5, 0, 4), (5, 1, 3), (6, 0, 5), (6, 2, 3)])   # odd and even totals
+def test_scatter_nd_leaves_what_lies_next_to_a_slice_alone(dtype, bits, start, slice_, n, rows_, first, second):
     from tilefusion_amd.ops import scatter_nd
     ints = torch.int32 if dtype == torch.float32 else torch.int16
-    buf = torch.full((start + 5 * slice_ + 3,), bits, dtype=ints, device=DEV)
-    inside = buf[start:start + 5 * slice_]
+    buf = torch.full((start + rows_ * slice_ + 3,), bits, dtype=ints, device=DEV)
+    inside = buf[start:start + rows_ * slice_]
     inside.fill_(1)
-    data = inside.view(dtype).view(5, slice_)
+    data = inside.view(dtype).view(rows_, slice_)
     data[first], data[second] = 1.0, 2.0
     want = buf.clone()
-    rows = want.view(dtype)[start:start + 5 * slice_].view(5, slice_)
+    rows = want.view(dtype)[start:start + rows_ * slice_].view(rows_, slice_)
     rows[first], rows[second] = 4.0, 6.0
     upd = torch.zeros(n, slice_, dtype=dtype, device=DEV)
     upd[0], upd[1] = 3.0, 4.0

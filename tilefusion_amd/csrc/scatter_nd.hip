@@ -32,6 +32,12 @@ struct Strides {
 
 constexpr int kScatterThreads = 256;
 
+// How the words of slices lie.  kPairs: every word holds elements of one slice (always so in fp32).  kSplit: 16-bit
+// slices of which a word may hold one half (an odd slice length or an odd start).  kSplitShared: as before, and
+// the first or the last word of `data` holds 16 bits that are not its own.  (That check in every atomic's
+// way costs up to 8%: 676 fp16 updates of 3755 into 82 rows 10.4 us and 11.3.)
+enum class Layout { kPairs, kSplit, kSplitShared };
+
 // One 32-bit word of a slice: an fp32 element or an aligned pair of 16-bit ones.
 template <typename T>
 struct Word {
@@ -83,10 +89,10 @@ TFK_DEVICE void atomic_add_word(T* p, const Word<T>& w) {
 }
 
 // The words of one slice's sum that a lane holds: loads and adds, and the atomics.
-template <typename T, bool kSplitPairs>
+template <typename T, Layout kLayout>
 TFK_DEVICE void add_word_of_slice(Word<T>& sum, const T* src, long long e0, long long slice) {
   constexpr int kElems = Word<T>::kElems;
-  if constexpr (kElems == 2 && !kSplitPairs) {
+  if constexpr (kElems == 2 && kLayout == Layout::kPairs) {
     typedef T t2 __attribute__((ext_vector_type(2)));
     if (e0 < slice) {
       const t2 x = *reinterpret_cast<const t2*>(src + e0);
@@ -99,13 +105,13 @@ TFK_DEVICE void add_word_of_slice(Word<T>& sum, const T* src, long long e0, long
       if (e0 + e >= 0 && e0 + e < slice) sum.v[e] += (float)src[e0 + e];
   }
 }
-// Adds word `w` at elements e0 .. of the slice at `dst`.  Of a word that the slice shares with memory outside the `total`
+// Adds word `w` at elements e0 .. of the slice at `dst`, the `at`-th element of `data`.  Of a word that the slice shares with memory outside the `total`
 // elements of `data` the other half keeps its bits, whatever they stand for: compare-and-swap.  Only the first
 // and the last word of `data` can be such; for every word that two slices share it would cost far too
 // much (2048 bf16 updates of 33 into 64 rows 8 us and 40, 30000 of 77 into 131072 rows 25 and 1260).
 // kAnyMemory: every element by compare-and-swap.
-template <typename T, bool kSplitPairs, bool kAnyMemory>
-TFK_DEVICE void add_to_slice(T* dst, const Word<T>& w, long long e0, long long slice, const T* data, long long total) {
+template <typename T, Layout kLayout, bool kAnyMemory>
+TFK_DEVICE void add_to_slice(T* dst, const Word<T>& w, long long e0, long long slice, long long at, long long total) {
   T* const word = dst + e0;
   if constexpr (kAnyMemory) {
 #pragma unroll
@@ -113,8 +119,8 @@ TFK_DEVICE void add_to_slice(T* dst, const Word<T>& w, long long e0, long long s
       if (e0 + e >= 0 && e0 + e < slice) atomic_add_element(word + e, w.v[e]);
     return;
   }
-  if constexpr (kSplitPairs) {
-    const int outside = word < data ? 0 : word + 1 >= data + total ? 1 : -1;   // element of the word that is not data's
+  if constexpr (kLayout == Layout::kSplitShared) {
+    const int outside = at + e0 < 0 ? 0 : at + e0 + 1 >= total ? 1 : -1;   // element of the word that is not data's
     if (outside >= 0) {
       atomic_add_element(word + (1 - outside), outside ? w.v[0] : w.v[1]);
       return;
@@ -122,23 +128,24 @@ TFK_DEVICE void add_to_slice(T* dst, const Word<T>& w, long long e0, long long s
   }
   atomic_add_word(word, w);
 }
-// with kSplitPairs a slice may start in the upper half of its first word
-template <typename T, bool kSplitPairs>
+// unless kPairs, a slice may start in the upper half of its first word
+template <typename T, Layout kLayout>
 TFK_DEVICE int first_word_shift(const T* dst) {
-  return kSplitPairs ? (int)((reinterpret_cast<size_t>(dst) / sizeof(T)) % Word<T>::kElems) : 0;
+  return kLayout != Layout::kPairs ? (int)((reinterpret_cast<size_t>(dst) / sizeof(T)) % Word<T>::kElems) : 0;
 }
 
 // Few updates: a group of `lanes` adjacent lanes (a power of two up to 64) per update, one word per
 // lane, no sort.  The call is then the latency of a load of the index, one of the update and an atomic.
 // kAnyMemory: `data` is not known to be ordinary memory of this device; any number of updates.
-template <typename T, bool kSplitPairs, bool kAnyMemory>
+template <typename T, Layout kLayout, bool kAnyMemory>
 __global__ __launch_bounds__(kScatterThreads) void scatter_nd_direct_kernel(
     const T* __restrict__ updates, T* __restrict__ data, const long long* __restrict__ indices, Strides s, long long n,
     int k, long long slice, long long total, int lanes) {
   constexpr int kElems = Word<T>::kElems;
   const int lane = threadIdx.x & (lanes - 1);
-  const long long rows_step = gridDim.x * (long long)(kScatterThreads / lanes);
-  for (long long row = blockIdx.x * (long long)(kScatterThreads / lanes) + threadIdx.x / lanes; row < n; row += rows_step) {
+  long long row = blockIdx.x * (long long)(kScatterThreads / lanes) + threadIdx.x / lanes;
+  if (row >= n) return;
+  do {
     bool inside = true;
     unsigned long long at = 0;
     for (int j = 0; j < k; ++j) {
@@ -148,23 +155,24 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_nd_direct_kernel(
     }
     if (!inside) continue;
     T* const dst = data + at;
-    const int shift = first_word_shift<T, kSplitPairs>(dst);
+    const int shift = first_word_shift<T, kLayout>(dst);
     const long long step = (long long)gridDim.y * lanes * kElems;
     for (long long e0 = ((long long)blockIdx.y * lanes + lane) * kElems - shift; e0 < slice; e0 += step) {
       Word<T> w;
 #pragma unroll
       for (int e = 0; e < kElems; ++e) w.v[e] = -0.f;
-      add_word_of_slice<T, kSplitPairs>(w, updates + row * slice, e0, slice);
-      add_to_slice<T, kSplitPairs, kAnyMemory>(dst, w, e0, slice, data, total);
+      add_word_of_slice<T, kLayout>(w, updates + row * slice, e0, slice);
+      add_to_slice<T, kLayout, kAnyMemory>(dst, w, e0, slice, at, total);
     }
-  }
+  } while (kAnyMemory && (row += gridDim.x * (long long)(kScatterThreads / lanes)) < n);
 }
 
 // Many updates: kRows per workgroup; a group of `lanes` adjacent lanes (a power of two up to 64) takes one
-// distinct row at a time, kWords words per lane.  kSplitPairs: 16-bit slices whose words are not
-// pairs of the slice (an odd slice length or an odd start); their halves are loaded one by one.
-template <typename T, int kThreads, int kRows, int kWords, bool kSplitPairs>
-__global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
+// distinct row at a time, kWords words per lane.  Unless kPairs, the halves of words are loaded one by one.
+// Scalar registers: with more than 80 a SIMD holds fewer than eight wavefronts, and of workgroups of sixteen a CU
+// then holds one instead of two (83: 16598 bf16 updates of 627 into 318 rows 53 us, 78: 35).
+template <typename T, int kThreads, int kRows, int kWords, Layout kLayout>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_sgpr(80))) void scatter_nd_kernel(
     const T* __restrict__ updates, T* __restrict__ data, const long long* __restrict__ indices, Strides s, long long n,
     int k, long long slice, long long total, int lanes) {
   static_assert((kRows % kWaveSize == 0 || kRows < kWaveSize) && kRows <= kThreads,
@@ -228,13 +236,13 @@ __global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
     __syncthreads();
 
     const int groups = kThreads / lanes, lane = tid & (lanes - 1);
-    const long long words = (slice + kElems - 1 + (kSplitPairs ? 1 : 0)) / kElems;
+    const long long words = (slice + kElems - 1 + (kLayout != Layout::kPairs ? 1 : 0)) / kElems;
     for (long long word0 = (long long)blockIdx.y * lanes * kWords + lane; word0 - lane < words;
          word0 += (long long)gridDim.y * lanes * kWords) {
       for (int g = tid / lanes; g < count; g += groups) {
         const int begin = s_first[g], end = s_first[g + 1];
         T* const dst = data + s_sorted[begin];
-        const int shift = first_word_shift<T, kSplitPairs>(dst);
+        const int shift = first_word_shift<T, kLayout>(dst);
         Word<T> sum[kWords];
 #pragma unroll
         for (int v = 0; v < kWords; ++v)
@@ -246,7 +254,7 @@ __global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
 #pragma unroll
           for (int v = 0; v < kWords; ++v) {
             const long long e0 = (word0 + (long long)v * lanes) * kElems - shift;
-            add_word_of_slice<T, kSplitPairs>(sum[v], src, e0, slice);
+            add_word_of_slice<T, kLayout>(sum[v], src, e0, slice);
           }
         }
 #pragma unroll
@@ -262,12 +270,12 @@ __global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
               Word<T> w;
 #pragma unroll
               for (int e = 0; e < kElems; ++e) w.v[e] = -0.f;
-              add_word_of_slice<T, kSplitPairs>(w, updates + (row0 + s_order[p]) * slice, e0, slice);
-              add_to_slice<T, kSplitPairs, false>(dst, w, e0, slice, data, total);
+              add_word_of_slice<T, kLayout>(w, updates + (row0 + s_order[p]) * slice, e0, slice);
+              add_to_slice<T, kLayout, false>(dst, w, e0, slice, (long long)s_sorted[begin], total);
             }
             continue;
           }
-          add_to_slice<T, kSplitPairs, false>(dst, sum[v], e0, slice, data, total);
+          add_to_slice<T, kLayout, false>(dst, sum[v], e0, slice, (long long)s_sorted[begin], total);
         }
       }
     }
@@ -275,25 +283,25 @@ __global__ __launch_bounds__(kThreads) void scatter_nd_kernel(
   }
 }
 
-template <typename T, int kThreads, int kRows, int kWords, bool kSplitPairs>
+template <typename T, int kThreads, int kRows, int kWords, Layout kLayout>
 int launch_shape(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
                  long long slice, long long total, int lanes, long long words, hipStream_t st) {
   const long long per = (long long)lanes * kWords;
   const dim3 grid((unsigned)std::min<long long>((n + kRows - 1) / kRows, 1 << 20),
                   (unsigned)std::min<long long>((words + per - 1) / per, 1024));
-  hipLaunchKernelGGL((scatter_nd_kernel<T, kThreads, kRows, kWords, kSplitPairs>), grid, dim3(kThreads), 0, st,
+  hipLaunchKernelGGL((scatter_nd_kernel<T, kThreads, kRows, kWords, kLayout>), grid, dim3(kThreads), 0, st,
                      static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
 
-template <typename T, bool kSplitPairs, bool kAnyMemory>
+template <typename T, Layout kLayout, bool kAnyMemory>
 int launch_direct(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
                   long long slice, long long total, int lanes, long long words, hipStream_t st) {
   const int per = kScatterThreads / lanes;
   const dim3 grid((unsigned)std::min<long long>((n + per - 1) / per, 1 << 20),
                   (unsigned)std::min<long long>((words + lanes - 1) / lanes, 1024));
-  hipLaunchKernelGGL((scatter_nd_direct_kernel<T, kSplitPairs, kAnyMemory>), grid, dim3(kScatterThreads), 0, st,
+  hipLaunchKernelGGL((scatter_nd_direct_kernel<T, kLayout, kAnyMemory>), grid, dim3(kScatterThreads), 0, st,
                      static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
@@ -311,28 +319,28 @@ bool is_ordinary_device_memory(const void* p) {
   return a.type == hipMemoryTypeDevice && !a.isManaged && a.device == device && a.allocationFlags == hipDeviceMallocDefault;
 }
 
-template <typename T, bool kSplitPairs>
+template <typename T, Layout kLayout>
 int launch_rows(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
                 long long slice, long long targets, int lanes, long long words, hipStream_t st) {
   if (!is_ordinary_device_memory(data))
-    return launch_direct<T, kSplitPairs, true>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+    return launch_direct<T, kLayout, true>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   // Times in us with log-uniform indices (threads / updates a workgroup).  Few updates: no sort (806 of
   // 34 fp32: direct 3.3, 256/16 5.6).  From 1024 on contention shows (2048 of 64 bf16 into 64 rows:
   // direct 10.8, 256/16 6.3, 512/64 8.2), beyond 2048 more updates per sort pay (4096 of 1024 bf16
   // into 1000 rows: direct 26, 256/16 17.6, 512/64 12.9).
   if (n <= 1024)
-    return launch_direct<T, kSplitPairs, false>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+    return launch_direct<T, kLayout, false>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   if (n <= 2048)
-    return launch_shape<T, 256, 16, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+    return launch_shape<T, 256, 16, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   // Every target hit at least eight times on average: the deeper sort (59764 of 21 fp32 into 219 rows:
   // 512/64 43, 1024/128 31; 49954 of 622 fp32 into 77: 175 and 143).
   if (n / 8 >= targets)
-    return launch_shape<T, 1024, 128, 2, kSplitPairs>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+    return launch_shape<T, 1024, 128, 2, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   // A workgroup of eight wavefronts hides its own latencies where there are few of them (16384 of 64
   // bf16: 256/64 13.8, 512/64 12.5); enough of four do it better (8192 of 1024 fp32: 31.9 and 40.1).
   if ((n / 64) * ((words + lanes - 1) / lanes) < 1024)
-    return launch_shape<T, 512, 64, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  return launch_shape<T, 256, 64, 1, kSplitPairs>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+    return launch_shape<T, 512, 64, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+  return launch_shape<T, 256, 64, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
 }
 
 template <typename T>
@@ -346,9 +354,12 @@ int launch(const void* updates, void* data, const long long* indices, const Stri
   int lanes = 1;
   while (lanes < kWaveSize && lanes < words) lanes *= 2;
   if constexpr (kElems == 2) {
-    if (!pairs) return launch_rows<T, true>(updates, data, indices, s, n, k, slice, targets, lanes, words, st);
+    const size_t first = reinterpret_cast<size_t>(data), behind = first + (size_t)(slice * targets) * sizeof(T);
+    if (!pairs && (first % 4 != 0 || behind % 4 != 0))
+      return launch_rows<T, Layout::kSplitShared>(updates, data, indices, s, n, k, slice, targets, lanes, words, st);
+    if (!pairs) return launch_rows<T, Layout::kSplit>(updates, data, indices, s, n, k, slice, targets, lanes, words, st);
   }
-  return launch_rows<T, false>(updates, data, indices, s, n, k, slice, targets, lanes, words, st);
+  return launch_rows<T, Layout::kPairs>(updates, data, indices, s, n, k, slice, targets, lanes, words, st);
 }
 
 }  // namespace
