@@ -109,7 +109,8 @@ def test_decode_plan():
     assert _plan(512, 32768, 128, 3) == (3, 4)       # the caller's limit
     assert _plan(512, 32768, 128, 1) == (1, 4)
     assert _plan(512, 8192, 128, 64) == (1, 4)       # 4 MiB a slice: not cut
-    assert _plan(256, 8193, 128, 64)[0] > 1          # beyond
+    assert _plan(768, 8193, 128, 64)[0] == 3         # beyond, and 2.75 GB together
+    assert _plan(512, 10000, 128, 64) == (1, 4)      # less together
     assert _plan(0, 64, 128, 4)[0] == 0 and _plan(4, 64, 96, 4)[0] == 0
     for bh, lkv, d, splits in [(1, 1, 64, 64), (3, 100000, 128, 5), (65535, 7, 64, 9), (40, 40000, 128, 65536)]:
         n, waves = _plan(bh, lkv, d, splits)

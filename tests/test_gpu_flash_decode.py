@@ -107,12 +107,12 @@ def test_c5_full_size():
 
 # The cut is the library's: one workgroup of 8 or (from 512 slices on) 4 wavefronts per slice and no
 # partials, or up to num_splits ranges reduced by workgroups of 8 (fewer than 1024 of them) or 4
-# wavefronts; slices of more than 4 MiB that would do without a cut come in ranges of 2 MiB.  Lengths around the
+# wavefronts; slices of more than 4 MiB, 2.75 GB together, come in ranges of 2 MiB in any case.  Lengths around the
 # rows of a load step (32 or 64) and of the two batches in flight.
 CUTS = [(3, 31, 128, 64), (3, 65, 64, 64), (513, 33, 128, 64), (520, 63, 64, 3),
         (600, 300, 64, 64), (4, 2047, 128, 64), (5, 4097, 64, 64),
         (2, 9000, 128, 2), (40, 6000, 64, 64), (270, 2100, 128, 9), (1, 1, 64, 2),
-        (136, 4099, 64, 64), (256, 8192, 128, 64), (256, 8193, 128, 64),
+        (136, 4099, 64, 64), (256, 8192, 128, 64), (256, 8193, 128, 64), (768, 8200, 128, 64),
         (250, 17001, 64, 2), (130, 16500, 64, 64)]
 
 

@@ -11,7 +11,7 @@
 //     its own running (max, sum, o[D]) over the rows it sees; the groups of a wavefront are merged with
 //     lane swaps, the wavefronts through LDS.  The dot product is v_dot2 (fp16 or bf16) +
 //     a DPP reduction inside the lane group;
-//     two batches of 4 rows per group are in flight (16 KiB per wavefront), the next one
+//     two batches of 4 or 6 rows per group are in flight (16 or 24 KiB per wavefront), the next one
 //     requested before the current one is consumed; the partials leave through streaming
 //     stores (ordinary stores in the middle of the read stream cost 7% of its bandwidth);
 //   * combine kernel: grid batch_heads, merges the fp32 partials.
@@ -28,9 +28,10 @@
 namespace tfk {
 namespace {
 
-// Rows per lane group in one batch of loads; two batches are in flight.  Eight instead of four took 214
-// registers and two wavefronts per SIMD (802 slices of 2574 x 128 in 4 splits: 171 us, with four 165).
-constexpr int kBatchRows = 4;
+// Rows per lane group in one batch of loads, of which up to two are in flight.  More cost registers and with them
+// wavefronts; six pay where a CU often has one workgroup only (fp16, four / six / eight rows: 157 slices of 6530 x 128
+// 84.1 / 79.9 / 79.9 us, 186 of 11138 x 128 160.9 / 152.1 / 151.6, 33 of 662 x 64 5.5 / 5.8 / 7.2).
+__host__ __device__ constexpr int batch_rows(int waves, bool whole) { return whole && waves == 8 ? 6 : 4; }
 using float2_t = float __attribute__((ext_vector_type(2)));
 
 constexpr int kD = 128;   // head dimension of the benchmark configuration (and of the static entry point)
@@ -124,6 +125,7 @@ __global__ __launch_bounds__(kDecWaves * kWaveSize) void flash_decode_split_kern
   constexpr int kLanesPerRow = D / 8;                   // 16-byte vectors per row
   constexpr int kRowsPerWave = kWaveSize / kLanesPerRow;  // rows one wavefront load instruction covers
   constexpr int kRowsPerStep = kDecWaves * kRowsPerWave;  // ... and one workgroup load step
+  constexpr int kBatchRows = batch_rows(kDecWaves, kWhole);
   __shared__ float s_o[kDecWaves][D];
   __shared__ float s_m[kDecWaves], s_l[kDecWaves];
 
@@ -144,44 +146,37 @@ __global__ __launch_bounds__(kDecWaves * kWaveSize) void flash_decode_split_kern
   // Two register sets of kBatchRows rows per group: the loads of batch b+1 are issued before
   // batch b is consumed, so a wavefront always has loads on their way (a load-all / wait-all /
   // compute loop leaves the memory pipe of that wavefront empty while it computes).
-  // `base` is workgroup-uniform.  A batch that lies inside the chunk is addressed as a scalar
-  // base plus one per-lane 32-bit offset computed once (no per-load 64-bit arithmetic, no
-  // clamps, no masks); only a batch that crosses the end of the chunk takes the clamped and
-  // masked form.
-  constexpr int64_t kBatchSpan = (int64_t)kBatchRows * kRowsPerStep;
-  const int64_t lane_row = wave * kRowsPerWave + gw;
-  const unsigned lane_off = (unsigned)(lane_row * D + 8 * lv) * 2u;   // bytes inside a batch
+  // The loop asks past the end of the range as well: the bounds check of a buffer load returns zeros there and
+  // fetches nothing.  (With a branch around the loads of a short batch the compiler waits for all loads
+  // in flight where its two ways meet.  Zeros, because the weight of such a row is zero, and zero
+  // times another row's infinity would be NaN.)
+  constexpr int kBatchSpan = kBatchRows * kRowsPerStep;
+  constexpr int kRowBytes = D * 2;
+  const int lane_row = wave * kRowsPerWave + gw;
+  unsigned lane_off[kBatchRows];   // bytes inside a batch
+#pragma unroll
+  for (int u = 0; u < kBatchRows; ++u) lane_off[u] = (unsigned)((lane_row + u * kRowsPerStep) * kRowBytes + 16 * lv);
   const char* k_slice = reinterpret_cast<const char*>(K + bh * Lkv * D);
   const char* v_slice = reinterpret_cast<const char*>(V + bh * Lkv * D);
+  auto rows_left = [&](int64_t base) __attribute__((always_inline)) {   // of a batch
+    return (int)max((int64_t)0, min((int64_t)kBatchSpan, row_end - base));
+  };
   auto load_batch = [&](V8* kd, V8* vd, int64_t base) __attribute__((always_inline)) {
-    if (base + kBatchSpan <= row_end) {
-      const char* kb = k_slice + base * (D * 2);
-      const char* vb = v_slice + base * (D * 2);
+    const unsigned bytes = (unsigned)rows_left(base) * kRowBytes;
 #pragma unroll
-      for (int u = 0; u < kBatchRows; ++u)
-        kd[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(kb + lane_off + u * (kRowsPerStep * D * 2)));
+    for (int u = 0; u < kBatchRows; ++u) kd[u] = load_below<V8>(k_slice + base * kRowBytes, bytes, lane_off[u]);
 #pragma unroll
-      for (int u = 0; u < kBatchRows; ++u)
-        vd[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(vb + lane_off + u * (kRowsPerStep * D * 2)));
-    } else {
-      // rows behind the end of the chunk come as zeros from the bounds check of a buffer load: their weight is
-      // zero, and zero times another row's infinity would be NaN
-      const unsigned left = (unsigned)((row_end - base) * (D * 2));
-#pragma unroll
-      for (int u = 0; u < kBatchRows; ++u) kd[u] = load_below<V8>(k_slice + base * (D * 2), left, lane_off + u * (kRowsPerStep * D * 2));
-#pragma unroll
-      for (int u = 0; u < kBatchRows; ++u) vd[u] = load_below<V8>(v_slice + base * (D * 2), left, lane_off + u * (kRowsPerStep * D * 2));
-    }
+    for (int u = 0; u < kBatchRows; ++u) vd[u] = load_below<V8>(v_slice + base * kRowBytes, bytes, lane_off[u]);
     __builtin_amdgcn_sched_barrier(0);   // the requests leave before the other batch is consumed
   };
   auto consume = [&](const V8* kd, const V8* vd, int64_t base) __attribute__((always_inline)) {
-    const bool full = base + kBatchSpan <= row_end;   // workgroup-uniform
+    const int left = rows_left(base) - lane_row;
     float s[kBatchRows];
     float mx = -INFINITY;
 #pragma unroll
     for (int u = 0; u < kBatchRows; ++u) {
       const float d = group_sum<kLanesPerRow>(dot8<T>(kd[u], q8)) * scale_log2;
-      s[u] = (full || base + lane_row + (int64_t)u * kRowsPerStep < row_end) ? d : -INFINITY;
+      s[u] = u * kRowsPerStep < left ? d : -INFINITY;
       mx = fmaxf(mx, s[u]);
     }
     const float m_new = fmaxf(m_run, mx);
@@ -201,15 +196,15 @@ __global__ __launch_bounds__(kDecWaves * kWaveSize) void flash_decode_split_kern
     __builtin_amdgcn_sched_barrier(0);
   };
   V8 k_a[kBatchRows], v_a[kBatchRows], k_b[kBatchRows], v_b[kBatchRows];
-  if (row_begin < row_end) load_batch(k_a, v_a, row_begin);
-  for (int64_t base = row_begin; base < row_end; base += 2 * kBatchSpan) {
-    const bool more1 = base + kBatchSpan < row_end;
-    if (more1) load_batch(k_b, v_b, base + kBatchSpan);
+  load_batch(k_a, v_a, row_begin);
+  int64_t base = row_begin;
+  for (; base + kBatchSpan < row_end; base += 2 * kBatchSpan) {
+    load_batch(k_b, v_b, base + kBatchSpan);
     consume(k_a, v_a, base);
-    if (!more1) break;
-    if (base + 2 * kBatchSpan < row_end) load_batch(k_a, v_a, base + 2 * kBatchSpan);
+    load_batch(k_a, v_a, base + 2 * kBatchSpan);
     consume(k_b, v_b, base + kBatchSpan);
   }
+  if (base < row_end) consume(k_a, v_a, base);
 
   // merge the lane groups of the wavefront, then the wavefronts
   const auto add = [](float a, float b) { return a + b; };
@@ -348,11 +343,12 @@ struct DecodePlan {
 // launch cost ~4 us.  Measured (fp16, us, one workgroup per slice / best split): 33 slices of 662 x 64
 // 6.5 / 8.1, 964 of 913 x 128 68 / 73, 11 of 825 x 128 10.4 / 8.5, 64 of 8192 x 128 85 / 44.  Slices that the
 // CUs cannot share evenly cost about a third of the unevenness (802 of 2574 x 128: 180 / 165).
-// Of a slice beyond 4 MiB one workgroup never gets far while all the others do the same: hundreds of streams,
-// megabytes apart, and a first pass over memory whose translations no cache holds yet pays for each (512 of
-// 32768 x 128: 1460-1500 us, in 8 ranges 1320-1370; 155 of 36332 x 128 636 / 569, 180 of 50000 x 128 886 / 807).
-// Passes after that take as long as with one workgroup per slice (1237 / 1235; over ten caches in turn too).
-// So such slices come in ranges of at most 2 MiB.  (512 of 8192 x 128, 4 MiB: first pass 375 whole and 384 cut.)
+// Where the slices are large and many, one workgroup in each means hundreds of streams, megabytes apart, and a first
+// pass over memory whose translations no cache holds yet pays for each (512 of 32768 x 128: 1460-1500 us, in 8
+// ranges 1320-1370; 155 of 36332 x 128 636 / 569, 180 of 50000 x 128 886 / 807).  Passes after that take as long
+// either way (512 of 32768 x 128 1237 / 1235, over ten caches in turn too).  So slices of more than 4 MiB, of
+// more than 2.75 GB together, come in ranges of at most 2 MiB.  (Below neither was ahead at first: 512 of 8192 x 128 375 whole
+// and 384 cut, 512 of 10000 x 128 484 and 491, 200 of 12000 x 128 246 and 242 - then 190 and 196.)
 // Otherwise the cut aims at 1024 workgroups, and at no more than 256 KiB of keys and values in each: they
 // come in rounds, and the last one fills the chip badly (584 of 16256 x 64: 4 splits 411, 16 364; 136 of
 // 36053 x 64: 8 splits 201, 32 192), but at 32 KiB at least (32 of 1999 x 64: 16 splits 10.2, 64 12.8),
@@ -366,7 +362,7 @@ DecodePlan plan_decode(int64_t batch_heads, int64_t Lkv, int num_splits) {
   // 32768 x 128: 1254 and 1203 us; 33 of 662 x 64: 6.5 and 8.1)
   const DecodePlan whole = {1, Lkv, batch_heads >= 512 ? 4 : 8};
   const bool shared_evenly = 2.5 + std::max(alone_us, stream_us * uneven) <= 6.5 + stream_us;
-  if (num_splits == 1 || (shared_evenly && slice_bytes <= 4194304.0)) return whole;
+  if (num_splits == 1 || (shared_evenly && (slice_bytes <= 4194304.0 || slice_bytes * batch_heads <= 2.75e9))) return whole;
   constexpr int64_t kStep = 8 * (kWaveSize / (D / 8));   // rows of one load step of the larger workgroup
   const int64_t fill = (1024 + batch_heads - 1) / batch_heads;
   const int64_t least = shared_evenly ? (int64_t)std::ceil(slice_bytes / 2097152.0) : (int64_t)(slice_bytes / 262144.0) + 1;
