@@ -86,11 +86,13 @@ def test_gemm_edge_cases_reach_every_kernel_of_the_table():
     from tests.test_gpu_gemm import EDGES
     lib = _capi.load()
     for kernel, problems in EDGES.items():
-        assert [lib.tf_gemm_kernel_index(*mnk) for mnk in problems] == [kernel] * len(problems)
+        assert [lib.tf_gemm_kernel_index(*mnk, 0) for mnk in problems] == [kernel] * len(problems)
     text = open(os.path.join(ROOT, "tilefusion_amd", "csrc", "gemm.hip")).read()
     table = re.search(r"constexpr GemmKernel kGemmKernels\[\] = \{\n(.*?)\n\};", text, re.S).group(1)
-    assert sorted(EDGES) == list(range(len(table.splitlines())))
-    assert lib.tf_gemm_kernel_index(0, 64, 64) == -1 and lib.tf_gemm_kernel_index(64, 64, 1 << 22) == -1
+    assert sorted(EDGES) == list(range(len(table.splitlines()) + 1))   # and the bounds-checked kernel
+    assert lib.tf_gemm_kernel_index(0, 64, 64, 0) == -1 and lib.tf_gemm_kernel_index(64, 64, 1 << 22, 0) == -1
+    # the grid of the bounds-checked kernel ends at 65535 columns of tiles
+    assert lib.tf_gemm_kernel_index(512, 65535 * 64, 8, 1) == 15 and lib.tf_gemm_kernel_index(512, 65535 * 64 + 1, 8, 1) != 15
 
 
 def _plan(bh, lkv, d, splits):

@@ -132,26 +132,31 @@ def test_identity_operand():
     assert torch.equal(c, b.T)
 
 
-# Ragged problems for every kernel and tile that the dispatch can pick (position in its table: m, n, k), at the
-# edges where each can go wrong: fewer rows or columns than a tile, a last tile that overlaps its neighbour
-# by all but one row, K that completes its first (ring kernels) or last (split-K kernels) 64-deep k-tile
-# with 8 to 56 zeros, fewer k-tiles than wavefronts.  Small integers: exact in fp32, whatever the order of the sums.
+# Ragged problems for every kernel and tile that the dispatch can pick (for a 16-bit result; position in its table: m, n,
+# k), at the edges where each can go wrong: fewer rows or columns than a tile, a last tile that overlaps its
+# neighbour by all but one row, K that completes its first (ring kernels) or last (split-K kernels)
+# 64-deep k-tile with 8 to 56 zeros, fewer k-tiles than wavefronts.  Small integers: exact in fp32, whatever the
+# order of the sums.
 EDGES = {
     0: [(1, 1, 8), (72, 1, 72), (17, 33, 8), (3, 577, 200)],                # 16 x 16, four wavefronts
     1: [(1, 264, 264), (15, 72, 4264), (33, 31, 1000), (44, 650, 1160)],    # 16 x 16, eight
     2: [(5390, 1, 200)],                                                    # 32 x 16
-    3: [(33, 4449, 72), (131, 1433, 64), (925, 768, 64), (129, 4095, 120), (128, 6400, 64)],   # 32 x 32, one
+    3: [(33, 4449, 72), (131, 1433, 64), (925, 768, 64), (129, 4095, 120), (128, 6400, 64), (65, 6209, 8),
+        (7000, 65, 24), (517, 3009, 64)],                                                    # 32 x 32, one
     4: [(17, 4561, 72), (257, 513, 328)],                                   # 32 x 32, four
     5: [(6426, 54, 4480), (165, 1765, 7616)],                               # 64 x 32
     6: [(3578, 101, 1000), (1088, 577, 1032), (50, 6432, 5688)],            # 64 x 64
     7: [(205, 5613, 1904)],                                                 # 128 x 128, requests four tiles ahead
-    8: [(4794, 235, 72), (2048, 2048, 136)],                                # 128 x 128, two ahead
-    9: [(4939, 3091, 80), (5216, 6236, 256)],                               # 128 x 128, two per CU
-    10: [(812, 4675, 72), (2999, 1544, 1032)],                              # 192 x 128
-    11: [(1398, 5437, 72)],                                                 # 192 x 192
-    12: [(982, 5472, 72), (3333, 2288, 1944)],                              # 256 x 128
-    13: [(4929, 1741, 72), (4097, 2305, 264)],                              # 256 x 192
-    14: [(4882, 2468, 72)],                                                 # 256 x 256
+    8: [(2048, 2048, 136), (2177, 513, 136), (4939, 3091, 80), (1398, 5437, 72), (4929, 1741, 72),
+        (4882, 2468, 72)],                                                  # 128 x 128, two ahead
+    9: [(5216, 6236, 256)],                                                 # 128 x 128, two per CU
+    10: [(2999, 1544, 1032), (2689, 1409, 136)],                            # 192 x 128
+    11: [(2305, 3265, 136), (1537, 4611, 152)],                             # 192 x 192
+    12: [(3333, 2288, 1944), (6145, 897, 144)],                             # 256 x 128
+    13: [(4097, 2305, 264), (5378, 1537, 144)],                             # 256 x 192
+    14: [(4865, 2305, 136), (2305, 4867, 136)],                             # 256 x 256
+    15: [(517, 3008, 64), (982, 5472, 72), (4097, 2305, 40), (3301, 2817, 8), (4794, 235, 72),
+         (812, 4675, 72)],                                                  # bounds-checked
 }
 
 
@@ -160,7 +165,7 @@ EDGES = {
 def test_every_kernel_at_its_edges_is_exact(kernel, m, n, k, dtype):
     from tilefusion_amd import _capi
     lib = _capi.load()
-    assert lib.tf_gemm_kernel_index(m, n, k) == kernel
+    assert lib.tf_gemm_kernel_index(m, n, k, 0) == kernel
     g = torch.Generator().manual_seed(m + n + k)
     a = torch.randint(-2, 3, (m, k), generator=g).to(dtype).to(DEV)
     b = torch.randint(-2, 3, (n, k), generator=g).to(dtype).to(DEV)

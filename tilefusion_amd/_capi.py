@@ -33,7 +33,7 @@ SIGNATURES = {
     "tf_flash_decode_static_prepare": (_i, []),
     "tf_flash_decode_static_f16": (_i, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _d, _vp]),
     "tf_scatter_nd": (_i, [_vp, _vp, _vp, ctypes.POINTER(_i64), _i, _i64, _i, _i, _vp]),
-    "tf_gemm_kernel_index": (_i, [_i64, _i64, _i64]),
+    "tf_gemm_kernel_index": (_i, [_i64, _i64, _i64, _i]),
     "tf_flash_decode_plan": (_i, [_i64, _i64, _i64, _i, ctypes.POINTER(_i)]),
     "tf_flash_attention_wide_rows": (_i, [_i64, _i64, _i]),
     "tf_jit_compile": (_i, [ctypes.c_char_p, ctypes.c_char_p, ctypes.POINTER(ctypes.c_char_p), _i,

@@ -678,7 +678,7 @@ int launch_split_k(const void* A, const void* B, void* C, int M, int N, int K, h
 }
 
 // ------------------------------------------------------------------------------------------
-// Operands that do not start at a 16-byte boundary: any M, N; K % 8 == 0.  Register-staged,
+// Operands that do not start at a 16-byte boundary, and short K with many outputs: any M, N; K % 8 == 0.  Register-staged,
 // bounds-checked, one LDS stage.
 // ------------------------------------------------------------------------------------------
 template <typename S, typename OutT, typename InT>
@@ -817,7 +817,54 @@ float expected_us(const GemmKernel& g, int64_t tiles, int ktiles, bool unaligned
   return g.start + std::max(rounds * chain * g.step, per_cu * ktiles * (g.shared + unaligned)) + per_cu * g.round;
 }
 
-int pick_gemm_kernel(int M, int N, int K) {
+// Up to K = 128 (16-bit results: 120) with many outputs, what counts is how C leaves, in which the table above does not go by the type (it was
+// fitted to 16-bit results), and the bounds-checked kernel is in the race: its k-tiles are 32 deep, and
+// several of its workgroups share a CU.  Microseconds, fitted to 521 problems (7 to 13% root mean square): start +
+// round per round of the chip + per tile of a CU: tile, depth a k-tile, wide for an fp32 result, odd_k where K is no
+// multiple of 64, odd_n where rows of C do not start at 16-byte boundaries.  Picks are 1.6% behind the best
+// of all kernels on average and 20% at most; those of the table above 8% and 83% (517 x 3008 x 64, fp32 result:
+// 128 x 128 ring 5.9 us, bounds-checked kernel 4.05; 1664 x 1472 x 64 6.2 and 4.8).
+struct ShortKKernel {
+  int index;                // into kGemmKernels; behind its end: the bounds-checked kernel
+  int bm, bn, k_tile;
+  float start, round, tile, depth, wide, odd_k, odd_n;
+};
+constexpr ShortKKernel kShortKKernels[] = {
+    {3, 32, 32, 64, 2.93f, 0.f, 0.163f, 0.064f, 0.070f, 0.f, 0.010f},
+    {8, 128, 128, 64, 3.34f, 1.31f, 0.303f, 0.415f, 1.54f, 0.178f, 0.277f},
+    {11, 192, 192, 64, 2.83f, 3.90f, 0.288f, 0.896f, 3.32f, 0.584f, 0.811f},
+    {12, 256, 128, 64, 2.54f, 3.80f, 0.153f, 0.853f, 3.18f, 0.559f, 0.640f},
+    {13, 256, 192, 64, 2.68f, 5.32f, 0.f, 1.262f, 4.89f, 0.768f, 0.871f},
+    {kNumGemmKernels, 64, 64, 32, 3.23f, 0.f, 0.254f, 0.168f, 0.296f, 0.f, 0.139f},
+};
+
+int pick_short_k_kernel(int M, int N, int K, bool c_is_f32) {
+  const int64_t row_bytes = (int64_t)N * (c_is_f32 ? 4 : 2);
+  int best = 3;
+  float best_us = INFINITY;
+#pragma unroll
+  for (const ShortKKernel& g : kShortKKernels) {
+    if (kGemmKernels[g.index % kNumGemmKernels].ring && (M < g.bm || N < g.bn || K < 64)) continue;
+    if (g.index == kNumGemmKernels) {
+      if (N > 65535 * 64) continue;   // its grid has columns of tiles in y
+      // Its tiles are 64 columns wide, so rows of C that are no whole 128-byte lines leave it in parts of lines, which
+      // costs from ~32 MiB of C on (5898 x 5498 x 64, fp32 result: 58 us, 128 x 128 ring 33; 8192 x 4160 x 64 33 and 36).
+      if (K >= 64 && row_bytes % 128 != 0 && M * row_bytes > (int64_t)32 << 20) continue;
+    }
+    const int64_t tiles = (int64_t)((M + g.bm - 1) / g.bm) * ((N + g.bn - 1) / g.bn);
+    const float per_tile = g.tile + (K + g.k_tile - 1) / g.k_tile * g.depth + (c_is_f32 ? g.wide : 0.f) +
+                           (K % 64 != 0 ? g.odd_k : 0.f) + (row_bytes % 16 != 0 ? g.odd_n : 0.f);
+    const float us = g.start + (tiles + 255) / 256 * g.round + tiles / 256.f * per_tile;
+    if (us < best_us) {
+      best = g.index;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+int pick_gemm_kernel(int M, int N, int K, bool c_is_f32) {
+  if (K <= (c_is_f32 ? 128 : 120) && (int64_t)((M + 63) / 64) * ((N + 63) / 64) >= 96) return pick_short_k_kernel(M, N, K, c_is_f32);
   int best = 0;
   float best_us = INFINITY;
   const int ktiles = (K + 63) / 64;
@@ -848,14 +895,15 @@ int dispatch(const void* A, const void* B, void* C, int M, int N, int K, hipStre
       launch_ring64<Ring64Shape<128, 128, 2>, OutT, InT>, launch_ring64<Ring64Shape<192, 128, 2>, OutT, InT>,
       launch_ring64<Ring64Shape<192, 192, 2>, OutT, InT>, launch_ring64<Ring64Shape<256, 128, 2>, OutT, InT>,
       launch_ring64<Ring64Shape<256, 192, 2>, OutT, InT>, launch_ring64<Ring64Shape<256, 256, 2>, OutT, InT>,
+      launch_guarded<ShapeSmall, OutT, InT>,
   };
-  static_assert(sizeof(kLaunchers) / sizeof(kLaunchers[0]) == kNumGemmKernels, "one launcher per row of kGemmKernels");
+  static_assert(sizeof(kLaunchers) / sizeof(kLaunchers[0]) == kNumGemmKernels + 1, "one launcher per row of kGemmKernels");
   // LDS-direct requests take 16 bytes at a 16-byte boundary.  (2^35 elements of C with a K below the ring
   // kernels' are more threads than a launch of the split-K kernels may have.)
   if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) % 16 != 0 ||
       (K < 64 && (int64_t)M * N >= (int64_t)1 << 35))
-    return launch_guarded<ShapeSmall, OutT, InT>(A, B, C, M, N, K, st);
-  return kLaunchers[pick_gemm_kernel(M, N, K)](A, B, C, M, N, K, st);
+    return kLaunchers[kNumGemmKernels](A, B, C, M, N, K, st);
+  return kLaunchers[pick_gemm_kernel(M, N, K, sizeof(OutT) == 4)](A, B, C, M, N, K, st);
 }
 
 }  // namespace
@@ -907,7 +955,7 @@ extern "C" int tf_gemm(const void* A, const void* B, void* C, int dtype, int c_i
   return dispatch<bf16_t, bf16_t>(A, B, C, (int)M, (int)N, (int)K, st);
 }
 
-extern "C" int tf_gemm_kernel_index(int64_t M, int64_t N, int64_t K) {
+extern "C" int tf_gemm_kernel_index(int64_t M, int64_t N, int64_t K, int c_is_f32) {
   if (M <= 0 || N <= 0 || K <= 0 || M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 22)) return -1;
-  return tfk::pick_gemm_kernel((int)M, (int)N, (int)K);
+  return tfk::pick_gemm_kernel((int)M, (int)N, (int)K, c_is_f32 != 0);
 }
