@@ -328,7 +328,7 @@ class Decode:
                           "softmax(qK^T)V per slice with K, V upcast per slice (value = sampled bytes / sampled time; "
                           "rate of the best and of the median slice beside it)" % len(idx)}
 
-    config = {"workload": "flash-decoding fp16 B=16 H=32 q_len=1 KV=32768 D=128, 64 splits + LSE combine (2 kernels per step)",
+    config = {"workload": "flash-decoding fp16 B=16 H=32 q_len=1 KV=32768 D=128, num_splits 64 (the library cuts each slice into 8 ranges) + LSE combine (2 kernels per step)",
               "inputs": "N(0,1) drawn on the device, seed 1005; 8 GiB of K,V (exceeds the last-level cache)"}
 
 

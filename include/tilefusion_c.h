@@ -127,9 +127,11 @@ TF_API int tf_flash_attention_fwd_wide(const void* Q, const void* K, const void*
                                        int64_t Lq, int64_t Lkv, int64_t D, double softmax_scale, int causal,
                                        void* stream);
 
-/* Single-query (decoding) attention with the KV range split into `num_splits` chunks:
- * kernel 1 writes per-split partial (o, max, sum) in fp32 into `workspace`, kernel 2 merges
- * them with a log-sum-exp weighted sum into O.
+/* Single-query (decoding) attention with the KV range cut into up to `num_splits` ranges:
+ * kernel 1 writes a partial (o, max, sum) per range in fp32 into `workspace`, kernel 2 merges
+ * them with a log-sum-exp weighted sum into O.  `num_splits` is an upper bound: the library takes fewer and
+ * longer ranges where that is sooner, or one (then kernel 1 writes O and there is no kernel 2); tf_flash_decode_plan
+ * tells.  The workspace always has to hold num_splits partials a slice.
  * Q [batch_heads, D]; K, V [batch_heads, Lkv, D]; O [batch_heads, D]; D must be 128 or 64.
  * All offsets are 64-bit (K alone has 2^31 elements at the benchmark size).
  * No counterpart in the reference (it has no decoding kernel); built on the same online
@@ -154,7 +156,7 @@ TF_API int tf_flash_decode(const void* Q, const void* K, const void* V, void* O,
  * owns `stream` must be current.  The first call on a device looks up the array's address there
  * (hipGetSymbolAddress, which may load the code object): make that first call - or
  * tf_flash_decode_static_prepare(), which does only the lookup for the current device - OUTSIDE any
- * stream capture; afterwards a call is two kernel launches and nothing else.  No call allocates or
+ * stream capture; afterwards a call is one or two kernel launches and nothing else.  No call allocates or
  * frees.  The array is part of the library's code object: every process that loads the library
  * holds it on every GPU it uses, whether or not it calls this entry point.  batch_heads * num_splits above
  * TF_FLASH_DECODE_STATIC_MAX_PARTIALS is rejected with TF_ERR_INVALID_ARG; D must be 128.  Same kernels and

@@ -141,3 +141,24 @@ def test_infinite_values_in_any_split_stay_infinite(bh, lkv, d, splits, dtype):
     want = torch.zeros(d, device=DEV)
     want[1], want[2], want[3] = math.inf, -math.inf, math.inf
     assert torch.equal(torch.where(o.isfinite(), torch.zeros_like(o), o).float(), want.expand(bh, d))
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, (1e-3, 2e-2)), (torch.bfloat16, (4e-3, 4e-2))])
+@pytest.mark.parametrize("start", [1, 2, 5])
+@pytest.mark.parametrize("bh,lkv,d,splits", [(5, 301, 128, 64), (5, 4097, 64, 64), (3, 2000, 128, 1)])
+def test_operands_that_start_anywhere(bh, lkv, d, splits, start, dtype, tol):
+    # operands at the alignment of their elements, between numbers that must not count
+    g = torch.Generator(device=DEV).manual_seed(start + lkv)
+
+    def inside(*shape):
+        n = math.prod(shape)
+        buf = torch.full((n + 16,), 100.0, device=DEV, dtype=dtype)
+        x = buf[start:start + n].view(*shape)
+        return x.copy_(torch.randn(*shape, device=DEV, generator=g))
+
+    q, k, v = inside(bh, d), inside(bh, lkv, d), inside(bh, lkv, d)
+    assert k.data_ptr() % 16 == start * 2
+    scores = (k.float() * q.float()[:, None]).sum(-1) / math.sqrt(d)
+    ref = (torch.softmax(scores, -1)[..., None] * v.float()).sum(1)
+    o = c_decode(q, k, v, splits)
+    assert N.rel_l2(o, ref) <= tol[0] and N.max_abs(o, ref) <= tol[1]

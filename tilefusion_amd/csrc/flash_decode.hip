@@ -463,7 +463,7 @@ extern "C" int tf_flash_decode(const void* Q, const void* K, const void* V, void
                                num_splits, softmax_scale, stream);
 }
 
-// ---- the same pair of kernels with the partials in a static device array -------------------
+// ---- the same kernels with the partials in a static device array -------------------
 //
 // For callers that cannot allocate device memory (code under HIP graph capture, tight serving
 // loops, harnesses that forbid hipMalloc): no workspace argument, nothing allocated.  Every GPU

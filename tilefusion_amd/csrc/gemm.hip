@@ -111,8 +111,8 @@ TFK_DEVICE float16_t mfma32_t(in8_t<InT> a, in8_t<InT> b, float16_t c) {
 // ------------------------------------------------------------------------------------------
 //
 // The same kernel serves smaller tiles (2 x 2 wavefronts of half a tile each way), for grids that 256 x 256
-// tiles would leave CUs idle on: 3333 x 2288 x 1944 takes 45.5 us with 126 tiles of 256 x 256 and 36.7 with
-// 216 of 192 x 192; 2999 x 1544 x 1032 27.6 and, with 192 x 128, 18.7 (the bounds-checked kernel that ran
+// tiles would leave CUs idle on: 3333 x 2288 x 1944 takes 45.5 us with 126 tiles of 256 x 256, 36.7 with
+// 216 of 192 x 192 and 36.4 with 252 of 256 x 128; 2999 x 1544 x 1032 27.6 and, with 192 x 128, 18.7 (the bounds-checked kernel that ran
 // these shapes before: 37.8).  Units then have the size of the larger operand.  128 x 128 tiles have k-steps
 // four times shorter; where a workgroup has its CU to itself their requests run kAhead = 4 tiles
 // ahead (a ring of 2 * kAhead + 1 = 9 units).

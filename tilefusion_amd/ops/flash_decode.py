@@ -17,8 +17,9 @@ def flash_decode(
 ) -> torch.Tensor:
     """Single-query attention: query [..., 1, D] or [..., D]; key, value [..., Lkv, D].
 
-    The key/value range is cut into `num_splits` chunks that are reduced independently and
-    merged by a log-sum-exp combine kernel.  Returns a tensor shaped like `query`."""
+    The key/value range is cut into at most `num_splits` ranges that are reduced independently and
+    merged by a log-sum-exp combine kernel; where one workgroup per slice is done sooner it is not
+    cut.  Returns a tensor shaped like `query`."""
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(query.size(-1))
     out = torch.empty_like(query)
