@@ -126,6 +126,13 @@ TF_API int tf_flash_attention_fwd(const void* Q, const void* K, const void* V, v
 TF_API int tf_flash_attention_fwd_wide(const void* Q, const void* K, const void* V, void* O, int dtype, int64_t batch,
                                        int64_t Lq, int64_t Lkv, int64_t D, double softmax_scale, int causal,
                                        void* stream);
+/* The tuned kernels for D == Dv == 128, 96 or 64 on a key stored [batch, D, Lkv] (what the reference's Python wrapper is
+ * called with, python/ops/flash_attention.py:64-74), V in its natural layout: bit for bit the results of
+ * tf_flash_attention_fwd on the transposed key.  Any Lq, Lkv % 8 == 0, operands at 16-byte boundaries, else
+ * TF_ERR_UNSUPPORTED. */
+TF_API int tf_flash_attention_fwd_kt(const void* Q, const void* K, const void* V, void* O, int dtype, int64_t batch,
+                                     int64_t Lq, int64_t Lkv, int64_t D, double softmax_scale, int causal,
+                                     void* stream);
 
 /* Single-query (decoding) attention with the KV range cut into up to `num_splits` ranges:
  * kernel 1 writes a partial (o, max, sum) per range in fp32 into `workspace`, kernel 2 merges

@@ -9,6 +9,7 @@ import torch
 import oracle
 from oracle import numerics as N
 from tests.gpu_util import DEV, c_attention
+from tilefusion_amd import ops
 
 pytestmark = pytest.mark.gpu
 
@@ -84,6 +85,25 @@ def test_causal_pairs_and_single_tiles_agree(bh, lq, d):
         assert torch.equal(o[i:i + 1], alone), i
     ok, r, m = N.check_close(o[-1:].cpu(), N.attention_ref(q[-1:].cpu(), k[-1:].cpu(), v[-1:].cpu(), causal=True))
     assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
+
+
+# A key stored [D, Lkv] is read as it is: the same products in the same order as on the transposed key, so the same
+# bits; a length that is no multiple of 8, or a key that starts off a 16-byte boundary, takes the copy.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [64, 96, 128])
+@pytest.mark.parametrize("lq,lkv", [(1, 8), (17, 72), (128, 64), (129, 128), (300, 200), (520, 520), (257, 333)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_key_stored_transposed(lq, lkv, d, causal, dtype):
+    q, k, v = (x.to(DEV, dtype) for x in _inputs(3, lq, lkv, d, lq + lkv + d))
+    kt = k.transpose(-1, -2).contiguous()
+    o = ops.flash_attention(q, kt, v, 1, 1, d, d, d ** -0.5, causal)
+    want = ops.flash_attention(q, k.transpose(-1, -2), v, 1, 1, d, d, d ** -0.5, causal)
+    assert torch.equal(o, want)
+    odd = torch.empty(kt.numel() + 1, device=DEV, dtype=dtype)[1:].view_as(kt).copy_(kt)
+    assert torch.equal(ops.flash_attention(q, odd, v, 1, 1, d, d, d ** -0.5, causal), want)
+    rel = 1e-3 if dtype == torch.float16 else 4e-3
+    ref = N.attention_ref(q.cpu(), k.cpu(), v.cpu(), causal=causal)
+    assert (o.float().cpu() - ref.float()).norm() <= rel * ref.float().norm()
 
 
 def test_scale_and_large_logits():

@@ -55,6 +55,10 @@ __host__ __device__ constexpr int swz_v(int row, int c) {
   if constexpr (CH >= 16) return c ^ ((row & 7) << 1);
   return c ^ (((row >> 1) & 3) << 1);
 }
+// K^T tile [D][64] read the same way, where the half wavefront's 8 rows are 0-3 and 8-11 (or 4-7 and 12-15) of 16.
+__host__ __device__ constexpr int swz_kt(int row, int c) {
+  return c ^ ((((row >> 1) & 1) | ((row >> 2) & 2)) << 1);
+}
 
 typedef __fp16 fp16x4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
 
@@ -151,7 +155,14 @@ TFK_DEVICE SplitWeight<T> split_weight(float p) {
 // of 1024 x 1024 x 256: 45 us without either, 51 with the remainder, 57 with the true maximum.
 // The scale is applied to the fp32 scores there: Q stays as it came, a second rounding of Q
 // would make a 16-bit result measurably worse.
-template <typename T, int D, int DV, bool kVT, bool kCausal, int kWavesT, int kQB>
+//
+// kKT: K comes as [D][Lkv].  Its tile keeps that layout in LDS ([D][kBN], 128-byte rows, as the V^T tile) and the
+// K fragments are transposed on their way to registers as those of V are: two ds_read_b64_tr_b16 for a
+// ds_read_b128, the same bytes.  Bound as the other instances are; the extra read instructions and their
+// addresses cost 0-12%, a transposed copy of K in front of the kernel costs more at every size (fp16, us, K
+// as [Lkv][D] / as [D][Lkv] / copied first: 64 slices of 4096 x 4096 x 128 444 / 449 / 534, causal 241 / 254 / 340; 16 of
+// 1024 x 1024 x 128 29 / 31 / 40; 32 of 100 x 8192 x 128 157 / 176 / 266; 64 of 1336 x 1336 x 64 causal 30 / 31 / 45).
+template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB>
 __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
     T* __restrict__ O, int Lq, int Lkv, float scale_log2, int q_tiles, int total_items, int paired) {
@@ -164,9 +175,10 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   constexpr int kRowsPerWave = 16 * kQB;  // kQB 16-query blocks per wavefront
   constexpr int kBMq = kWavesT * kRowsPerWave;
   constexpr int DP = lds_pitch(D), DVP = lds_pitch(DV);   // LDS row pitch of the K / natural V tile
-  constexpr int kKChunks = DP / 8;
+  static_assert(!kKT || !kWide, "K^T tiles are 64 keys wide");
+  constexpr int kKChunks = kKT ? kBN / 8 : DP / 8;
   constexpr int kVChunks = kVT ? kBN / 8 : DVP / 8;
-  constexpr int kKBytes = kBN * DP * 2;
+  constexpr int kKBytes = kKT ? D * kBN * 2 : kBN * DP * 2;
   constexpr int kVBytes = kVT ? DV * kBN * 2 : kBN * DVP * 2;
   constexpr int kStageBytes = kKBytes + kVBytes;
   constexpr int kKB = kBN / 16;   // 16-key blocks per tile (rows of S^T)
@@ -260,12 +272,15 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   unsigned req_off[kLoadsPerTile];   // per-lane byte offset inside the tile (global side)
   unsigned req_lds[kLoadsPerTile];   // wave-uniform byte offset inside the stage (LDS side)
 #pragma unroll
-  for (int t = 0; t < kKPerWave; ++t) {  // K tile: [kBN][D]
+  for (int t = 0; t < kKPerWave; ++t) {
     const int i = (wave + kWavesT * t) % kKInstr;
     constexpr int kRowsPerInstr = 64 / kKChunks;
     const int row = i * kRowsPerInstr + lane / kKChunks;
-    // (a physical chunk whose logical chunk lies beyond D is never read: it re-fetches the last one)
-    req_off[t] = (unsigned)(row * D + min(swz_k<kKChunks>(row, lane % kKChunks), D / 8 - 1) * 8) * 2u;
+    if constexpr (kKT)  // K^T tile: [D][kBN] out of a [D][Lkv] matrix
+      req_off[t] = ((unsigned)row * (unsigned)Lkv + swz_kt(row, lane % kKChunks) * 8) * 2u;
+    else                // K tile: [kBN][D]
+      // (a physical chunk whose logical chunk lies beyond D is never read: it re-fetches the last one)
+      req_off[t] = (unsigned)(row * D + min(swz_k<kKChunks>(row, lane % kKChunks), D / 8 - 1) * 8) * 2u;
     req_lds[t] = i * 1024;
   }
 #pragma unroll
@@ -283,7 +298,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     const int n0 = min(tile, num_tiles - 1) * kBN;  // clamped past the end (never read)
     const unsigned dst = smem_base + (tile % kStages) * kStageBytes + req_lds[r];
     if (n0 + kBN <= Lkv) {
-      const char* base = r < kKPerWave ? reinterpret_cast<const char*>(K + (size_t)n0 * D)
+      const char* base = r < kKPerWave ? reinterpret_cast<const char*>(K + (size_t)n0 * (kKT ? 1 : D))
                          : kVT         ? reinterpret_cast<const char*>(V + n0)
                                        : reinterpret_cast<const char*>(V + (size_t)n0 * DV);
       // the LDS destination is an M0 INPUT of the statement: the compiler writes M0 itself and
@@ -299,9 +314,14 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
       const int i = (wave + kWavesT * r) % kKInstr;
       constexpr int kRowsPerInstr = 64 / kKChunks;
       const int row = i * kRowsPerInstr + lane / kKChunks;
-      const int cc = min(swz_k<kKChunks>(row, lane % kKChunks), D / 8 - 1);
-      const int gr = min(n0 + row, Lkv - 1);
-      lds_dma_16B(K + (size_t)gr * D + cc * 8, dst);
+      if constexpr (kKT) {
+        const int gc = min(n0 + swz_kt(row, lane % kKChunks) * 8, Lkv - 8);
+        lds_dma_16B(K + (size_t)row * Lkv + gc, dst);
+      } else {
+        const int cc = min(swz_k<kKChunks>(row, lane % kKChunks), D / 8 - 1);
+        const int gr = min(n0 + row, Lkv - 1);
+        lds_dma_16B(K + (size_t)gr * D + cc * 8, dst);
+      }
     } else {
       const int i = (wave + kWavesT * (r - kKPerWave)) % kVInstr;
       constexpr int kRowsPerInstr = 64 / kVChunks;
@@ -324,7 +344,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   // cycles per request with the pipe idle.
   auto issue_request_lean = [&](int tile, int r) __attribute__((always_inline)) {
     const unsigned dst = smem_base + (tile % kStages) * kStageBytes + req_lds[r];
-    const char* base = r < kKPerWave ? reinterpret_cast<const char*>(K) + (size_t)tile * (kBN * D * 2)
+    const char* base = r < kKPerWave ? reinterpret_cast<const char*>(K) + (size_t)tile * (kBN * (kKT ? 1 : D) * 2)
                        : kVT         ? reinterpret_cast<const char*>(V) + (size_t)tile * (kBN * 2)
                                      : reinterpret_cast<const char*>(V) + (size_t)tile * (kBN * DV * 2);
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
@@ -342,9 +362,21 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   // swizzles only XOR lane-dependent bits into the chunk index, so the lane part is computed
   // once here and the tile loop spends no VALU on addresses beyond adding the stage base.
   //   K fragment (kb, kk) - A operand, 16 keys x 32 dims: row 16*kb + lr, logical chunk 4*kk + lg.
-  unsigned k_off[kKK];
+  //     K kept [dim][key]: rows 32*kk + 8*lg (+4) .. +3, columns 16*kb .. +15, transposed by the read; lane r of
+  //     a 16-lane group addresses row r/4, columns 4*(r%4) .. +3 of that block.  The lane part is kept per kb.
+  constexpr int kKOffs = kKT ? kKB : kKK;
+  unsigned k_off[kKOffs];
+  if constexpr (kKT) {
+    const int row_l = 8 * lg + (lr >> 2);
 #pragma unroll
-  for (int kk = 0; kk < kKK; ++kk) k_off[kk] = lr * DP * 2 + swz_k<kKChunks>(lr, 4 * kk + lg) * 16;
+    for (int kb = 0; kb < kKB; ++kb) {
+      const int col = kb * 16 + 4 * (lr & 3);
+      k_off[kb] = row_l * kBN * 2 + swz_kt(row_l, col / 8) * 16 + (col % 8) * 2;
+    }
+  } else {
+#pragma unroll
+    for (int kk = 0; kk < kKK; ++kk) k_off[kk] = lr * DP * 2 + swz_k<kKChunks>(lr, 4 * kk + lg) * 16;
+  }
   //   Reduction step j of the second product covers keys 32*j .. +31; slot t of lane group lg
   //   is key 32*j + 4*lg + t (t < 4) or 32*j + 16 + 4*lg + (t - 4): exactly the keys whose
   //   scores the lane already holds in its accumulators of key blocks 2*j and 2*j + 1.
@@ -405,10 +437,28 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   constexpr int kKAhead = kWide ? 2 : 1;
   V8 kf[kKAhead + 1][kKB];   // K fragments of reduction step kk (buffer kk % (kKAhead + 1))
   V8 vf[2][kDB];   // V fragments of reduction step j (buffer j & 1)
-  auto k_reads = [&](int buf, int it, int kk) __attribute__((always_inline)) {
-    const unsigned ka = opaque(smem_base + (it % kStages) * kStageBytes + k_off[kk]);
+  // lane address of the fragments of step kk (kKT: recomputed per fragment)
+  auto k_addr = [&](int it, int kk) __attribute__((always_inline)) {
+    const unsigned stage_base = smem_base + (it % kStages) * kStageBytes;
+    return kKT ? stage_base : opaque(stage_base + k_off[kk]);
+  };
+  auto k_read = [&](int buf, unsigned ka, int kk, int kb) __attribute__((always_inline)) {
+    if constexpr (kKT) {
+      const unsigned a = opaque(ka + k_off[kb]) + 32 * kk * kBN * 2;
+      const V4 lo = lds_read_tr4<V4>(a), hi = lds_read_tr4<V4>(a + 4 * kBN * 2);
 #pragma unroll
-    for (int kb = 0; kb < kKB; ++kb) kf[buf][kb] = lds_read_b128<V8>(ka + kb * 16 * DP * 2);
+      for (int t = 0; t < 4; ++t) {
+        kf[buf][kb][t] = lo[t];
+        kf[buf][kb][4 + t] = hi[t];
+      }
+    } else {
+      kf[buf][kb] = lds_read_b128<V8>(ka + kb * 16 * DP * 2);
+    }
+  };
+  auto k_reads = [&](int buf, int it, int kk) __attribute__((always_inline)) {
+    const unsigned ka = k_addr(it, kk);
+#pragma unroll
+    for (int kb = 0; kb < kKB; ++kb) k_read(buf, ka, kk, kb);
   };
   auto first_k_reads = [&](int it) __attribute__((always_inline)) {
 #pragma unroll
@@ -457,13 +507,13 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
 #pragma unroll
     for (int kk = 0; kk < kKK; ++kk) {
       const int next = kk + kKAhead;
-      const unsigned ka = next < kKK ? opaque(smem_base + (it % kStages) * kStageBytes + k_off[next < kKK ? next : 0]) : 0u;
+      const unsigned ka = next < kKK ? k_addr(it, next < kKK ? next : 0) : 0u;
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int kb = 0; kb < kKB; ++kb) {
 #pragma unroll
         for (int qb = 0; qb < kQB; ++qb) s[kb][qb] = mfma_t<T>(kf[kk % (kKAhead + 1)][kb], qf[kk][qb], s[kb][qb]);
-        if (next < kKK) kf[next % (kKAhead + 1)][kb] = lds_read_b128<V8>(ka + kb * 16 * DP * 2);
+        if (next < kKK) k_read(next % (kKAhead + 1), ka, next, kb);
         if constexpr (kWide) {
 #pragma unroll
           for (int db = 0; db < kDB; ++db)
@@ -772,12 +822,12 @@ inline bool pair_query_tiles(int64_t q_tiles, int64_t batch) {
   return paired <= 1.04 * single;
 }
 
-template <typename T, int D, int DV, bool kVT, bool kCausal, int kWavesT, int kQB>
+template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB>
 int launch_w(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv,
              float scale_log2, hipStream_t st) {
-  auto kern = flash_attention_fwd_kernel<T, D, DV, kVT, kCausal, kWavesT, kQB>;
+  auto kern = flash_attention_fwd_kernel<T, D, DV, kKT, kVT, kCausal, kWavesT, kQB>;
   constexpr int kBN = key_tile(D);
-  constexpr int lds = ring_stages(kWavesT) * (kBN * lds_pitch(D) * 2 + (kVT ? DV * kBN * 2 : kBN * lds_pitch(DV) * 2));
+  constexpr int lds = ring_stages(kWavesT) * (kBN * (kKT ? D : lds_pitch(D)) * 2 + (kVT ? DV * kBN * 2 : kBN * lds_pitch(DV) * 2));
   static_assert(lds <= kMaxLdsBytes, "tiles do not fit in LDS");
   TFK_LDS_OPT_IN(kern, lds);
   constexpr int bm = kWavesT * 16 * kQB;
@@ -793,11 +843,11 @@ int launch_w(const void* Q, const void* K, const void* V, void* O, int batch, in
   return TF_OK;
 }
 
-template <typename T, int D, int DV, bool kVT, bool kCausal>
+template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal>
 int launch(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv,
            float scale_log2, hipStream_t st) {
-  if (Lq > 128) return launch_w<T, D, DV, kVT, kCausal, 8, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
-  return launch_w<T, D, DV, kVT, kCausal, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+  if (Lq > 128) return launch_w<T, D, DV, kKT, kVT, kCausal, 8, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+  return launch_w<T, D, DV, kKT, kVT, kCausal, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
 }
 
 // Head dimensions above 128 (V as it comes, whole key tiles): 64 or 128 queries a workgroup, the larger one
@@ -818,11 +868,11 @@ int launch_wide(const void* Q, const void* K, const void* V, void* O, int batch,
                 bool causal, hipStream_t st) {
   const bool wide_tile = wide_takes_128_queries(batch, Lq, causal);
   if (causal) {
-    if (wide_tile) return launch_w<T, D, D, false, true, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
-    return launch_w<T, D, D, false, true, 4, 1>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+    if (wide_tile) return launch_w<T, D, D, false, false, true, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+    return launch_w<T, D, D, false, false, true, 4, 1>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
   }
-  if (wide_tile) return launch_w<T, D, D, false, false, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
-  return launch_w<T, D, D, false, false, 4, 1>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+  if (wide_tile) return launch_w<T, D, D, false, false, false, 4, 2>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+  return launch_w<T, D, D, false, false, false, 4, 1>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
 }
 
 template <typename T>
@@ -837,11 +887,25 @@ template <typename T, int D, int DV>
 int pick(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv,
          float scale_log2, bool vt, bool causal, hipStream_t st) {
   if (vt) {
-    if (causal) return launch<T, D, DV, true, true>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
-    return launch<T, D, DV, true, false>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+    if (causal) return launch<T, D, DV, false, true, true>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+    return launch<T, D, DV, false, true, false>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
   }
-  if (causal) return launch<T, D, DV, false, true>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
-  return launch<T, D, DV, false, false>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+  if (causal) return launch<T, D, DV, false, false, true>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+  return launch<T, D, DV, false, false, false>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+}
+
+// K as [D][Lkv], V as it comes
+template <typename T>
+int pick_kt(const void* Q, const void* K, const void* V, void* O, int batch, int Lq, int Lkv, int D,
+            float scale_log2, bool causal, hipStream_t st) {
+  auto run = [&](auto d) -> int {
+    constexpr int kD = decltype(d)::value;
+    if (causal) return launch<T, kD, kD, true, false, true>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+    return launch<T, kD, kD, true, false, false>(Q, K, V, O, batch, Lq, Lkv, scale_log2, st);
+  };
+  if (D == 128) return run(std::integral_constant<int, 128>{});
+  if (D == 96) return run(std::integral_constant<int, 96>{});
+  return run(std::integral_constant<int, 64>{});
 }
 
 }  // namespace
@@ -962,6 +1026,28 @@ extern "C" int tf_flash_attention_fwd_wide(const void* Q, const void* K, const v
   if (dtype == TF_DTYPE_BF16)
     return pick_wide<bf16_t>(Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, scale_log2, causal != 0, st);
   return pick_wide<half_t>(Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, scale_log2, causal != 0, st);
+}
+
+extern "C" int tf_flash_attention_fwd_kt(const void* Q, const void* K, const void* V, void* O, int dtype,
+                                         int64_t batch, int64_t Lq, int64_t Lkv, int64_t D, double softmax_scale,
+                                         int causal, void* stream) {
+  using namespace tfk;
+  if (int rc = check_attention_args("tf_flash_attention_fwd_kt", Q, K, V, O, batch, Lq, Lkv, D, D, 1, 1, 1, 1,
+                                    softmax_scale))
+    return rc;
+  TFK_REQUIRE(dtype == TF_DTYPE_F16 || dtype == TF_DTYPE_BF16, TF_ERR_UNSUPPORTED,
+              "tf_flash_attention_fwd_kt: dtype must be TF_DTYPE_F16 or TF_DTYPE_BF16");
+  TFK_REQUIRE((D == 64 || D == 96 || D == 128) && Lkv % 8 == 0, TF_ERR_UNSUPPORTED,
+              "tf_flash_attention_fwd_kt: needs a head dimension of 64, 96 or 128 and Lkv %% 8 == 0 "
+              "(got D=%lld Lkv=%lld)", (long long)D, (long long)Lkv);
+  TFK_REQUIRE((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V) |
+               reinterpret_cast<uintptr_t>(O)) % 16 == 0, TF_ERR_UNSUPPORTED,
+              "tf_flash_attention_fwd_kt: operands must start at a 16-byte boundary");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const float scale_log2 = (float)(softmax_scale * 1.4426950408889634);
+  if (dtype == TF_DTYPE_BF16)
+    return pick_kt<bf16_t>(Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, scale_log2, causal != 0, st);
+  return pick_kt<half_t>(Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, scale_log2, causal != 0, st);
 }
 
 extern "C" int tf_flash_attention_wide_rows(int64_t batch, int64_t Lq, int causal) {

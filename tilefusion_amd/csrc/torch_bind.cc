@@ -1,5 +1,5 @@
 // PyTorch operator bindings: registers torch.ops.tilefusion.{gemm, fused_two_gemms,
-// flash_attention, flash_attention_fwd, flash_decode} for the CUDA dispatch key (HIP tensors
+// flash_attention, flash_attention_fwd, flash_attention_fwd_kt, flash_decode} for the CUDA dispatch key (HIP tensors
 // are "cuda" tensors on PyTorch-ROCm) and forwards to the C ABI in tilefusion_c.h on the
 // caller's current stream.
 //
@@ -157,7 +157,7 @@ TILEFUSION_EXPORT void fused_two_gemms(const at::Tensor& A, const at::Tensor& B,
 
 namespace {
 void attention_impl(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& V, at::Tensor& O,
-                    bool v_transposed, int64_t tq, int64_t tkv, int64_t thqk, int64_t thv,
+                    bool k_transposed, bool v_transposed, int64_t tq, int64_t tkv, int64_t thqk, int64_t thv,
                     double softmax_scale, bool causal, const char* op) {
   CHECK_INPUT(Q);
   CHECK_INPUT(K);
@@ -170,15 +170,29 @@ void attention_impl(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& 
   TORCH_CHECK(Q.dim() >= 2 && Q.dim() == K.dim() && Q.dim() == V.dim() && Q.dim() == O.dim(),
               op, " expects tensors of equal rank >= 2.");
   const int64_t batch = leading_numel(Q, 2);
-  const int64_t lq = Q.size(-2), d = Q.size(-1), lkv = K.size(-2);
+  const int64_t lq = Q.size(-2), d = Q.size(-1), lkv = k_transposed ? K.size(-1) : K.size(-2);
   const int64_t dv = v_transposed ? V.size(-2) : V.size(-1);
   const int64_t v_len = v_transposed ? V.size(-1) : V.size(-2);
-  TORCH_CHECK(K.size(-1) == d, "K must be [Lkv, D].");
+  TORCH_CHECK((k_transposed ? K.size(-2) : K.size(-1)) == d, k_transposed ? "K must be [D, Lkv]." : "K must be [Lkv, D].");
   TORCH_CHECK(v_len == lkv, "V does not match the key length.");
   TORCH_CHECK(O.size(-2) == lq && O.size(-1) == dv, "O must be [Lq, Dv].");
   TORCH_CHECK(leading_numel(K, 2) == batch && leading_numel(V, 2) == batch &&
                   leading_numel(O, 2) == batch,
               "batch dimensions must match.");
+  // K as [D, Lkv]: read as it is where a kernel takes it, otherwise made [Lkv, D] first.
+  if (k_transposed) {
+    if (!v_transposed && d == dv) {
+      const int status = tf_flash_attention_fwd_kt(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dtype, batch,
+                                                   lq, lkv, d, softmax_scale, causal ? 1 : 0, current_stream());
+      if (status != TF_ERR_UNSUPPORTED) {
+        check_status(status, op);
+        return;
+      }
+    }
+    attention_impl(Q, K.transpose(-1, -2).contiguous(), V, O, false, v_transposed, tq, tkv, thqk, thv, softmax_scale,
+                   causal, op);
+    return;
+  }
   // Head dimensions up to 128 without a tuned kernel are zero-padded to the next tuned size (64,
   // 96 or 128): zeros change neither the scores nor the kept output columns, and the tuned kernel
   // on the padded problem is well ahead of the header kernel compiled at run time on the exact
@@ -251,14 +265,20 @@ void attention_impl(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& 
 TILEFUSION_EXPORT void flash_attention(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& V, at::Tensor& O,
                      int64_t tile_length_q, int64_t tile_length_kv, int64_t tile_hidden_qk,
                      int64_t tile_hidden_v, double softmax_scale, bool causal) {
-  attention_impl(Q, K, V, O, true, tile_length_q, tile_length_kv, tile_hidden_qk, tile_hidden_v,
+  attention_impl(Q, K, V, O, false, true, tile_length_q, tile_length_kv, tile_hidden_qk, tile_hidden_v,
                  softmax_scale, causal, "flash_attention");
 }
 
 // flash_attention_fwd: same computation with V in its natural [.., Lkv, Dv] layout.
 void flash_attention_fwd(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& V,
                          at::Tensor& O, double softmax_scale, bool causal) {
-  attention_impl(Q, K, V, O, false, 1, 1, 1, 1, softmax_scale, causal, "flash_attention_fwd");
+  attention_impl(Q, K, V, O, false, false, 1, 1, 1, 1, softmax_scale, causal, "flash_attention_fwd");
+}
+
+// flash_attention_fwd_kt: the same with K as [.., D, Lkv], the layout the Python wrapper is called with.
+void flash_attention_fwd_kt(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& V,
+                            at::Tensor& O, double softmax_scale, bool causal) {
+  attention_impl(Q, K, V, O, true, false, 1, 1, 1, 1, softmax_scale, causal, "flash_attention_fwd_kt");
 }
 
 // flash_decode(Q [.., D], K [.., Lkv, D], V [.., Lkv, D], O [.., D]); the fp32 split-KV
@@ -369,6 +389,10 @@ REGISTER_OP(flash_attention_fwd,
             "flash_attention_fwd(Tensor Q, Tensor K, Tensor V, Tensor(a!) O, "
             "float softmax_scale, bool causal) -> ()",
             &kernels::flash_attention_fwd);
+REGISTER_OP(flash_attention_fwd_kt,
+            "flash_attention_fwd_kt(Tensor Q, Tensor K, Tensor V, Tensor(a!) O, "
+            "float softmax_scale, bool causal) -> ()",
+            &kernels::flash_attention_fwd_kt);
 REGISTER_OP(flash_decode,
             "flash_decode(Tensor Q, Tensor K, Tensor V, Tensor(a!) O, "
             "int num_splits, float softmax_scale) -> ()",

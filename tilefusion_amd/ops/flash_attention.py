@@ -29,9 +29,9 @@ class FlashAttention:
         tests/python/test_flash_attn.py:173-175), value [..., Lkv, Dv] -> [..., Lq, Dv].
 
         The reference transposes both key and value before its op
-        (python/ops/flash_attention.py:73-74); here only the key is made [Lkv, D]-contiguous
-        and the value is consumed in its natural layout (the kernel transposes it on the way
-        from LDS to registers).  Tile sizes are validated against the problem."""
+        (python/ops/flash_attention.py:73-74); here the value is consumed in its natural layout, and
+        the key either as a transposed view of a [Lkv, D] tensor or stored [D, Lkv] (the kernel
+        transposes both on the way from LDS to registers).  Tile sizes are validated against the problem."""
         length_q, hidden_qk = query.size(-2), query.size(-1)
         length_kv, hidden_v = value.size(-2), value.size(-1)
         for what, dim, tile in (("length_q", length_q, self.tile_length_q),
@@ -41,9 +41,15 @@ class FlashAttention:
             if tile <= 0 or dim % tile != 0:
                 raise RuntimeError(f"tile size {tile} does not divide {what} = {dim}")
         output = torch.empty(*query.shape[:-1], hidden_v, dtype=query.dtype, device=query.device)
+        key_rows = key.transpose(-1, -2)
+        if key.is_contiguous() and not key_rows.is_contiguous():
+            torch.ops.tilefusion.flash_attention_fwd_kt(
+                query.contiguous(), key, value.contiguous(), output, self.softmax_scale, self.causal
+            )
+            return output
         torch.ops.tilefusion.flash_attention_fwd(
             query.contiguous(),
-            key.transpose(-1, -2).contiguous(),
+            key_rows.contiguous(),
             value.contiguous(),
             output,
             self.softmax_scale,
