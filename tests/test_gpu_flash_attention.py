@@ -9,7 +9,7 @@ import torch
 import oracle
 from oracle import numerics as N
 from tests.gpu_util import DEV, c_attention
-from tilefusion_amd import ops
+from tilefusion_amd import _capi, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -104,6 +104,27 @@ def test_key_stored_transposed(lq, lkv, d, causal, dtype):
     rel = 1e-3 if dtype == torch.float16 else 4e-3
     ref = N.attention_ref(q.cpu(), k.cpu(), v.cpu(), causal=causal)
     assert (o.float().cpu() - ref.float()).norm() <= rel * ref.float().norm()
+
+
+# The three workgroup sizes (256, 128, 64 query rows), at remainders of their tiles and of the key tiles, with all
+# orders of K and V; the library's pick is checked with them.
+@pytest.mark.parametrize("rows,b,lq,lkv,d", [
+    (64, 2, 1, 8, 64), (64, 3, 63, 200, 96), (64, 2, 65, 64, 128), (64, 5, 257, 136, 64), (64, 3, 300, 328, 128),
+    (128, 250, 128, 72, 64), (128, 130, 128, 192, 96), (128, 128, 129, 264, 128), (128, 64, 449, 448, 128),
+    (128, 300, 70, 128, 64), (256, 256, 200, 200, 128), (256, 512, 513, 72, 64), (256, 256, 250, 320, 96)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_every_workgroup_size(rows, b, lq, lkv, d, causal):
+    if not causal:
+        assert _capi.load().tf_flash_attention_rows(b, lq, lkv, d, 0) == rows
+    q, k, v = _inputs(b, lq, lkv, d, rows + lq + lkv)
+    o = c_attention(q.to(DEV), k.to(DEV), v.to(DEV), causal)
+    pick = [0, b // 2, b - 1]
+    ok, r, m = N.check_close(o[pick], N.attention_ref(q[pick], k[pick], v[pick], causal=causal))
+    assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
+    vt = v.transpose(-1, -2).contiguous().to(DEV)
+    assert torch.equal(c_attention(q.to(DEV), k.to(DEV), vt, causal, None, True), o)
+    kt = k.transpose(-1, -2).contiguous().to(DEV)
+    assert torch.equal(ops.flash_attention(q.to(DEV), kt, v.to(DEV), 1, 1, d, d, d ** -0.5, causal), o)
 
 
 def test_scale_and_large_logits():

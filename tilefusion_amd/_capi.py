@@ -36,6 +36,7 @@ SIGNATURES = {
     "tf_scatter_nd": (_i, [_vp, _vp, _vp, ctypes.POINTER(_i64), _i, _i64, _i, _i, _vp]),
     "tf_gemm_kernel_index": (_i, [_i64, _i64, _i64, _i]),
     "tf_flash_decode_plan": (_i, [_i64, _i64, _i64, _i, ctypes.POINTER(_i)]),
+    "tf_flash_attention_rows": (_i, [_i64, _i64, _i64, _i64, _i]),
     "tf_flash_attention_wide_rows": (_i, [_i64, _i64, _i]),
     "tf_jit_compile": (_i, [ctypes.c_char_p, ctypes.c_char_p, ctypes.POINTER(ctypes.c_char_p), _i,
                             ctypes.POINTER(ctypes.c_char_p), _i, ctypes.POINTER(_vp)]),
