@@ -72,8 +72,8 @@ TF_API int tf_fused_two_gemms(const void* A, const void* B, const void* C, void*
                               int64_t batch, int64_t M, int64_t N, int64_t K, int64_t P, int tm,
                               int tn, int tk, int tp, void* stream);
 
-/* tf_fused_two_gemms with a caller-provided device workspace.  Long-N problems (K = P = 128, N
- * a multiple of 64, too few row blocks to fill the chip) are then cut along N wherever that is the
+/* tf_fused_two_gemms with a caller-provided device workspace.  Problems of narrow K and P (up to
+ * 128) with too few row blocks to fill the chip are then cut along N wherever that is the
  * faster way: each workgroup takes a range of N for its rows, fp32 partial results go to the
  * workspace and a second kernel adds them up into D (fp16 and bf16).  tf_fused_two_gemms_workspace_bytes says how many bytes that takes
  * for a problem (0: it would not be cut); with a null or smaller workspace, and for every other
@@ -89,6 +89,13 @@ TF_API int tf_fused_two_gemms_ws(const void* A, const void* B, const void* C, vo
                                  int64_t batch, int64_t M, int64_t N, int64_t K, int64_t P, int tm,
                                  int tn, int tk, int tp, void* workspace, size_t workspace_bytes,
                                  void* stream);
+
+/* The same for 32 < K <= 128 and P <= 128 that are multiples of 8 only, as N (tf_fused_two_gemms_ws asks for K and N of
+ * whole 32, P of whole 16), operands at 16-byte boundaries; no tile sizes.  TF_ERR_UNSUPPORTED for everything else and for
+ * problems that tf_fused_two_gemms runs in one n-tile.  The workspace is that of tf_fused_two_gemms_workspace_bytes. */
+TF_API int tf_fused_two_gemms_narrow(const void* A, const void* B, const void* C, void* D, int dtype, int64_t batch,
+                                     int64_t M, int64_t N, int64_t K, int64_t P, void* workspace,
+                                     size_t workspace_bytes, void* stream);
 
 /* O = softmax(scale * Q K^T (+ causal mask)) V for `batch` independent (batch x head)
  * slices laid out back to back.  fp16 in/out, fp32 scores, fp32 running max / sum.

@@ -7,6 +7,7 @@ import torch
 import oracle
 from oracle import numerics as N
 from tests.gpu_util import DEV, c_fused, c_fused_dtype, c_fused_ws
+from tilefusion_amd import _capi, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -166,6 +167,49 @@ def test_every_plain_kernel_instance_is_exact(dtype, k, p, n):
     for _ in range(2):
         d = c_fused_dtype(a.to(dtype).to(DEV), b.to(dtype).to(DEV), c.to(dtype).to(DEV)).cpu()
         assert torch.equal(d.float(), ref)
+
+
+# Narrow K and P that are multiples of 8 only run the streaming kernel as they are: every instance (two to four steps of
+# K, 4, 6 and 8 column blocks, 64 and 128 rows), half-full last steps, last n-tiles that overlap their neighbour or are the
+# only one, uncut, cut, one tile a part, one row.  Integers again; an infinity in the last column of C reaches that
+# row of C only, whatever the overlapping columns and the chunks beyond K are multiplied with.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("batch,m,n,k,p", [
+    (1, 70, 320, 64, 64), (2, 1, 200, 48, 80), (1, 129, 8, 40, 8), (1, 65, 72, 104, 128), (1, 300, 1000, 96, 48), (3, 200, 584, 72, 96),
+    (1, 64, 4096, 128, 24), (1, 1000, 2056, 120, 120), (1, 33000, 328, 56, 64), (2, 17000, 136, 88, 88), (1, 40000, 264, 128, 128)])
+def test_narrow_shapes_exact(batch, m, n, k, p, dtype):
+    g = torch.Generator().manual_seed(m + n + k + p)
+    a = torch.randint(-2, 3, (batch, m, k), generator=g).to(dtype)
+    b = torch.zeros(batch, n, k)
+    b.scatter_(2, torch.randint(0, k, (batch, n, 5), generator=g), 1.0)      # five entries of a row of A
+    b[:, :, -1] = 1.0
+    c = torch.zeros(batch, p, n)
+    c.scatter_(2, torch.randint(0, n, (batch, p, 4), generator=g), 1.0)
+    c[:, :, -1] = -1.0
+    b, c = b.to(dtype), c.to(dtype)
+    rows = torch.cat([torch.arange(0, min(m, 130)), torch.arange(max(0, m - 70), m)])
+    inter = a[:, rows].float() @ b.float().transpose(1, 2)
+    ref = inter @ c.float().transpose(1, 2)
+    assert float(inter.abs().max()) <= 256 and float(ref.abs().max()) <= 256   # exact in bf16 too
+    ad, bd, cd = a.to(DEV), b.to(DEV), c.to(DEV)
+    d = torch.full((batch, m, p), float("nan"), device=DEV, dtype=dtype)
+    lead = (lambda t: t[0]) if batch == 1 else (lambda t: t)
+    ops.fused_two_gemms(lead(ad), lead(bd), lead(cd), lead(d), 1, 1, 1, 1)
+    assert torch.equal(d.cpu()[:, rows].float(), ref)
+    assert not torch.isnan(d).any()
+    code = _capi.TF_DTYPE_BF16 if dtype == torch.bfloat16 else _capi.TF_DTYPE_F16
+    lib, st = _capi.load(), torch.cuda.current_stream().cuda_stream
+    d2 = torch.full_like(d, float("nan"))
+    _capi.check(lib.tf_fused_two_gemms_narrow(ad.data_ptr(), bd.data_ptr(), cd.data_ptr(), d2.data_ptr(), code, batch, m, n, k,
+                                              p, None, 0, st), "tf_fused_two_gemms_narrow")                     # uncut
+    assert torch.equal(d, d2)
+    cd[:, p // 2, n - 1] = float("inf")
+    ops.fused_two_gemms(lead(ad), lead(bd), lead(cd), lead(d2), 1, 1, 1, 1)
+    s = inter[..., n - 1]   # infinity times this: +-inf, or NaN for zero
+    got = d2.cpu()[:, rows, p // 2].float()
+    assert torch.equal(torch.isnan(got), s == 0) and torch.equal(got[s != 0], torch.sign(s[s != 0]) * float("inf"))
+    keep = [i for i in range(p) if i != p // 2]
+    assert torch.equal(d2[..., keep], d[..., keep])
 
 
 def test_bf16_random_inputs_within_tolerance():

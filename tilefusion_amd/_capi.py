@@ -24,6 +24,7 @@ SIGNATURES = {
     "tf_fused_two_gemms": (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i64, _i64, _i64, _i64, _i, _i, _i, _i, _vp]),
     "tf_fused_two_gemms_workspace_bytes": (_sz, [_i, _i64, _i64, _i64, _i64, _i64]),
     "tf_fused_two_gemms_ws": (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i64, _i64, _i64, _i64, _i, _i, _i, _i, _vp, _sz, _vp]),
+    "tf_fused_two_gemms_narrow": (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i64, _i64, _i64, _i64, _vp, _sz, _vp]),
     "tf_flash_attention_fwd": (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i64, _i64, _i64, _i64, _i, _i, _i, _i, _i, _d, _i, _vp]),
     "tf_flash_attention_fwd_wide": (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i64, _i64, _i64, _d, _i, _vp]),
     "tf_flash_attention_fwd_kt": (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i64, _i64, _i64, _d, _i, _vp]),

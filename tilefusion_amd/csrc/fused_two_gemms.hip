@@ -13,11 +13,13 @@
 //   * B and C chunks go global -> LDS directly (global_load_lds_dwordx4) into XOR-swizzled
 //     tiles shared by the 4 wavefronts; A fragments are private to a wavefront and are read
 //     straight from global memory into registers;
-//   * D is staged through LDS so that global stores are 16 bytes per lane along rows.
+//   * D leaves from registers, four adjacent lanes to 64 contiguous bytes of a row.
+// Problems of several n-tiles stream (fused_two_gemms_stream.hip).
 #include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
+#include "fused_two_gemms_stream.hpp"
 
 namespace tfk {
 namespace {
@@ -42,83 +44,6 @@ template <int CH>
 __host__ __device__ constexpr int swz(int row, int c) {
   constexpr int kRowsPer256B = CH >= 16 ? 1 : 16 / CH;
   return c ^ ((row / kRowsPer256B) % CH);
-}
-
-// Cooperative direct global->LDS copy of a [ROWS x COLS] fp16 tile (row stride `ld` elements
-// in global memory) into a swizzled LDS tile with COLS-element rows.
-template <typename T, int ROWS, int COLS>
-TFK_DEVICE void tile_to_lds(const T* __restrict__ g, size_t ld, char* lds, int wave, int lane) {
-  constexpr int CH = COLS / 8;
-  constexpr int kRowsPerInstr = 64 / CH;
-  constexpr int kInstr = ROWS * CH / 64;
-  static_assert(ROWS * CH % 64 == 0, "tile must be a whole number of 1 KiB wavefront loads");
-  for (int i = wave; i < kInstr; i += kWaves) {
-    const int row = i * kRowsPerInstr + lane / CH;
-    const int c = swz<CH>(row, lane % CH);
-    load_global_to_lds_16B(g + (size_t)row * ld + c * 8, lds + i * 1024);
-  }
-}
-
-// The two products of one n-tile for one wavefront, with the LDS fragment reads issued one
-// step ahead of the MFMAs that use them (a wavefront alone on its SIMD has nobody to hide the
-// LDS latency behind; requesting step s+1 before multiplying step s takes it off the critical
-// path).  sB: [TN][KC] tile, sC: [TP][TN] tile, both XOR-swizzled.
-//   first_product:  acc1[nt] += S^T tile (rows n from B, columns m from A) over the KC / 32 steps
-//   second_product: acc2[pt] += (fp16 of acc1) * C over the TN / 32 steps; lane (m = lr, group
-//                   lg) holds A*B[m][16*nt + 4*lg + r] in acc1[nt][r], and reduction step s uses
-//                   n = 32*s + {4*lg + 0..3, 16 + 4*lg + 0..3} as its 8 slots.
-template <typename T, int TN, int KC>
-TFK_DEVICE void first_product(const char* sB, const vec8_t<T>* af, float4_t* acc1, int lr, int lg) {
-  constexpr int kNT = TN / 16, kKSteps = KC / 32, kCh = KC / 8;
-  vec8_t<T> bf[2][kNT];
-  auto read_b = [&](int buf, int ks) __attribute__((always_inline)) {
-#pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) {
-      const int row = nt * 16 + lr;
-      bf[buf][nt] = *reinterpret_cast<const vec8_t<T>*>(sB + row * KC * 2 + swz<kCh>(row, ks * 4 + lg) * 16);
-    }
-  };
-  read_b(0, 0);
-#pragma unroll
-  for (int ks = 0; ks < kKSteps; ++ks) {
-    if (ks + 1 < kKSteps) read_b((ks + 1) & 1, ks + 1);
-#pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) acc1[nt] = mfma_t<T>(bf[ks & 1][nt], af[ks], acc1[nt]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-template <typename T, int TN, int TP>
-TFK_DEVICE void second_product(const char* sC, const float4_t* acc1, float4_t* acc2, int lr, int lg) {
-  constexpr int kPT = TP / 16, kSteps = TN / 32, kCh = TN / 8;
-  vec8_t<T> cf[2][kPT];
-  auto read_c = [&](int buf, int s2) __attribute__((always_inline)) {
-#pragma unroll
-    for (int pt = 0; pt < kPT; ++pt) {
-      const int row = pt * 16 + lr;
-      const char* base = sC + row * TN * 2 + (lg & 1) * 8;
-      const vec4_t<T> lo = *reinterpret_cast<const vec4_t<T>*>(base + swz<kCh>(row, 4 * s2 + (lg >> 1)) * 16);
-      const vec4_t<T> hi = *reinterpret_cast<const vec4_t<T>*>(base + swz<kCh>(row, 4 * s2 + 2 + (lg >> 1)) * 16);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        cf[buf][pt][r] = lo[r];
-        cf[buf][pt][4 + r] = hi[r];
-      }
-    }
-  };
-  read_c(0, 0);
-#pragma unroll
-  for (int s2 = 0; s2 < kSteps; ++s2) {
-    if (s2 + 1 < kSteps) read_c((s2 + 1) & 1, s2 + 1);
-    vec8_t<T> pa;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      pa[r] = (T)acc1[2 * s2][r];
-      pa[4 + r] = (T)acc1[2 * s2 + 1][r];
-    }
-#pragma unroll
-    for (int pt = 0; pt < kPT; ++pt) acc2[pt] = mfma_t<T>(pa, cf[s2 & 1][pt], acc2[pt]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -387,260 +312,6 @@ int launch(const void* A, const void* B, const void* C, void* D, int batch, int 
   return TF_OK;
 }
 
-// ------------------------------------------------------------------------------------------
-// Streaming variant for long N (K = P = 128, N a multiple of 64, at least four n-tiles): n-tiles
-// of 64 (a B tile [64][128] and a C tile [128][64], whole 128-byte lines either way) go global ->
-// LDS through a four-stage ring, three tiles ahead of the one being multiplied, one barrier per
-// n-tile; A fragments are loaded once.  A workgroup alone on a CU has to hide the L2 latency
-// with bytes in flight: two 64 KiB stages (one tile ahead) ran at a quarter of this speed.
-// ------------------------------------------------------------------------------------------
-// kSplit = 2: a second set of kWavesT wavefronts takes every other n-tile of the same rows (the
-// pair w, w + kWavesT shares a SIMD), and the two partial D tiles are added through LDS at the
-// end.  A wavefront's chain per tile - fragment reads, 16 MFMAs, fp16 conversion, 16 MFMAs that
-// depend on it - leaves the matrix pipe idle most of the time; a second, independent chain on
-// the same SIMD fills it.  Only the first set issues the tile requests.
-// kPartial: blockIdx.y selects a part of `tiles_per_part` n-tiles, and the workgroup writes its fp32
-// partial sums to part blockIdx.y of the workspace W [batch][parts][M][128] instead of D; a second
-// kernel adds the parts up.  M / 64 workgroups do not fill the chip for the shapes this kernel is
-// for, and a workgroup is bound by how many tile bytes its ring keeps in flight, not by arithmetic.
-template <typename T, int kWavesT, int kSplit, bool kPartial>
-__global__ __launch_bounds__(kWavesT * kSplit * 64) void fused_two_gemms_stream_kernel(
-    const T* __restrict__ A, const T* __restrict__ B, const T* __restrict__ C,
-    T* __restrict__ D, float* __restrict__ W, int M, int N, int tiles_per_part) {
-  constexpr int K = 128, P = 128, TN = 64, kStagesS = 4;
-  constexpr int kRows = 16 * kWavesT;
-  constexpr int kBBytes = TN * K * 2;                // 16 KiB: B tile [n][k], 256-byte rows
-  constexpr int kCBytes = P * TN * 2;                // 16 KiB: C tile [p][n], 128-byte rows
-  constexpr int kStageBytes = kBBytes + kCBytes;
-  constexpr int kBInstr = kBBytes / 1024, kCInstr = kCBytes / 1024;   // 1 KiB wavefront requests
-  // the first kReqWaves wavefronts issue the tile requests (all of them when there are four)
-  constexpr int kReqWaves = kWavesT > 4 ? 4 : kWavesT;
-  constexpr int kReqPerWave = (kBInstr + kCInstr) / kReqWaves;
-  static_assert((kBInstr / kReqWaves) % 4 == 0 && (kCInstr / kReqWaves) % 4 == 0,
-                "a wavefront's requests of a tile come in groups of four consecutive instructions");
-  // tiles requested ahead of the one being multiplied: the ring allows kStagesS - 1, the 6-bit
-  // vmcnt allows 63 requests of one wavefront to stay in flight behind the awaited tile
-  constexpr int kAhead = (kStagesS - 2) * kReqPerWave <= 63 ? kStagesS - 1 : 63 / kReqPerWave + 1;
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
-  T* sD = reinterpret_cast<T*>(smem + kStagesS * kStageBytes);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave = wave_id % kWavesT;      // which 16 rows
-  const int half = wave_id / kWavesT;      // which n-tiles (t % kSplit == half)
-  const int lr = lane & 15, lg = lane >> 4;
-  const int m0 = blockIdx.x * kRows;
-  const size_t batch = blockIdx.z;
-  A += batch * (size_t)M * K;
-  B += batch * (size_t)N * K;
-  C += batch * (size_t)P * N;
-  D += batch * (size_t)M * P;
-  const unsigned smem_base = lds_address(smem);
-
-  const int a_row = min(m0 + wave * 16 + lr, M - 1);  // clamped: rows past M are never stored
-  vec8_t<T> af[4];
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
-    af[ks] = *reinterpret_cast<const vec8_t<T>*>(A + (size_t)a_row * K + 8 * lg + ks * 32);
-
-  // this workgroup's n-tiles: [t_begin, t_begin + n_tiles)
-  const int t_begin = kPartial ? (int)blockIdx.y * tiles_per_part : 0;
-  const int n_tiles = kPartial ? min(tiles_per_part, N / TN - t_begin) : N / TN;
-  // Requests of n-tile t (clamped past the end: the surplus lands in a stage nobody reads
-  // again).  Instruction i of the B tile covers rows 4i .. 4i+3 (16 chunks each), of the C tile
-  // rows 8i .. 8i+7 (8 chunks each); lane l fills physical chunk l % 16 (l % 8) and fetches the
-  // logical chunk the swizzle maps there.  The swizzle XORs row bits into the chunk index, so the
-  // per-lane byte offsets of all instructions follow from one base by an XOR with a constant
-  // (B: 4 variants, C: 2); everything else - the tile origin, the rows 4i or 8i, the part
-  // cancelled by the immediate offset - is scalar.  Four instructions share one M0 value.
-  const unsigned voff_b0 = (lane / 16) * (K * 2) + (((lane % 16) ^ (lane / 16)) << 4);
-  const unsigned voff_c0 = (lane / 8) * (unsigned)N * 2u + (((lane % 8) ^ (lane / 16)) << 4);
-  auto request_tile = [&](int t) __attribute__((always_inline)) {
-    if (wave_id >= kReqWaves) return;
-    const unsigned stage = smem_base + (t % kStagesS) * kStageBytes;
-    const int n0 = (t_begin + min(t, n_tiles - 1)) * TN;
-    const char* b_src = reinterpret_cast<const char*>(B) + (size_t)n0 * (K * 2);
-    const char* c_src = reinterpret_cast<const char*>(C) + (size_t)n0 * 2;
-#pragma unroll
-    for (int q = 0; q < kBInstr / kReqWaves; ++q) {
-      // instructions are dealt in blocks of kBInstr / kReqWaves consecutive ones per wavefront
-      const int i_first = wave_id * (kBInstr / kReqWaves);
-      const unsigned voff = voff_b0 ^ (unsigned)(((q % 4) * 4) << 4);        // row 4i: chunk ^= 4 * (i % 4)
-      const char* src = b_src + (size_t)(i_first + q) * 1024 - (q % 4) * 1024;   // + rows, - what the immediate adds
-      // four requests share one M0 value (an input of each statement, so the compiler keeps it
-      // there) and differ in the immediate offset
-      asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%2"
-                   :
-                   : "v"(voff), "s"(src), "n"(1024 * (q % 4)), "{m0}"(stage + (i_first + q - q % 4) * 1024)
-                   : "memory");
-    }
-#pragma unroll
-    for (int q = 0; q < kCInstr / kReqWaves; ++q) {
-      const int i_first = wave_id * (kCInstr / kReqWaves);
-      const unsigned voff = voff_c0 ^ (unsigned)(((q % 2) * 4) << 4);        // row 8i: chunk ^= 4 * (i % 2)
-      const char* src = c_src + (size_t)(i_first + q) * 8 * (size_t)N * 2 - (q % 4) * 1024;
-      asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%2"
-                   :
-                   : "v"(voff), "s"(src), "n"(1024 * (q % 4)), "{m0}"(stage + kBBytes + (i_first + q - q % 4) * 1024)
-                   : "memory");
-    }
-  };
-
-  float4_t acc2[8];
-#pragma unroll
-  for (int pt = 0; pt < 8; ++pt) acc2[pt] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-#pragma unroll
-  for (int t = 0; t < kAhead; ++t) request_tile(t);
-  for (int t = 0; t < n_tiles; ++t) {
-    // this wavefront's requests of tile t have landed (kAhead - 1 younger tiles stay in flight); after
-    // the barrier everybody's have, and everybody is done with tile t-1, whose stage is refilled
-    wait_vmem<(kAhead - 1) * kReqPerWave>();
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    request_tile(t + kAhead);
-    const char* sB = smem + (t % kStagesS) * kStageBytes;
-    const char* sC = sB + kBBytes;
-
-    if (kSplit > 1 && t % kSplit != half) continue;
-    float4_t acc1[TN / 16];
-#pragma unroll
-    for (int nt = 0; nt < TN / 16; ++nt) acc1[nt] = float4_t{0.f, 0.f, 0.f, 0.f};
-    first_product<T, TN, K>(sB, af, acc1, lr, lg);
-    second_product<T, TN, P>(sC, acc1, acc2, lr, lg);
-  }
-  wait_vmem_all();  // the surplus requests must not outlive the workgroup's LDS
-  if constexpr (kSplit > 1) {
-    // add the second set's partial sums to the first set's (the ring is free by now)
-    __syncthreads();
-    constexpr int kPartElems = kWavesT * 8 * 64;   // float4 per wavefront set
-    static_assert((kSplit - 1) * kPartElems * 16 <= kStagesS * kStageBytes, "partial sums fit in the ring");
-    float4_t* part = reinterpret_cast<float4_t*>(smem) + (size_t)wave * 8 * 64 + lane;
-    if (half != 0) {
-#pragma unroll
-      for (int pt = 0; pt < 8; ++pt) part[(half - 1) * kPartElems + pt * 64] = acc2[pt];
-    }
-    __syncthreads();
-    if (half == 0) {
-#pragma unroll
-      for (int h = 1; h < kSplit; ++h)
-#pragma unroll
-        for (int pt = 0; pt < 8; ++pt) acc2[pt] += part[(h - 1) * kPartElems + pt * 64];
-    }
-  }
-
-  // Epilogue: acc2[pt][r] = D[m0 + 16*wave + 4*lg + r][16*pt + lr]
-  if constexpr (kPartial) {
-    // fp32 partial sums straight from the accumulators: 16 adjacent lanes write 64 contiguous bytes
-    if (half == 0) {
-      float* w = W + ((batch * gridDim.y + blockIdx.y) * (size_t)M + m0 + wave * 16 + 4 * lg) * P + lr;
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (m0 + wave * 16 + 4 * lg + r < M) {
-#pragma unroll
-          for (int pt = 0; pt < 8; ++pt) __builtin_nontemporal_store(acc2[pt][r], w + (size_t)r * P + pt * 16);
-        }
-    }
-    return;
-  }
-  // fp16 result, staged through LDS for 16-byte stores along rows
-  if (half == 0) {
-#pragma unroll
-    for (int pt = 0; pt < 8; ++pt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sD[(wave * 16 + 4 * lg + r) * P + pt * 16 + lr] = (T)acc2[pt][r];
-  }
-  __syncthreads();
-  constexpr int kDChunks = P / 8;
-  for (int f = tid; f < kRows * kDChunks; f += kWavesT * kSplit * 64) {
-    const int row = f / kDChunks, c = f % kDChunks;
-    if (m0 + row < M)
-      __builtin_nontemporal_store(*reinterpret_cast<const uint4_t*>(sD + row * P + c * 8),
-                                  reinterpret_cast<uint4_t*>(D + (size_t)(m0 + row) * P + c * 8));
-  }
-}
-
-// D[b][i] = fp16(sum over parts of W[b][part][i]), i over the M * 128 elements of a problem
-template <typename T>
-__global__ __launch_bounds__(256) void fused_two_gemms_reduce_kernel(const float* __restrict__ W,
-                                                                     T* __restrict__ D, int parts,
-                                                                     size_t elems) {
-  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (i >= elems) return;
-  const float* w = W + (size_t)blockIdx.z * parts * elems + i;
-  float4_t acc = __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(w));
-  for (int part = 1; part < parts; ++part)
-    acc += __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(w + (size_t)part * elems));
-  vec4_t<T> h = {(T)acc[0], (T)acc[1], (T)acc[2], (T)acc[3]};
-  *reinterpret_cast<vec4_t<T>*>(D + (size_t)blockIdx.z * elems + i) = h;
-}
-
-template <typename T, int kWavesT, int kSplit>
-int launch_stream(const void* A, const void* B, const void* C, void* D, int batch, int M, int N,
-                  hipStream_t st) {
-  auto kern = fused_two_gemms_stream_kernel<T, kWavesT, kSplit, false>;
-  constexpr int lds = 4 * (64 * 128 * 2 + 128 * 64 * 2) + 16 * kWavesT * 128 * 2;
-  static_assert(lds <= kMaxLdsBytes, "ring does not fit in LDS");
-  TFK_LDS_OPT_IN(kern, lds);
-  dim3 grid((M + 16 * kWavesT - 1) / (16 * kWavesT), 1, batch);
-  hipLaunchKernelGGL(kern, grid, dim3(kWavesT * kSplit * 64), lds, st, static_cast<const T*>(A),
-                     static_cast<const T*>(B), static_cast<const T*>(C),
-                     static_cast<T*>(D), static_cast<float*>(nullptr), M, N, 0);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
-}
-
-// How a long-N problem (K = P = 128) is cut when a workspace is available: `parts` ranges of
-// `tiles_per_part` 64-wide n-tiles for row blocks of `rows` rows.  A workgroup takes a CU to itself
-// (the ring fills its LDS) and is bound by the tile bytes it keeps in flight, so the cut aims at one
-// workgroup per CU (row blocks x parts <= 256) and keeps at least the four tiles per part that
-// fill the ring.  Measured on the reference's sweep, a launch takes about 9.6 + 0.9 t us with
-// 64-row blocks and 11.8 + 1.23 t us with 128-row blocks (eight wavefronts share every tile), t the
-// tiles a workgroup walks, against 4 + 0.8 t uncut: the second launch and the trip of the partial
-// sums through memory are in the constants.  The cheapest of the three is taken; 128-row blocks
-// only from eight tiles per part on (shorter walks are dominated by filling the ring, and eight
-// wavefronts fill it no faster than four).  parts == 1: no cut.
-struct SplitPlan { int parts, tiles_per_part, rows; };
-SplitPlan fused_split_plan(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t P) {
-  const SplitPlan uncut = {1, 0, 64};
-  if (!(K == 128 && P == 128 && N % 64 == 0 && N >= 512)) return uncut;
-  const int64_t n_tiles = N / 64;
-  auto cut = [&](int rows) -> SplitPlan {
-    const int64_t row_blocks = (M + rows - 1) / rows * batch;
-    int64_t parts = std::min<int64_t>(256 / std::max<int64_t>(row_blocks, 1), n_tiles / 4);
-    if (parts <= 1) return {1, 0, rows};
-    const int64_t per = (n_tiles + parts - 1) / parts;
-    return {(int)((n_tiles + per - 1) / per), (int)per, rows};
-  };
-  const SplitPlan p64 = cut(64), p128 = cut(128);
-  double best = 4.0 + 0.8 * (double)n_tiles;
-  SplitPlan plan = uncut;
-  if (p64.parts > 1 && 9.6 + 0.9 * p64.tiles_per_part < best) {
-    best = 9.6 + 0.9 * p64.tiles_per_part;
-    plan = p64;
-  }
-  if (p128.parts > 1 && p128.tiles_per_part >= 8 && 11.8 + 1.23 * p128.tiles_per_part < best) plan = p128;
-  return plan;
-}
-
-template <typename T, int kWavesT, int kSplit>
-int launch_stream_split(const void* A, const void* B, const void* C, void* D, float* W, SplitPlan plan, int batch,
-                        int M, int N, hipStream_t st) {
-  auto kern = fused_two_gemms_stream_kernel<T, kWavesT, kSplit, true>;
-  constexpr int lds = 4 * (64 * 128 * 2 + 128 * 64 * 2) + 16 * kWavesT * 128 * 2;
-  TFK_LDS_OPT_IN(kern, lds);
-  dim3 grid((M + 16 * kWavesT - 1) / (16 * kWavesT), plan.parts, batch);
-  hipLaunchKernelGGL(kern, grid, dim3(kWavesT * kSplit * 64), lds, st, static_cast<const T*>(A),
-                     static_cast<const T*>(B), static_cast<const T*>(C),
-                     static_cast<T*>(D), W, M, N, plan.tiles_per_part);
-  TFK_HIP_TRY(hipGetLastError());
-  const size_t elems = (size_t)M * 128;
-  hipLaunchKernelGGL(fused_two_gemms_reduce_kernel<T>, dim3((unsigned)((elems / 4 + 255) / 256), 1, batch), dim3(256), 0,
-                     st, W, static_cast<T*>(D), plan.parts, elems);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
-}
-
 template <typename T, int TN, int TP>
 int pick_kc(const void* A, const void* B, const void* C, void* D, int batch, int M, int N, int K,
             int P, hipStream_t st) {
@@ -681,27 +352,85 @@ int check_fused_args(const char* who, const void* A, const void* B, const void* 
 
 namespace tfk {
 namespace {
-// the tuned kernels for element type T (arguments already checked)
+// The plain kernel for element type T (arguments already checked)
 template <typename T>
-int run_fused(const void* A, const void* B, const void* C, void* D, int64_t batch, int64_t M, int64_t N, int64_t K,
+int run_plain(const void* A, const void* B, const void* C, void* D, int64_t batch, int64_t M, int64_t N, int64_t K,
               int64_t P, hipStream_t st) {
-  // long N: stream the B / C tiles through the LDS ring (8-15% faster than the plain kernel's
-  // load - wait - multiply per n-tile; both are bound by the latencies of one wavefront per SIMD)
-  if (K == 128 && P == 128 && N % 64 == 0 && N >= 256) {
-    // enough rows for a 128-row block per CU: eight wavefronts share every tile (1.23 us per tile
-    // for 128 rows against 0.8 us for 64)
-    if (N >= 512 && (M + 127) / 128 * batch >= 256)
-      return launch_stream<T, 8, 1>(A, B, C, D, (int)batch, (int)M, (int)N, st);
-    return launch_stream<T, 4, 2>(A, B, C, D, (int)batch, (int)M, (int)N, st);
-  }
   if (N % 128 == 0) return pick_tp<T, 128>(A, B, C, D, (int)batch, (int)M, (int)N, (int)K, (int)P, st);
   return pick_tp<T, 32>(A, B, C, D, (int)batch, (int)M, (int)N, (int)K, (int)P, st);
 }
-template <typename T>
-int run_fused_split(const void* A, const void* B, const void* C, void* D, float* W, SplitPlan plan, int64_t batch,
-                    int64_t M, int64_t N, hipStream_t st) {
-  if (plan.rows == 128) return launch_stream_split<T, 8, 1>(A, B, C, D, W, plan, (int)batch, (int)M, (int)N, st);
-  return launch_stream_split<T, 4, 2>(A, B, C, D, W, plan, (int)batch, (int)M, (int)N, st);
+
+// Which problems stream (fused_two_gemms_stream.hip), and how they are cut.
+//
+// The plain kernel is made for one n-tile: it starts ~1 us sooner and several of its workgroups share a CU, but it
+// loads, waits and multiplies one tile after the other, by k-chunks of 32 unless K % 128 == 0, once for every 16
+// columns of D unless P % 64 == 0.  us, bf16, plain / streaming: N = 128, K = P = 128, 16384 rows 5.1 / 6.2, 262144 rows
+// 36 / 50; N = 256, K = P = 64, 32768 rows 5.9 / 6.5; N = 320 10.5 / 6.9; N = 256, K = 96, P = 48, 16384 rows 5.7 / 6.2,
+// 32768 rows 11.0 / 6.5; N = 192, K = P = 128, 64 rows 7.6 / 5.8.
+bool takes_plain(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t P) {
+  if (N % 32 != 0 || K % 32 != 0 || P % 16 != 0) return false;   // (it would have to be padded in memory)
+  return (N <= 128 || (N <= 256 && N % 128 == 0 && K < 128)) && (P % 64 == 0 || M * batch <= 16384);
+}
+bool may_stream(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t P) {
+  return K > 32 && K <= 128 && P <= 128 && K % 8 == 0 && P % 8 == 0 && N % 8 == 0 &&
+         (M + 63) / 64 < (1 << 20) && !takes_plain(batch, M, N, K, P);
+}
+
+// Rows per workgroup (64 or 128) and the cut along N, by expected time: a workgroup takes its tiles in turn, one on
+// a CU; parts cost a second launch and a trip of fp32 sums through memory (and with the workspace ~10.5 us of the calling
+// thread, against 6-7 for one launch).  Fitted to 330 problems (64..32768
+// rows, N 16..8192, the K and P of the sweep), 1.2% behind the best of up to 12 plans each on average.  Without room for
+// partial sums (`may_cut` false) there is one part.
+FusedPlan plan_stream(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t P, bool may_cut) {
+  const int64_t tiles = (N + 63) / 64;
+  const double k_steps = (double)((K + 31) / 32), p_blocks = P <= 64 ? 4 : P <= 96 ? 6 : 8;
+  FusedPlan plan = {64, 1, (int)tiles};
+  double best = 0;
+  auto consider = [&](int rows, int64_t wanted) {
+    const int64_t row_blocks = (M + rows - 1) / rows * batch;
+    const int64_t per = (tiles + wanted - 1) / wanted, parts = (tiles + per - 1) / per;
+    const int64_t groups = row_blocks * parts, rounds = (groups + 255) / 256;
+    const double tile = rows == 64 ? 0.128 + 0.038 * k_steps + 0.027 * p_blocks : 0.131 + 0.027 * k_steps + 0.052 * p_blocks;
+    const double fill = 0.847 + 0.153 * std::min(1.0, (double)groups / 256.0);
+    double t = (rows == 64 ? 5.5 : 5.7) + (rows == 64 ? 1.1 : 1.6) * (double)(rounds - 1) + (double)(rounds * per) * tile * fill;
+    if (parts > 1) t = std::max(10.5, t + 3.0 + 0.315e-6 * 4.0 * (double)(parts * batch * M * P));
+    if (best == 0 || t < best) {
+      best = t;
+      plan = {rows, (int)parts, (int)per};
+    }
+  };
+  for (int rows : {64, 128}) {
+    const int64_t row_blocks = (M + rows - 1) / rows * batch;
+    consider(rows, 1);
+    if (!may_cut) continue;
+    for (int64_t target : {256, 512})
+      if (target / row_blocks > 1) consider(rows, std::min(tiles, target / row_blocks));
+    if (row_blocks <= 256)
+      for (int64_t parts = 2; parts < tiles && parts * row_blocks <= 512; parts *= 2) consider(rows, parts);
+  }
+  return plan;
+}
+
+bool aligned16(const void* A, const void* B, const void* C, const void* D) {
+  return (reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C) |
+          reinterpret_cast<uintptr_t>(D)) % 16 == 0;
+}
+
+size_t partial_bytes(const FusedPlan& plan, int64_t batch, int64_t M, int64_t P) {
+  return plan.parts > 1 ? (size_t)plan.parts * (size_t)batch * (size_t)M * (size_t)P * sizeof(float) : 0;
+}
+
+int run_fused(const void* A, const void* B, const void* C, void* D, bool bf16, int64_t batch, int64_t M, int64_t N,
+              int64_t K, int64_t P, void* workspace, size_t workspace_bytes, hipStream_t st) {
+  if (may_stream(batch, M, N, K, P) && aligned16(A, B, C, D)) {
+    FusedPlan plan = plan_stream(batch, M, N, K, P, true);
+    if (workspace == nullptr || workspace_bytes < partial_bytes(plan, batch, M, P))
+      plan = plan_stream(batch, M, N, K, P, false);
+    const FusedCall call = {A, B, C, D, workspace, bf16, (int)batch, (int)M, (int)N, (int)K, (int)P, st};
+    return run_fused_stream(call, plan);
+  }
+  if (bf16) return run_plain<bf16_t>(A, B, C, D, batch, M, N, K, P, st);
+  return run_plain<half_t>(A, B, C, D, batch, M, N, K, P, st);
 }
 }  // namespace
 }  // namespace tfk
@@ -711,15 +440,15 @@ extern "C" int tf_fused_two_gemms_f16(const void* A, const void* B, const void* 
                                       int tm, int tn, int tk, int tp, void* stream) {
   using namespace tfk;
   if (int rc = check_fused_args("tf_fused_two_gemms_f16", A, B, C, D, batch, M, N, K, P, tm, tn, tk, tp)) return rc;
-  return run_fused<half_t>(A, B, C, D, batch, M, N, K, P, static_cast<hipStream_t>(stream));
+  return run_fused(A, B, C, D, false, batch, M, N, K, P, nullptr, 0, static_cast<hipStream_t>(stream));
 }
 
 extern "C" size_t tf_fused_two_gemms_workspace_bytes(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
                                                      int64_t P) {
   using namespace tfk;
-  if ((dtype != TF_DTYPE_F16 && dtype != TF_DTYPE_BF16) || batch <= 0 || M <= 0 || N <= 0) return 0;
-  const SplitPlan plan = fused_split_plan(batch, M, N, K, P);
-  return plan.parts > 1 ? (size_t)plan.parts * (size_t)batch * (size_t)M * 128 * sizeof(float) : 0;
+  if ((dtype != TF_DTYPE_F16 && dtype != TF_DTYPE_BF16) || batch <= 0 || M <= 0 || N <= 0 || K <= 0 || P <= 0) return 0;
+  if (!may_stream(batch, M, N, K, P)) return 0;
+  return partial_bytes(plan_stream(batch, M, N, K, P, true), batch, M, P);
 }
 
 extern "C" int tf_fused_two_gemms_ws(const void* A, const void* B, const void* C, void* D, int dtype, int64_t batch,
@@ -732,11 +461,29 @@ extern "C" int tf_fused_two_gemms_ws(const void* A, const void* B, const void* C
   if (int rc = check_fused_args("tf_fused_two_gemms_ws", A, B, C, D, batch, M, N, K, P, tm, tn, tk, tp)) return rc;
   TFK_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, TF_ERR_INVALID_ARG,
               "tf_fused_two_gemms_ws: workspace must be 16-byte aligned");
-  const SplitPlan plan = fused_split_plan(batch, M, N, K, P);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dtype == TF_DTYPE_BF16)
-    return run_fused_split<bf16_t>(A, B, C, D, static_cast<float*>(workspace), plan, batch, M, N, st);
-  return run_fused_split<half_t>(A, B, C, D, static_cast<float*>(workspace), plan, batch, M, N, st);
+  return run_fused(A, B, C, D, dtype == TF_DTYPE_BF16, batch, M, N, K, P, workspace, workspace_bytes,
+                   static_cast<hipStream_t>(stream));
+}
+
+extern "C" int tf_fused_two_gemms_narrow(const void* A, const void* B, const void* C, void* D, int dtype, int64_t batch,
+                                         int64_t M, int64_t N, int64_t K, int64_t P, void* workspace,
+                                         size_t workspace_bytes, void* stream) {
+  using namespace tfk;
+  TFK_REQUIRE(A && B && C && D, TF_ERR_INVALID_ARG, "tf_fused_two_gemms_narrow: null pointer");
+  TFK_REQUIRE(batch > 0 && M > 0 && N > 0 && K > 0 && P > 0, TF_ERR_INVALID_ARG,
+              "tf_fused_two_gemms_narrow: sizes must be positive");
+  TFK_REQUIRE(batch < 65536 && M < (1 << 30) && N < (1 << 24), TF_ERR_INVALID_ARG,
+              "tf_fused_two_gemms_narrow: dimension too large");
+  TFK_REQUIRE(dtype == TF_DTYPE_F16 || dtype == TF_DTYPE_BF16, TF_ERR_UNSUPPORTED,
+              "tf_fused_two_gemms_narrow: dtype must be TF_DTYPE_F16 or TF_DTYPE_BF16");
+  TFK_REQUIRE(may_stream(batch, M, N, K, P) && aligned16(A, B, C, D), TF_ERR_UNSUPPORTED,
+              "tf_fused_two_gemms_narrow: needs 32 < K <= 128, P <= 128, multiples of 8 (got K=%lld N=%lld P=%lld) and "
+              "operands at 16-byte boundaries, and takes no problem that tf_fused_two_gemms runs in one n-tile",
+              (long long)K, (long long)N, (long long)P);
+  TFK_REQUIRE(workspace == nullptr || reinterpret_cast<uintptr_t>(workspace) % 16 == 0, TF_ERR_INVALID_ARG,
+              "tf_fused_two_gemms_narrow: workspace must be 16-byte aligned");
+  return run_fused(A, B, C, D, dtype == TF_DTYPE_BF16, batch, M, N, K, P, workspace, workspace_bytes,
+                   static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tf_fused_two_gemms(const void* A, const void* B, const void* C, void* D, int dtype, int64_t batch,
@@ -748,5 +495,5 @@ extern "C" int tf_fused_two_gemms(const void* A, const void* B, const void* C, v
               "tf_fused_two_gemms: dtype must be TF_DTYPE_F16 or TF_DTYPE_BF16");
   // bf16: the same kernels with the bf16 MFMA, a bf16 intermediate and bf16 output
   if (int rc = check_fused_args("tf_fused_two_gemms", A, B, C, D, batch, M, N, K, P, tm, tn, tk, tp)) return rc;
-  return run_fused<bf16_t>(A, B, C, D, batch, M, N, K, P, static_cast<hipStream_t>(stream));
+  return run_fused(A, B, C, D, true, batch, M, N, K, P, nullptr, 0, static_cast<hipStream_t>(stream));
 }

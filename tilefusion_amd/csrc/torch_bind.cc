@@ -121,21 +121,28 @@ TILEFUSION_EXPORT void fused_two_gemms(const at::Tensor& A, const at::Tensor& B,
   TORCH_CHECK(leading_numel(B, 2) == batch && leading_numel(C, 2) == batch &&
                   leading_numel(D, 2) == batch,
               "batch dimensions must match.");
-  // The kernels reduce 32 values of k (and of n, in the second product) per MFMA and write 16
+  // long-N problems are cut along N when the library is handed a workspace for the partial sums
+  const size_t ws_bytes = tf_fused_two_gemms_workspace_bytes(dtype, batch, m, n, k, p);
+  at::Tensor ws;
+  if (ws_bytes > 0) ws = at::empty({(int64_t)ws_bytes}, A.options().dtype(at::kByte));
+  void* ws_ptr = ws_bytes > 0 ? ws.data_ptr() : nullptr;
+  // The plain kernels reduce 32 values of k (and of n, in the second product) per MFMA and write 16
   // columns per base tile.  Shapes the reference accepts with 16-wide base tiles (K or N = 48,
-  // ...) are zero-padded here: zeros add nothing to either product.  A padded P goes through a
-  // temporary D.
+  // ...) run the streaming kernel where K and P are narrow and all are multiples of 8, and are zero-padded here
+  // otherwise: zeros add nothing to either product.  A padded P goes through a temporary D.
   const int64_t kp = round_up(k, 32), np = round_up(n, 32), pp = round_up(p, 16);
   const int64_t mp = m;
   if (kp == k && np == n && pp == p && mp == m) {
-    // long-N problems are cut along N when the library is handed a workspace for the partial sums
-    const size_t ws_bytes = tf_fused_two_gemms_workspace_bytes(dtype, batch, m, n, k, p);
-    at::Tensor ws;
-    if (ws_bytes > 0) ws = at::empty({(int64_t)ws_bytes}, A.options().dtype(at::kByte));
     check_status(tf_fused_two_gemms_ws(A.data_ptr(), B.data_ptr(), C.data_ptr(), D.data_ptr(), dtype, batch,
-                                       m, n, k, p, (int)tm, (int)tn, (int)tk, (int)tp,
-                                       ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, current_stream()),
+                                       m, n, k, p, (int)tm, (int)tn, (int)tk, (int)tp, ws_ptr, ws_bytes,
+                                       current_stream()),
                  "fused_two_gemms");
+    return;
+  }
+  const int status = tf_fused_two_gemms_narrow(A.data_ptr(), B.data_ptr(), C.data_ptr(), D.data_ptr(), dtype, batch,
+                                               m, n, k, p, ws_ptr, ws_bytes, current_stream());
+  if (status != TF_ERR_UNSUPPORTED) {
+    check_status(status, "fused_two_gemms");
     return;
   }
   // constant_pad_nd pads from the last dimension backwards: {last_lo, last_hi, prev_lo, prev_hi}
