@@ -42,8 +42,8 @@ def test_out_of_range_rows_are_skipped_and_shapes_checked():
         scatter_nd(data, idx.int(), upd)
 
 
-# Up to 1024 updates go straight to memory; beyond, workgroups sort 16 (up to 2048), 64 or, with at
-# least eight updates per target, 128 at a time (64: with 256 or 512 threads); lanes take words of 32
+# Up to 1024 updates go straight to memory; beyond, workgroups sort 16 at a time (a few 16-bit updates, up to 2048) or own a
+# share of the targets; lanes take words of 32
 # bits, so odd slices and an odd start of a 16-bit array split pairs.  Values of
 # -1, 0, 1 keep every partial sum well below 256 (the hottest row takes 1367 of them: a standard
 # deviation of 30): exact in all types, whatever the order.
@@ -67,6 +67,39 @@ def test_scatter_nd_sorted_workgroups(dtype, rows, slice_, n, start):
     scatter_nd(dev, bad.to(DEV), upd.to(DEV))
     assert torch.equal(dev.float().cpu(), want)
     assert buf[-1].item() == 3.0 and (start == 0 or buf[0].item() == 3.0)
+
+
+# Owners of targets: one and several chunks of 2048 updates, the last as long as the others or shorter, chunks of 8192 from
+# 20000 on (and narrow slices hit often, which the sort of 128 keeps), slices of a few lanes, of one word a lane and two,
+# of more column ranges than one, indices of one and of three numbers, all updates to one target, and to none.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("dims,depth,n,start", [
+    ((500, 40), 1, 2048, 0), ((500, 3), 1, 2049, 1), ((6, 5, 7, 260), 3, 4097, 0), ((3000, 517), 1, 4096, 1), ((300, 1026), 1, 2500, 0),
+    ((1200, 34), 1, 9001, 1), ((5000, 66), 1, 19999, 0), ((5000, 65), 1, 20001, 0), ((70, 60, 130), 2, 20000, 0), ((2000, 8), 1, 33000, 0),
+    ((900, 6), 1, 16385, 0)])
+def test_scatter_nd_owners_of_targets(dtype, dims, depth, n, start):
+    from tilefusion_amd.ops import scatter_nd
+    g = torch.Generator().manual_seed(n + dims[0])
+    data = torch.randint(-2, 3, dims, generator=g).to(dtype)
+    idx = torch.stack([torch.randint(0, dims[j], (n,), generator=g) for j in range(depth)], dim=1)
+    idx[::97] = torch.tensor([d // 2 for d in dims[:depth]])      # a target of every chunk
+    idx[5], idx[n - 1] = -1, dims[0]                              # skipped
+    upd = torch.randint(-1, 2, (n, *dims[depth:]), generator=g).to(dtype)
+    keep = (idx >= 0).all(1) & (idx[:, 0] < dims[0])
+    want = N.scatter_nd_ref(data, idx[keep], upd[keep])
+    buf = torch.full((start + data.numel() + 1,), 3.0, dtype=dtype, device=DEV)
+    dev = buf[start:start + data.numel()].view(dims)
+    dev.copy_(data)
+    scatter_nd(dev, idx.to(DEV), upd.to(DEV))
+    assert torch.equal(dev.float().cpu(), want)
+    assert buf[-1].item() == 3.0 and (start == 0 or buf[0].item() == 3.0)
+    one = torch.zeros(3, *dims[depth:], dtype=dtype, device=DEV)   # every update to one target: alternating signs
+    at = torch.ones(n, 1, dtype=torch.int64, device=DEV)
+    sign = (1 - 2 * (torch.arange(n, device=DEV) % 2)).to(dtype).view(-1, *[1] * (len(dims) - depth))
+    scatter_nd(one, at, (sign * torch.ones(n, *dims[depth:], dtype=dtype, device=DEV)).contiguous())
+    assert torch.equal(one[1].float().cpu(), torch.full(dims[depth:], float(n % 2))) and not one[[0, 2]].any()
+    scatter_nd(one, at * 3, sign.expand(n, *dims[depth:]).contiguous())
+    assert not one[[0, 2]].any()
 
 
 def test_scatter_nd_fp16_sum_of_duplicates_beyond_its_range():

@@ -11,10 +11,11 @@
 // What bounds it: atomics on one 128-byte line are served one after another, ~20 ns each (the eight
 // L2s are not coherent with each other, so a device-wide atomic is done on the memory side).  With
 // indices that repeat as word frequencies do, the most frequent row of 8192 updates is hit ~550
-// times.  So a workgroup takes kRows updates, sorts their rows in LDS and issues ONE hardware atomic
+// times.  So a workgroup sorts updates by their rows in LDS and issues ONE hardware atomic
 // per word and distinct row (16-bit types: packed pairs; a compare-and-swap loop per element, tried
 // first, retries for as long as others win).  8192 bf16 updates of 1024 into 32000 rows, log-uniform
-// indices: 2200 to 3000 us with compare-and-swap, 41 with a packed atomic per update and word, 20 as here.
+// indices: 2200 to 3000 us with compare-and-swap, 41 with a packed atomic per update and word, 20 with every 64
+// updates sorted as they come, 17 with workgroups that own rows (scatter_nd_owner_kernel).
 // What is left is the rate of the atomics themselves, ~0.9 TB/s with distinct rows as well.
 #include <algorithm>
 #include <type_traits>
@@ -167,7 +168,7 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_nd_direct_kernel(
   } while (kAnyMemory && (row += gridDim.x * (long long)(kScatterThreads / lanes)) < n);
 }
 
-// Many updates: kRows per workgroup; a group of `lanes` adjacent lanes (a power of two up to 64) takes one
+// The next kRows updates per workgroup, as they come; a group of `lanes` adjacent lanes (a power of two up to 64) takes one
 // distinct row at a time, kWords words per lane.  Unless kPairs, the halves of words are loaded one by one.
 // Scalar registers: with more than 80 a SIMD holds fewer than eight wavefronts, and of workgroups of sixteen a CU
 // then holds one instead of two (83: 16598 bf16 updates of 627 into 318 rows 53 us, 78: 35).
@@ -283,6 +284,184 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_sgpr(80))) void
   }
 }
 
+// Many updates: a workgroup owns a share of the TARGETS (a bucket of a hash of their numbers) and 64 or 128 words of
+// their slices, looks through a chunk of 1024 * kMine updates for those of its targets, sorts them by target in LDS and adds them up
+// window by window of kWindow updates: one atomic per word and target of a chunk, and one more for every window that a
+// target's updates run across, where a workgroup that takes the next 64 updates as they come issues one per word and
+// distinct row of those 64 (8192 log-uniform updates of 32000 rows: 3252 distinct rows, 6944 over groups of 64).
+// A window is the same work however often its targets repeat, and its loads are all in flight.
+// What bounds it: the atomics as before where there are many; below ~4 MB the chain of loading indices, sorting (five
+// barriers), loading updates and the atomics, ~6 us.  us, before / now: 8192 bf16 updates of 1024 into 32000 rows 20.5 / 17.2,
+// 65536 of 1000 into 131072 194 / 90, 16384 of 4096 into 20000 162 / 62, 49954 fp32 of 622 into 77 145 / 52, 4413 fp32 of 65
+// into 72 20.3 / 9; all indices distinct: 8192 of 1024 18.7 / 20, 16384 of 4096 110 / 117 (nothing to merge).
+// The sort is by hash, not by number: two targets of one slot may lie mixed, which costs them more
+// atomics and nothing else.
+constexpr int kOwnerThreads = 1024;
+template <typename T, int kMine, int kWords, Layout kLayout>
+__global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
+    const T* __restrict__ updates, T* __restrict__ data, const long long* __restrict__ indices, Strides s, long long n,
+    int k, long long slice, long long total, int lanes, int bucket_bits, int chunk) {
+  constexpr int kElems = Word<T>::kElems;
+  constexpr int kChunk = kMine * kOwnerThreads, kSlots = 2 * kOwnerThreads, kSlotShift = 32 - 11;
+  constexpr int kWindow = kMine > 2 ? 16 : 8;   // longer where more updates of a target meet
+  constexpr int kFlight = kWindow / kWords;     // updates whose loads are in flight
+  constexpr float kLargest = std::is_same_v<T, half_t> ? 65504.f : std::is_same_v<T, bf16_t> ? 0x1.FEp127f : 0x1.FFFFFEp127f;
+  __shared__ unsigned s_target[kChunk];          // target numbers, sorted
+  __shared__ unsigned short s_update[kChunk];    // numbers in the chunk of their updates
+  __shared__ int s_slot[kSlots];                 // updates of a slot, then the position of its first
+  __shared__ int s_wave[kOwnerThreads / kWaveSize];
+  const int tid = threadIdx.x;
+  const unsigned bucket = blockIdx.x & ((1u << bucket_bits) - 1);
+  const long long row0 = (long long)(blockIdx.x >> bucket_bits) * chunk;
+  const long long row_end = std::min(row0 + chunk, n);   // (chunk <= kChunk)
+
+  // ---- this bucket's updates ----
+  for (int i = tid; i < kSlots; i += kOwnerThreads) s_slot[i] = 0;
+  unsigned target[kMine];
+  bool inside[kMine];
+#pragma unroll
+  for (int j = 0; j < kMine; ++j) {
+    target[j] = 0;
+    inside[j] = row0 + j * kOwnerThreads + tid < row_end;
+  }
+  for (int d = 0; d < k; ++d) {
+    long long ix[kMine];   // all of them in flight
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) ix[j] = indices[std::min<long long>(row0 + j * kOwnerThreads + tid, row_end - 1) * k + d];
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) {
+      inside[j] &= ix[j] >= 0 && ix[j] < s.dim[d];
+      target[j] += (unsigned)ix[j] * (unsigned)s.stride[d];   // (below 2^32 where inside)
+    }
+  }
+  __syncthreads();
+  int rank[kMine];
+#pragma unroll
+  for (int j = 0; j < kMine; ++j) {
+    // (bucket_bits + 11 <= 32; a shift by 32 - 0 is not one)
+    const unsigned long long hash = (unsigned long long)(target[j] * 0x9E3779B1u) << bucket_bits;
+    inside[j] &= (unsigned)(hash >> 32) == bucket;
+    target[j] = inside[j] ? target[j] : 0;
+    rank[j] = inside[j] ? atomicAdd(&s_slot[(unsigned)hash >> kSlotShift], 1) : 0;
+  }
+  __syncthreads();
+  // ---- positions of the slots: two slots a thread ----
+  const int c0 = s_slot[2 * tid], c1 = s_slot[2 * tid + 1];
+  int sum = c0 + c1;
+#pragma unroll
+  for (int d = 1; d < kWaveSize; d *= 2) {
+    const int below = __shfl_up(sum, d);
+    if (tid % kWaveSize >= d) sum += below;
+  }
+  if (tid % kWaveSize == kWaveSize - 1) s_wave[tid / kWaveSize] = sum;
+  __syncthreads();
+  int before = 0, count = 0;
+#pragma unroll
+  for (int w = 0; w < kOwnerThreads / kWaveSize; ++w) {
+    if (w < tid / kWaveSize) before += s_wave[w];
+    count += s_wave[w];
+  }
+  s_slot[2 * tid] = before + sum - c0 - c1;
+  s_slot[2 * tid + 1] = before + sum - c1;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kMine; ++j)
+    if (inside[j]) {
+      const unsigned hash = (unsigned)((unsigned long long)(target[j] * 0x9E3779B1u) << bucket_bits);
+      const int at = s_slot[hash >> kSlotShift] + rank[j];
+      s_target[at] = target[j];
+      s_update[at] = (unsigned short)(j * kOwnerThreads + tid);
+    }
+  __syncthreads();
+
+  // ---- windows of sorted updates; a group of `lanes` adjacent lanes takes one at a time, kWords words a lane ----
+  const int groups = kOwnerThreads / lanes;
+  const long long word0 = (long long)blockIdx.y * lanes * kWords + (tid & (lanes - 1));
+  auto first_elem = [&](unsigned t, int v) -> long long {   // element of the slice at word v of this lane
+    return (word0 + (long long)v * lanes) * kElems - first_word_shift<T, kLayout>(data + (size_t)t * slice);
+  };
+  auto load = [&](long long row, long long e0) -> unsigned {
+    const T* src = updates + row * slice;
+    if constexpr (kLayout == Layout::kPairs) {
+      return e0 < slice ? *reinterpret_cast<const unsigned*>(src + e0) : 0u;
+    } else {
+      // (one load of two elements, at any even address, inside the slice; slice > 1)
+      typedef unsigned any_u32 __attribute__((aligned(2)));
+      const unsigned w = *reinterpret_cast<const any_u32*>(src + std::min(std::max(e0, 0ll), slice - 2));
+      // a half that is not the slice's has nothing to add: -0.0
+      return e0 < 0 ? w << 16 | 0x8000u : e0 + 1 < slice ? w : w >> 16 | 0x80000000u;
+    }
+  };
+  auto unpack = [](unsigned w) -> Word<T> {
+    Word<T> x;
+    if constexpr (kElems == 1) {
+      x.v[0] = __builtin_bit_cast(float, w);
+    } else {
+      x.v[0] = (float)__builtin_bit_cast(T, (unsigned short)w);
+      x.v[1] = (float)__builtin_bit_cast(T, (unsigned short)(w >> 16));
+    }
+    return x;
+  };
+  for (int first = tid / lanes * kWindow; first < count; first += groups * kWindow) {
+    const int end = min(first + kWindow, count);
+    Word<T> sum[kWords];
+    int from = first;   // of the updates that `sum` holds
+    auto clear = [&]() {
+#pragma unroll
+      for (int v = 0; v < kWords; ++v)
+#pragma unroll
+        for (int e = 0; e < kElems; ++e) sum[v].v[e] = -0.f;
+    };
+    clear();
+    // adds what `sum` holds of updates [from, to), all of one target
+    auto flush = [&](int to) {
+      const unsigned t = s_target[from];
+      T* const dst = data + (size_t)t * slice;
+      const long long at = (long long)((size_t)t * slice);
+#pragma unroll
+      for (int v = 0; v < kWords; ++v) {
+        const long long e0 = first_elem(t, v);
+        if (e0 >= slice) continue;
+        // A sum that T does not hold is added as its single updates, which `data` may bring back into range.
+        bool held = true;
+#pragma unroll
+        for (int e = 0; e < kElems; ++e) held &= __builtin_fabsf(sum[v].v[e]) <= kLargest;
+        if (held) {
+          add_to_slice<T, kLayout, false>(dst, sum[v], e0, slice, at, total);
+        } else {
+          for (int p = from; p < to; ++p)
+            add_to_slice<T, kLayout, false>(dst, unpack(load(row0 + s_update[p], e0)), e0, slice, at, total);
+        }
+      }
+      from = to;
+      clear();
+    };
+    for (int p0 = first; p0 < end; p0 += kFlight) {
+      unsigned raw[kFlight][kWords];
+#pragma unroll
+      for (int i = 0; i < kFlight; ++i) {
+        const int p = min(p0 + i, end - 1);   // (behind the end: the last update again, not added)
+        const unsigned t = s_target[p];
+#pragma unroll
+        for (int v = 0; v < kWords; ++v) raw[i][v] = load(row0 + s_update[p], first_elem(t, v));
+      }
+#pragma unroll
+      for (int i = 0; i < kFlight; ++i) {
+        if (p0 + i < end) {
+          if (s_target[p0 + i] != s_target[from]) flush(p0 + i);
+#pragma unroll
+          for (int v = 0; v < kWords; ++v) {
+            const Word<T> x = unpack(raw[i][v]);
+#pragma unroll
+            for (int e = 0; e < kElems; ++e) sum[v].v[e] += x.v[e];
+          }
+        }
+      }
+    }
+    flush(end);
+  }
+}
+
 template <typename T, int kThreads, int kRows, int kWords, Layout kLayout>
 int launch_shape(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
                  long long slice, long long total, int lanes, long long words, hipStream_t st) {
@@ -291,6 +470,25 @@ int launch_shape(const void* updates, void* data, const long long* indices, cons
                   (unsigned)std::min<long long>((words + per - 1) / per, 1024));
   hipLaunchKernelGGL((scatter_nd_kernel<T, kThreads, kRows, kWords, kLayout>), grid, dim3(kThreads), 0, st,
                      static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
+  TFK_HIP_TRY(hipGetLastError());
+  return TF_OK;
+}
+
+// As many buckets (a power of two, at least two) as bring about 224 workgroups: one a CU.
+template <typename T, int kMine, int kWords, Layout kLayout>
+int launch_owner(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
+                 long long slice, long long total, int lanes, long long words, hipStream_t st) {
+  Strides numbers = s;
+  for (int d = 0; d < k; ++d) numbers.stride[d] /= slice;   // the number of a target, not its first element
+  const long long chunks = (n + kMine * kOwnerThreads - 1) / (kMine * kOwnerThreads);
+  const long long columns = (words + lanes * kWords - 1) / (lanes * kWords);
+  int bits = 1;
+  while (bits < 8 && chunks * columns * 3 << bits <= 2 * 224) ++bits;
+  const int chunk = (int)((n + chunks - 1) / chunks);   // (even ones: no nearly empty last chunk)
+  const dim3 grid((unsigned)((n + chunk - 1) / chunk) << bits, (unsigned)columns);
+  hipLaunchKernelGGL((scatter_nd_owner_kernel<T, kMine, kWords, kLayout>), grid, dim3(kOwnerThreads), 0, st,
+                     static_cast<const T*>(updates), static_cast<T*>(data), indices, numbers, n, k, slice, total, lanes, bits,
+                     chunk);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
@@ -324,23 +522,34 @@ int launch_rows(const void* updates, void* data, const long long* indices, const
                 long long slice, long long targets, int lanes, long long words, hipStream_t st) {
   if (!is_ordinary_device_memory(data))
     return launch_direct<T, kLayout, true>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  // Times in us with log-uniform indices (threads / updates a workgroup).  Few updates: no sort (806 of
-  // 34 fp32: direct 3.3, 256/16 5.6).  From 1024 on contention shows (2048 of 64 bf16 into 64 rows:
-  // direct 10.8, 256/16 6.3, 512/64 8.2), beyond 2048 more updates per sort pay (4096 of 1024 bf16
-  // into 1000 rows: direct 26, 256/16 17.6, 512/64 12.9).
+  // Times in us with log-uniform indices.  Few updates: no sort (806 of 34 fp32: direct 3.3, 16 of 256 threads' updates
+  // sorted 5.6).  From 1024 on contention shows (2048 of 64 bf16 into 64 rows: direct 10.8, sorted 6.3).
   if (n <= 1024)
     return launch_direct<T, kLayout, false>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  if (n <= 2048)
+  // Beyond, owners of targets, except: a few 16-bit updates (1489 of 1206 bf16 into 1412 rows: 9.4 sorted by 16, 10.4 by
+  // owners; 1894 of 3924 21.8 and 14.6; 1077 fp32 of 26 into 95 5.6 and 6.1, 1469 of 68 into 350 8.1 and 6.9), and narrow slices whose targets are hit often, for which the sort of the next 128
+  // finds as much to merge (58345 of 55 fp16 into 306 rows: 42 and 54).  (Target numbers are 32 bits there.)
+  const bool owners_fit = targets < (1ll << 32) && n < (1ll << 31) && (kLayout == Layout::kPairs || slice > 1) &&
+                          words <= 1024ll * lanes;
+  if ((n <= 2048 && ((sizeof(T) == 2 && n * words < 2 << 20) || !owners_fit)) || n <= 1280)
     return launch_shape<T, 256, 16, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  // Every target hit at least eight times on average: the deeper sort (59764 of 21 fp32 into 219 rows:
-  // 512/64 43, 1024/128 31; 49954 of 622 fp32 into 77: 175 and 143).
-  if (n / 8 >= targets)
+  if (!owners_fit || (words <= 32 && n > 8192 && n / 16 >= targets))
     return launch_shape<T, 1024, 128, 2, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  // A workgroup of eight wavefronts hides its own latencies where there are few of them (16384 of 64
-  // bf16: 256/64 13.8, 512/64 12.5); enough of four do it better (8192 of 1024 fp32: 31.9 and 40.1).
-  if ((n / 64) * ((words + lanes - 1) / lanes) < 1024)
-    return launch_shape<T, 512, 64, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  return launch_shape<T, 256, 64, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+  // Longer chunks find more to merge and cost workgroups (16384 bf16 of 4096 into 20000 rows: 2048 updates a chunk 72,
+  // 8192 61; 8192 of 1024 into 32000 17.2 and 19.2); unpaired halves lose by them (45202 bf16 of 365 into 64 rows 49, 92).
+  // Two words a lane, likewise, halve the workgroups that look through the same indices, from 256 words on.
+  auto owners = [&](auto mine, auto per_lane) -> int {
+    return launch_owner<T, decltype(mine)::value, decltype(per_lane)::value, kLayout>(
+        updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+  };
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  if constexpr (kLayout == Layout::kPairs) {
+    using Eight = std::integral_constant<int, 8>;
+    if (n >= 20000) return words > 256 ? owners(Eight{}, Two{}) : owners(Eight{}, One{});
+    if (words > 256) return owners(Two{}, Two{});
+  }
+  return owners(Two{}, One{});
 }
 
 template <typename T>
