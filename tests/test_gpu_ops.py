@@ -334,3 +334,58 @@ def test_fused_two_gemms_and_flash_attention_ops_bf16():
         assert o.dtype == torch.bfloat16
         ref = N.attention_ref(q, k, v, 1 / math.sqrt(128), causal)
         assert _close_bf16(o, ref), (causal, N.rel_l2(o, ref), N.max_abs(o, ref))
+
+
+# The wrappers call the implementations directly where nothing is to see the call; a mode, a profiler, autocast, a gradient
+# or a subclass gets the op itself.  Same results and same errors either way.
+def test_direct_calls_and_ops_agree_and_observers_see_the_ops():
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from tilefusion_amd import _direct, ops
+    g = torch.Generator().manual_seed(3)
+    a, b = (torch.randn(n, 96, generator=g).half().to(DEV) for n in (70, 40))
+    c, c2 = (torch.empty(70, 40, device=DEV, dtype=torch.float32) for _ in range(2))
+    q, k, v = (torch.randn(2, n, 64, generator=g).half().to(DEV) for n in (1, 200, 200))
+    e, f = torch.randn(64, 40, generator=g).half().to(DEV), torch.empty(70, 64, device=DEV, dtype=torch.float16)
+    idx, upd = torch.tensor([[1], [3], [1]], device=DEV), torch.ones(3, 8, device=DEV)
+    data = torch.zeros(5, 8, device=DEV)
+    calls = {
+        "gemm": lambda: (ops.gemm(a, b, c2, 1, 1, 1, 1, 1), c2)[1],
+        "fused_two_gemms": lambda: (ops.fused_two_gemms(a, b, e, f, 1, 1, 1, 1), f)[1],
+        "flash_attention_fwd": lambda: ops.flash_attention(q, k.transpose(-1, -2), v, 1, 1, 64, 64, 0.125, False),
+        "flash_attention_fwd_kt": lambda: ops.flash_attention(q, k.transpose(-1, -2).contiguous(), v, 1, 1, 64, 64, 0.125, False),
+        "flash_decode": lambda: ops.flash_decode(q, k, v, 2),
+        "scatter_nd": lambda: (data.zero_(), ops.scatter_nd(data, idx, upd), data)[2],
+    }
+    assert _direct.gemm(a, b, c, 1, 1, 1, 1, 1)
+    seen = []
+
+    class Log(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+    for name, call in calls.items():
+        direct = call().clone()
+        with Log():
+            through_op = call().clone()
+        assert any(s.startswith(f"tilefusion.{name}.") for s in seen), (name, seen)
+        assert torch.equal(direct, through_op), name
+        with torch.autograd.profiler.profile() as prof:
+            call()
+        assert any(x.name == f"tilefusion::{name}" for x in prof.function_events), name
+    ok, r, m = N.check_close(c, (a.float() @ b.float().T).cpu())
+    assert ok
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert not _direct.gemm(a, b, c, 1, 1, 1, 1, 1)
+    assert not _direct.gemm(a.clone().requires_grad_(), b, c, 1, 1, 1, 1, 1)
+    assert not _direct.gemm(a, b, c.cpu(), 1, 1, 1, 1, 1)
+    assert not _direct.gemm(a, b, c, 1, 1, 1, 1, True) and not _direct.gemm(a, b, c, 1, 1, 1, 1)
+    assert not torch.vmap(lambda x: torch.tensor(_direct.gemm(x, b, c, 1, 1, 1, 1, 1)))(torch.stack([a, a])).any()
+    for bad in (lambda: ops.gemm(a.t(), b, c, 1, 1, 1, 1, 1), lambda: ops.gemm(a, b, c, 64, 64, 64, 1, 1),
+                lambda: ops.gemm(a.float(), b, c, 1, 1, 1, 1, 1), lambda: ops.flash_decode(q, k, v[:1], 2),
+                lambda: ops.flash_attention(q, k, v, 1, 1, 64, 64, 0.125, False), lambda: ops.scatter_nd(data, idx.int(), upd)):
+        with pytest.raises(RuntimeError) as direct:
+            bad()
+        with Log(), pytest.raises(RuntimeError) as through_op:
+            bad()
+        assert str(direct.value).splitlines()[0] == str(through_op.value).splitlines()[0]

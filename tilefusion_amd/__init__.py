@@ -32,6 +32,8 @@ def _load_library(filename: str) -> Any:
 
 
 _lib = _load_library("libtilefusion.so")
+if not os.path.exists(os.path.join(_HERE, "_direct.so")):
+    raise RuntimeError(f"{_HERE}/_direct.so is missing: build it with `make -C tilefusion_amd/csrc all bind`")
 
 from . import _capi, jit, ops  # noqa: E402
 

@@ -1,0 +1,175 @@
+// Python module tilefusion_amd._direct: the ops' implementations called without the dispatcher.
+//
+// A call of torch.ops.tilefusion.* from Python costs ~2 us beside the launch (matching the arguments to the schema,
+// boxing them, three dispatch keys that fall through), as much as the launch of a small kernel.  The functions
+// here take a call only where the dispatcher would do nothing but call the implementation: plain
+// device tensors, no gradient asked for, nothing that watches or rewrites ops (see `plain`).  Otherwise they
+// return False (None), having done nothing, and the wrapper in tilefusion_amd/ops goes through torch.ops, as it does for
+// torch.compile and torch.jit.script.  (An implementation that a program registers for the CUDA key in place of the
+// library's is seen through torch.ops only.)
+// us a call in a loop, through torch.ops / as here: gemm 128 x 64 x 256 4.5 / 3.3, fused 16384 x 128 x 128 x 128
+// 6.2 / 4.4 (its kernel), decoding 32 x 1999 x 64 10.7 / 8.4 (two launches).
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/record_function.h>
+#include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cmath>
+#include <vector>
+
+#include "torch_bind.hpp"
+
+namespace {
+
+// Dispatch keys under which these ops, which register an implementation for CUDA only, do what is written
+// here: the implementation, and keys that fall through to it when no gradient is asked for.
+const c10::DispatchKeySet kPlainKeys =
+    c10::DispatchKeySet(c10::DispatchKey::CUDA) | c10::DispatchKeySet(c10::DispatchKey::AutogradCUDA) |
+    c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView) | c10::DispatchKeySet(c10::DispatchKey::BackendSelect);
+
+// Takes the tensors out of args[0 .. n); false unless every one is an ordinary torch.Tensor (no subclass) on a GPU that
+// wants no gradient, and no mode, transform, autocast, tracer or profiler is to see the call.
+bool plain(PyObject* const* args, int n, at::Tensor* out) {
+  c10::DispatchKeySet keys;
+  for (int i = 0; i < n; ++i) {
+    if (!THPVariable_CheckExact(args[i])) return false;
+    const at::Tensor& t = THPVariable_Unpack(args[i]);
+    if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided) return false;
+    if (t.requires_grad() || t._fw_grad(0).defined()) return false;
+    keys = keys | t.key_set();
+    out[i] = t;   // (held while the interpreter is unlocked)
+  }
+  const auto local = c10::impl::tls_local_dispatch_key_set();
+  keys = ((keys | local.included_) - local.excluded_) - kPlainKeys;
+  return keys.highestFunctionalityKey() == c10::DispatchKey::Undefined && !at::impl::torch_function_mode_enabled() &&
+         !at::hasCallbacks();
+}
+
+// ints only (a bool, a numpy number or a tensor is the dispatcher's business)
+bool ints(PyObject* const* args, int n, int64_t* out) {
+  for (int i = 0; i < n; ++i) {
+    if (!PyLong_CheckExact(args[i])) return false;
+    out[i] = PyLong_AsLongLong(args[i]);
+    if (out[i] == -1 && PyErr_Occurred()) {
+      PyErr_Clear();
+      return false;
+    }
+  }
+  return true;
+}
+
+struct NoGil {   // as the dispatcher: other threads run while a call is prepared
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
+bool is_half_type(const at::Tensor& t) { return t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16; }
+
+PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  at::Tensor t[3];
+  int64_t i[5];
+  if (nargs != 8 || !plain(args, 3, t) || !ints(args + 3, 5, i)) Py_RETURN_FALSE;
+  {
+    NoGil unlocked;
+    tilefusion::kernels::gemm(t[0], t[1], t[2], i[0], i[1], i[2], i[3], i[4]);
+  }
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* fused_two_gemms(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  at::Tensor t[4];
+  int64_t i[4];
+  if (nargs != 8 || !plain(args, 4, t) || !ints(args + 4, 4, i)) Py_RETURN_FALSE;
+  for (const at::Tensor& x : t)   // (other types: the wrapper's own errors)
+    if (!is_half_type(x) || x.scalar_type() != t[0].scalar_type()) Py_RETURN_FALSE;
+  {
+    NoGil unlocked;
+    tilefusion::kernels::fused_two_gemms(t[0], t[1], t[2], t[3], i[0], i[1], i[2], i[3]);
+  }
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* scatter_nd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {   // data, updates, indices
+  HANDLE_TH_ERRORS
+  at::Tensor t[3];
+  if (nargs != 3 || !plain(args, 3, t)) Py_RETURN_FALSE;
+  {
+    NoGil unlocked;
+    tilefusion::kernels::scatter_nd(t[0], t[1], t[2]);
+  }
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
+// (query, key [.., D, Lkv], value, tile_length_q, tile_length_kv, tile_hidden_qk, tile_hidden_v, softmax_scale, causal)
+// -> output, or None
+PyObject* flash_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  at::Tensor t[3];
+  int64_t tile[4];
+  if (nargs != 9 || !plain(args, 3, t) || !ints(args + 3, 4, tile) || !PyFloat_CheckExact(args[7]) || !PyBool_Check(args[8]))
+    Py_RETURN_NONE;
+  const at::Tensor &q = t[0], &k = t[1], &v = t[2];
+  if (q.dim() < 2 || k.dim() < 2 || v.dim() < 2) Py_RETURN_NONE;
+  const int64_t extent[4] = {q.size(-2), v.size(-2), q.size(-1), v.size(-1)};
+  for (int i = 0; i < 4; ++i)
+    if (tile[i] <= 0 || extent[i] % tile[i] != 0) Py_RETURN_NONE;
+  const double scale = PyFloat_AS_DOUBLE(args[7]);
+  const bool causal = args[8] == Py_True;
+  at::Tensor out;
+  {
+    NoGil unlocked;
+    std::vector<int64_t> shape(q.sizes().begin(), q.sizes().end());
+    shape.back() = v.size(-1);
+    out = at::empty(shape, q.options());
+    const at::Tensor key_rows = k.transpose(-1, -2);
+    if (k.is_contiguous() && !key_rows.is_contiguous())
+      tilefusion::kernels::flash_attention_fwd_kt(q.contiguous(), k, v.contiguous(), out, scale, causal);
+    else
+      tilefusion::kernels::flash_attention_fwd(q.contiguous(), key_rows.contiguous(), v.contiguous(), out, scale, causal);
+  }
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// (query, key, value, num_splits, softmax_scale or None) -> output, or None
+PyObject* flash_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  at::Tensor t[3];
+  int64_t num_splits;
+  if (nargs != 5 || !plain(args, 3, t) || !ints(args + 3, 1, &num_splits)) Py_RETURN_NONE;
+  if (args[4] != Py_None && !PyFloat_CheckExact(args[4])) Py_RETURN_NONE;
+  const at::Tensor &q = t[0], &k = t[1], &v = t[2];
+  if (q.dim() < 1 || q.size(-1) < 1) Py_RETURN_NONE;
+  const double scale = args[4] == Py_None ? 1.0 / std::sqrt((double)q.size(-1)) : PyFloat_AS_DOUBLE(args[4]);
+  at::Tensor out;
+  {
+    NoGil unlocked;
+    out = at::empty_like(q);
+    tilefusion::kernels::flash_decode(q.contiguous(), k.contiguous(), v.contiguous(), out, num_splits, scale);
+  }
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+template <PyObject* (*kFunction)(PyObject*, PyObject* const*, Py_ssize_t)>
+constexpr PyMethodDef method(const char* name) {
+  return {name, (PyCFunction)(void (*)(void))kFunction, METH_FASTCALL, nullptr};
+}
+PyMethodDef methods[] = {method<gemm>("gemm"), method<fused_two_gemms>("fused_two_gemms"), method<scatter_nd>("scatter_nd"),
+                         method<flash_attention>("flash_attention"), method<flash_decode>("flash_decode"),
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_direct", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__direct() { return PyModule_Create(&module); }

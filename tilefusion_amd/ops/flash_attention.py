@@ -2,6 +2,8 @@
 
 import torch
 
+from .. import _direct
+
 __all__ = ["FlashAttention", "flash_attention"]
 
 
@@ -32,6 +34,13 @@ class FlashAttention:
         (python/ops/flash_attention.py:73-74); here the value is consumed in its natural layout, and
         the key either as a transposed view of a [Lkv, D] tensor or stored [D, Lkv] (the kernel
         transposes both on the way from LDS to registers).  Tile sizes are validated against the problem."""
+        if not torch.compiler.is_compiling():
+            direct = _direct.flash_attention(
+                query, key, value, self.tile_length_q, self.tile_length_kv, self.tile_hidden_qk, self.tile_hidden_v,
+                self.softmax_scale, self.causal
+            )
+            if direct is not None:
+                return direct
         length_q, hidden_qk = query.size(-2), query.size(-1)
         length_kv, hidden_v = value.size(-2), value.size(-1)
         for what, dim, tile in (("length_q", length_q, self.tile_length_q),

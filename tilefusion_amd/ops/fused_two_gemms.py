@@ -2,6 +2,8 @@
 
 import torch
 
+from .. import _direct
+
 __all__ = ["fused_two_gemms"]
 
 
@@ -40,6 +42,11 @@ def fused_two_gemms(
 
     All four tensors are float16 (as in the reference) or all bfloat16.
     """
+    if not torch.jit.is_scripting():
+        if not torch.compiler.is_compiling() and _direct.fused_two_gemms(
+            input_a, input_b, input_c, output, tm, tn, tk, tp
+        ):
+            return
     dtype = torch.bfloat16 if input_a.dtype == torch.bfloat16 else torch.float16
     _validate_tensor(input_a, "input_a", dtype)
     _validate_tensor(input_b, "input_b", dtype)

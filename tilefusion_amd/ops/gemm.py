@@ -2,6 +2,8 @@
 
 import torch
 
+from .. import _direct
+
 __all__ = ["gemm"]
 
 
@@ -26,6 +28,11 @@ def gemm(
         num_stages: 1..3, pipeline_level: 0..2 - validated, kept for signature parity (LDS
             double buffering is always on).
     """
+    if not torch.jit.is_scripting():
+        if not torch.compiler.is_compiling() and _direct.gemm(
+            tensor_a, tensor_b, tensor_c, tile_m, tile_n, tile_k, num_stages, pipeline_level
+        ):
+            return
     torch.ops.tilefusion.gemm(
         tensor_a, tensor_b, tensor_c, tile_m, tile_n, tile_k, num_stages, pipeline_level
     )

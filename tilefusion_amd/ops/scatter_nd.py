@@ -2,6 +2,8 @@
 
 import torch
 
+from .. import _direct
+
 __all__ = ["scatter_nd"]
 
 
@@ -13,4 +15,7 @@ def scatter_nd(scatter_data: torch.Tensor, scatter_indices: torch.Tensor, scatte
     ([.., d(k), .., d(r-1)]) is added.  Duplicate index rows accumulate, like the reference
     kernel's atomicAdd (src/kernels/scatter_nd.cu:30); rows outside the tensor are skipped.
     """
+    if not torch.jit.is_scripting():
+        if not torch.compiler.is_compiling() and _direct.scatter_nd(scatter_data, scatter_updates, scatter_indices):
+            return
     torch.ops.tilefusion.scatter_nd(scatter_data, scatter_updates, scatter_indices)
