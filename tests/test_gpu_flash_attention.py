@@ -127,6 +127,25 @@ def test_every_workgroup_size(rows, b, lq, lkv, d, causal):
     assert torch.equal(ops.flash_attention(q.to(DEV), kt, v.to(DEV), 1, 1, d, d, d ** -0.5, causal), o)
 
 
+# Single causal tiles dealt by XCD (slice counts that 8 does not divide) and not, and pairs of 64-query tiles of wide
+# heads: every tile of every slice is done once, with the bits of the slice alone.
+@pytest.mark.parametrize("bh,lq", [(31, 320), (30, 160), (63, 192), (61, 544), (9, 96), (150, 384), (225, 256)])
+@pytest.mark.parametrize("d", [64, 128, 192, 256])
+def test_causal_orders_agree(bh, lq, d):
+    q, k, v = (x.to(DEV) for x in _inputs(bh, lq, lq, d, bh + lq + d))
+    o = torch.full_like(q, float("nan"))
+    torch.ops.tilefusion.flash_attention_fwd(q, k, v, o, d ** -0.5, True)
+    assert not torch.isnan(o).any()
+    for i in (0, 7, 8, bh // 2, bh - 1):
+        alone = torch.empty_like(o[i:i + 1])
+        torch.ops.tilefusion.flash_attention_fwd(q[i:i + 1].contiguous(), k[i:i + 1].contiguous(), v[i:i + 1].contiguous(), alone,
+                                                 d ** -0.5, True)
+        assert torch.equal(o[i:i + 1], alone), i
+    ref = torch.softmax((q.float() @ k.float().transpose(1, 2).contiguous() * d ** -0.5).masked_fill(
+        torch.ones(lq, lq, dtype=torch.bool, device=DEV).triu(1), float("-inf")), -1) @ v.float()
+    assert (o.float() - ref).norm() <= 1e-3 * ref.norm()
+
+
 def test_scale_and_large_logits():
     # scale enters the logits; big logits need the running max (exp would overflow otherwise)
     q, k, v = _inputs(2, 128, 256, 128, 77)

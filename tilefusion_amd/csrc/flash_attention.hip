@@ -115,18 +115,21 @@ int run_tuned(const void* Q, const void* K, const void* V, void* O, bool bf16, i
   return D == 128 ? run_attention_d128(c) : D == 96 ? run_attention_d96(c) : run_attention_d64(c);
 }
 
-// Head dimensions above 128 (V as it comes, whole key tiles): single tiles (pairs lost everywhere: 64 slices of 2048 x
-// 2048 308 / 271, 80 of 1024 169 / 107), 64 or 128 queries a workgroup, the larger one
-// where it saves a round of the CUs.  bf16, D = 256, 64 / 128 queries: 8 slices of 2048 x 2048 69 / 95 us, 32 of
-// 1024 x 1024 89 / 64, 100 of 384 x 384 58 / 56; causal, 32 of 1024 x 1024 49 / 64 (193 by the kernel compiled
-// at run time, with its transposed copy of V), 40 of them 67 / 63, 64 of them 100 / 81.
-inline bool wide_takes_128_queries(int64_t batch, int64_t Lq, bool causal) {
-  auto rounds = [&](int rows) -> double {
-    const int64_t items = (Lq + rows - 1) / rows * batch;
-    if (causal) return std::max(1.0, (double)items / 512.0);   // a tile is half of the heaviest on average
-    return (double)((items + 255) / 256);
-  };
-  return 1.1 * rounds(128) < rounds(64);
+// Head dimensions above 128 (V as it comes, whole key tiles): workgroups of 64 queries, two to a CU; 128 (8 wavefronts, one
+// to a CU) where those are just one for every CU: the tiles come from the L2 half as often, and nothing is left for a second
+// round.  bf16, 64 / 128 queries: 128 slices of 256 x 4096 x 160 162 / 147 us, 256 of 128 x 2048 x 192 106 / 99, 32 of 1000 x
+// 1024 x 256 52 / 54; 320 workgroups of 128 are 25% behind.
+// Causal: pairs of tiles where they fill rounds of two a CU, and single tiles, heaviest first, otherwise.  D = 256,
+// singles / pairs: 341 slices of 384 (1024 pairs) 80 / 60, 150 of 384 (450) 32.7 / 30.5, 192 of 256 (384) 24.2 / 25.3, 320 of
+// 1024 39 / 51.  (128 queries a workgroup are up to 30% behind the better of the two.)
+AttentionPlan plan_wide(int64_t batch, int64_t Lq, bool causal) {
+  const int64_t tiles = (Lq + 63) / 64;
+  if (causal) {
+    const int64_t pairs = tiles / 2 * batch, rounds = (pairs + 511) / 512;
+    return {64, tiles % 2 == 0 && 100 * pairs >= 86 * 512 * rounds};
+  }
+  const int64_t large = (tiles + 1) / 2 * batch;
+  return {tiles % 2 == 0 && large >= 244 && large <= 256 ? 128 : 64, false};
 }
 
 int check_attention_args(const char* who, const void* Q, const void* K, const void* V, const void* O, int64_t batch,
@@ -222,9 +225,9 @@ extern "C" int tf_flash_attention_fwd_wide(const void* Q, const void* K, const v
                reinterpret_cast<uintptr_t>(O)) % 16 == 0, TF_ERR_UNSUPPORTED,
               "tf_flash_attention_fwd_wide: operands must start at a 16-byte boundary");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const AttentionPlan plan = plan_wide(batch, Lq, causal != 0);
   const AttentionCall c = {Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (float)(softmax_scale * 1.4426950408889634),
-                           dtype == TF_DTYPE_BF16, false, false, causal != 0,
-                           wide_takes_128_queries(batch, Lq, causal != 0) ? 128 : 64, false, st};
+                           dtype == TF_DTYPE_BF16, false, false, causal != 0, plan.rows, plan.paired, st};
   return run_attention_wide(c, (int)D);
 }
 
@@ -253,5 +256,6 @@ extern "C" int tf_flash_attention_rows(int64_t batch, int64_t Lq, int64_t Lkv, i
 }
 
 extern "C" int tf_flash_attention_wide_rows(int64_t batch, int64_t Lq, int causal) {
-  return tfk::wide_takes_128_queries(batch, Lq, causal != 0) ? 128 : 64;
+  const tfk::AttentionPlan plan = tfk::plan_wide(batch, Lq, causal != 0);
+  return plan.paired ? 2 * plan.rows : plan.rows;
 }

@@ -34,8 +34,9 @@ namespace {
 // 32 keys leave room for a ring of four.
 __host__ __device__ constexpr int key_tile(int d) { return d <= 128 ? 64 : 32; }
 // LDS ring depth: the 8-wavefront kernel keeps two tiles live (its two wavefront sets are half a
-// tile apart) and three in flight; the 4-wavefront kernel one live and three in flight.
-__host__ __device__ constexpr int ring_stages(int waves) { return waves == 8 ? 5 : 4; }
+// tile apart) and three in flight; the 4-wavefront kernel one live and three in flight, or, with head dimensions above
+// 128, one live and one in flight, so that two workgroups share a CU.
+__host__ __device__ constexpr int ring_stages(int waves, int d) { return waves == 8 ? 5 : d > 128 ? 2 : 4; }
 // Row pitch (in elements) of a [key][dim] tile in LDS: the next power of two.  The swizzles XOR
 // chunk indices, which needs a power-of-two chunk count, and a 1 KiB request must cover whole
 // rows.  A head dimension of 96 is kept in 128-element rows whose last quarter is never read (160 and
@@ -61,6 +62,9 @@ __host__ __device__ constexpr int swz_v(int row, int c) {
 __host__ __device__ constexpr int swz_kt(int row, int c) {
   return c ^ ((((row >> 1) & 1) | ((row >> 2) & 2)) << 1);
 }
+
+// What a workgroup's number stands for (causal; see the kernel).
+enum : int { kSingle = 0, kPairs = 1, kByXcd = 2 };
 
 typedef __fp16 fp16x4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
 
@@ -142,14 +146,12 @@ TFK_DEVICE SplitWeight<T> split_weight(float p) {
 // kWavesT wavefronts x 16 * kQB queries per workgroup.  8 x 32 (256 queries) read K and V fragments
 // least often per query and put two wavefronts on every SIMD, so one wavefront's softmax
 // (VALU) overlaps the other's MFMAs; 8 x 16 and 4 x 16 take less time for a key tile (D = 128: 0.9 and 0.77 us
-// against 1.3) but more for a query, and serve problems that do not fill the chip with 256; 4 wavefronts with
-// 32 or 16 queries each serve head dimensions above 128.
+// against 1.3) but more for a query, and serve problems that do not fill the chip with 256, and head dimensions above 128.
 //
-// Above 128 (kWide) the output accumulators and Q fragments of 32 queries take 192 registers, which two
-// wavefronts on a SIMD do not have.  What bounds these instances: the four wavefronts read the whole
-// K and V tile each, 128 KiB of LDS reads a key tile (1024 cycles) for 100 MFMAs (1600 cycles) on each SIMD with 32
-// queries a wavefront and 50 (800) with 16, and one wavefront per SIMD puts the softmax behind them
-// instead of beside them.
+// Above 128 (kWide) two 4-wavefront workgroups share a CU, each with a ring of two tiles, so that one's softmax runs
+// beside the other's MFMAs: what bounds them then is the LDS reads, 128 KiB a key tile of a workgroup (1024 cycles; its MFMAs
+// take 800 on each SIMD).  64 slices of 512 x 4096 x 256, bf16: 290 us with one workgroup a CU, 64 or 128 queries, and a ring
+// of four tiles, 256 with two, 203 without the wait of q_is_there; causal, 32 of 1024 x 1024 x 256: 53, 51 and 39.
 // The weights enter the second product as a 16-bit number and a 16-bit remainder (pb_rest): rounded to 16
 // bits once, against a reference that is raised lazily, they made the result 5% worse (relative error of
 // 4 slices of 1024 x 1024 x 256, bf16, against 64 bits: 2.33e-3, against the true running maximum, whose
@@ -166,15 +168,16 @@ TFK_DEVICE SplitWeight<T> split_weight(float p) {
 // as [Lkv][D] / as [D][Lkv] / copied first: 64 slices of 4096 x 4096 x 128 444 / 449 / 534, causal 241 / 254 / 340; 16 of
 // 1024 x 1024 x 128 29 / 31 / 40; 32 of 100 x 8192 x 128 157 / 176 / 266; 64 of 1336 x 1336 x 64 causal 30 / 31 / 45).
 template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB>
-__global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
+__global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1) void flash_attention_fwd_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
-    T* __restrict__ O, int Lq, int Lkv, float scale_log2, int q_tiles, int total_items, int paired) {
+    T* __restrict__ O, int Lq, int Lkv, float scale_log2, int q_tiles, int total_items, int order) {
   using V2 = typename Vec<T>::v2;
   using V4 = typename Vec<T>::v4;
   using V8 = typename Vec<T>::v8;
   constexpr bool kWide = D > 128;
   constexpr int kBN = key_tile(D);
-  constexpr int kStages = ring_stages(kWavesT);
+  constexpr int kStages = ring_stages(kWavesT, D);
+  constexpr bool kPairOnCU = kStages == 2;
   constexpr int kRowsPerWave = 16 * kQB;  // kQB 16-query blocks per wavefront
   constexpr int kBMq = kWavesT * kRowsPerWave;
   constexpr int DP = lds_pitch(D), DVP = lds_pitch(DV);   // LDS row pitch of the K / natural V tile
@@ -208,11 +211,11 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   //               same amount of work, no sorting by weight is needed and the slice-major
   //               order (with its L2 locality) is kept.  Where that is done sooner (the
   //               caller tells) and with an odd number of query tiles, one tile per workgroup,
-  //               heaviest first over all slices.
+  //               heaviest first over all slices (kSingle) or over those of an XCD (kByXcd).
   int qt_of_pass[2] = {0, 0};
   int num_passes = 1;
   size_t bh;
-  if (!kCausal || (D <= 128 && paired)) {
+  if (!kCausal || order == kPairs) {
     const int per_slice = kCausal ? q_tiles / 2 : q_tiles;
     const int per_xcd = (total_items + 7) / 8;
     const int item = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
@@ -227,10 +230,18 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
       qt_of_pass[0] = p;
     }
   } else {
-    if ((int)blockIdx.x >= total_items) return;
     const int slices = total_items / q_tiles;
-    qt_of_pass[0] = q_tiles - 1 - (int)blockIdx.x / slices;
-    bh = blockIdx.x % slices;
+    if (order == kByXcd) {
+      const int xcd = (int)blockIdx.x % 8, p = (int)blockIdx.x / 8;
+      const int own = (slices - xcd + 7) / 8;   // slices of this XCD
+      if (p >= own * q_tiles) return;
+      qt_of_pass[0] = q_tiles - 1 - p / own;
+      bh = xcd + 8 * (p % own);
+    } else {
+      if ((int)blockIdx.x >= total_items) return;
+      qt_of_pass[0] = q_tiles - 1 - (int)blockIdx.x / slices;
+      bh = blockIdx.x % slices;
+    }
   }
   Q += bh * (size_t)Lq * D;
   K += bh * (size_t)Lkv * D;
@@ -367,7 +378,9 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   //   K fragment (kb, kk) - A operand, 16 keys x 32 dims: row 16*kb + lr, logical chunk 4*kk + lg.
   //     K kept [dim][key]: rows 32*kk + 8*lg (+4) .. +3, columns 16*kb .. +15, transposed by the read; lane r of
   //     a 16-lane group addresses row r/4, columns 4*(r%4) .. +3 of that block.  The lane part is kept per kb.
-  constexpr int kKOffs = kKT ? kKB : kKK;
+  //     (256-element rows: the swizzles reach the low 16 of 32 chunks, so that steps and blocks half a row apart
+  //     differ by a constant and share an offset)
+  constexpr int kKOffs = kKT ? kKB : kKChunks > 16 ? 4 : kKK;
   unsigned k_off[kKOffs];
   if constexpr (kKT) {
     const int row_l = 8 * lg + (lr >> 2);
@@ -378,7 +391,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     }
   } else {
 #pragma unroll
-    for (int kk = 0; kk < kKK; ++kk) k_off[kk] = lr * DP * 2 + swz_k<kKChunks>(lr, 4 * kk + lg) * 16;
+    for (int kk = 0; kk < kKOffs; ++kk) k_off[kk] = lr * DP * 2 + swz_k<kKChunks>(lr, 4 * kk + lg) * 16;
   }
   //   Reduction step j of the second product covers keys 32*j .. +31; slot t of lane group lg
   //   is key 32*j + 4*lg + t (t < 4) or 32*j + 16 + 4*lg + (t - 4): exactly the keys whose
@@ -389,12 +402,12 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   //     columns 4*(r%4) .. +3 of that block.  One offset per (db & 1, db / 2 via XOR) would not
   //     be constant, so the lane part is kept per db.
   //     V kept [dim][key]: row 16*db + lr, keys 32*j + 4*lg (+16) .. +3 (8 bytes each).
-  constexpr int kVOffs = kVT ? 2 * kJ : kDB;
+  constexpr int kVOffs = kVT ? 2 * kJ : kVChunks > 16 ? 8 : kDB;
   unsigned v_off[kVOffs];
   if constexpr (!kVT) {
     const int row_l = 4 * lg + (lr >> 2);
 #pragma unroll
-    for (int db = 0; db < kDB; ++db) {
+    for (int db = 0; db < kVOffs; ++db) {
       const int col = db * 16 + 4 * (lr & 3);
       v_off[db] = row_l * DVP * 2 + swz_v<kVChunks>(row_l, col / 8) * 16 + (col % 8) * 2;
     }
@@ -437,13 +450,13 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
   // kWide: one wavefront a SIMD and few MFMAs a step, so K fragments are requested two steps ahead, and the V
   // fragments during the QK product, behind whose MFMAs they arrive (causal, D = 256, before the
   // weights had a remainder: 32 slices of 1024 x 1024 52.5 -> 47.0 us, 8 of 4096 173 -> 157; D = 160: 46.2 -> 44.8).
-  constexpr int kKAhead = kWide ? 2 : 1;
+  constexpr int kKAhead = kWide && D <= 192 && kWavesT == 4 ? 2 : 1;
   V8 kf[kKAhead + 1][kKB];   // K fragments of reduction step kk (buffer kk % (kKAhead + 1))
-  V8 vf[2][kDB];   // V fragments of reduction step j (buffer j & 1)
+  V8 vf[kJ > 1 ? 2 : 1][kDB];   // V fragments of reduction step j (buffer j & 1)
   // lane address of the fragments of step kk (kKT: recomputed per fragment)
   auto k_addr = [&](int it, int kk) __attribute__((always_inline)) {
     const unsigned stage_base = smem_base + (it % kStages) * kStageBytes;
-    return kKT ? stage_base : opaque(stage_base + k_off[kk]);
+    return kKT ? stage_base : opaque(stage_base + k_off[kk % kKOffs]) + kk / kKOffs * 256;
   };
   auto k_read = [&](int buf, unsigned ka, int kk, int kb) __attribute__((always_inline)) {
     if constexpr (kKT) {
@@ -472,7 +485,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     {
       V4 lo, hi;
       if constexpr (!kVT) {
-        const unsigned va = opaque(stage_base + v_off[db]) + kKBytes;
+        const unsigned va = opaque(stage_base + v_off[db % kVOffs]) + db / kVOffs * 256 + kKBytes;
         lo = lds_read_tr4<V4>(va + (32 * j) * DVP * 2);
         hi = lds_read_tr4<V4>(va + (32 * j + 16) * DVP * 2);
       } else {
@@ -642,7 +655,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
 #pragma unroll
     for (int j = 0; j < kJ; ++j) {
       if (j + 1 < kJ) v_reads((j + 1) & 1, it, j + 1);
-      else first_k_reads(it_next);
+      else if (!kPairOnCU) first_k_reads(it_next);
 #pragma unroll
       for (int db = 0; db < kDB; ++db)
 #pragma unroll
@@ -661,6 +674,17 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     }
   };
 
+  // kWide: Q comes into its registers as it is, and the compiler would wait for it at its first use, in the tile loop
+  // and in every iteration: a wait for vmcnt(0), which there drains the requests of the tiles ahead (64 slices of
+  // 512 x 4096 x 256: 256 us with it, 203 without).  This is a use in front of the loop.
+  auto q_is_there = [&]() __attribute__((always_inline)) {
+    if constexpr (kWide) {
+#pragma unroll
+      for (int kk = 0; kk < kKK; ++kk)
+#pragma unroll
+        for (int qb = 0; qb < kQB; ++qb) asm volatile("" : "+v"(qf[kk][qb]));
+    }
+  };
   // Tiles [0, n_plain) need no mask for this wavefront's rows, [n_plain, n_compute) cross
   // the diagonal or the end of the keys, and [n_compute, num_tiles) lie above the diagonal:
   // the wavefront only keeps the ring (barrier + loads) going for its workgroup.
@@ -692,6 +716,7 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
 #pragma unroll
     for (int t = 0; t < 3; ++t) issue_tile_loads(t);
     barrier_keep_vmem<2 * kLoadsPerTile>();  // tile 0 has landed
+    q_is_there();
     const bool second_set = wave >= 4;
     if (second_set) barrier_only();  // slot 0: set 0 alone
     first_k_reads(0);
@@ -724,37 +749,40 @@ __global__ __launch_bounds__(kWavesT * 64) void flash_attention_fwd_kernel(
     }
     if (!second_set) barrier_only();  // the slot in which set 1 finishes its last tile
   } else {
-    // One wavefront per SIMD.  Ring of 4 tiles: iteration `it` starts with the ring barrier (tile
-    // it has landed, the stage of tile it-1 is free) and QK(it) carries the requests of tile it+3.
+    // One wavefront of the workgroup per SIMD.  Ring of 4 tiles: iteration `it` starts with the ring barrier (tiles
+    // it and it+1 have landed, the stage of tile it-1 is free) and QK(it) carries the requests of tile it+3.
+    // Two stages (kPairOnCU): tile it has landed, and QK(it) carries the requests of tile it+1.
 #pragma unroll
     for (int t = 0; t < kStages - 1; ++t) issue_tile_loads(t);
     barrier_keep_vmem<(kStages - 2) * kLoadsPerTile>();  // tile 0 has landed
-    auto ring_barrier = [&]() __attribute__((always_inline)) {
-      barrier_keep_vmem<(kStages - 3) * kLoadsPerTile>();
+    q_is_there();
+    auto ring_barrier = [&](int it) __attribute__((always_inline)) {
+      barrier_keep_vmem<kPairOnCU ? 0 : (kStages - 3) * kLoadsPerTile>();
+      if (kPairOnCU) first_k_reads(it);
     };
     const int n_lean = min(n_plain, n_fast - (kStages - 1));
     int it = 0;
-    first_k_reads(0);
+    if (!kPairOnCU) first_k_reads(0);
     for (; it < n_lean; ++it) {
-      ring_barrier();
+      ring_barrier(it);
       qk_tile(it, it + kStages - 1, std::true_type{});
       softmax_tile(it, std::false_type{});
       pv_tile(it, it + 1);
     }
     for (; it < n_plain; ++it) {
-      ring_barrier();
+      ring_barrier(it);
       qk_tile(it, it + kStages - 1, std::false_type{});
       softmax_tile(it, std::false_type{});
       pv_tile(it, it + 1);
     }
     for (; it < n_compute; ++it) {
-      ring_barrier();
+      ring_barrier(it);
       qk_tile(it, it + kStages - 1, std::false_type{});
       softmax_tile(it, std::true_type{});
       pv_tile(it, it + 1);
     }
     for (; it < num_tiles; ++it) {
-      ring_barrier();
+      ring_barrier(it);
       issue_tile_loads(it + kStages - 1);
     }
   }
@@ -812,18 +840,22 @@ template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWave
 int launch_w(const AttentionCall& c) {
   auto kern = flash_attention_fwd_kernel<T, D, DV, kKT, kVT, kCausal, kWavesT, kQB>;
   constexpr int kBN = key_tile(D);
-  constexpr int lds = ring_stages(kWavesT) * (kBN * (kKT ? D : lds_pitch(D)) * 2 + (kVT ? DV * kBN * 2 : kBN * lds_pitch(DV) * 2));
+  constexpr int lds = ring_stages(kWavesT, D) * (kBN * (kKT ? D : lds_pitch(D)) * 2 + (kVT ? DV * kBN * 2 : kBN * lds_pitch(DV) * 2));
   static_assert(lds <= kMaxLdsBytes, "tiles do not fit in LDS");
   TFK_LDS_OPT_IN(kern, lds);
   constexpr int bm = kWavesT * 16 * kQB;
   const int q_tiles = (c.Lq + bm - 1) / bm;
-  const bool paired = kCausal && D <= 128 && c.paired;
+  const bool paired = kCausal && c.paired;
   const int total_items = paired ? (q_tiles / 2) * c.batch : q_tiles * c.batch;
-  const dim3 grid(8 * ((total_items + 7) / 8));
+  // Single causal tiles: a slice's stay on one XCD by themselves where 8 divides the slices, and where it does not if
+  // that leaves the XCDs within 4% of each other (bf16, 150 slices of 384 x 384 x 256: 39.4 / 31.4 us).
+  const int per_xcd = (c.batch + 7) / 8;
+  const bool by_xcd = kCausal && !paired && c.batch % 8 != 0 && 8 * per_xcd * 100 <= c.batch * 104;
+  const dim3 grid(by_xcd ? 8 * per_xcd * q_tiles : 8 * ((total_items + 7) / 8));
   hipLaunchKernelGGL(kern, grid, dim3(kWavesT * 64), lds, c.stream,
                      static_cast<const T*>(c.Q), static_cast<const T*>(c.K),
                      static_cast<const T*>(c.V), static_cast<T*>(c.O), c.Lq, c.Lkv, c.scale_log2,
-                     q_tiles, total_items, paired ? 1 : 0);
+                     q_tiles, total_items, paired ? kPairs : by_xcd ? kByXcd : kSingle);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }

@@ -12,7 +12,7 @@ struct AttentionCall {
   int batch, Lq, Lkv;
   float scale_log2;
   bool bf16, k_transposed, v_transposed, causal;   // K as [D][Lkv]; V as [Dv][Lkv]; not both
-  int rows;                                        // query rows per workgroup: 256, 128 or 64 (wide: 128 or 64)
+  int rows;                                        // query rows per workgroup: 256, 128 or 64 (wide, causal: 64)
   bool paired;                                     // causal: two query tiles per workgroup (even tile counts)
   hipStream_t stream;
 };

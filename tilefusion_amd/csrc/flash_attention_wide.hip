@@ -5,11 +5,8 @@ namespace tfk {
 namespace {
 template <typename T, int D>
 int launch_wide(const AttentionCall& c) {
-  if (c.causal) {
-    if (c.rows == 128) return launch_w<T, D, D, false, false, true, 4, 2>(c);
-    return launch_w<T, D, D, false, false, true, 4, 1>(c);
-  }
-  if (c.rows == 128) return launch_w<T, D, D, false, false, false, 4, 2>(c);
+  if (c.causal) return launch_w<T, D, D, false, false, true, 4, 1>(c);
+  if (c.rows == 128) return launch_w<T, D, D, false, false, false, 8, 1>(c);
   return launch_w<T, D, D, false, false, false, 4, 1>(c);
 }
 template <typename T>
