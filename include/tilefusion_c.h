@@ -141,6 +141,10 @@ TF_API int tf_flash_attention_fwd_kt(const void* Q, const void* K, const void* V
                                      int64_t Lq, int64_t Lkv, int64_t D, double softmax_scale, int causal,
                                      void* stream);
 
+/* out[b][c][r] = in[b][r][c] for a batch of [rows, cols] matrices of 16-bit elements: makes a key stored [D, Lkv] a [Lkv, D] one
+ * where tf_flash_attention_fwd_kt does not take it.  `out` at a 16-byte boundary. */
+TF_API int tf_transpose_16bit(const void* in, void* out, int64_t batch, int64_t rows, int64_t cols, void* stream);
+
 /* Single-query (decoding) attention with the KV range cut into up to `num_splits` ranges:
  * kernel 1 writes a partial (o, max, sum) per range in fp32 into `workspace`, kernel 2 merges
  * them with a log-sum-exp weighted sum into O.  `num_splits` is an upper bound: the library takes fewer and

@@ -106,6 +106,21 @@ def test_key_stored_transposed(lq, lkv, d, causal, dtype):
     assert (o.float().cpu() - ref.float()).norm() <= rel * ref.float().norm()
 
 
+# The copy of a key [D, Lkv] that no kernel reads as it is: edges of the 64 x 64 tiles, rows off every boundary, the
+# stores of 16 bytes (D a multiple of 8) and of 2.  Nothing beyond the copy may be written.
+@pytest.mark.parametrize("b,rows,cols", [(1, 1, 1), (2, 7, 9), (3, 64, 64), (2, 72, 65), (1, 63, 127), (4, 160, 333),
+                                         (2, 256, 96), (5, 130, 70), (70, 80, 3)])
+def test_transposed_copy(b, rows, cols):
+    x = torch.randint(-2 ** 15, 2 ** 15, (b * rows * cols + 1,), dtype=torch.int16, device=DEV)
+    for start in (0, 1):
+        src = x[start:start + b * rows * cols].view(b, rows, cols)
+        out = torch.full((b * rows * cols + 64,), 77, dtype=torch.int16, device=DEV)
+        _capi.check(_capi.load().tf_transpose_16bit(src.data_ptr(), out.data_ptr(), b, rows, cols,
+                                                    torch.cuda.current_stream().cuda_stream), "transpose")
+        assert torch.equal(out[:-64].view(b, cols, rows), src.transpose(1, 2))
+        assert bool((out[-64:] == 77).all())
+
+
 # The three workgroup sizes (256, 128, 64 query rows), at remainders of their tiles and of the key tiles, with all
 # orders of K and V; the library's pick is checked with them.
 @pytest.mark.parametrize("rows,b,lq,lkv,d", [

@@ -197,8 +197,11 @@ void attention_impl(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& 
         return;
       }
     }
-    attention_impl(Q, K.transpose(-1, -2).contiguous(), V, O, false, v_transposed, tq, tkv, thqk, thv, softmax_scale,
-                   causal, op);
+    std::vector<int64_t> k_shape(K.sizes().begin(), K.sizes().end());
+    std::swap(k_shape[k_shape.size() - 1], k_shape[k_shape.size() - 2]);
+    const at::Tensor rows = at::empty(k_shape, K.options());
+    check_status(tf_transpose_16bit(K.data_ptr(), rows.data_ptr(), batch, d, lkv, current_stream()), op);
+    attention_impl(Q, rows, V, O, false, v_transposed, tq, tkv, thqk, thv, softmax_scale, causal, op);
     return;
   }
   // Head dimensions up to 128 without a tuned kernel are zero-padded to the next tuned size (64,
