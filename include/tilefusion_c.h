@@ -141,6 +141,13 @@ TF_API int tf_flash_attention_fwd_kt(const void* Q, const void* K, const void* V
                                      int64_t Lq, int64_t Lkv, int64_t D, double softmax_scale, int causal,
                                      void* stream);
 
+/* The same for head dimensions between the tuned ones: D = Dv a multiple of 8 in 40..120 other than 64 and 96, K and V
+ * as [Lkv, D]; rows are read and written as they are, nothing is padded.  Operands at 16-byte boundaries (else, and for
+ * other head dimensions, TF_ERR_UNSUPPORTED). */
+TF_API int tf_flash_attention_fwd_d8(const void* Q, const void* K, const void* V, void* O, int dtype, int64_t batch,
+                                     int64_t Lq, int64_t Lkv, int64_t D, double softmax_scale, int causal,
+                                     void* stream);
+
 /* out[b][c][r] = in[b][r][c] for a batch of [rows, cols] matrices of 16-bit elements: makes a key stored [D, Lkv] a [Lkv, D] one
  * where tf_flash_attention_fwd_kt does not take it.  `out` at a 16-byte boundary. */
 TF_API int tf_transpose_16bit(const void* in, void* out, int64_t batch, int64_t rows, int64_t cols, void* stream);

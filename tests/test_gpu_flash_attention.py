@@ -121,6 +121,33 @@ def test_transposed_copy(b, rows, cols):
         assert bool((out[-64:] == 77).all())
 
 
+# Head dimensions between the tuned ones take the next tuned kernel on rows as they are: the bits of the operands padded
+# with zeros, at every workgroup size and remainder, with K and V of other heads (and nothing of them) around; an
+# infinity in the last chunk of K meets no zero of the padding, and no element beyond O is written.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,lq,lkv,d", [(2, 1, 8, 40), (3, 17, 72, 80), (2, 64, 64, 88), (5, 129, 130, 72), (3, 300, 333, 104),
+                                        (1, 513, 520, 48), (130, 128, 192, 80), (256, 250, 320, 112), (2, 70, 1, 56)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_rows_between_head_dimensions(b, lq, lkv, d, causal, dtype):
+    q, k, v = (x.to(DEV, dtype) for x in _inputs(b, lq, lkv, d, lq + lkv + d))
+    k[0, lkv // 2, d - 1] = float("inf")
+    store = torch.full((q.numel() + 64,), 77, device=DEV, dtype=dtype)
+    _capi.check(_capi.load().tf_flash_attention_fwd_d8(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), store.data_ptr(),
+        _capi.TF_DTYPE_F16 if dtype == torch.float16 else _capi.TF_DTYPE_BF16, b, lq, lkv, d,
+        d ** -0.5, int(causal), torch.cuda.current_stream().cuda_stream), "between")
+    pad = (64 if d < 64 else 96 if d < 96 else 128) - d
+    want = c_attention(*(torch.nn.functional.pad(x, (0, pad)) for x in (q, k, v)), causal, d ** -0.5)[..., :d]
+    o = store[:-64].view_as(q)
+    assert torch.equal(o.isnan(), want.isnan()) and torch.equal(o.nan_to_num(), want.nan_to_num())
+    assert bool((store[-64:] == 77).all())
+    for key in (k.transpose(1, 2), k.transpose(1, 2).contiguous()):
+        assert torch.equal(ops.flash_attention(q, key, v, 1, 1, d, d, d ** -0.5, causal).nan_to_num(), want.nan_to_num())
+    if b > 1:
+        ref = N.attention_ref(q[-1:].cpu(), k[-1:].cpu(), v[-1:].cpu(), causal=causal)
+        assert (o[-1:].float().cpu() - ref.float()).norm() <= (1e-3 if dtype == torch.float16 else 4e-3) * ref.float().norm()
+
+
 # The three workgroup sizes (256, 128, 64 query rows), at remainders of their tiles and of the key tiles, with all
 # orders of K and V; the library's pick is checked with them.
 @pytest.mark.parametrize("rows,b,lq,lkv,d", [

@@ -106,13 +106,17 @@ AttentionPlan plan_attention(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D, 
   return plan;
 }
 
-// the tuned kernels for D = Dv = 64, 96 or 128 (arguments already checked)
+int64_t next_tuned(int64_t D) { return D <= 64 ? 64 : D <= 96 ? 96 : 128; }
+
+// the tuned kernels for D = Dv = 64, 96 or 128, and, K and V as they come, for multiples of 8 in between and above 32 (arguments
+// already checked)
 int run_tuned(const void* Q, const void* K, const void* V, void* O, bool bf16, int64_t batch, int64_t Lq, int64_t Lkv,
               int64_t D, bool k_transposed, bool v_transposed, double softmax_scale, bool causal, hipStream_t st) {
-  const AttentionPlan plan = plan_attention(batch, Lq, Lkv, D, causal);
-  const AttentionCall c = {Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (float)(softmax_scale * 1.4426950408889634),
+  const AttentionPlan plan = plan_attention(batch, Lq, Lkv, next_tuned(D), causal);
+  const AttentionCall c = {Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, (float)(softmax_scale * 1.4426950408889634),
                            bf16, k_transposed, v_transposed, causal, plan.rows, plan.paired, st};
-  return D == 128 ? run_attention_d128(c) : D == 96 ? run_attention_d96(c) : run_attention_d64(c);
+  if (D == next_tuned(D)) return D == 128 ? run_attention_d128(c) : D == 96 ? run_attention_d96(c) : run_attention_d64(c);
+  return D > 96 ? run_attention_below128(c) : D > 64 ? run_attention_below96(c) : run_attention_below64(c);
 }
 
 // Head dimensions above 128 (V as it comes, whole key tiles): workgroups of 64 queries, two to a CU; 128 (8 wavefronts, one
@@ -226,7 +230,7 @@ extern "C" int tf_flash_attention_fwd_wide(const void* Q, const void* K, const v
               "tf_flash_attention_fwd_wide: operands must start at a 16-byte boundary");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const AttentionPlan plan = plan_wide(batch, Lq, causal != 0);
-  const AttentionCall c = {Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (float)(softmax_scale * 1.4426950408889634),
+  const AttentionCall c = {Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, (float)(softmax_scale * 1.4426950408889634),
                            dtype == TF_DTYPE_BF16, false, false, causal != 0, plan.rows, plan.paired, st};
   return run_attention_wide(c, (int)D);
 }
@@ -247,6 +251,25 @@ extern "C" int tf_flash_attention_fwd_kt(const void* Q, const void* K, const voi
                reinterpret_cast<uintptr_t>(O)) % 16 == 0, TF_ERR_UNSUPPORTED,
               "tf_flash_attention_fwd_kt: operands must start at a 16-byte boundary");
   return run_tuned(Q, K, V, O, dtype == TF_DTYPE_BF16, batch, Lq, Lkv, D, true, false, softmax_scale, causal != 0,
+                   static_cast<hipStream_t>(stream));
+}
+
+extern "C" int tf_flash_attention_fwd_d8(const void* Q, const void* K, const void* V, void* O, int dtype, int64_t batch,
+                                         int64_t Lq, int64_t Lkv, int64_t D, double softmax_scale, int causal,
+                                         void* stream) {
+  using namespace tfk;
+  if (int rc = check_attention_args("tf_flash_attention_fwd_d8", Q, K, V, O, batch, Lq, Lkv, D, D, 1, 1, 1, 1,
+                                    softmax_scale))
+    return rc;
+  TFK_REQUIRE(dtype == TF_DTYPE_F16 || dtype == TF_DTYPE_BF16, TF_ERR_UNSUPPORTED,
+              "tf_flash_attention_fwd_d8: dtype must be TF_DTYPE_F16 or TF_DTYPE_BF16");
+  TFK_REQUIRE(D > 32 && D < 128 && D % 8 == 0 && D != 64 && D != 96, TF_ERR_UNSUPPORTED,
+              "tf_flash_attention_fwd_d8: needs a head dimension of 40..120, a multiple of 8 other than 64 and 96 "
+              "(got %lld)", (long long)D);
+  TFK_REQUIRE((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V) |
+               reinterpret_cast<uintptr_t>(O)) % 16 == 0, TF_ERR_UNSUPPORTED,
+              "tf_flash_attention_fwd_d8: operands must start at a 16-byte boundary");
+  return run_tuned(Q, K, V, O, dtype == TF_DTYPE_BF16, batch, Lq, Lkv, D, false, false, softmax_scale, causal != 0,
                    static_cast<hipStream_t>(stream));
 }
 

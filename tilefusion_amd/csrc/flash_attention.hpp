@@ -167,10 +167,18 @@ TFK_DEVICE SplitWeight<T> split_weight(float p) {
 // addresses cost 0-12%, a transposed copy of K in front of the kernel costs more at every size (fp16, us, K
 // as [Lkv][D] / as [D][Lkv] / copied first: 64 slices of 4096 x 4096 x 128 444 / 449 / 534, causal 241 / 254 / 340; 16 of
 // 1024 x 1024 x 128 29 / 31 / 40; 32 of 100 x 8192 x 128 157 / 176 / 266; 64 of 1336 x 1336 x 64 causal 30 / 31 / 45).
-template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB>
+//
+// kTail: rows of Q, K, V and O have d < D elements (a multiple of 8, more than D - 32): they are read and written
+// as they are, the last reduction step takes zeros for what is missing of Q and K, columns of V beyond d are those of its
+// last chunk and are not stored.  The same bits as on operands padded with zeros, without the three padded copies and the
+// copy of the result (bf16, us, padded / as they are: 40 slices of 500 x 500 x 80 46 / 13.5, 16 of 4096 x 4096 x 80 125 / 89,
+// 32 of 100 x 2048 x 80 68 / 27, 64 of 1024 x 1024 x 80 causal 67 / 25, 32 of 1024 x 1024 x 112 causal 58 / 22; the kernel
+// alone on padded operands is 0-5% ahead of the one on rows as they are).  With K as [D][Lkv] such instances were at most 15%
+// ahead of a transposed copy in front (none in the largest case), and are left out.
+template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB, bool kTail>
 __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1) void flash_attention_fwd_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
-    T* __restrict__ O, int Lq, int Lkv, float scale_log2, int q_tiles, int total_items, int order) {
+    T* __restrict__ O, int Lq, int Lkv, float scale_log2, int q_tiles, int total_items, int order, int d) {
   using V2 = typename Vec<T>::v2;
   using V4 = typename Vec<T>::v4;
   using V8 = typename Vec<T>::v8;
@@ -182,6 +190,8 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   constexpr int kBMq = kWavesT * kRowsPerWave;
   constexpr int DP = lds_pitch(D), DVP = lds_pitch(DV);   // LDS row pitch of the K / natural V tile
   static_assert(!kKT || !kWide, "K^T tiles are 64 keys wide");
+  static_assert(!kTail || (D == DV && !kWide && !kKT && !kVT), "");
+  const int d_row = kTail ? d : D, dv_row = kTail ? d : DV;   // elements of a row in memory
   constexpr int kKChunks = kKT ? kBN / 8 : DP / 8;
   constexpr int kVChunks = kVT ? kBN / 8 : DVP / 8;
   constexpr int kKBytes = kKT ? D * kBN * 2 : kBN * DP * 2;
@@ -243,10 +253,10 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
       bh = blockIdx.x % slices;
     }
   }
-  Q += bh * (size_t)Lq * D;
-  K += bh * (size_t)Lkv * D;
-  V += bh * (size_t)Lkv * DV;
-  O += bh * (size_t)Lq * DV;
+  Q += bh * (size_t)Lq * d_row;
+  K += bh * (size_t)Lkv * d_row;
+  V += bh * (size_t)Lkv * dv_row;
+  O += bh * (size_t)Lq * dv_row;
 
   for (int pass = 0; pass < num_passes; ++pass) {
   const int qt = qt_of_pass[pass];
@@ -264,7 +274,9 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
     const int m_ld = min(q_row0 + 16 * qb + lr, Lq - 1);
 #pragma unroll
     for (int kk = 0; kk < kKK; ++kk) {
-      const V8 raw = *reinterpret_cast<const V8*>(Q + (size_t)m_ld * D + kk * 32 + lg * 8);
+      const int col = kk * 32 + lg * 8;
+      V8 raw = *reinterpret_cast<const V8*>(Q + (size_t)m_ld * d_row + (kTail ? min(col, d_row - 8) : col));
+      if (kTail && col >= d_row) raw = V8{};
       if constexpr (kWide) {
         qf[kk][qb] = raw;
       } else {
@@ -283,6 +295,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   // base (start of the tile in global memory) + a per-lane 32-bit offset computed once here.
   // Only a tile that crosses the end of the keys takes the slow form with clamped addresses.
   const unsigned smem_base = lds_address(smem);
+  const int k_last = d_row / 8 - 1, v_last = dv_row / 8 - 1;   // last 16-byte chunk of a row
   unsigned req_off[kLoadsPerTile];   // per-lane byte offset inside the tile (global side)
   unsigned req_lds[kLoadsPerTile];   // wave-uniform byte offset inside the stage (LDS side)
 #pragma unroll
@@ -293,8 +306,8 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
     if constexpr (kKT)  // K^T tile: [D][kBN] out of a [D][Lkv] matrix
       req_off[t] = ((unsigned)row * (unsigned)Lkv + swz_kt(row, lane % kKChunks) * 8) * 2u;
     else                // K tile: [kBN][D]
-      // (a physical chunk whose logical chunk lies beyond D is never read: it re-fetches the last one)
-      req_off[t] = (unsigned)(row * D + min(swz_k<kKChunks>(row, lane % kKChunks), D / 8 - 1) * 8) * 2u;
+      // (a physical chunk whose logical chunk lies beyond the row is never read: it re-fetches the last one)
+      req_off[t] = (unsigned)(row * d_row + min(swz_k<kKChunks>(row, lane % kKChunks), k_last) * 8) * 2u;
     req_lds[t] = i * 1024;
   }
 #pragma unroll
@@ -303,7 +316,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
     constexpr int kRowsPerInstr = 64 / kVChunks;
     const int row = i * kRowsPerInstr + lane / kVChunks;
     if constexpr (!kVT)  // V tile: [kBN][DV]
-      req_off[kKPerWave + t] = (unsigned)(row * DV + min(swz_v<kVChunks>(row, lane % kVChunks), DV / 8 - 1) * 8) * 2u;
+      req_off[kKPerWave + t] = (unsigned)(row * dv_row + min(swz_v<kVChunks>(row, lane % kVChunks), v_last) * 8) * 2u;
     else                 // V^T tile: [DV][kBN] out of a [DV][Lkv] matrix
       req_off[kKPerWave + t] = ((unsigned)row * (unsigned)Lkv + swz_k<kVChunks>(row, lane % kVChunks) * 8) * 2u;
     req_lds[kKPerWave + t] = kKBytes + i * 1024;
@@ -312,9 +325,9 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
     const int n0 = min(tile, num_tiles - 1) * kBN;  // clamped past the end (never read)
     const unsigned dst = smem_base + (tile % kStages) * kStageBytes + req_lds[r];
     if (n0 + kBN <= Lkv) {
-      const char* base = r < kKPerWave ? reinterpret_cast<const char*>(K + (size_t)n0 * (kKT ? 1 : D))
+      const char* base = r < kKPerWave ? reinterpret_cast<const char*>(K + (size_t)n0 * (kKT ? 1 : d_row))
                          : kVT         ? reinterpret_cast<const char*>(V + n0)
-                                       : reinterpret_cast<const char*>(V + (size_t)n0 * DV);
+                                       : reinterpret_cast<const char*>(V + (size_t)n0 * dv_row);
       // the LDS destination is an M0 INPUT of the statement: the compiler writes M0 itself and
       // cannot use the register for anything else between that write and the request; the
       // s_nop is the wait state an M0 write needs in front of an LDS-direct load
@@ -332,18 +345,18 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
         const int gc = min(n0 + swz_kt(row, lane % kKChunks) * 8, Lkv - 8);
         lds_dma_16B(K + (size_t)row * Lkv + gc, dst);
       } else {
-        const int cc = min(swz_k<kKChunks>(row, lane % kKChunks), D / 8 - 1);
+        const int cc = min(swz_k<kKChunks>(row, lane % kKChunks), k_last);
         const int gr = min(n0 + row, Lkv - 1);
-        lds_dma_16B(K + (size_t)gr * D + cc * 8, dst);
+        lds_dma_16B(K + (size_t)gr * d_row + cc * 8, dst);
       }
     } else {
       const int i = (wave + kWavesT * (r - kKPerWave)) % kVInstr;
       constexpr int kRowsPerInstr = 64 / kVChunks;
       const int row = i * kRowsPerInstr + lane / kVChunks;
       if constexpr (!kVT) {
-        const int cc = min(swz_v<kVChunks>(row, lane % kVChunks), DV / 8 - 1);
+        const int cc = min(swz_v<kVChunks>(row, lane % kVChunks), v_last);
         const int gr = min(n0 + row, Lkv - 1);
-        lds_dma_16B(V + (size_t)gr * DV + cc * 8, dst);
+        lds_dma_16B(V + (size_t)gr * dv_row + cc * 8, dst);
       } else {
         const int cc = swz_k<kVChunks>(row, lane % kVChunks);
         const int gc = min(n0 + cc * 8, Lkv - 8);
@@ -358,9 +371,9 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   // cycles per request with the pipe idle.
   auto issue_request_lean = [&](int tile, int r) __attribute__((always_inline)) {
     const unsigned dst = smem_base + (tile % kStages) * kStageBytes + req_lds[r];
-    const char* base = r < kKPerWave ? reinterpret_cast<const char*>(K) + (size_t)tile * (kBN * (kKT ? 1 : D) * 2)
+    const char* base = r < kKPerWave ? reinterpret_cast<const char*>(K) + (size_t)tile * (kBN * (kKT ? 1 : d_row) * 2)
                        : kVT         ? reinterpret_cast<const char*>(V) + (size_t)tile * (kBN * 2)
-                                     : reinterpret_cast<const char*>(V) + (size_t)tile * (kBN * DV * 2);
+                                     : reinterpret_cast<const char*>(V) + (size_t)tile * (kBN * dv_row * 2);
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
                  : "v"(req_off[r]), "s"(base), "{m0}"(dst)
@@ -452,6 +465,15 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   // weights had a remainder: 32 slices of 1024 x 1024 52.5 -> 47.0 us, 8 of 4096 173 -> 157; D = 160: 46.2 -> 44.8).
   constexpr int kKAhead = kWide && D <= 192 && kWavesT == 4 ? 2 : 1;
   V8 kf[kKAhead + 1][kKB];   // K fragments of reduction step kk (buffer kk % (kKAhead + 1))
+  // kTail: all ones where this lane's dims of the last reduction step exist (K may hold infinities there)
+  const int tail_mask = kTail && (kKK - 1) * 32 + lg * 8 >= d_row ? 0 : -1;
+  auto k_frag = [&](int buf, int kk, int kb) __attribute__((always_inline)) {
+    if constexpr (kTail) {
+      typedef int int4v_t __attribute__((ext_vector_type(4)));
+      if (kk == kKK - 1) return __builtin_bit_cast(V8, __builtin_bit_cast(int4v_t, kf[buf][kb]) & tail_mask);
+    }
+    return kf[buf][kb];
+  };
   V8 vf[kJ > 1 ? 2 : 1][kDB];   // V fragments of reduction step j (buffer j & 1)
   // lane address of the fragments of step kk (kKT: recomputed per fragment)
   auto k_addr = [&](int it, int kk) __attribute__((always_inline)) {
@@ -527,8 +549,9 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int kb = 0; kb < kKB; ++kb) {
+        const V8 k_now = k_frag(kk % (kKAhead + 1), kk, kb);
 #pragma unroll
-        for (int qb = 0; qb < kQB; ++qb) s[kb][qb] = mfma_t<T>(kf[kk % (kKAhead + 1)][kb], qf[kk][qb], s[kb][qb]);
+        for (int qb = 0; qb < kQB; ++qb) s[kb][qb] = mfma_t<T>(k_now, qf[kk][qb], s[kb][qb]);
         if (next < kKK) k_read(next % (kKAhead + 1), ka, next, kb);
         if constexpr (kWide) {
 #pragma unroll
@@ -805,21 +828,21 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
     for (int qb = 0; qb < kQB; ++qb) {
       const float inv = 1.f / l_acc[qb][0];   // of this lane's own row lr
       const int m_row = q_row0 + 16 * qb + st_row;   // the row this lane stores
-      T* o_lane = O + (size_t)m_row * DV + 8 * st_seg;
+      T* o_lane = O + (size_t)m_row * dv_row + 8 * st_seg;
 #pragma unroll
       for (int db = 0; db < kDB; db += 2) {
         unsigned x[2], y[2];
 #pragma unroll
-        for (int d = 0; d < 2; ++d) {
-          const V2 hx = {(T)(o_acc[db][qb][2 * d] * inv), (T)(o_acc[db][qb][2 * d + 1] * inv)};
-          const V2 hy = {(T)(o_acc[db + 1][qb][2 * d] * inv), (T)(o_acc[db + 1][qb][2 * d + 1] * inv)};
-          x[d] = __builtin_bit_cast(unsigned, hx);
-          y[d] = __builtin_bit_cast(unsigned, hy);
+        for (int h = 0; h < 2; ++h) {
+          const V2 hx = {(T)(o_acc[db][qb][2 * h] * inv), (T)(o_acc[db][qb][2 * h + 1] * inv)};
+          const V2 hy = {(T)(o_acc[db + 1][qb][2 * h] * inv), (T)(o_acc[db + 1][qb][2 * h + 1] * inv)};
+          x[h] = __builtin_bit_cast(unsigned, hx);
+          y[h] = __builtin_bit_cast(unsigned, hy);
 #if defined(__HIP_DEVICE_COMPILE__)
           // x of the odd groups <-> y of the even groups
-          auto sw = __builtin_amdgcn_permlane16_swap(x[d], y[d], false, false);
-          x[d] = sw[0];
-          y[d] = sw[1];
+          auto sw = __builtin_amdgcn_permlane16_swap(x[h], y[h], false, false);
+          x[h] = sw[0];
+          y[h] = sw[1];
 #endif
         }
         uint4_t v;
@@ -827,7 +850,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
         v[1] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)x[1]);
         v[2] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)y[0]);
         v[3] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)y[1]);
-        if (m_row < Lq) *reinterpret_cast<uint4_t*>(o_lane + 16 * db) = v;
+        if (m_row < Lq && (!kTail || 16 * db + 8 * st_seg < dv_row)) *reinterpret_cast<uint4_t*>(o_lane + 16 * db) = v;
       }
     }
   }
@@ -836,9 +859,9 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   }  // pass
 }
 
-template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB>
+template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB, bool kTail>
 int launch_w(const AttentionCall& c) {
-  auto kern = flash_attention_fwd_kernel<T, D, DV, kKT, kVT, kCausal, kWavesT, kQB>;
+  auto kern = flash_attention_fwd_kernel<T, D, DV, kKT, kVT, kCausal, kWavesT, kQB, kTail>;
   constexpr int kBN = key_tile(D);
   constexpr int lds = ring_stages(kWavesT, D) * (kBN * (kKT ? D : lds_pitch(D)) * 2 + (kVT ? DV * kBN * 2 : kBN * lds_pitch(DV) * 2));
   static_assert(lds <= kMaxLdsBytes, "tiles do not fit in LDS");
@@ -855,20 +878,20 @@ int launch_w(const AttentionCall& c) {
   hipLaunchKernelGGL(kern, grid, dim3(kWavesT * 64), lds, c.stream,
                      static_cast<const T*>(c.Q), static_cast<const T*>(c.K),
                      static_cast<const T*>(c.V), static_cast<T*>(c.O), c.Lq, c.Lkv, c.scale_log2,
-                     q_tiles, total_items, paired ? kPairs : by_xcd ? kByXcd : kSingle);
+                     q_tiles, total_items, paired ? kPairs : by_xcd ? kByXcd : kSingle, c.d);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
 
-template <typename T, int D, bool kKT, bool kVT, bool kCausal>
+template <typename T, int D, bool kKT, bool kVT, bool kCausal, bool kTail>
 int launch_rows(const AttentionCall& c) {
-  if (c.rows == 256) return launch_w<T, D, D, kKT, kVT, kCausal, 8, 2>(c);
-  if (c.rows == 128) return launch_w<T, D, D, kKT, kVT, kCausal, 8, 1>(c);
-  return launch_w<T, D, D, kKT, kVT, kCausal, 4, 1>(c);
+  if (c.rows == 256) return launch_w<T, D, D, kKT, kVT, kCausal, 8, 2, kTail>(c);
+  if (c.rows == 128) return launch_w<T, D, D, kKT, kVT, kCausal, 8, 1, kTail>(c);
+  return launch_w<T, D, D, kKT, kVT, kCausal, 4, 1, kTail>(c);
 }
-template <typename T, int D, bool kKT, bool kVT>
+template <typename T, int D, bool kKT, bool kVT, bool kTail = false>
 int launch_causal(const AttentionCall& c) {
-  return c.causal ? launch_rows<T, D, kKT, kVT, true>(c) : launch_rows<T, D, kKT, kVT, false>(c);
+  return c.causal ? launch_rows<T, D, kKT, kVT, true, kTail>(c) : launch_rows<T, D, kKT, kVT, false, kTail>(c);
 }
 template <typename T, int D>
 int launch_layout(const AttentionCall& c) {
@@ -879,6 +902,11 @@ int launch_layout(const AttentionCall& c) {
 template <int D>
 int launch(const AttentionCall& c) {
   return c.bf16 ? launch_layout<bf16_t, D>(c) : launch_layout<half_t, D>(c);
+}
+// rows of c.d < D elements (K and V as they come)
+template <int D>
+int launch_tail(const AttentionCall& c) {
+  return c.bf16 ? launch_causal<bf16_t, D, false, false, true>(c) : launch_causal<half_t, D, false, false, true>(c);
 }
 
 }  // namespace

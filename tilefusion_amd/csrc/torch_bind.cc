@@ -204,11 +204,20 @@ void attention_impl(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& 
     attention_impl(Q, rows, V, O, false, v_transposed, tq, tkv, thqk, thv, softmax_scale, causal, op);
     return;
   }
-  // Head dimensions up to 128 without a tuned kernel are zero-padded to the next tuned size (64,
+  const bool tuned = d == dv && (d == 128 || d == 96 || d == 64);
+  // Multiples of 8 between the tuned ones have kernels that read and write rows as they are.
+  if (d == dv && !v_transposed && d > 32 && d < 128 && d % 8 == 0 && !tuned) {
+    const int status = tf_flash_attention_fwd_d8(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dtype, batch,
+                                                 lq, lkv, d, softmax_scale, causal ? 1 : 0, current_stream());
+    if (status != TF_ERR_UNSUPPORTED) {
+      check_status(status, op);
+      return;
+    }
+  }
+  // Other head dimensions up to 128 without a tuned kernel are zero-padded to the next tuned size (64,
   // 96 or 128): zeros change neither the scores nor the kept output columns, and the tuned kernel
   // on the padded problem is well ahead of the header kernel compiled at run time on the exact
   // one, copies included.
-  const bool tuned = d == dv && (d == 128 || d == 96 || d == 64);
   if (!tuned && d <= 128 && dv <= 128 && (!v_transposed || lkv % 8 == 0)) {
     const int64_t hmax = std::max(d, dv);
     const int64_t hp = hmax <= 64 ? 64 : hmax <= 96 ? 96 : 128;

@@ -1,5 +1,5 @@
 // Transposes a batch of matrices of 16-bit elements: out[b][c][r] = in[b][r][c], for keys stored [D, Lkv] that no
-// attention kernel reads as they are (lengths that are no multiple of 8, wide heads).
+// attention kernel reads as they are (lengths that are no multiple of 8, wide heads, heads between the tuned sizes).
 //
 // A workgroup takes a 64 x 64 tile through LDS: rows come as 8-byte loads at any even address (rows of an odd length have
 // no alignment), leave as 16-byte stores.  Bound by memory: [64, 128, 4096] in 20.5 us (6.5 TB/s;
