@@ -148,6 +148,15 @@ TF_API int tf_flash_attention_fwd_d8(const void* Q, const void* K, const void* V
                                      int64_t Lq, int64_t Lkv, int64_t D, double softmax_scale, int causal,
                                      void* stream);
 
+/* Without a mask, V as [Lkv, D], for problems with too few queries to fill the chip: the keys in parts, merged by a second kernel
+ * (D a multiple of 8 in 40..128; K as [Lkv, D], or as [D, Lkv] with D 64, 96 or 128 and Lkv % 8 == 0).  `workspace` has
+ * tf_flash_attention_split_workspace bytes for the problem, 0 where the keys are not split (then, and for operands off a
+ * 16-byte boundary, TF_ERR_UNSUPPORTED). */
+TF_API int64_t tf_flash_attention_split_workspace(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D);
+TF_API int tf_flash_attention_fwd_split(const void* Q, const void* K, const void* V, void* O, int dtype, int64_t batch,
+                                        int64_t Lq, int64_t Lkv, int64_t D, int k_is_transposed, double softmax_scale,
+                                        void* workspace, void* stream);
+
 /* out[b][c][r] = in[b][r][c] for a batch of [rows, cols] matrices of 16-bit elements: makes a key stored [D, Lkv] a [Lkv, D] one
  * where tf_flash_attention_fwd_kt does not take it.  `out` at a 16-byte boundary. */
 TF_API int tf_transpose_16bit(const void* in, void* out, int64_t batch, int64_t rows, int64_t cols, void* stream);

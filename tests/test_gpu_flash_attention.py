@@ -126,7 +126,7 @@ def test_transposed_copy(b, rows, cols):
 # infinity in the last chunk of K meets no zero of the padding, and no element beyond O is written.
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("b,lq,lkv,d", [(2, 1, 8, 40), (3, 17, 72, 80), (2, 64, 64, 88), (5, 129, 130, 72), (3, 300, 333, 104),
-                                        (1, 513, 520, 48), (130, 128, 192, 80), (256, 250, 320, 112), (2, 70, 1, 56)])
+                                        (1, 513, 440, 48), (130, 128, 192, 80), (256, 250, 320, 112), (2, 70, 1, 56)])
 @pytest.mark.parametrize("causal", [False, True])
 def test_rows_between_head_dimensions(b, lq, lkv, d, causal, dtype):
     q, k, v = (x.to(DEV, dtype) for x in _inputs(b, lq, lkv, d, lq + lkv + d))
@@ -146,6 +146,53 @@ def test_rows_between_head_dimensions(b, lq, lkv, d, causal, dtype):
     if b > 1:
         ref = N.attention_ref(q[-1:].cpu(), k[-1:].cpu(), v[-1:].cpu(), causal=causal)
         assert (o[-1:].float().cpu() - ref.float()).norm() <= (1e-3 if dtype == torch.float16 else 4e-3) * ref.float().norm()
+
+
+# Keys in parts (few queries, many keys), against 64 bits and the kernel on all keys, with the workspace full of NaN:
+# remainders of queries, keys and parts, both orders of K, rows between the tuned sizes.  The error is that of 16-bit weights and
+# results in either case: the same bound, and no more than 1.1 of the other's (samples of 16 x 40 elements and up).
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,lq,lkv,d", [(1, 16, 1500, 40), (1, 63, 5056, 128), (9, 65, 648, 128), (3, 129, 2001, 64),
+                                        (12, 20, 1280, 96), (5, 300, 4104, 80), (70, 64, 4096, 128), (2, 1708, 1664, 96)])
+def test_keys_in_parts(b, lq, lkv, d, dtype):
+    lib, stream = _capi.load(), torch.cuda.current_stream().cuda_stream
+    bytes_ = lib.tf_flash_attention_split_workspace(b, lq, lkv, d)
+    assert bytes_ > 0
+    q, k, v = (x.to(DEV, dtype) for x in _inputs(b, lq, lkv, d, lq + lkv + d))
+    want = torch.softmax(q.double() @ k.double().transpose(1, 2).contiguous() * d ** -0.5, -1) @ v.double()
+    code = _capi.TF_DTYPE_F16 if dtype == torch.float16 else _capi.TF_DTYPE_BF16
+    if d in (64, 96, 128):
+        whole = c_attention(q, k, v)
+    else:
+        whole = torch.empty_like(q)
+        _capi.check(lib.tf_flash_attention_fwd_d8(q.data_ptr(), k.data_ptr(), v.data_ptr(), whole.data_ptr(), code, b, lq, lkv,
+                                                  d, d ** -0.5, 0, stream), "whole")
+    bound = 1.1 * (whole.double() - want).norm()
+    for kt in (False, True):
+        if kt and (lkv % 8 or d not in (64, 96, 128)):
+            continue
+        key = k.transpose(1, 2).contiguous() if kt else k
+        room = torch.full((bytes_ // 4 + 64,), float("nan"), device=DEV)
+        store = torch.full((q.numel() + 64,), 77, device=DEV, dtype=dtype)
+        _capi.check(lib.tf_flash_attention_fwd_split(q.data_ptr(), key.data_ptr(), v.data_ptr(), store.data_ptr(), code, b, lq,
+                                                     lkv, d, int(kt), d ** -0.5, room.data_ptr(), stream), "parts")
+        o = store[:-64].view_as(q)
+        assert (o.double() - want).norm() <= bound
+        assert bool((store[-64:] == 77).all()) and bool(room[-64:].isnan().all())
+        assert torch.equal(ops.flash_attention(q, k.transpose(1, 2) if not kt else key, v, 1, 1, d, d, d ** -0.5, False), o)
+
+
+# ... a part whose scores are all -inf takes no weight, and a row without a score is NaN as it is in one piece
+def test_keys_in_parts_without_scores():
+    q, k, v = (x.to(DEV) for x in _inputs(2, 40, 4096, 64, 5))
+    q[..., 0] = 1.0
+    k[0, 512:3000, 0] = float("-inf")
+    k[1, :, 0] = float("-inf")
+    assert _capi.load().tf_flash_attention_split_workspace(2, 40, 4096, 64) > 0
+    o = ops.flash_attention(q, k.transpose(1, 2), v, 1, 1, 64, 64, 0.125, False)
+    whole = c_attention(q, k, v, False, 0.125)
+    assert bool(o[1].isnan().all()) and bool(whole[1].isnan().all())
+    assert (o[0].float() - whole[0].float()).norm() <= 1e-3 * whole[0].float().norm()
 
 
 # The three workgroup sizes (256, 128, 64 query rows), at remainders of their tiles and of the key tiles, with all

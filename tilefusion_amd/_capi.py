@@ -35,6 +35,8 @@ SIGNATURES = {
     "tf_flash_decode_static_prepare": (_i, []),
     "tf_flash_decode_static_f16": (_i, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _d, _vp]),
     "tf_flash_attention_fwd_d8": (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i64, _i64, _i64, _d, _i, _vp]),
+    "tf_flash_attention_split_workspace": (_i64, [_i64, _i64, _i64, _i64]),
+    "tf_flash_attention_fwd_split": (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i64, _i64, _i64, _i, _d, _vp, _vp]),
     "tf_transpose_16bit": (_i, [_vp, _vp, _i64, _i64, _i64, _vp]),
     "tf_scatter_nd": (_i, [_vp, _vp, _vp, ctypes.POINTER(_i64), _i, _i64, _i, _i, _vp]),
     "tf_gemm_kernel_index": (_i, [_i64, _i64, _i64, _i]),

@@ -44,6 +44,8 @@ constexpr HeadCost kHeadCost[3] = {
      {{8.3, 1.186, 1.636, 0.225, 9.8, 1.883}, {6.5, 0.873, 1.044, 0.125, 8.3, 1.121}, {6.0, 0.690, 0.368, 0.193, 6.4, 0.879}},
      {{7.2, 1.167, 0.536, 8.0}, {3.0, 0.835, 0.225, 8.7}, {1.0, 0.772, 0.0, 8.3}}}};
 
+constexpr double kSplitMergeUs = 3.5, kSplitBytesPerUs = 2e6;
+
 double expected_single(const SingleCost& c, int64_t batch, int64_t Lq, int64_t Lkv, bool causal, int rows) {
   const int64_t q_tiles = (Lq + rows - 1) / rows, items = q_tiles * batch, rounds = (items + 255) / 256;
   const int64_t all = (Lkv + 63) / 64;   // key tiles of a slice
@@ -106,7 +108,40 @@ AttentionPlan plan_attention(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D, 
   return plan;
 }
 
+// Keys in parts, workgroups of 64 queries: where the workgroups of whole problems leave CUs idle and the cost model, for `s` times
+// as many slices of 1 / s of the keys plus the second kernel (a launch, and the fp32 rows written and read), sees more than 10%.
+// 70 problems that it splits (1..110 slices, 16..4726 queries, 640..7732 keys): 1.06x to 4.8x, 1.86x on average, e.g. 17
+// slices of 114 x 7732 x 128 99 / 27 us, 10 of 497 x 6123 x 128 80 / 36, 60 of 41 x 4096 x 128 55 / 28, 9 of 65 x 640 x 128
+// 12.9 / 11.9; relative errors against 64 bits 0.96..1.05 of those in one piece (0.985 on average).
+struct SplitPlan { int splits, chunk; };
+SplitPlan plan_split(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D) {
+  const int64_t items = (Lq + 63) / 64 * batch, tiles = (Lkv + 63) / 64;
+  if (items >= 256 || tiles < 8) return {1, 0};
+  const HeadCost& cost = kHeadCost[D == 64 ? 0 : D == 96 ? 1 : 2];
+  double best = 1e30;
+  for (int i = Lq <= 64 ? 2 : Lq <= 128 ? 1 : 0; i < 3; ++i)
+    best = std::min(best, expected_single(cost.plain[i], batch, Lq, Lkv, false, kRowChoices[i]));
+  best *= 0.9;
+  SplitPlan plan = {1, 0};
+  const double row_us = (double)(batch * Lq * D * 4) / kSplitBytesPerUs;
+  for (int64_t s = 2; s <= 16 && s <= tiles / 2 && s * items <= 1024; ++s) {
+    const int64_t chunk = (tiles + s - 1) / s, parts = (tiles + chunk - 1) / chunk;
+    if (parts != s) continue;
+    const double t = expected_single(cost.plain[2], batch * s, Lq, 64 * chunk, false, 64) + kSplitMergeUs + (double)s * row_us;
+    if (t < best) {
+      best = t;
+      plan = {(int)s, (int)(64 * chunk)};
+    }
+  }
+  return plan;
+}
+
 int64_t next_tuned(int64_t D) { return D <= 64 ? 64 : D <= 96 ? 96 : 128; }
+
+int run_by_head(const AttentionCall& c) {
+  if (c.d == next_tuned(c.d)) return c.d == 128 ? run_attention_d128(c) : c.d == 96 ? run_attention_d96(c) : run_attention_d64(c);
+  return c.d > 96 ? run_attention_below128(c) : c.d > 64 ? run_attention_below96(c) : run_attention_below64(c);
+}
 
 // the tuned kernels for D = Dv = 64, 96 or 128, and, K and V as they come, for multiples of 8 in between and above 32 (arguments
 // already checked)
@@ -115,8 +150,7 @@ int run_tuned(const void* Q, const void* K, const void* V, void* O, bool bf16, i
   const AttentionPlan plan = plan_attention(batch, Lq, Lkv, next_tuned(D), causal);
   const AttentionCall c = {Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, (float)(softmax_scale * 1.4426950408889634),
                            bf16, k_transposed, v_transposed, causal, plan.rows, plan.paired, st};
-  if (D == next_tuned(D)) return D == 128 ? run_attention_d128(c) : D == 96 ? run_attention_d96(c) : run_attention_d64(c);
-  return D > 96 ? run_attention_below128(c) : D > 64 ? run_attention_below96(c) : run_attention_below64(c);
+  return run_by_head(c);
 }
 
 // Head dimensions above 128 (V as it comes, whole key tiles): workgroups of 64 queries, two to a CU; 128 (8 wavefronts, one
@@ -271,6 +305,38 @@ extern "C" int tf_flash_attention_fwd_d8(const void* Q, const void* K, const voi
               "tf_flash_attention_fwd_d8: operands must start at a 16-byte boundary");
   return run_tuned(Q, K, V, O, dtype == TF_DTYPE_BF16, batch, Lq, Lkv, D, false, false, softmax_scale, causal != 0,
                    static_cast<hipStream_t>(stream));
+}
+
+extern "C" int64_t tf_flash_attention_split_workspace(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D) {
+  using namespace tfk;
+  if (batch <= 0 || batch >= 65536 || Lq <= 0 || Lq >= 1 << 21 || Lkv <= 0 || Lkv >= 1 << 24 || D <= 32 || D > 128 || D % 8 != 0)
+    return 0;
+  const SplitPlan plan = plan_split(batch, Lq, Lkv, next_tuned(D));
+  return plan.splits > 1 ? (int64_t)plan.splits * batch * Lq * (next_tuned(D) + 2) * 4 : 0;
+}
+
+extern "C" int tf_flash_attention_fwd_split(const void* Q, const void* K, const void* V, void* O, int dtype, int64_t batch,
+                                            int64_t Lq, int64_t Lkv, int64_t D, int k_is_transposed, double softmax_scale,
+                                            void* workspace, void* stream) {
+  using namespace tfk;
+  if (int rc = check_attention_args("tf_flash_attention_fwd_split", Q, K, V, O, batch, Lq, Lkv, D, D, 1, 1, 1, 1,
+                                    softmax_scale))
+    return rc;
+  TFK_REQUIRE(dtype == TF_DTYPE_F16 || dtype == TF_DTYPE_BF16, TF_ERR_UNSUPPORTED,
+              "tf_flash_attention_fwd_split: dtype must be TF_DTYPE_F16 or TF_DTYPE_BF16");
+  const bool between = D != next_tuned(D);
+  TFK_REQUIRE(tf_flash_attention_split_workspace(batch, Lq, Lkv, D) > 0 && (!k_is_transposed || (Lkv % 8 == 0 && !between)),
+              TF_ERR_UNSUPPORTED, "tf_flash_attention_fwd_split: the keys of [%lld, %lld, %lld, %lld] are not split",
+              (long long)batch, (long long)Lq, (long long)Lkv, (long long)D);
+  TFK_REQUIRE(workspace, TF_ERR_INVALID_ARG, "tf_flash_attention_fwd_split: null workspace");
+  TFK_REQUIRE((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V) |
+               reinterpret_cast<uintptr_t>(O) | reinterpret_cast<uintptr_t>(workspace)) % 16 == 0, TF_ERR_UNSUPPORTED,
+              "tf_flash_attention_fwd_split: operands must start at a 16-byte boundary");
+  const SplitPlan plan = plan_split(batch, Lq, Lkv, next_tuned(D));
+  const AttentionCall c = {Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, (float)(softmax_scale * 1.4426950408889634),
+                           dtype == TF_DTYPE_BF16, k_is_transposed != 0, false, false, 64, false,
+                           static_cast<hipStream_t>(stream), static_cast<float*>(workspace), plan.splits, plan.chunk};
+  return run_by_head(c);
 }
 
 extern "C" int tf_flash_attention_rows(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D, int causal) {

@@ -66,6 +66,7 @@ __host__ __device__ constexpr int swz_kt(int row, int c) {
 // What a workgroup's number stands for (causal; see the kernel).
 enum : int { kSingle = 0, kPairs = 1, kByXcd = 2 };
 
+typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef __fp16 fp16x4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
 
 // The kernel moves 16-bit elements without looking at them; the element type T (half_t or bf16_t)
@@ -175,10 +176,13 @@ TFK_DEVICE SplitWeight<T> split_weight(float p) {
 // 32 of 100 x 2048 x 80 68 / 27, 64 of 1024 x 1024 x 80 causal 67 / 25, 32 of 1024 x 1024 x 112 causal 58 / 22; the kernel
 // alone on padded operands is 0-5% ahead of the one on rows as they are).  With K as [D][Lkv] such instances were at most 15%
 // ahead of a transposed copy in front (none in the largest case), and are left out.
-template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB, bool kTail>
+//
+// kSplit: a workgroup takes `chunk` keys (whole tiles; the last of a slice's `splits` parts may be shorter) and leaves its
+// un-normalised fp32 rows, minus their reference and their weights' sum in `part`; merge_parts_kernel puts them together.
+template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB, bool kTail, bool kSplit>
 __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1) void flash_attention_fwd_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
-    T* __restrict__ O, int Lq, int Lkv, float scale_log2, int q_tiles, int total_items, int order, int d) {
+    T* __restrict__ O, int Lq, int Lkv, float scale_log2, int q_tiles, int total_items, int order, int d, float* __restrict__ part, int splits, int chunk) {
   using V2 = typename Vec<T>::v2;
   using V4 = typename Vec<T>::v4;
   using V8 = typename Vec<T>::v8;
@@ -191,6 +195,9 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   constexpr int DP = lds_pitch(D), DVP = lds_pitch(DV);   // LDS row pitch of the K / natural V tile
   static_assert(!kKT || !kWide, "K^T tiles are 64 keys wide");
   static_assert(!kTail || (D == DV && !kWide && !kKT && !kVT), "");
+  static_assert(!kSplit || (!kCausal && !kVT && !kWide && kWavesT == 4 && kQB == 1), "");
+  // A row's reference is set by its first tile with a score above -inf, whichever that is; else by the first tile.
+  constexpr bool kLateReference = kWide || kSplit;
   const int d_row = kTail ? d : D, dv_row = kTail ? d : DV;   // elements of a row in memory
   constexpr int kKChunks = kKT ? kBN / 8 : DP / 8;
   constexpr int kVChunks = kVT ? kBN / 8 : DVP / 8;
@@ -225,6 +232,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   int qt_of_pass[2] = {0, 0};
   int num_passes = 1;
   size_t bh;
+  int split = 0;
   if (!kCausal || order == kPairs) {
     const int per_slice = kCausal ? q_tiles / 2 : q_tiles;
     const int per_xcd = (total_items + 7) / 8;
@@ -232,6 +240,10 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
     if (item >= total_items) return;
     const int p = item % per_slice;
     bh = item / per_slice;
+    if constexpr (kSplit) {
+      split = (int)(bh % splits);
+      bh /= splits;
+    }
     if (kCausal) {
       qt_of_pass[0] = q_tiles - 1 - p;
       qt_of_pass[1] = p;
@@ -257,6 +269,13 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   K += bh * (size_t)Lkv * d_row;
   V += bh * (size_t)Lkv * dv_row;
   O += bh * (size_t)Lq * dv_row;
+
+  const int kv_pitch = Lkv;   // row length of a transposed K or V
+  if constexpr (kSplit) {
+    K += (size_t)split * chunk * (kKT ? 1 : d_row);
+    V += (size_t)split * chunk * dv_row;
+    Lkv = min(chunk, Lkv - split * chunk);
+  }
 
   for (int pass = 0; pass < num_passes; ++pass) {
   const int qt = qt_of_pass[pass];
@@ -304,7 +323,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
     constexpr int kRowsPerInstr = 64 / kKChunks;
     const int row = i * kRowsPerInstr + lane / kKChunks;
     if constexpr (kKT)  // K^T tile: [D][kBN] out of a [D][Lkv] matrix
-      req_off[t] = ((unsigned)row * (unsigned)Lkv + swz_kt(row, lane % kKChunks) * 8) * 2u;
+      req_off[t] = ((unsigned)row * (unsigned)kv_pitch + swz_kt(row, lane % kKChunks) * 8) * 2u;
     else                // K tile: [kBN][D]
       // (a physical chunk whose logical chunk lies beyond the row is never read: it re-fetches the last one)
       req_off[t] = (unsigned)(row * d_row + min(swz_k<kKChunks>(row, lane % kKChunks), k_last) * 8) * 2u;
@@ -318,7 +337,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
     if constexpr (!kVT)  // V tile: [kBN][DV]
       req_off[kKPerWave + t] = (unsigned)(row * dv_row + min(swz_v<kVChunks>(row, lane % kVChunks), v_last) * 8) * 2u;
     else                 // V^T tile: [DV][kBN] out of a [DV][Lkv] matrix
-      req_off[kKPerWave + t] = ((unsigned)row * (unsigned)Lkv + swz_k<kVChunks>(row, lane % kVChunks) * 8) * 2u;
+      req_off[kKPerWave + t] = ((unsigned)row * (unsigned)kv_pitch + swz_k<kVChunks>(row, lane % kVChunks) * 8) * 2u;
     req_lds[kKPerWave + t] = kKBytes + i * 1024;
   }
   auto issue_request = [&](int tile, int r) __attribute__((always_inline)) {
@@ -343,7 +362,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
       const int row = i * kRowsPerInstr + lane / kKChunks;
       if constexpr (kKT) {
         const int gc = min(n0 + swz_kt(row, lane % kKChunks) * 8, Lkv - 8);
-        lds_dma_16B(K + (size_t)row * Lkv + gc, dst);
+        lds_dma_16B(K + (size_t)row * kv_pitch + gc, dst);
       } else {
         const int cc = min(swz_k<kKChunks>(row, lane % kKChunks), k_last);
         const int gr = min(n0 + row, Lkv - 1);
@@ -360,7 +379,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
       } else {
         const int cc = swz_k<kVChunks>(row, lane % kVChunks);
         const int gc = min(n0 + cc * 8, Lkv - 8);
-        lds_dma_16B(V + (size_t)row * Lkv + gc, dst);
+        lds_dma_16B(V + (size_t)row * kv_pitch + gc, dst);
       }
     }
   };
@@ -445,7 +464,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   // another wavefront of the SIMD streams MFMAs - against 8 for an ordinary VALU instruction.)
   float neg_m[kQB];
   float4_t l_acc[kQB];
-  bool unset[kQB];    // kWide: no finite score seen yet (the row's reference is not set)
+  bool unset[kQB];    // kLateReference: no finite score seen yet (the row's reference is not set)
 #pragma unroll
   for (int qb = 0; qb < kQB; ++qb) {
     unset[qb] = true;
@@ -620,20 +639,20 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
 #pragma unroll
         for (int r = 0; r < 4; ++r) mx[qb] = fmaxf(mx[qb], s[kb][qb][r]);
       grow |= mx[qb] > kLazy;
-      if constexpr (kWide) grow |= unset[qb];
+      if constexpr (kLateReference) grow |= unset[qb];
     }
     // The first tile sets the reference to the row's true maximum, whichever way that is from
     // the initial 0 (every row has at least key 0 unmasked there; nothing is accumulated yet).
-    // kWide: a row whose scores were all -inf so far takes its reference from the first tile that has another.
-    const bool first = !kWide && it == 0;
+    // kLateReference: a row whose scores were all -inf so far takes its reference from the first tile that has another.
+    const bool first = !kLateReference && it == 0;
     if (first || __builtin_amdgcn_ballot_w64(grow) != 0) {
 #pragma unroll
       for (int qb = 0; qb < kQB; ++qb) {
         const float qmax = quad_max(mx[qb]) - kUp;
-        const bool set = kWide ? unset[qb] : first;
+        const bool set = kLateReference ? unset[qb] : first;
         float shift = set ? qmax : fmaxf(0.f, qmax);  // afterwards the reference only rises
         const float alpha = set ? 1.f : __builtin_amdgcn_exp2f(-shift);
-        if constexpr (kWide) {
+        if constexpr (kLateReference) {
           if (set && qmax == -INFINITY) shift = 0.f;
           unset[qb] = set && qmax == -INFINITY;
         }
@@ -820,7 +839,21 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   // 8-15 of block db and groups 1/3 the same of block db+1, 16 bytes per lane; ds_bpermute then
   // moves the 16 bytes of (row r, segment s) to lane 4*r + s, and four adjacent lanes store 64
   // contiguous bytes of a row.
-  {
+  if constexpr (kSplit) {
+    // (fp32: the 64 bytes that four lanes of a row hold are stored as they are)
+    const size_t rows = (size_t)(total_items / q_tiles / splits) * Lq;
+    const int m_row = q_row0 + lr;
+    if (m_row < Lq) {
+      const size_t row = split * rows + bh * Lq + m_row;
+#pragma unroll
+      for (int db = 0; db < kDB; ++db) *reinterpret_cast<float4_t*>(part + row * DV + 16 * db + 4 * lg) = o_acc[db][0];
+      if (lg == 0) {
+        float* stats = part + splits * rows * DV + 2 * row;
+        stats[0] = neg_m[0];
+        stats[1] = l_acc[0][0];
+      }
+    }
+  } else {
     const int st_row = lane >> 2, st_seg = lane & 3;
     // segment s of a row lives in group {0, 2, 1, 3}[s] after the swap
     const int src_lane = st_row + 16 * (((st_seg & 1) << 1) | (st_seg >> 1));
@@ -859,9 +892,47 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   }  // pass
 }
 
-template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB, bool kTail>
+// O = sum over parts of 2^(m_part - m) rows / the same of their sums, m the largest reference; a part without a score
+// above -inf (sum 0) has none.  A thread takes 8 elements of a row.  Bound by its launch and the
+// latency of two dependent reads: its rows are in the L2 (33 MB at most), the rule that asks for it counts 3.5 us for it.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void merge_parts_kernel(const float* __restrict__ part, T* __restrict__ O, size_t rows, int d,
+                                                          int splits) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const int per_row = d / 8;
+  const size_t row = i / per_row;
+  const int col = (int)(i % per_row) * 8;
+  if (row >= rows) return;
+  const float2_t* stats = reinterpret_cast<const float2_t*>(part + splits * rows * D);
+  float m = -INFINITY;
+#pragma unroll 8
+  for (int s = 0; s < splits; ++s) {
+    const float2_t x = stats[s * rows + row];
+    if (x[1] != 0.f) m = fmaxf(m, -x[0]);
+  }
+  float sum = 0.f;
+  float4_t acc[2] = {};
+#pragma unroll 4
+  for (int s = 0; s < splits; ++s) {
+    const float2_t x = stats[s * rows + row];
+    const float4_t* src = reinterpret_cast<const float4_t*>(part + (s * rows + row) * D + col);
+    const float w = x[1] != 0.f ? __builtin_amdgcn_exp2f(-x[0] - m) : 0.f;
+    sum = fmaf(w, x[1], sum);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[h][e] = fmaf(w, src[h][e], acc[h][e]);
+  }
+  typename Vec<T>::v8 out;
+  const float inv = 1.f / sum;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) out[e] = (T)(acc[e / 4][e % 4] * inv);
+  *reinterpret_cast<typename Vec<T>::v8*>(O + row * d + col) = out;
+}
+
+template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB, bool kTail, bool kSplit = false>
 int launch_w(const AttentionCall& c) {
-  auto kern = flash_attention_fwd_kernel<T, D, DV, kKT, kVT, kCausal, kWavesT, kQB, kTail>;
+  auto kern = flash_attention_fwd_kernel<T, D, DV, kKT, kVT, kCausal, kWavesT, kQB, kTail, kSplit>;
   constexpr int kBN = key_tile(D);
   constexpr int lds = ring_stages(kWavesT, D) * (kBN * (kKT ? D : lds_pitch(D)) * 2 + (kVT ? DV * kBN * 2 : kBN * lds_pitch(DV) * 2));
   static_assert(lds <= kMaxLdsBytes, "tiles do not fit in LDS");
@@ -869,7 +940,7 @@ int launch_w(const AttentionCall& c) {
   constexpr int bm = kWavesT * 16 * kQB;
   const int q_tiles = (c.Lq + bm - 1) / bm;
   const bool paired = kCausal && c.paired;
-  const int total_items = paired ? (q_tiles / 2) * c.batch : q_tiles * c.batch;
+  const int total_items = paired ? (q_tiles / 2) * c.batch : q_tiles * c.batch * (kSplit ? c.splits : 1);
   // Single causal tiles: a slice's stay on one XCD by themselves where 8 divides the slices, and where it does not if
   // that leaves the XCDs within 4% of each other (bf16, 150 slices of 384 x 384 x 256: 39.4 / 31.4 us).
   const int per_xcd = (c.batch + 7) / 8;
@@ -878,7 +949,7 @@ int launch_w(const AttentionCall& c) {
   hipLaunchKernelGGL(kern, grid, dim3(kWavesT * 64), lds, c.stream,
                      static_cast<const T*>(c.Q), static_cast<const T*>(c.K),
                      static_cast<const T*>(c.V), static_cast<T*>(c.O), c.Lq, c.Lkv, c.scale_log2,
-                     q_tiles, total_items, paired ? kPairs : by_xcd ? kByXcd : kSingle, c.d);
+                     q_tiles, total_items, paired ? kPairs : by_xcd ? kByXcd : kSingle, c.d, c.part, c.splits, c.chunk);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
@@ -899,13 +970,28 @@ int launch_layout(const AttentionCall& c) {
   if (c.v_transposed) return launch_causal<T, D, false, true>(c);
   return launch_causal<T, D, false, false>(c);
 }
+template <typename T, int D, bool kTail>
+int launch_split(const AttentionCall& c) {
+  int rc;
+  if constexpr (kTail) rc = launch_w<T, D, D, false, false, false, 4, 1, true, true>(c);
+  else rc = c.k_transposed ? launch_w<T, D, D, true, false, false, 4, 1, false, true>(c)
+                           : launch_w<T, D, D, false, false, false, 4, 1, false, true>(c);
+  if (rc != TF_OK) return rc;
+  const size_t rows = (size_t)c.batch * c.Lq, threads = rows * (c.d / 8);
+  hipLaunchKernelGGL((merge_parts_kernel<T, D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, c.stream, c.part,
+                     static_cast<T*>(c.O), rows, c.d, c.splits);
+  TFK_HIP_TRY(hipGetLastError());
+  return TF_OK;
+}
 template <int D>
 int launch(const AttentionCall& c) {
+  if (c.splits > 1) return c.bf16 ? launch_split<bf16_t, D, false>(c) : launch_split<half_t, D, false>(c);
   return c.bf16 ? launch_layout<bf16_t, D>(c) : launch_layout<half_t, D>(c);
 }
 // rows of c.d < D elements (K and V as they come)
 template <int D>
 int launch_tail(const AttentionCall& c) {
+  if (c.splits > 1) return c.bf16 ? launch_split<bf16_t, D, true>(c) : launch_split<half_t, D, true>(c);
   return c.bf16 ? launch_causal<bf16_t, D, false, false, true>(c) : launch_causal<half_t, D, false, false, true>(c);
 }
 

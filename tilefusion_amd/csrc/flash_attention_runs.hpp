@@ -15,6 +15,8 @@ struct AttentionCall {
   int rows;                                        // query rows per workgroup: 256, 128 or 64 (wide, causal: 64)
   bool paired;                                     // causal: two query tiles per workgroup (even tile counts)
   hipStream_t stream;
+  float* part = nullptr;                           // splits > 1 (no mask, V as it comes): parts of `chunk` keys, workgroups
+  int splits = 1, chunk = 0;                       // of 64 queries; room for their fp32 rows
 };
 int run_attention_d64(const AttentionCall& c);
 int run_attention_d96(const AttentionCall& c);

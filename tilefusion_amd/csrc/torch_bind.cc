@@ -187,6 +187,20 @@ void attention_impl(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& 
   TORCH_CHECK(leading_numel(K, 2) == batch && leading_numel(V, 2) == batch &&
                   leading_numel(O, 2) == batch,
               "batch dimensions must match.");
+  // Few queries against many keys: the keys in parts, where that fills the chip better.
+  if (!causal && !v_transposed && d == dv && (!k_transposed || (lkv % 8 == 0 && (d == 64 || d == 96 || d == 128)))) {
+    const int64_t bytes = tf_flash_attention_split_workspace(batch, lq, lkv, d);
+    if (bytes > 0) {
+      const at::Tensor room = at::empty({bytes}, Q.options().dtype(at::kByte));
+      const int status = tf_flash_attention_fwd_split(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dtype, batch, lq,
+                                                      lkv, d, k_transposed ? 1 : 0, softmax_scale, room.data_ptr(),
+                                                      current_stream());
+      if (status != TF_ERR_UNSUPPORTED) {
+        check_status(status, op);
+        return;
+      }
+    }
+  }
   // K as [D, Lkv]: read as it is where a kernel takes it, otherwise made [Lkv, D] first.
   if (k_transposed) {
     if (!v_transposed && d == dv) {
