@@ -149,7 +149,7 @@ TF_API int tf_flash_attention_fwd_d8(const void* Q, const void* K, const void* V
                                      void* stream);
 
 /* Without a mask, V as [Lkv, D], for problems with too few queries to fill the chip: the keys in parts, merged by a second kernel
- * (D a multiple of 8 in 40..128; K as [Lkv, D], or as [D, Lkv] with D 64, 96 or 128 and Lkv % 8 == 0).  `workspace` has
+ * (D a multiple of 8 in 40..128, or 160, 192, 256 with Lkv % 32 == 0; K as [Lkv, D], or as [D, Lkv] with D 64, 96 or 128 and Lkv % 8 == 0).  `workspace` has
  * tf_flash_attention_split_workspace bytes for the problem, 0 where the keys are not split (then, and for operands off a
  * 16-byte boundary, TF_ERR_UNSUPPORTED). */
 TF_API int64_t tf_flash_attention_split_workspace(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D);

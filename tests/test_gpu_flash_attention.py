@@ -153,7 +153,8 @@ def test_rows_between_head_dimensions(b, lq, lkv, d, causal, dtype):
 # results in either case: the same bound, and no more than 1.1 of the other's (samples of 16 x 40 elements and up).
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("b,lq,lkv,d", [(1, 16, 1500, 40), (1, 63, 5056, 128), (9, 65, 648, 128), (3, 129, 2001, 64),
-                                        (12, 20, 1280, 96), (5, 300, 4104, 80), (70, 64, 4096, 128), (2, 1708, 1664, 96)])
+                                        (12, 20, 1280, 96), (5, 300, 4104, 80), (70, 64, 4096, 128), (2, 1708, 1664, 96),
+                                        (16, 63, 4096, 256), (3, 130, 1056, 192), (8, 250, 768, 160)])
 def test_keys_in_parts(b, lq, lkv, d, dtype):
     lib, stream = _capi.load(), torch.cuda.current_stream().cuda_stream
     bytes_ = lib.tf_flash_attention_split_workspace(b, lq, lkv, d)
@@ -163,6 +164,10 @@ def test_keys_in_parts(b, lq, lkv, d, dtype):
     code = _capi.TF_DTYPE_F16 if dtype == torch.float16 else _capi.TF_DTYPE_BF16
     if d in (64, 96, 128):
         whole = c_attention(q, k, v)
+    elif d > 128:
+        whole = torch.empty_like(q)
+        _capi.check(lib.tf_flash_attention_fwd_wide(q.data_ptr(), k.data_ptr(), v.data_ptr(), whole.data_ptr(), code, b, lq, lkv,
+                                                    d, d ** -0.5, 0, stream), "whole")
     else:
         whole = torch.empty_like(q)
         _capi.check(lib.tf_flash_attention_fwd_d8(q.data_ptr(), k.data_ptr(), v.data_ptr(), whole.data_ptr(), code, b, lq, lkv,

@@ -136,7 +136,32 @@ SplitPlan plan_split(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D) {
   return plan;
 }
 
-int64_t next_tuned(int64_t D) { return D <= 64 ? 64 : D <= 96 ? 96 : 128; }
+bool is_wide(int64_t D) { return D == 160 || D == 192 || D == 256; }
+
+// Head dimensions above 128, by the same rule: a workgroup takes `alone` us for 64 keys, `shared` where two are on a CU.  bf16, us,
+// whole / in parts (how many): 16 slices of 64 x 4096 x 256 99.7 / 21.6 (13), 60 100 / 49.6 (4), 128 160 / 112 (2), 240 of 64 x
+// 2048 97 / 112 (2, not taken), 100 of 128 x 1024 29.7 / 36.8 (2, not taken), 8 of 256 x 768 x 160 17.0 / 13.7 (4).
+// 50 problems that it splits: 1.15x to 7.1x, 2.37x on average; errors against 64 bits as in one piece.
+SplitPlan plan_split_wide(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D) {
+  const int64_t items = (Lq + 63) / 64 * batch, tiles = (Lkv + 63) / 64;
+  if (items >= 256 || tiles < 8 || Lkv % 32 != 0) return {1, 0};
+  const double alone = D == 160 ? 1.17 : D == 192 ? 1.32 : 1.53, shared = D == 160 ? 2.3 : D == 192 ? 2.6 : 3.2;
+  SplitPlan plan = {1, 0};
+  double best = 0.9 * (double)tiles * alone;
+  const double row_us = (double)(batch * Lq * D * 4) / kSplitBytesPerUs;
+  for (int64_t s = 2; s <= 16 && s <= tiles / 2 && s * items <= 512; ++s) {
+    const int64_t chunk = (tiles + s - 1) / s;
+    if ((tiles + chunk - 1) / chunk != s) continue;
+    const double t = (double)chunk * (s * items <= 256 ? alone : shared) + kSplitMergeUs + (double)s * row_us;
+    if (t < best) {
+      best = t;
+      plan = {(int)s, (int)(64 * chunk)};
+    }
+  }
+  return plan;
+}
+
+int64_t next_tuned(int64_t D) { return D <= 64 ? 64 : D <= 96 ? 96 : D <= 128 ? 128 : D; }
 
 int run_by_head(const AttentionCall& c) {
   if (c.d == next_tuned(c.d)) return c.d == 128 ? run_attention_d128(c) : c.d == 96 ? run_attention_d96(c) : run_attention_d64(c);
@@ -309,9 +334,10 @@ extern "C" int tf_flash_attention_fwd_d8(const void* Q, const void* K, const voi
 
 extern "C" int64_t tf_flash_attention_split_workspace(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D) {
   using namespace tfk;
-  if (batch <= 0 || batch >= 65536 || Lq <= 0 || Lq >= 1 << 21 || Lkv <= 0 || Lkv >= 1 << 24 || D <= 32 || D > 128 || D % 8 != 0)
+  if (batch <= 0 || batch >= 65536 || Lq <= 0 || Lq >= 1 << 21 || Lkv <= 0 || Lkv >= 1 << 24 || D <= 32 || (D > 128 && !is_wide(D)) ||
+      D % 8 != 0)
     return 0;
-  const SplitPlan plan = plan_split(batch, Lq, Lkv, next_tuned(D));
+  const SplitPlan plan = is_wide(D) ? plan_split_wide(batch, Lq, Lkv, D) : plan_split(batch, Lq, Lkv, next_tuned(D));
   return plan.splits > 1 ? (int64_t)plan.splits * batch * Lq * (next_tuned(D) + 2) * 4 : 0;
 }
 
@@ -325,18 +351,18 @@ extern "C" int tf_flash_attention_fwd_split(const void* Q, const void* K, const 
   TFK_REQUIRE(dtype == TF_DTYPE_F16 || dtype == TF_DTYPE_BF16, TF_ERR_UNSUPPORTED,
               "tf_flash_attention_fwd_split: dtype must be TF_DTYPE_F16 or TF_DTYPE_BF16");
   const bool between = D != next_tuned(D);
-  TFK_REQUIRE(tf_flash_attention_split_workspace(batch, Lq, Lkv, D) > 0 && (!k_is_transposed || (Lkv % 8 == 0 && !between)),
+  TFK_REQUIRE(tf_flash_attention_split_workspace(batch, Lq, Lkv, D) > 0 && (!k_is_transposed || (Lkv % 8 == 0 && !between && !is_wide(D))),
               TF_ERR_UNSUPPORTED, "tf_flash_attention_fwd_split: the keys of [%lld, %lld, %lld, %lld] are not split",
               (long long)batch, (long long)Lq, (long long)Lkv, (long long)D);
   TFK_REQUIRE(workspace, TF_ERR_INVALID_ARG, "tf_flash_attention_fwd_split: null workspace");
   TFK_REQUIRE((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V) |
                reinterpret_cast<uintptr_t>(O) | reinterpret_cast<uintptr_t>(workspace)) % 16 == 0, TF_ERR_UNSUPPORTED,
               "tf_flash_attention_fwd_split: operands must start at a 16-byte boundary");
-  const SplitPlan plan = plan_split(batch, Lq, Lkv, next_tuned(D));
+  const SplitPlan plan = is_wide(D) ? plan_split_wide(batch, Lq, Lkv, D) : plan_split(batch, Lq, Lkv, next_tuned(D));
   const AttentionCall c = {Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, (float)(softmax_scale * 1.4426950408889634),
                            dtype == TF_DTYPE_BF16, k_is_transposed != 0, false, false, 64, false,
                            static_cast<hipStream_t>(stream), static_cast<float*>(workspace), plan.splits, plan.chunk};
-  return run_by_head(c);
+  return is_wide(D) ? run_attention_wide(c, (int)D) : run_by_head(c);
 }
 
 extern "C" int tf_flash_attention_rows(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D, int causal) {

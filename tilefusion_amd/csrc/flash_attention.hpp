@@ -178,7 +178,7 @@ TFK_DEVICE SplitWeight<T> split_weight(float p) {
 // ahead of a transposed copy in front (none in the largest case), and are left out.
 //
 // kSplit: a workgroup takes `chunk` keys (whole tiles; the last of a slice's `splits` parts may be shorter) and leaves its
-// un-normalised fp32 rows, minus their reference and their weights' sum in `part`; merge_parts_kernel puts them together.
+// un-normalised fp32 rows, minus their reference and their weights' sum in `part` (V as it comes, all head dimensions); merge_parts_kernel puts them together.
 template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB, bool kTail, bool kSplit>
 __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1) void flash_attention_fwd_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   constexpr int DP = lds_pitch(D), DVP = lds_pitch(DV);   // LDS row pitch of the K / natural V tile
   static_assert(!kKT || !kWide, "K^T tiles are 64 keys wide");
   static_assert(!kTail || (D == DV && !kWide && !kKT && !kVT), "");
-  static_assert(!kSplit || (!kCausal && !kVT && !kWide && kWavesT == 4 && kQB == 1), "");
+  static_assert(!kSplit || (!kCausal && !kVT && kWavesT == 4 && kQB == 1), "");
   // A row's reference is set by its first tile with a score above -inf, whichever that is; else by the first tile.
   constexpr bool kLateReference = kWide || kSplit;
   const int d_row = kTail ? d : D, dv_row = kTail ? d : DV;   // elements of a row in memory
@@ -974,6 +974,7 @@ template <typename T, int D, bool kTail>
 int launch_split(const AttentionCall& c) {
   int rc;
   if constexpr (kTail) rc = launch_w<T, D, D, false, false, false, 4, 1, true, true>(c);
+  else if constexpr (D > 128) rc = launch_w<T, D, D, false, false, false, 4, 1, false, true>(c);
   else rc = c.k_transposed ? launch_w<T, D, D, true, false, false, 4, 1, false, true>(c)
                            : launch_w<T, D, D, false, false, false, 4, 1, false, true>(c);
   if (rc != TF_OK) return rc;

@@ -5,6 +5,7 @@ namespace tfk {
 namespace {
 template <typename T, int D>
 int launch_wide(const AttentionCall& c) {
+  if (c.splits > 1) return launch_split<T, D, false>(c);
   if (c.causal) return launch_w<T, D, D, false, false, true, 4, 1, false>(c);
   if (c.rows == 128) return launch_w<T, D, D, false, false, false, 8, 1, false>(c);
   return launch_w<T, D, D, false, false, false, 4, 1, false>(c);
