@@ -43,7 +43,7 @@ def test_out_of_range_rows_are_skipped_and_shapes_checked():
 
 
 # Up to 1024 updates go straight to memory; beyond, workgroups sort 16 at a time (a few 16-bit updates, up to 2048) or own a
-# share of the targets; lanes take words of 32
+# share of the targets of a chunk; lanes take words of 32
 # bits, so odd slices and an odd start of a 16-bit array split pairs.  Values of
 # -1, 0, 1 keep every partial sum well below 256 (the hottest row takes 1367 of them: a standard
 # deviation of 30): exact in all types, whatever the order.
@@ -69,9 +69,8 @@ def test_scatter_nd_sorted_workgroups(dtype, rows, slice_, n, start):
     assert buf[-1].item() == 3.0 and (start == 0 or buf[0].item() == 3.0)
 
 
-# Owners of targets: one and several chunks of 2048 updates, the last as long as the others or shorter, chunks of 8192 from
-# 20000 on (and narrow slices hit often, which the sort of 128 keeps), slices of a few lanes, of one word a lane and two,
-# of more column ranges than one, indices of one and of three numbers, all updates to one target, and to none.
+# Owners of targets: one and several chunks of 1024 and 2048 updates, the last as long as the others or shorter, chunks of 4096
+# from 20000 on, slices of a few lanes, of one word a lane and two, of more column ranges than one, indices of one and of three numbers, all updates to one target, and to none.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=lambda d: str(d).split(".")[-1])
 @pytest.mark.parametrize("dims,depth,n,start", [
     ((500, 40), 1, 2048, 0), ((500, 3), 1, 2049, 1), ((6, 5, 7, 260), 3, 4097, 0), ((3000, 517), 1, 4096, 1), ((300, 1026), 1, 2500, 0),
@@ -100,6 +99,49 @@ def test_scatter_nd_owners_of_targets(dtype, dims, depth, n, start):
     assert torch.equal(one[1].float().cpu(), torch.full(dims[depth:], float(n % 2))) and not one[[0, 2]].any()
     scatter_nd(one, at * 3, sign.expand(n, *dims[depth:]).contiguous())
     assert not one[[0, 2]].any()
+
+
+# Targets with a large part of a chunk's updates: half of them to one row, an eighth to a second and a thirtieth to a third, in
+# chunks of 1024, 2048 and 4096 updates, one and two words a lane, unpaired halves, slices of one element.  All workgroups of a
+# chunk have to agree on who adds what: every update once.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("rows,slice_,n,start", [
+    (900, 20, 1281, 0), (900, 520, 2049, 0), (300, 1, 2500, 0), (300, 1, 9000, 1), (5000, 64, 4096, 0), (70, 33, 5000, 1), (2000, 1026, 3000, 0),
+    (4000, 640, 9001, 0), (4000, 8, 8193, 0), (4000, 40, 20011, 0), (3000, 530, 20000, 0), (500, 7, 33001, 0), (8, 16, 24000, 0)])
+def test_scatter_nd_hot_targets(dtype, rows, slice_, n, start):
+    from tilefusion_amd.ops import scatter_nd
+    g = torch.Generator().manual_seed(rows + n)
+    data = torch.randint(-2, 3, (rows, slice_), generator=g).to(dtype)
+    idx = torch.randint(0, rows, (n,), generator=g)
+    u = torch.rand(n, generator=g)
+    idx[u < 0.5], idx[(u >= 0.5) & (u < 0.625)], idx[(u >= 0.625) & (u < 0.658)] = rows // 3, rows - 1, 0
+    idx[7], idx[n - 1] = -1, rows
+    keep = (idx >= 0) & (idx < rows)
+    upd = torch.randint(-1, 2, (n, slice_), generator=g).to(dtype)
+    upd[(idx == rows // 3).nonzero()[100:, 0]] = 0.0               # sums stay exact in bf16 in any order
+    upd[(idx == rows - 1).nonzero()[100:, 0]] = 0.0
+    want = N.scatter_nd_ref(data, idx[keep].unsqueeze(1), upd[keep])
+    assert float(want.abs().max()) <= 128
+    for shift in (0, n // 3):                                      # the updates that count at the front, and elsewhere
+        buf = torch.full((start + data.numel() + 1,), 3.0, dtype=dtype, device=DEV)
+        dev = buf[start:start + data.numel()].view(rows, slice_)
+        dev.copy_(data)
+        scatter_nd(dev, idx.roll(shift).unsqueeze(1).to(DEV), upd.roll(shift, 0).to(DEV))
+        assert torch.equal(dev.float().cpu(), want)
+        assert buf[-1].item() == 3.0 and (start == 0 or buf[0].item() == 3.0)
+
+
+# Updates of one target are added up, 128 at least, before they are rounded to the target's type: whole numbers up to
+# 256 times 128 come out exactly in bf16, which added eight at a time stop at 2048.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("n", [4096, 8192, 16384, 24576])
+@pytest.mark.parametrize("slice_", [1, 33, 40, 520])
+def test_scatter_nd_sums_one_target_before_rounding(dtype, n, slice_):
+    from tilefusion_amd.ops import scatter_nd
+    data = torch.zeros(300, slice_, dtype=dtype, device=DEV)
+    scatter_nd(data, torch.full((n, 1), 150, device=DEV), torch.ones(n, slice_, dtype=dtype, device=DEV))
+    assert torch.equal(data[150].float(), torch.full((slice_,), float(n), device=DEV))
+    assert not data[:150].any() and not data[151:].any()
 
 
 def test_scatter_nd_fp16_sum_of_duplicates_beyond_its_range():

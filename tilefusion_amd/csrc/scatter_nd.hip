@@ -14,8 +14,8 @@
 // times.  So a workgroup sorts updates by their rows in LDS and issues ONE hardware atomic
 // per word and distinct row (16-bit types: packed pairs; a compare-and-swap loop per element, tried
 // first, retries for as long as others win).  8192 bf16 updates of 1024 into 32000 rows, log-uniform
-// indices: 2200 to 3000 us with compare-and-swap, 41 with a packed atomic per update and word, 20 with every 64
-// updates sorted as they come, 17 with workgroups that own rows (scatter_nd_owner_kernel).
+// indices: 2200 to 3000 us with compare-and-swap, 41 with a packed atomic per update and word, 21 with every 64
+// updates sorted as they come, 17 with chunks sorted whole (scatter_nd_owner_kernel).
 // What is left is the rate of the atomics themselves, ~0.9 TB/s with distinct rows as well.
 #include <algorithm>
 #include <type_traits>
@@ -284,39 +284,59 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_sgpr(80))) void
   }
 }
 
-// Many updates: a workgroup owns a share of the TARGETS (a bucket of a hash of their numbers) and 64 or 128 words of
-// their slices, looks through a chunk of 1024 * kMine updates for those of its targets, sorts them by target in LDS and adds them up
-// window by window of kWindow updates: one atomic per word and target of a chunk, and one more for every window that a
-// target's updates run across, where a workgroup that takes the next 64 updates as they come issues one per word and
-// distinct row of those 64 (8192 log-uniform updates of 32000 rows: 3252 distinct rows, 6944 over groups of 64).
-// A window is the same work however often its targets repeat, and its loads are all in flight.
-// What bounds it: the atomics as before where there are many; below ~4 MB the chain of loading indices, sorting (five
-// barriers), loading updates and the atomics, ~6 us.  us, before / now: 8192 bf16 updates of 1024 into 32000 rows 20.5 / 17.2,
-// 65536 of 1000 into 131072 194 / 90, 16384 of 4096 into 20000 162 / 62, 49954 fp32 of 622 into 77 145 / 52, 4413 fp32 of 65
-// into 72 20.3 / 9; all indices distinct: 8192 of 1024 18.7 / 20, 16384 of 4096 110 / 117 (nothing to merge).
-// The sort is by hash, not by number: two targets of one slot may lie mixed, which costs them more
-// atomics and nothing else.
+// Many updates: every workgroup of a chunk of 1024 * kMine updates sorts the chunk by target in LDS, into slots of a hash,
+// and owns some of them and 64 or 128 words of their slices, which it adds up window by window of kWindow updates: one
+// atomic per word and target of a window.  A window is the same work however often its targets repeat, and its loads are
+// all in flight.
+//
+// Who owns what must come out alike in every workgroup: the order of updates within a slot does not (it is that of LDS atomics).
+// So a slot belongs whole to the share of the sorted positions in which it begins, and the updates of a hot slot (a
+// twelfth of the chunk or more), which would keep its owner busy behind all others, go by their numbers in the chunk.
+// Windows of one target that follow each other are added up in LDS before they leave, up to 16 of them.  That is for speed
+// (atomics on one line are served one after another) and for the sum: a 16-bit target of many updates is rounded
+// with every atomic.  (With a hash to pick the owner and 8 updates an atomic, all of 8192 x 1024 bf16 into
+// one row took 50 us and came out at half its value; 12 us and 0.2% as here; every 64 as they come 18.6, 1.2%.)
+//
+// What bounds it: the atomics where there are many; below ~4 MB the chain of loading indices, sorting (five barriers,
+// an LDS atomic per update in every workgroup), loading updates and the atomics, ~6 us.  us, log-uniform indices, sorted
+// 64 or 128 as they come / hash owners / as here: 8192 bf16 of 1024 into 32000 rows 20.8 / 16.8 / 17.3, 65536 of 1000 into
+// 131072 187 / 90 / 96, 16384 of 4096 into 20000 158 / 74 / 69, 60000 of 40 into 131072 35.9 / 26.6 / 12.8, 49954 fp32 of 622
+// into 77 154 / 60 / 44; all indices distinct: 8192 of 1024 20.1 / 22.5 / 20.6, 32768 fp16 of 512 32.9 / 39.7 / 35.4; half
+// of them one row: 8192 of 1024 20.5 / 34.5 / 21.2, 60000 of 40 23.2 / 74.9 / 18.6; all: 18.7 / 50.3 / 12.2, 25.4 / 136 / 15.7.
+// Two targets of one slot may lie mixed, which costs them more atomics and nothing else.  kSingle: 16-bit slices of one element.
 constexpr int kOwnerThreads = 1024;
-template <typename T, int kMine, int kWords, Layout kLayout>
+template <typename T, int kMine, int kWords, Layout kLayout, bool kSingle>
 __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
     const T* __restrict__ updates, T* __restrict__ data, const long long* __restrict__ indices, Strides s, long long n,
-    int k, long long slice, long long total, int lanes, int bucket_bits, int chunk) {
+    int k, long long slice, long long total, int lanes, int share_bits, int chunk) {
   constexpr int kElems = Word<T>::kElems;
   constexpr int kChunk = kMine * kOwnerThreads, kSlots = 2 * kOwnerThreads, kSlotShift = 32 - 11;
   constexpr int kWindow = kMine > 2 ? 16 : 8;   // longer where more updates of a target meet
   constexpr int kFlight = kWindow / kWords;     // updates whose loads are in flight
+  constexpr int kHotSlots = 12, kHot = kChunk / kHotSlots;   // a hot slot has kHot updates or more
+  constexpr int kLinks = 16;                    // windows of one target that are added up before they leave
   constexpr float kLargest = std::is_same_v<T, half_t> ? 65504.f : std::is_same_v<T, bf16_t> ? 0x1.FEp127f : 0x1.FFFFFEp127f;
-  __shared__ unsigned s_target[kChunk];          // target numbers, sorted
-  __shared__ unsigned short s_update[kChunk];    // numbers in the chunk of their updates
-  __shared__ int s_slot[kSlots];                 // updates of a slot, then the position of its first
+  __shared__ unsigned s_target[kChunk];          // target numbers of this workgroup's updates, sorted
+  __shared__ unsigned short s_update[kChunk];    // numbers in the chunk of these updates
+  __shared__ int s_slot[kSlots];                 // updates of a slot; then the position of its first, or -1 - number of a hot slot
+  __shared__ int s_hot[kHotSlots];               // this workgroup's updates of a hot slot
   __shared__ int s_wave[kOwnerThreads / kWaveSize];
+  __shared__ int s_hots;                         // number of hot slots
+  __shared__ bool s_links;                       // windows of one target may follow each other here
+  __shared__ int s_front, s_end;                 // positions of the first slot of this workgroup and behind its last one
+  __shared__ alignas(16) bool s_linked[kOwnerThreads];
   const int tid = threadIdx.x;
-  const unsigned bucket = blockIdx.x & ((1u << bucket_bits) - 1);
-  const long long row0 = (long long)(blockIdx.x >> bucket_bits) * chunk;
+  const int shares = 1 << share_bits, share = blockIdx.x & (shares - 1);
+  const long long row0 = (long long)(blockIdx.x >> share_bits) * chunk;
   const long long row_end = std::min(row0 + chunk, n);   // (chunk <= kChunk)
 
-  // ---- this bucket's updates ----
+  // ---- updates of every slot ----
   for (int i = tid; i < kSlots; i += kOwnerThreads) s_slot[i] = 0;
+  if (tid < kHotSlots) s_hot[tid] = 0;
+  if (tid == 0) {
+    s_hots = s_front = s_end = 0;
+    s_links = false;
+  }
   unsigned target[kMine];
   bool inside[kMine];
 #pragma unroll
@@ -335,19 +355,15 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
     }
   }
   __syncthreads();
-  int rank[kMine];
+  auto slot_of = [](unsigned t) { return (t * 0x9E3779B1u) >> kSlotShift; };
+  int rank[kMine];   // (in the order of arrival: another one in every workgroup)
 #pragma unroll
-  for (int j = 0; j < kMine; ++j) {
-    // (bucket_bits + 11 <= 32; a shift by 32 - 0 is not one)
-    const unsigned long long hash = (unsigned long long)(target[j] * 0x9E3779B1u) << bucket_bits;
-    inside[j] &= (unsigned)(hash >> 32) == bucket;
-    target[j] = inside[j] ? target[j] : 0;
-    rank[j] = inside[j] ? atomicAdd(&s_slot[(unsigned)hash >> kSlotShift], 1) : 0;
-  }
+  for (int j = 0; j < kMine; ++j) rank[j] = inside[j] ? atomicAdd(&s_slot[slot_of(target[j])], 1) : 0;
   __syncthreads();
-  // ---- positions of the slots: two slots a thread ----
+  // ---- positions of the slots, the hot ones left out: two slots a thread ----
   const int c0 = s_slot[2 * tid], c1 = s_slot[2 * tid + 1];
-  int sum = c0 + c1;
+  const int n0 = c0 < kHot ? c0 : 0, n1 = c1 < kHot ? c1 : 0;
+  int sum = n0 + n1;
 #pragma unroll
   for (int d = 1; d < kWaveSize; d *= 2) {
     const int below = __shfl_up(sum, d);
@@ -361,21 +377,53 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
     if (w < tid / kWaveSize) before += s_wave[w];
     count += s_wave[w];
   }
-  s_slot[2 * tid] = before + sum - c0 - c1;
-  s_slot[2 * tid + 1] = before + sum - c1;
+  // this workgroup has the slots that begin at positions [begin, behind)
+  const int per_share = (((count + shares - 1) >> share_bits) + kWindow - 1) / kWindow * kWindow;
+  const int begin = share * per_share, behind = min(begin + per_share, count);
+  auto place = [&](int slot, int c, int n_slot, int pos) {
+    s_slot[slot] = c < kHot ? pos : -1 - atomicAdd(&s_hots, 1);
+    // (the exchange costs 2 * kWords barriers: below four windows a word, the atomics that it saves cost less)
+    if (pos >= begin && pos < behind && n_slot >= 4 * kWords * kWindow) s_links = true;
+    if (pos < begin && begin <= pos + n_slot) s_front = pos + n_slot;
+    if (pos < behind && behind <= pos + n_slot) s_end = pos + n_slot;
+  };
+  place(2 * tid, c0, n0, before + sum - n0 - n1);
+  place(2 * tid + 1, c1, n1, before + sum - n1);
   __syncthreads();
+  const bool links = s_links || s_hots > 0;
+  const int hots = s_hots, front = s_front, own = begin < count ? s_end - front : 0;
+  // ... and of the hot ones the updates [share * per_hot, (share + 1) * per_hot) of the chunk.  These come first: their runs are
+  // cut as seldom as can be, and leave no small rest that a large target would round away.
+  int base = 0;
+  if (hots > 0) {
+    const int per_hot = (((chunk + shares - 1) >> share_bits) + kLinks * kWindow - 1) / (kLinks * kWindow) * (kLinks * kWindow);
 #pragma unroll
-  for (int j = 0; j < kMine; ++j)
-    if (inside[j]) {
-      const unsigned hash = (unsigned)((unsigned long long)(target[j] * 0x9E3779B1u) << bucket_bits);
-      const int at = s_slot[hash >> kSlotShift] + rank[j];
-      s_target[at] = target[j];
-      s_update[at] = (unsigned short)(j * kOwnerThreads + tid);
+    for (int j = 0; j < kMine; ++j) {
+      const int pos = inside[j] ? s_slot[slot_of(target[j])] : 0;
+      if (pos < 0) rank[j] = (j * kOwnerThreads + tid) / per_hot == share ? atomicAdd(&s_hot[-1 - pos], 1) : -1;
     }
+    __syncthreads();
+    for (int h = 0; h < hots; ++h) base += s_hot[h];
+  }
+#pragma unroll
+  for (int j = 0; j < kMine; ++j) {
+    if (!inside[j] || rank[j] < 0) continue;
+    const int pos = s_slot[slot_of(target[j])];
+    int at = rank[j];
+    if (pos >= 0) {
+      if (pos < begin || pos >= behind) continue;
+      at += base + pos - front;
+    } else {
+      for (int h = 0; h < -1 - pos; ++h) at += s_hot[h];
+    }
+    s_target[at] = target[j];
+    s_update[at] = (unsigned short)(j * kOwnerThreads + tid);
+  }
   __syncthreads();
+  const int stop = base + own;
 
   // ---- windows of sorted updates; a group of `lanes` adjacent lanes takes one at a time, kWords words a lane ----
-  const int groups = kOwnerThreads / lanes;
+  const int groups = kOwnerThreads / lanes, group = tid / lanes;
   const long long word0 = (long long)blockIdx.y * lanes * kWords + (tid & (lanes - 1));
   auto first_elem = [&](unsigned t, int v) -> long long {   // element of the slice at word v of this lane
     return (word0 + (long long)v * lanes) * kElems - first_word_shift<T, kLayout>(data + (size_t)t * slice);
@@ -385,10 +433,14 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
     if constexpr (kLayout == Layout::kPairs) {
       return e0 < slice ? *reinterpret_cast<const unsigned*>(src + e0) : 0u;
     } else {
-      // (one load of two elements, at any even address, inside the slice; slice > 1)
+      // a half that is not the slice's has nothing to add: -0.0
+      if constexpr (kSingle) {
+        const unsigned w = *reinterpret_cast<const unsigned short*>(src);
+        return e0 < 0 ? w << 16 | 0x8000u : w | 0x80000000u;
+      }
+      // (one load of two elements, at any even address, inside the slice)
       typedef unsigned any_u32 __attribute__((aligned(2)));
       const unsigned w = *reinterpret_cast<const any_u32*>(src + std::min(std::max(e0, 0ll), slice - 2));
-      // a half that is not the slice's has nothing to add: -0.0
       return e0 < 0 ? w << 16 | 0x8000u : e0 + 1 < slice ? w : w >> 16 | 0x80000000u;
     }
   };
@@ -402,8 +454,8 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
     }
     return x;
   };
-  for (int first = tid / lanes * kWindow; first < count; first += groups * kWindow) {
-    const int end = min(first + kWindow, count);
+  for (int round = 0; round < stop; round += groups * kWindow) {
+    const int first = round + group * kWindow, end = min(first + kWindow, stop);
     Word<T> sum[kWords];
     int from = first;   // of the updates that `sum` holds
     auto clear = [&]() {
@@ -458,7 +510,43 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
         }
       }
     }
-    flush(end);
+    // A window that is all of the target in front of it leaves its sums to that one's group.
+    const bool linked = links && first < end && from == first && group % kLinks != 0 && s_target[first - 1] == s_target[first];
+    int last = end;
+    if (links) {
+      if ((tid & (lanes - 1)) == 0) s_linked[group] = linked;
+      float* const sums = reinterpret_cast<float*>(s_slot) + tid;
+      int follow = 0;   // linked windows that follow this one
+#pragma unroll
+      for (int v = 0; v < kWords; ++v) {
+        if (linked) {
+#pragma unroll
+          for (int e = 0; e < kElems; ++e) sums[e * kOwnerThreads] = sum[v].v[e];
+        }
+        __syncthreads();
+        if (v == 0) {
+          const uint4_t flags = *reinterpret_cast<const uint4_t*>(s_linked + group / kLinks * kLinks);
+          unsigned bits = 0;   // of the kLinks windows around this one
+#pragma unroll
+          for (int w = 0; w < 4; ++w) bits |= ((flags[w] * 0x10204080u) >> 28) << (4 * w);
+          follow = linked ? 0 : __builtin_ctz(~(bits >> (group % kLinks + 1)));
+          last = min(end + follow * kWindow, stop);
+        }
+        for (int h0 = 0; h0 < follow; h0 += 4) {
+          float more[4][kElems];
+#pragma unroll
+          for (int h = 0; h < 4; ++h)
+#pragma unroll
+            for (int e = 0; e < kElems; ++e) more[h][e] = sums[e * kOwnerThreads + min(h0 + h + 1, follow) * lanes];
+#pragma unroll
+          for (int h = 0; h < 4; ++h)
+#pragma unroll
+            for (int e = 0; e < kElems; ++e) sum[v].v[e] += h0 + h < follow ? more[h][e] : -0.f;
+        }
+        __syncthreads();
+      }
+    }
+    if (first < end && !linked) flush(last);
   }
 }
 
@@ -474,8 +562,8 @@ int launch_shape(const void* updates, void* data, const long long* indices, cons
   return TF_OK;
 }
 
-// As many buckets (a power of two, at least two) as bring about 224 workgroups: one a CU.
-template <typename T, int kMine, int kWords, Layout kLayout>
+// As many shares (a power of two, at least two) as bring about 224 workgroups: one a CU.
+template <typename T, int kMine, int kWords, Layout kLayout, bool kSingle>
 int launch_owner(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
                  long long slice, long long total, int lanes, long long words, hipStream_t st) {
   Strides numbers = s;
@@ -486,7 +574,7 @@ int launch_owner(const void* updates, void* data, const long long* indices, cons
   while (bits < 8 && chunks * columns * 3 << bits <= 2 * 224) ++bits;
   const int chunk = (int)((n + chunks - 1) / chunks);   // (even ones: no nearly empty last chunk)
   const dim3 grid((unsigned)((n + chunk - 1) / chunk) << bits, (unsigned)columns);
-  hipLaunchKernelGGL((scatter_nd_owner_kernel<T, kMine, kWords, kLayout>), grid, dim3(kOwnerThreads), 0, st,
+  hipLaunchKernelGGL((scatter_nd_owner_kernel<T, kMine, kWords, kLayout, kSingle>), grid, dim3(kOwnerThreads), 0, st,
                      static_cast<const T*>(updates), static_cast<T*>(data), indices, numbers, n, k, slice, total, lanes, bits,
                      chunk);
   TFK_HIP_TRY(hipGetLastError());
@@ -526,30 +614,43 @@ int launch_rows(const void* updates, void* data, const long long* indices, const
   // sorted 5.6).  From 1024 on contention shows (2048 of 64 bf16 into 64 rows: direct 10.8, sorted 6.3).
   if (n <= 1024)
     return launch_direct<T, kLayout, false>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  // Beyond, owners of targets, except: a few 16-bit updates (1489 of 1206 bf16 into 1412 rows: 9.4 sorted by 16, 10.4 by
-  // owners; 1894 of 3924 21.8 and 14.6; 1077 fp32 of 26 into 95 5.6 and 6.1, 1469 of 68 into 350 8.1 and 6.9), and narrow slices whose targets are hit often, for which the sort of the next 128
-  // finds as much to merge (58345 of 55 fp16 into 306 rows: 42 and 54).  (Target numbers are 32 bits there.)
-  const bool owners_fit = targets < (1ll << 32) && n < (1ll << 31) && (kLayout == Layout::kPairs || slice > 1) &&
-                          words <= 1024ll * lanes;
-  if ((n <= 2048 && ((sizeof(T) == 2 && n * words < 2 << 20) || !owners_fit)) || n <= 1280)
+  // Beyond, chunks sorted whole, except: a few 16-bit updates (1489 of 1206 bf16 into 1412 rows: 9.4 sorted by 16, 10.4 by
+  // the chunk; 1894 of 3924 21.8 and 14.6; 1077 fp32 of 26 into 95 5.6 and 6.1, 1469 of 68 into 350 8.1 and 6.9), and what its target
+  // numbers (32 bits) and columns do not hold: 2100 bf16 of 140000 into 300 rows 364 sorted by 64, 527 by 128, all to one row 591 and 2010.
+  const bool chunks_fit = targets < (1ll << 32) && n < (1ll << 31) && words <= 1024ll * lanes;
+  if ((n <= 2048 && ((sizeof(T) == 2 && n * words < 2 << 20) || !chunks_fit)) || n <= 1280)
     return launch_shape<T, 256, 16, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  if (!owners_fit || (words <= 32 && n > 8192 && n / 16 >= targets))
-    return launch_shape<T, 1024, 128, 2, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  // Longer chunks find more to merge and cost workgroups (16384 bf16 of 4096 into 20000 rows: 2048 updates a chunk 72,
-  // 8192 61; 8192 of 1024 into 32000 17.2 and 19.2); unpaired halves lose by them (45202 bf16 of 365 into 64 rows 49, 92).
-  // Two words a lane, likewise, halve the workgroups that look through the same indices, from 256 words on.
-  auto owners = [&](auto mine, auto per_lane) -> int {
-    return launch_owner<T, decltype(mine)::value, decltype(per_lane)::value, kLayout>(
+  if (!chunks_fit) {
+    // Every target hit at least eight times on average: the deeper sort.  A workgroup of eight wavefronts hides its own
+    // latencies where there are few of them, enough of four do it better.
+    if (n / 8 >= targets)
+      return launch_shape<T, 1024, 128, 2, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+    if ((n / 64) * ((words + lanes - 1) / lanes) < 1024)
+      return launch_shape<T, 512, 64, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+    return launch_shape<T, 256, 64, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+  }
+  // Longer chunks find more to merge, shorter ones are sorted sooner, in every workgroup.  4096 updates instead of 2048 from
+  // 20000 on (40000 bf16 of 1000 into 131072 rows 80 and 67, distinct indices 83 and 85; 8192 a chunk 69 and 88), 1024 where there are
+  // few (4096 fp32 of 64 into 8000 rows 7.7 and 7.1, 4096 bf16 of 1024 13.7 and 11.2; 3000 fp32 of 4096 27.3 and 31.5).
+  // Two words a lane halve the workgroups that sort the same indices, from 256 words on.
+  auto owners = [&](auto mine, auto per_lane, auto single) -> int {
+    return launch_owner<T, decltype(mine)::value, decltype(per_lane)::value, kLayout, decltype(single)::value>(
         updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   };
   using One = std::integral_constant<int, 1>;
   using Two = std::integral_constant<int, 2>;
   if constexpr (kLayout == Layout::kPairs) {
-    using Eight = std::integral_constant<int, 8>;
-    if (n >= 20000) return words > 256 ? owners(Eight{}, Two{}) : owners(Eight{}, One{});
-    if (words > 256) return owners(Two{}, Two{});
+    using Four = std::integral_constant<int, 4>;
+    using Many = std::false_type;
+    if (words > 256) {
+      if (n >= 20000) return owners(Four{}, Two{}, Many{});
+      return n <= 4096 && n * words <= 8 << 20 ? owners(One{}, Two{}, Many{}) : owners(Two{}, Two{}, Many{});
+    }
+    if (n >= 20000) return owners(Four{}, One{}, Many{});
+    return n <= 8192 ? owners(One{}, One{}, Many{}) : owners(Two{}, One{}, Many{});
+  } else {
+    return slice == 1 ? owners(Two{}, One{}, std::true_type{}) : owners(Two{}, One{}, std::false_type{});
   }
-  return owners(Two{}, One{});
 }
 
 template <typename T>
