@@ -336,6 +336,26 @@ def test_fused_two_gemms_and_flash_attention_ops_bf16():
         assert _close_bf16(o, ref), (causal, N.rel_l2(o, ref), N.max_abs(o, ref))
 
 
+# Tile sizes that are not positive are refused whichever kernel the shape runs, the plain one, the streaming one or
+# (operands off a 16-byte boundary) that on padded copies, and leave the output alone.
+@pytest.mark.parametrize("k,n,p", [(64, 128, 64), (64, 320, 64), (48, 320, 64), (56, 136, 40), (24, 40, 40)])
+@pytest.mark.parametrize("at", [0, 1, 2, 3])
+@pytest.mark.parametrize("tile", [0, -1, -64])
+def test_fused_two_gemms_refuses_tiles_that_are_not_positive(k, n, p, at, tile):
+    from tilefusion_amd.ops import fused_two_gemms
+    store = torch.ones(64 * k + 1, device=DEV, dtype=torch.float16)
+    b, c = torch.ones(n, k, device=DEV, dtype=torch.float16), torch.ones(p, n, device=DEV, dtype=torch.float16)
+    d = torch.full((64, p), 7.0, device=DEV, dtype=torch.float16)
+    tiles = [1, 1, 1, 1]
+    tiles[at] = tile
+    for start in (0, 1):
+        with pytest.raises(RuntimeError, match="tile sizes must be positive"):
+            fused_two_gemms(store[start:start + 64 * k].view(64, k), b, c, d, *tiles)
+    assert bool((d == 7.0).all())
+    fused_two_gemms(store[:64 * k].view(64, k), b, c, d, 1, 1, 1, 1)
+    assert bool((d == float(n * k)).all())
+
+
 # The wrappers call the implementations directly where nothing is to see the call; a mode, a profiler, autocast, a gradient
 # or a subclass gets the op itself.  Same results and same errors either way.
 def test_direct_calls_and_ops_agree_and_observers_see_the_ops():

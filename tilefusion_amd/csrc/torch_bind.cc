@@ -140,6 +140,9 @@ TILEFUSION_EXPORT void fused_two_gemms(const at::Tensor& A, const at::Tensor& B,
                  "fused_two_gemms");
     return;
   }
+  // (tiles that do not divide such a shape have always been taken, as none divides the padded one; others than positive ones are
+  // an error here as above)
+  TORCH_CHECK(tm > 0 && tn > 0 && tk > 0 && tp > 0, "fused_two_gemms: tile sizes must be positive.");
   const int status = tf_fused_two_gemms_narrow(A.data_ptr(), B.data_ptr(), C.data_ptr(), D.data_ptr(), dtype, batch,
                                                m, n, k, p, ws_ptr, ws_bytes, current_stream());
   if (status != TF_ERR_UNSUPPORTED) {
