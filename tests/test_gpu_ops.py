@@ -409,3 +409,37 @@ def test_direct_calls_and_ops_agree_and_observers_see_the_ops():
         with Log(), pytest.raises(RuntimeError) as through_op:
             bad()
         assert str(direct.value).splitlines()[0] == str(through_op.value).splitlines()[0]
+
+
+# What a program registers for an op is what the wrappers call: an implementation for the CUDA key in place of the library's, and
+# a kernel under the autograd keys, which the op's own call goes through whether a gradient is wanted or not.
+@pytest.mark.filterwarnings("ignore:Warning only once for all operators")
+@pytest.mark.parametrize("key", ["CUDA", "AutogradCUDA", "Autograd"])
+def test_registered_implementations_are_called(key):
+    from tilefusion_amd import ops
+    g = torch.Generator().manual_seed(4)
+    a, b = (torch.randn(n, 96, generator=g).half().to(DEV) for n in (70, 40))
+    c = torch.zeros(70, 40, device=DEV, dtype=torch.float32)
+    q, k, v = (torch.randn(2, n, 64, generator=g).half().to(DEV) for n in (1, 200, 200))
+    e, f = torch.randn(64, 40, generator=g).half().to(DEV), torch.zeros(70, 64, device=DEV, dtype=torch.float16)
+    data, idx, upd = torch.zeros(5, 8, device=DEV), torch.tensor([[1], [3], [1]], device=DEV), torch.ones(3, 8, device=DEV)
+    calls = {
+        "gemm": lambda: ops.gemm(a, b, c, 1, 1, 1, 1, 1),
+        "fused_two_gemms": lambda: ops.fused_two_gemms(a, b, e, f, 1, 1, 1, 1),
+        "flash_attention_fwd": lambda: ops.flash_attention(q, k.transpose(-1, -2), v, 1, 1, 64, 64, 0.125, False),
+        "flash_attention_fwd_kt": lambda: ops.flash_attention(q, k.transpose(-1, -2).contiguous(), v, 1, 1, 64, 64, 0.125, False),
+        "flash_decode": lambda: ops.flash_decode(q, k, v, 2),
+        "scatter_nd": lambda: ops.scatter_nd(data, idx, upd),
+    }
+    for name, call in calls.items():
+        seen = []
+        lib = torch.library.Library("tilefusion", "IMPL")
+        try:
+            lib.impl(name, lambda *args: seen.append(len(args)), key)
+            call()
+        finally:
+            lib._destroy()
+        assert len(seen) == 1, name
+        call()                                                     # the library's own again
+        assert len(seen) == 1, name
+    assert bool(c.any()) and bool(f.any()) and bool(data.any())

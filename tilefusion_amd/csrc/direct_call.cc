@@ -1,18 +1,19 @@
-// Python module tilefusion_amd._direct: the ops' implementations called without the dispatcher.
+// Python module tilefusion_amd._direct: the ops called without the work that the dispatcher does for any op from Python.
 //
 // A call of torch.ops.tilefusion.* from Python costs ~2 us beside the launch (matching the arguments to the schema,
-// boxing them, three dispatch keys that fall through), as much as the launch of a small kernel.  The functions
-// here take a call only where the dispatcher would do nothing but call the implementation: plain
+// boxing them, three dispatch keys under which nothing is done), as much as the launch of a small kernel.  The functions
+// here take a call only where the dispatcher would do nothing but call what is registered for the CUDA key: plain
 // device tensors, no gradient asked for, nothing that watches or rewrites ops (see `plain`).  Otherwise they
 // return False (None), having done nothing, and the wrapper in tilefusion_amd/ops goes through torch.ops, as it does for
-// torch.compile and torch.jit.script.  (An implementation that a program registers for the CUDA key in place of the
-// library's is seen through torch.ops only.)
-// us a call in a loop, through torch.ops / as here: gemm 128 x 64 x 256 4.5 / 3.3, fused 16384 x 128 x 128 x 128
-// 6.2 / 4.4 (its kernel), decoding 32 x 1999 x 64 10.7 / 8.4 (two launches).
+// torch.compile and torch.jit.script.  What is called is the dispatcher's CUDA kernel of the op, an implementation that a
+// program registers in place of the library's included.
+// us a call in a loop, through torch.ops / as here: gemm 128 x 64 x 256 4.6 / 3.7; fused 16384 x 128 x 128 x 128 4.7 / 4.4 and decoding
+// 32 x 1999 x 64 9.4 / 9.4, whose kernels take as long.
 #include <Python.h>
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/record_function.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -22,19 +23,30 @@
 #include <cmath>
 #include <vector>
 
-#include "torch_bind.hpp"
-
 namespace {
 
-// Dispatch keys under which these ops, which register an implementation for CUDA only, do what is written
-// here: the implementation, and keys that fall through to it when no gradient is asked for.
-const c10::DispatchKeySet kPlainKeys =
-    c10::DispatchKeySet(c10::DispatchKey::CUDA) | c10::DispatchKeySet(c10::DispatchKey::AutogradCUDA) |
-    c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView) | c10::DispatchKeySet(c10::DispatchKey::BackendSelect);
+// Dispatch keys above CUDA that plain tensors come with: nothing is done under them where no gradient is asked for, unless a
+// program registers something there (has_observer).
+const c10::DispatchKeySet kPassed =
+    c10::DispatchKeySet(c10::DispatchKey::AutogradCUDA) | c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView) |
+    c10::DispatchKeySet(c10::DispatchKey::BackendSelect);
+const c10::DispatchKeySet kCuda(c10::DispatchKey::CUDA);
+
+// The ops of torch_bind.cc (loaded by the package before this module).
+template <typename Signature>
+c10::TypedOperatorHandle<Signature> find_op(const char* name) {
+  return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Signature>();
+}
+using AttentionOp = void(const at::Tensor&, const at::Tensor&, const at::Tensor&, at::Tensor&, double, bool);
+
+// A program has registered something under the keys that are passed.
+bool has_observer(const c10::OperatorHandle& op) {
+  return op.hasKernelForAnyDispatchKey(kPassed) || op.hasKernelForDispatchKey(c10::DispatchKey::Autograd);
+}
 
 // Takes the tensors out of args[0 .. n); false unless every one is an ordinary torch.Tensor (no subclass) on a GPU that
-// wants no gradient, and no mode, transform, autocast, tracer or profiler is to see the call.
-bool plain(PyObject* const* args, int n, at::Tensor* out) {
+// wants no gradient, and no mode, transform, autocast, tracer, profiler or observer of `op` is to see the call.
+bool plain(const c10::OperatorHandle& op, PyObject* const* args, int n, at::Tensor* out) {
   c10::DispatchKeySet keys;
   for (int i = 0; i < n; ++i) {
     if (!THPVariable_CheckExact(args[i])) return false;
@@ -45,9 +57,9 @@ bool plain(PyObject* const* args, int n, at::Tensor* out) {
     out[i] = t;   // (held while the interpreter is unlocked)
   }
   const auto local = c10::impl::tls_local_dispatch_key_set();
-  keys = ((keys | local.included_) - local.excluded_) - kPlainKeys;
+  keys = ((keys | local.included_) - local.excluded_) - (kPassed | kCuda);
   return keys.highestFunctionalityKey() == c10::DispatchKey::Undefined && !at::impl::torch_function_mode_enabled() &&
-         !at::hasCallbacks();
+         !at::hasCallbacks() && !has_observer(op);
 }
 
 // ints only (a bool, a numpy number or a tensor is the dispatcher's business)
@@ -74,10 +86,12 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   at::Tensor t[3];
   int64_t i[5];
-  if (nargs != 8 || !plain(args, 3, t) || !ints(args + 3, 5, i)) Py_RETURN_FALSE;
+  using Op = void(const at::Tensor&, const at::Tensor&, at::Tensor&, int64_t, int64_t, int64_t, int64_t, int64_t);
+  static const auto op = find_op<Op>("tilefusion::gemm");
+  if (nargs != 8 || !plain(op, args, 3, t) || !ints(args + 3, 5, i)) Py_RETURN_FALSE;
   {
     NoGil unlocked;
-    tilefusion::kernels::gemm(t[0], t[1], t[2], i[0], i[1], i[2], i[3], i[4]);
+    op.redispatch(kCuda, t[0], t[1], t[2], i[0], i[1], i[2], i[3], i[4]);
   }
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -87,12 +101,14 @@ PyObject* fused_two_gemms(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   at::Tensor t[4];
   int64_t i[4];
-  if (nargs != 8 || !plain(args, 4, t) || !ints(args + 4, 4, i)) Py_RETURN_FALSE;
+  using Op = void(const at::Tensor&, const at::Tensor&, const at::Tensor&, at::Tensor&, int64_t, int64_t, int64_t, int64_t);
+  static const auto op = find_op<Op>("tilefusion::fused_two_gemms");
+  if (nargs != 8 || !plain(op, args, 4, t) || !ints(args + 4, 4, i)) Py_RETURN_FALSE;
   for (const at::Tensor& x : t)   // (other types: the wrapper's own errors)
     if (!is_half_type(x) || x.scalar_type() != t[0].scalar_type()) Py_RETURN_FALSE;
   {
     NoGil unlocked;
-    tilefusion::kernels::fused_two_gemms(t[0], t[1], t[2], t[3], i[0], i[1], i[2], i[3]);
+    op.redispatch(kCuda, t[0], t[1], t[2], t[3], i[0], i[1], i[2], i[3]);
   }
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -101,10 +117,11 @@ PyObject* fused_two_gemms(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 PyObject* scatter_nd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {   // data, updates, indices
   HANDLE_TH_ERRORS
   at::Tensor t[3];
-  if (nargs != 3 || !plain(args, 3, t)) Py_RETURN_FALSE;
+  static const auto op = find_op<void(const at::Tensor&, at::Tensor&, const at::Tensor&)>("tilefusion::scatter_nd");
+  if (nargs != 3 || !plain(op, args, 3, t)) Py_RETURN_FALSE;
   {
     NoGil unlocked;
-    tilefusion::kernels::scatter_nd(t[0], t[1], t[2]);
+    op.redispatch(kCuda, t[0], t[1], t[2]);
   }
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -116,7 +133,10 @@ PyObject* flash_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   at::Tensor t[3];
   int64_t tile[4];
-  if (nargs != 9 || !plain(args, 3, t) || !ints(args + 3, 4, tile) || !PyFloat_CheckExact(args[7]) || !PyBool_Check(args[8]))
+  static const auto op = find_op<AttentionOp>("tilefusion::flash_attention_fwd");
+  static const auto op_kt = find_op<AttentionOp>("tilefusion::flash_attention_fwd_kt");
+  if (nargs != 9 || !plain(op, args, 3, t) || has_observer(op_kt) || !ints(args + 3, 4, tile) || !PyFloat_CheckExact(args[7]) ||
+      !PyBool_Check(args[8]))
     Py_RETURN_NONE;
   const at::Tensor &q = t[0], &k = t[1], &v = t[2];
   if (q.dim() < 2 || k.dim() < 2 || v.dim() < 2) Py_RETURN_NONE;
@@ -133,9 +153,9 @@ PyObject* flash_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     out = at::empty(shape, q.options());
     const at::Tensor key_rows = k.transpose(-1, -2);
     if (k.is_contiguous() && !key_rows.is_contiguous())
-      tilefusion::kernels::flash_attention_fwd_kt(q.contiguous(), k, v.contiguous(), out, scale, causal);
+      op_kt.redispatch(kCuda, q.contiguous(), k, v.contiguous(), out, scale, causal);
     else
-      tilefusion::kernels::flash_attention_fwd(q.contiguous(), key_rows.contiguous(), v.contiguous(), out, scale, causal);
+      op.redispatch(kCuda, q.contiguous(), key_rows.contiguous(), v.contiguous(), out, scale, causal);
   }
   return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
@@ -146,7 +166,9 @@ PyObject* flash_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   at::Tensor t[3];
   int64_t num_splits;
-  if (nargs != 5 || !plain(args, 3, t) || !ints(args + 3, 1, &num_splits)) Py_RETURN_NONE;
+  using Op = void(const at::Tensor&, const at::Tensor&, const at::Tensor&, at::Tensor&, int64_t, double);
+  static const auto op = find_op<Op>("tilefusion::flash_decode");
+  if (nargs != 5 || !plain(op, args, 3, t) || !ints(args + 3, 1, &num_splits)) Py_RETURN_NONE;
   if (args[4] != Py_None && !PyFloat_CheckExact(args[4])) Py_RETURN_NONE;
   const at::Tensor &q = t[0], &k = t[1], &v = t[2];
   if (q.dim() < 1 || q.size(-1) < 1) Py_RETURN_NONE;
@@ -155,7 +177,7 @@ PyObject* flash_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   {
     NoGil unlocked;
     out = at::empty_like(q);
-    tilefusion::kernels::flash_decode(q.contiguous(), k.contiguous(), v.contiguous(), out, num_splits, scale);
+    op.redispatch(kCuda, q.contiguous(), k.contiguous(), v.contiguous(), out, num_splits, scale);
   }
   return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS

@@ -17,7 +17,6 @@
 #include <vector>
 
 #include "tilefusion_c.h"
-#include "torch_bind.hpp"
 
 // The dtype switch of the reference (include/kernels/dispatch_macros.hpp:6-23).  This file is
 // built by the host compiler without the device headers, so the element types are ATen's.
