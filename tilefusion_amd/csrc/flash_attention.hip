@@ -163,6 +163,14 @@ SplitPlan plan_split_wide(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D) {
 
 int64_t next_tuned(int64_t D) { return D <= 64 ? 64 : D <= 96 ? 96 : D <= 128 ? 128 : D; }
 
+// (any arguments: one part for what is not split)
+SplitPlan plan_split_any(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D) {
+  if (batch <= 0 || batch >= 65536 || Lq <= 0 || Lq >= 1 << 21 || Lkv <= 0 || Lkv >= 1 << 24 || D <= 32 || (D > 128 && !is_wide(D)) ||
+      D % 8 != 0)
+    return {1, 0};
+  return is_wide(D) ? plan_split_wide(batch, Lq, Lkv, D) : plan_split(batch, Lq, Lkv, next_tuned(D));
+}
+
 int run_by_head(const AttentionCall& c) {
   if (c.d == next_tuned(c.d)) return c.d == 128 ? run_attention_d128(c) : c.d == 96 ? run_attention_d96(c) : run_attention_d64(c);
   return c.d > 96 ? run_attention_below128(c) : c.d > 64 ? run_attention_below96(c) : run_attention_below64(c);
@@ -334,10 +342,7 @@ extern "C" int tf_flash_attention_fwd_d8(const void* Q, const void* K, const voi
 
 extern "C" int64_t tf_flash_attention_split_workspace(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D) {
   using namespace tfk;
-  if (batch <= 0 || batch >= 65536 || Lq <= 0 || Lq >= 1 << 21 || Lkv <= 0 || Lkv >= 1 << 24 || D <= 32 || (D > 128 && !is_wide(D)) ||
-      D % 8 != 0)
-    return 0;
-  const SplitPlan plan = is_wide(D) ? plan_split_wide(batch, Lq, Lkv, D) : plan_split(batch, Lq, Lkv, next_tuned(D));
+  const SplitPlan plan = plan_split_any(batch, Lq, Lkv, D);
   return plan.splits > 1 ? (int64_t)plan.splits * batch * Lq * (next_tuned(D) + 2) * 4 : 0;
 }
 
@@ -351,14 +356,14 @@ extern "C" int tf_flash_attention_fwd_split(const void* Q, const void* K, const 
   TFK_REQUIRE(dtype == TF_DTYPE_F16 || dtype == TF_DTYPE_BF16, TF_ERR_UNSUPPORTED,
               "tf_flash_attention_fwd_split: dtype must be TF_DTYPE_F16 or TF_DTYPE_BF16");
   const bool between = D != next_tuned(D);
-  TFK_REQUIRE(tf_flash_attention_split_workspace(batch, Lq, Lkv, D) > 0 && (!k_is_transposed || (Lkv % 8 == 0 && !between && !is_wide(D))),
+  const SplitPlan plan = plan_split_any(batch, Lq, Lkv, D);
+  TFK_REQUIRE(plan.splits > 1 && (!k_is_transposed || (Lkv % 8 == 0 && !between && !is_wide(D))),
               TF_ERR_UNSUPPORTED, "tf_flash_attention_fwd_split: the keys of [%lld, %lld, %lld, %lld] are not split",
               (long long)batch, (long long)Lq, (long long)Lkv, (long long)D);
   TFK_REQUIRE(workspace, TF_ERR_INVALID_ARG, "tf_flash_attention_fwd_split: null workspace");
   TFK_REQUIRE((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V) |
                reinterpret_cast<uintptr_t>(O) | reinterpret_cast<uintptr_t>(workspace)) % 16 == 0, TF_ERR_UNSUPPORTED,
               "tf_flash_attention_fwd_split: operands must start at a 16-byte boundary");
-  const SplitPlan plan = is_wide(D) ? plan_split_wide(batch, Lq, Lkv, D) : plan_split(batch, Lq, Lkv, next_tuned(D));
   const AttentionCall c = {Q, K, V, O, (int)batch, (int)Lq, (int)Lkv, (int)D, (float)(softmax_scale * 1.4426950408889634),
                            dtype == TF_DTYPE_BF16, k_is_transposed != 0, false, false, 64, false,
                            static_cast<hipStream_t>(stream), static_cast<float*>(workspace), plan.splits, plan.chunk};
