@@ -128,6 +128,21 @@ def test_wide_attention_cases_reach_both_workgroup_sizes():
         (rows, causal) for rows in (64, 128) for causal in (False, True)}
 
 
+def test_fused_cases_reach_every_streaming_instance():
+    from tests.test_gpu_fused_two_gemms import STREAM_CASES
+    lib = _capi.load()
+    whole, cut = set(), set()
+    for m, n, k, p in STREAM_CASES:
+        size = lib.tf_fused_two_gemms_workspace_bytes(_capi.TF_DTYPE_F16, 1, m, n, k, p)
+        rows = lib.tf_fused_two_gemms_rows(1, m, n, k, p, size)
+        (cut if size else whole).add(((max(k, 64) + 31) // 32, 4 if p <= 64 else 6 if p <= 96 else 8, rows))
+    assert whole == {(steps, blocks, rows) for steps in (2, 3, 4) for blocks in (4, 6, 8) for rows in (64, 128)}
+    assert {x[:2] for x in cut} == {x[:2] for x in whole} and {x[2] for x in cut} == {64, 128}
+    assert lib.tf_fused_two_gemms_rows(1, 16384, 128, 128, 128, 0) == 0     # one n-tile: the plain kernel
+    assert lib.tf_fused_two_gemms_rows(1, 4000, 4096, 128, 128, 0) == 64    # no room for partial sums: other rows
+    assert lib.tf_fused_two_gemms_workspace_bytes(_capi.TF_DTYPE_F32, 1, 70, 2056, 64, 64) == 0
+
+
 def test_python_wrappers_validate_like_the_reference():
     # python/ops/fused_two_gemms.py:33-38: ValueError for a CPU tensor, TypeError for dtype
     import torch

@@ -169,9 +169,8 @@ def test_every_plain_kernel_instance_is_exact(dtype, k, p, n):
         assert torch.equal(d.float(), ref)
 
 
-# Narrow K and P that are multiples of 8 only run the streaming kernel as they are: every instance (two to four steps of
-# K, 4, 6 and 8 column blocks, 64 and 128 rows), half-full last steps, last n-tiles that overlap their neighbour or are the
-# only one, uncut, cut, one tile a part, one row.  Integers again; an infinity in the last column of C reaches that
+# Narrow K and P that are multiples of 8 only run the streaming kernel as they are: half-full last steps, last n-tiles that
+# overlap their neighbour or are the only one, uncut, cut, one tile a part, one row.  Integers again; an infinity in the last column of C reaches that
 # row of C only, whatever the overlapping columns and the chunks beyond K are multiplied with.
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("batch,m,n,k,p", [
@@ -210,6 +209,30 @@ def test_narrow_shapes_exact(batch, m, n, k, p, dtype):
     assert torch.equal(torch.isnan(got), s == 0) and torch.equal(got[s != 0], torch.sign(s[s != 0]) * float("inf"))
     keep = [i for i in range(p) if i != p // 2]
     assert torch.equal(d2[..., keep], d[..., keep])
+
+
+# Every instance of the streaming kernel (two to four steps of K, 4, 6 and 8 column blocks, 64 and 128 rows), with full and half-full last
+# steps and ragged rows, n-tiles and columns, uncut and cut along N.  Integers again: B and C have few entries in a row.
+STREAM_CASES = [(m, n, k, p) for m, n in [(70, 264), (17000, 264), (70, 2056), (1000, 2056), (9000, 2056)]
+                for k in (48, 64, 72, 96, 104, 128) for p in (40, 64, 80, 96, 128)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k,p", STREAM_CASES)
+def test_every_streaming_instance_is_exact(m, n, k, p, dtype):
+    g = torch.Generator().manual_seed(m + n + k + p)
+    a = torch.randint(-2, 3, (m, k), generator=g).to(dtype)
+    b = torch.zeros(n, k).scatter_(1, torch.randint(0, k, (n, 5), generator=g), 1.0)
+    c = torch.zeros(p, n).scatter_(1, torch.randint(0, n, (p, 6), generator=g), -1.0)
+    b[:, -1], c[:, -1], c[:, 0] = 1.0, 1.0, 1.0
+    rows = torch.cat([torch.arange(0, min(m, 130)), torch.arange(max(0, m - 70), m)])
+    ref = a[rows].float() @ b.T @ c.T
+    assert float(ref.abs().max()) <= 256   # exact in bf16 too
+    store = torch.full((m * p + 64,), float("nan"), device=DEV, dtype=dtype)
+    d = store[:-64].view(m, p)
+    ops.fused_two_gemms(a.to(DEV), b.to(DEV, dtype), c.to(DEV, dtype), d, 1, 1, 1, 1)
+    assert torch.equal(d[rows.to(DEV)].float().cpu(), ref)
+    assert not bool(torch.isnan(d).any()) and bool(torch.isnan(store[-64:]).all())
 
 
 def test_bf16_random_inputs_within_tolerance():

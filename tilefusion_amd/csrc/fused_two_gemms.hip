@@ -420,12 +420,16 @@ size_t partial_bytes(const FusedPlan& plan, int64_t batch, int64_t M, int64_t P)
   return plan.parts > 1 ? (size_t)plan.parts * (size_t)batch * (size_t)M * (size_t)P * sizeof(float) : 0;
 }
 
+// What a problem runs with `room` bytes for partial sums; rows = 0: the plain kernel.
+FusedPlan plan_fused(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t P, size_t room) {
+  if (!may_stream(batch, M, N, K, P)) return {0, 1, 0};
+  const FusedPlan plan = plan_stream(batch, M, N, K, P, room > 0);
+  return partial_bytes(plan, batch, M, P) <= room ? plan : plan_stream(batch, M, N, K, P, false);
+}
+
 int run_fused(const void* A, const void* B, const void* C, void* D, bool bf16, int64_t batch, int64_t M, int64_t N,
-              int64_t K, int64_t P, void* workspace, size_t workspace_bytes, hipStream_t st) {
-  if (may_stream(batch, M, N, K, P) && aligned16(A, B, C, D)) {
-    FusedPlan plan = plan_stream(batch, M, N, K, P, true);
-    if (workspace == nullptr || workspace_bytes < partial_bytes(plan, batch, M, P))
-      plan = plan_stream(batch, M, N, K, P, false);
+              int64_t K, int64_t P, FusedPlan plan, void* workspace, hipStream_t st) {
+  if (plan.rows > 0 && aligned16(A, B, C, D)) {
     const FusedCall call = {A, B, C, D, workspace, bf16, (int)batch, (int)M, (int)N, (int)K, (int)P, st};
     return run_fused_stream(call, plan);
   }
@@ -440,29 +444,32 @@ extern "C" int tf_fused_two_gemms_f16(const void* A, const void* B, const void* 
                                       int tm, int tn, int tk, int tp, void* stream) {
   using namespace tfk;
   if (int rc = check_fused_args("tf_fused_two_gemms_f16", A, B, C, D, batch, M, N, K, P, tm, tn, tk, tp)) return rc;
-  return run_fused(A, B, C, D, false, batch, M, N, K, P, nullptr, 0, static_cast<hipStream_t>(stream));
+  return run_fused(A, B, C, D, false, batch, M, N, K, P, plan_fused(batch, M, N, K, P, 0), nullptr, static_cast<hipStream_t>(stream));
 }
 
 extern "C" size_t tf_fused_two_gemms_workspace_bytes(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
                                                      int64_t P) {
   using namespace tfk;
   if ((dtype != TF_DTYPE_F16 && dtype != TF_DTYPE_BF16) || batch <= 0 || M <= 0 || N <= 0 || K <= 0 || P <= 0) return 0;
-  if (!may_stream(batch, M, N, K, P)) return 0;
-  return partial_bytes(plan_stream(batch, M, N, K, P, true), batch, M, P);
+  return partial_bytes(plan_fused(batch, M, N, K, P, SIZE_MAX), batch, M, P);
+}
+
+extern "C" int tf_fused_two_gemms_rows(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t P, size_t workspace_bytes) {
+  if (batch <= 0 || M <= 0 || N <= 0 || K <= 0 || P <= 0) return 0;
+  return tfk::plan_fused(batch, M, N, K, P, workspace_bytes).rows;
 }
 
 extern "C" int tf_fused_two_gemms_ws(const void* A, const void* B, const void* C, void* D, int dtype, int64_t batch,
                                      int64_t M, int64_t N, int64_t K, int64_t P, int tm, int tn, int tk, int tp,
                                      void* workspace, size_t workspace_bytes, void* stream) {
   using namespace tfk;
-  const size_t want = tf_fused_two_gemms_workspace_bytes(dtype, batch, M, N, K, P);
-  if (want == 0 || workspace == nullptr || workspace_bytes < want)
+  if (workspace == nullptr || workspace_bytes == 0 || (dtype != TF_DTYPE_F16 && dtype != TF_DTYPE_BF16))
     return tf_fused_two_gemms(A, B, C, D, dtype, batch, M, N, K, P, tm, tn, tk, tp, stream);
   if (int rc = check_fused_args("tf_fused_two_gemms_ws", A, B, C, D, batch, M, N, K, P, tm, tn, tk, tp)) return rc;
-  TFK_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, TF_ERR_INVALID_ARG,
+  const FusedPlan plan = plan_fused(batch, M, N, K, P, workspace_bytes);
+  TFK_REQUIRE(plan.parts == 1 || reinterpret_cast<uintptr_t>(workspace) % 16 == 0, TF_ERR_INVALID_ARG,
               "tf_fused_two_gemms_ws: workspace must be 16-byte aligned");
-  return run_fused(A, B, C, D, dtype == TF_DTYPE_BF16, batch, M, N, K, P, workspace, workspace_bytes,
-                   static_cast<hipStream_t>(stream));
+  return run_fused(A, B, C, D, dtype == TF_DTYPE_BF16, batch, M, N, K, P, plan, workspace, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tf_fused_two_gemms_narrow(const void* A, const void* B, const void* C, void* D, int dtype, int64_t batch,
@@ -482,8 +489,8 @@ extern "C" int tf_fused_two_gemms_narrow(const void* A, const void* B, const voi
               (long long)K, (long long)N, (long long)P);
   TFK_REQUIRE(workspace == nullptr || reinterpret_cast<uintptr_t>(workspace) % 16 == 0, TF_ERR_INVALID_ARG,
               "tf_fused_two_gemms_narrow: workspace must be 16-byte aligned");
-  return run_fused(A, B, C, D, dtype == TF_DTYPE_BF16, batch, M, N, K, P, workspace, workspace_bytes,
-                   static_cast<hipStream_t>(stream));
+  const FusedPlan plan = plan_fused(batch, M, N, K, P, workspace != nullptr ? workspace_bytes : 0);
+  return run_fused(A, B, C, D, dtype == TF_DTYPE_BF16, batch, M, N, K, P, plan, workspace, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tf_fused_two_gemms(const void* A, const void* B, const void* C, void* D, int dtype, int64_t batch,
@@ -495,5 +502,5 @@ extern "C" int tf_fused_two_gemms(const void* A, const void* B, const void* C, v
               "tf_fused_two_gemms: dtype must be TF_DTYPE_F16 or TF_DTYPE_BF16");
   // bf16: the same kernels with the bf16 MFMA, a bf16 intermediate and bf16 output
   if (int rc = check_fused_args("tf_fused_two_gemms", A, B, C, D, batch, M, N, K, P, tm, tn, tk, tp)) return rc;
-  return run_fused(A, B, C, D, true, batch, M, N, K, P, nullptr, 0, static_cast<hipStream_t>(stream));
+  return run_fused(A, B, C, D, true, batch, M, N, K, P, plan_fused(batch, M, N, K, P, 0), nullptr, static_cast<hipStream_t>(stream));
 }
