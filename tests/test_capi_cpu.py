@@ -128,6 +128,20 @@ def test_wide_attention_cases_reach_both_workgroup_sizes():
         (rows, causal) for rows in (64, 128) for causal in (False, True)}
 
 
+def test_attention_cases_reach_every_workgroup_form():
+    from tests.test_gpu_flash_attention import PAIR_CASES, RING_CASES, SINGLE_CASES
+    lib = _capi.load()
+    tuned = [(rows, d) for rows in (64, 128, 256) for d in (64, 96, 128)]
+    for cases, paired in ((PAIR_CASES, 1), (SINGLE_CASES, 0)):
+        for rows, b, lq, lkv, d in cases:
+            assert lib.tf_flash_attention_rows(b, lq, lkv, d, 1) == rows and lib.tf_flash_attention_pairs(b, lq, lkv, d, 1) == paired
+            assert lib.tf_flash_attention_pairs(1, lq, lkv, d, 1) == 0   # a slice alone
+        assert {(c[0], c[4]) for c in cases} == set(tuned)
+    for rows, b in RING_CASES:
+        for lkv in (8, 64, 72, 128, 192, 200, 256, 320, 384, 448):
+            assert {lib.tf_flash_attention_rows(b, 256, lkv, 128, causal) for causal in (0, 1)} == {rows}
+
+
 def test_fused_cases_reach_every_streaming_instance():
     from tests.test_gpu_fused_two_gemms import STREAM_CASES
     lib = _capi.load()

@@ -52,19 +52,27 @@ def test_shapes(b, lq, lkv, d, causal, v_transposed):
     assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
 
 
-# The 256-query workgroup keeps a five-tile ring with two tiles live and requests three tiles
+# The 256- and 128-query workgroups keep a five-tile ring with two tiles live and request three tiles
 # ahead: key ranges of one to seven tiles, with and without a ragged last tile, exercise its fill,
-# the clamped requests past the end and the hand-over between the two wavefront sets; 768 queries
-# (an odd number of query tiles) take the one-pass causal order, 512 and 1024 the paired one.
+# the clamped requests past the end and the hand-over between the two wavefront sets; the 64-query workgroup has
+# a ring of four tiles and one set.  (The number of slices decides which of them runs.)
+RING_CASES = [(64, 2), (128, 128), (256, 256)]   # query rows per workgroup, slices of 256 queries
+
+
 @pytest.mark.parametrize("lkv", [8, 64, 72, 128, 192, 200, 256, 320, 384, 448])
 @pytest.mark.parametrize("causal", [False, True])
-def test_short_key_ranges_through_the_eight_wavefront_ring(lkv, causal):
-    q, k, v = _inputs(2, 256, lkv, 128, 900 + lkv)
+@pytest.mark.parametrize("rows,b", RING_CASES)
+def test_short_key_ranges_through_the_eight_wavefront_ring(rows, b, lkv, causal):
+    assert _capi.load().tf_flash_attention_rows(b, 256, lkv, 128, int(causal)) == rows
+    q, k, v = _inputs(b, 256, lkv, 128, 900 + lkv)
     o = c_attention(q.to(DEV), k.to(DEV), v.to(DEV), causal, None, False)
-    ok, r, m = N.check_close(o, N.attention_ref(q, k, v, causal=causal))
+    assert not torch.isnan(o).any()
+    pick = sorted({0, b // 2, b - 1})
+    ok, r, m = N.check_close(o[pick], N.attention_ref(q[pick], k[pick], v[pick], causal=causal))
     assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
 
 
+# Single causal tiles of 64 queries: an odd and an even number of them, a ragged last one.
 @pytest.mark.parametrize("lq,d", [(512, 128), (768, 128), (1024, 64), (300, 128), (512, 96), (768, 96)])
 def test_causal_pass_orders(lq, d):
     q, k, v = _inputs(3, lq, lq, d, 77 + lq)
@@ -85,6 +93,40 @@ def test_causal_pairs_and_single_tiles_agree(bh, lq, d):
         assert torch.equal(o[i:i + 1], alone), i
     ok, r, m = N.check_close(o[-1:].cpu(), N.attention_ref(q[-1:].cpu(), k[-1:].cpu(), v[-1:].cpu(), causal=True))
     assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
+
+
+# Causal pairs and single tiles at every workgroup size and head dimension, with ragged last query and key tiles: the second
+# pass of a pair fills the ring behind the clamped requests of the first.  Every order of K and V, and rows of
+# fewer elements, against a slice alone, which runs single tiles (bit for bit), and the oracle.
+PAIR_CASES = [(64, 512, 250, 256, 64), (128, 229, 385, 392, 64), (256, 512, 300, 304, 64),
+              (64, 21, 1531, 1536, 96), (128, 52, 961, 968, 96), (256, 192, 300, 304, 96),
+              (64, 26, 1100, 1104, 128), (128, 43, 1217, 1224, 128), (256, 192, 300, 304, 128)]
+SINGLE_CASES = [(64, 5, 257, 264, 64), (128, 88, 129, 136, 64), (256, 88, 385, 392, 64),
+                (64, 5, 257, 264, 96), (128, 88, 129, 136, 96), (256, 88, 257, 264, 96),
+                (64, 5, 257, 264, 128), (128, 88, 129, 136, 128), (256, 88, 257, 264, 128)]
+
+
+@pytest.mark.parametrize("rows,b,lq,lkv,d", PAIR_CASES + SINGLE_CASES)
+@pytest.mark.parametrize("less", [0, 16])
+def test_causal_forms(rows, b, lq, lkv, d, less):
+    assert _capi.load().tf_flash_attention_rows(b, lq, lkv, d, 1) == rows
+    e = d - less
+    q, k, v = (x.to(DEV) for x in _inputs(b, lq, lkv, e, rows + b + lq + e))
+
+    def natural(q, k, v):
+        o = torch.full_like(q, float("nan"))
+        torch.ops.tilefusion.flash_attention_fwd(q, k, v, o, e ** -0.5, True)
+        return o
+    o = natural(q, k, v)
+    for i in (0, 7 % b, b // 2, b - 1):
+        one = slice(i, i + 1)
+        assert torch.equal(o[one], natural(q[one].contiguous(), k[one].contiguous(), v[one].contiguous())), i
+    ok, r, m = N.check_close(o[-1:].cpu(), N.attention_ref(q[-1:].cpu(), k[-1:].cpu(), v[-1:].cpu(), causal=True))
+    assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
+    assert not torch.isnan(o).any()
+    if not less:
+        assert torch.equal(ops.flash_attention(q, k.transpose(1, 2).contiguous(), v, 1, 1, d, d, d ** -0.5, True), o)
+        assert torch.equal(c_attention(q, k, v.transpose(1, 2).contiguous(), True, None, True), o)
 
 
 # A key stored [D, Lkv] is read as it is: the same products in the same order as on the transposed key, so the same

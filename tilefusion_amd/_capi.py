@@ -42,6 +42,7 @@ SIGNATURES = {
     "tf_gemm_kernel_index": (_i, [_i64, _i64, _i64, _i]),
     "tf_flash_decode_plan": (_i, [_i64, _i64, _i64, _i, ctypes.POINTER(_i)]),
     "tf_flash_attention_rows": (_i, [_i64, _i64, _i64, _i64, _i]),
+    "tf_flash_attention_pairs": (_i, [_i64, _i64, _i64, _i64, _i]),
     "tf_flash_attention_wide_rows": (_i, [_i64, _i64, _i]),
     "tf_fused_two_gemms_rows": (_i, [_i64, _i64, _i64, _i64, _i64, _sz]),
     "tf_jit_compile": (_i, [ctypes.c_char_p, ctypes.c_char_p, ctypes.POINTER(ctypes.c_char_p), _i,

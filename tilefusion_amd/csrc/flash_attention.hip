@@ -375,6 +375,11 @@ extern "C" int tf_flash_attention_rows(int64_t batch, int64_t Lq, int64_t Lkv, i
   return tfk::plan_attention(batch, Lq, Lkv, D, causal != 0).rows;
 }
 
+extern "C" int tf_flash_attention_pairs(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D, int causal) {
+  if (batch <= 0 || Lq <= 0 || Lkv <= 0 || (D != 64 && D != 96 && D != 128)) return 0;
+  return tfk::plan_attention(batch, Lq, Lkv, D, causal != 0).paired;
+}
+
 extern "C" int tf_flash_attention_wide_rows(int64_t batch, int64_t Lq, int causal) {
   const tfk::AttentionPlan plan = tfk::plan_wide(batch, Lq, causal != 0);
   return plan.paired ? 2 * plan.rows : plan.rows;
