@@ -15,7 +15,7 @@
 //     and exp2(S^T) converted to fp16 is already the B-operand fragment of the second MFMA
 //     O^T = V^T P^T;
 //   * K and V tiles go global -> LDS directly (global_load_lds_dwordx4) into a ring of 5 tiles
-//     (4 for the 4-wavefront workgroup);
+//     (4 for the 4-wavefront workgroup, 2 with head dimensions above 128);
 //     V is kept [key][dim] in LDS and transposed on the way to registers with
 //     ds_read_b64_tr_b16; both tiles are XOR-swizzled against bank conflicts;
 //   * causal: tiles right of the diagonal are skipped, only tiles crossing it are masked.
@@ -30,8 +30,8 @@
 namespace tfk {
 namespace {
 
-// Keys per tile.  Above a head dimension of 128 a tile of 64 keys is 64 KiB, of which the LDS holds two;
-// 32 keys leave room for a ring of four.
+// Keys per tile.  Above a head dimension of 128 a tile of 64 keys is 64 KiB, of which the LDS holds two; of 32 keys it
+// holds the five of the 8-wavefront ring, and the two of either 4-wavefront workgroup of a CU.
 __host__ __device__ constexpr int key_tile(int d) { return d <= 128 ? 64 : 32; }
 // LDS ring depth: the 8-wavefront kernel keeps two tiles live (its two wavefront sets are half a
 // tile apart) and three in flight; the 4-wavefront kernel one live and three in flight, or, with head dimensions above
@@ -479,8 +479,8 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   // Operand fragments are requested from LDS one step ahead of the MFMAs that use them, into
   // ping-pong registers, so that LDS latency is covered by the previous step's MFMAs (or by
   // the softmax arithmetic) instead of stalling the wavefront in front of every MFMA group.
-  // kWide: one wavefront a SIMD and few MFMAs a step, so K fragments are requested two steps ahead, and the V
-  // fragments during the QK product, behind whose MFMAs they arrive (causal, D = 256, before the
+  // kWide: few MFMAs a step, so K fragments are requested two steps ahead where the registers hold them, and the V
+  // fragments during the QK product, behind whose MFMAs they arrive (causal, D = 256, with one wavefront a SIMD and before the
   // weights had a remainder: 32 slices of 1024 x 1024 52.5 -> 47.0 us, 8 of 4096 173 -> 157; D = 160: 46.2 -> 44.8).
   constexpr int kKAhead = kWide && D <= 192 && kWavesT == 4 ? 2 : 1;
   V8 kf[kKAhead + 1][kKB];   // K fragments of reduction step kk (buffer kk % (kKAhead + 1))
@@ -894,7 +894,8 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
 
 // O = sum over parts of 2^(m_part - m) rows / the same of their sums, m the largest reference; a part without a score
 // above -inf (sum 0) has none.  A thread takes 8 elements of a row.  Bound by its launch and the
-// latency of two dependent reads: its rows are in the L2 (33 MB at most), the rule that asks for it counts 3.5 us for it.
+// latency of two dependent reads: the rows (33 MB at most) come from eight L2s that are not coherent with each other, through
+// the memory side.  The rule that asks for it counts 3.5 us and their way there and back.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void merge_parts_kernel(const float* __restrict__ part, T* __restrict__ O, size_t rows, int d,
                                                           int splits) {
