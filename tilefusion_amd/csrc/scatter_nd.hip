@@ -292,9 +292,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_sgpr(80))) void
 // Who owns what must come out alike in every workgroup: the order of updates within a slot does not (it is that of LDS atomics).
 // So a slot belongs whole to the share of the sorted positions in which it begins, and the updates of a hot slot (a
 // twelfth of the chunk or more), which would keep its owner busy behind all others, go by their numbers in the chunk.
-// Windows of one target that follow each other are added up in LDS before they leave, up to 16 of them.  That is for speed
-// (atomics on one line are served one after another) and for the sum: a 16-bit target of many updates is rounded
-// with every atomic.  (With a hash to pick the owner and 8 updates an atomic, all of 8192 x 1024 bf16 into
+// Windows of one target that follow each other are added up in LDS before they leave, up to 16 of them, with the updates of it
+// that the next window begins with.  That is for speed (atomics on one line are served one after another: 14576 bf16 of 218 into 7
+// rows 13.9 and, with those, 11.7 us) and for the sum: a 16-bit target of many updates is rounded with every atomic.  (With a hash to pick the owner and 8 updates an atomic, all of 8192 x 1024 bf16 into
 // one row took 50 us and came out at half its value; 12 us and 0.2% as here; every 64 as they come 18.6, 1.2%.)
 //
 // What bounds it: the atomics where there are many; below ~4 MB the chain of loading indices, sorting (five barriers,
@@ -325,6 +325,8 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
   __shared__ bool s_links;                       // windows of one target may follow each other here
   __shared__ int s_front, s_end;                 // positions of the first slot of this workgroup and behind its last one
   __shared__ alignas(16) bool s_linked[kOwnerThreads];
+  __shared__ unsigned char s_leading[kOwnerThreads];           // updates of a window that it leaves to the one in front
+  __shared__ float s_lead[kWords * kElems * kOwnerThreads];    // their sums
   const int tid = threadIdx.x;
   const int shares = 1 << share_bits, share = blockIdx.x & (shares - 1);
   const long long row0 = (long long)(blockIdx.x >> share_bits) * chunk;
@@ -424,14 +426,15 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
 
   // ---- windows of sorted updates; a group of `lanes` adjacent lanes takes one at a time, kWords words a lane ----
   const int groups = kOwnerThreads / lanes, group = tid / lanes;
-  const long long word0 = (long long)blockIdx.y * lanes * kWords + (tid & (lanes - 1));
-  auto first_elem = [&](unsigned t, int v) -> long long {   // element of the slice at word v of this lane
-    return (word0 + (long long)v * lanes) * kElems - first_word_shift<T, kLayout>(data + (size_t)t * slice);
+  const int len = (int)slice;   // (at most 65536 words)
+  const int word0 = (int)blockIdx.y * lanes * kWords + (tid & (lanes - 1));
+  auto first_elem = [&](unsigned t, int v) -> int {   // element of the slice at word v of this lane
+    return (word0 + v * lanes) * kElems - first_word_shift<T, kLayout>(data + (size_t)t * slice);
   };
-  auto load = [&](long long row, long long e0) -> unsigned {
+  auto load = [&](long long row, int e0) -> unsigned {
     const T* src = updates + row * slice;
     if constexpr (kLayout == Layout::kPairs) {
-      return e0 < slice ? *reinterpret_cast<const unsigned*>(src + e0) : 0u;
+      return e0 < len ? *reinterpret_cast<const unsigned*>(src + e0) : 0u;
     } else {
       // a half that is not the slice's has nothing to add: -0.0
       if constexpr (kSingle) {
@@ -440,8 +443,8 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
       }
       // (one load of two elements, at any even address, inside the slice)
       typedef unsigned any_u32 __attribute__((aligned(2)));
-      const unsigned w = *reinterpret_cast<const any_u32*>(src + std::min(std::max(e0, 0ll), slice - 2));
-      return e0 < 0 ? w << 16 | 0x8000u : e0 + 1 < slice ? w : w >> 16 | 0x80000000u;
+      const unsigned w = *reinterpret_cast<const any_u32*>(src + std::min(std::max(e0, 0), len - 2));
+      return e0 < 0 ? w << 16 | 0x8000u : e0 + 1 < len ? w : w >> 16 | 0x80000000u;
     }
   };
   auto unpack = [](unsigned w) -> Word<T> {
@@ -465,6 +468,9 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
         for (int e = 0; e < kElems; ++e) sum[v].v[e] = -0.f;
     };
     clear();
+    // This window's first target is the last one of the window in front, whose group takes the sums of both.
+    const bool led = links && first < end && group % kLinks != 0 && s_target[first - 1] == s_target[first];
+    int leading = 0;   // updates of it, where another target follows here
     // adds what `sum` holds of updates [from, to), all of one target
     auto flush = [&](int to) {
       const unsigned t = s_target[from];
@@ -472,8 +478,8 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
       const long long at = (long long)((size_t)t * slice);
 #pragma unroll
       for (int v = 0; v < kWords; ++v) {
-        const long long e0 = first_elem(t, v);
-        if (e0 >= slice) continue;
+        const int e0 = first_elem(t, v);
+        if (e0 >= len) continue;
         // A sum that T does not hold is added as its single updates, which `data` may bring back into range.
         bool held = true;
 #pragma unroll
@@ -500,7 +506,19 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
 #pragma unroll
       for (int i = 0; i < kFlight; ++i) {
         if (p0 + i < end) {
-          if (s_target[p0 + i] != s_target[from]) flush(p0 + i);
+          if (s_target[p0 + i] != s_target[from]) {
+            if (led && from == first) {
+#pragma unroll
+              for (int v = 0; v < kWords; ++v)
+#pragma unroll
+                for (int e = 0; e < kElems; ++e) s_lead[(v * kElems + e) * kOwnerThreads + tid] = sum[v].v[e];
+              from = p0 + i;
+              leading = from - first;
+              clear();
+            } else {
+              flush(p0 + i);
+            }
+          }
 #pragma unroll
           for (int v = 0; v < kWords; ++v) {
             const Word<T> x = unpack(raw[i][v]);
@@ -510,13 +528,15 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
         }
       }
     }
-    // A window that is all of the target in front of it leaves its sums to that one's group.
-    const bool linked = links && first < end && from == first && group % kLinks != 0 && s_target[first - 1] == s_target[first];
+    const bool linked = led && from == first;   // all of it is of the target in front
     int last = end;
     if (links) {
-      if ((tid & (lanes - 1)) == 0) s_linked[group] = linked;
+      if ((tid & (lanes - 1)) == 0) {
+        s_linked[group] = linked;
+        s_leading[group] = (unsigned char)leading;
+      }
       float* const sums = reinterpret_cast<float*>(s_slot) + tid;
-      int follow = 0;   // linked windows that follow this one
+      int follow = 0, behind_them = 0;   // linked windows that follow this one, leading updates of the next
 #pragma unroll
       for (int v = 0; v < kWords; ++v) {
         if (linked) {
@@ -530,7 +550,8 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
 #pragma unroll
           for (int w = 0; w < 4; ++w) bits |= ((flags[w] * 0x10204080u) >> 28) << (4 * w);
           follow = linked ? 0 : __builtin_ctz(~(bits >> (group % kLinks + 1)));
-          last = min(end + follow * kWindow, stop);
+          if (!linked && group % kLinks + follow + 1 < kLinks) behind_them = s_leading[group + follow + 1];
+          last = min(end + follow * kWindow, stop) + behind_them;
         }
         for (int h0 = 0; h0 < follow; h0 += 4) {
           float more[4][kElems];
@@ -542,6 +563,10 @@ __global__ __launch_bounds__(kOwnerThreads, 8) void scatter_nd_owner_kernel(
           for (int h = 0; h < 4; ++h)
 #pragma unroll
             for (int e = 0; e < kElems; ++e) sum[v].v[e] += h0 + h < follow ? more[h][e] : -0.f;
+        }
+        if (behind_them > 0) {
+#pragma unroll
+          for (int e = 0; e < kElems; ++e) sum[v].v[e] += s_lead[(v * kElems + e) * kOwnerThreads + tid + (follow + 1) * lanes];
         }
         __syncthreads();
       }
