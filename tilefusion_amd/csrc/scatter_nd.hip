@@ -587,7 +587,10 @@ int launch_shape(const void* updates, void* data, const long long* indices, cons
   return TF_OK;
 }
 
-// As many shares (a power of two, at least two) as bring about 224 workgroups: one a CU.
+// As many shares (a power of two, at least two) as bring about 224 workgroups: one a CU.  Twice as many, two a CU, for chunks of
+// 4096 and two words a lane, which have the most loads to wait for: us, one / two, 20837 fp32 of 2166 into 901 rows 75 / 59, 62413 of 994
+// into 1447 98 / 82, 27577 fp16 of 1990 into 35292 (uniform) 118 / 116; not beyond 512, which the chip does not hold at once (528: 22339 fp16 of 2710
+// 83 / 99), nor with shorter chunks (0-12% behind).
 template <typename T, int kMine, int kWords, Layout kLayout, bool kSingle>
 int launch_owner(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
                  long long slice, long long total, int lanes, long long words, hipStream_t st) {
@@ -597,6 +600,7 @@ int launch_owner(const void* updates, void* data, const long long* indices, cons
   const long long columns = (words + lanes * kWords - 1) / (lanes * kWords);
   int bits = 1;
   while (bits < 8 && chunks * columns * 3 << bits <= 2 * 224) ++bits;
+  if (kMine == 4 && kWords == 2 && bits < 8 && chunks * columns << bits <= 256) ++bits;
   const int chunk = (int)((n + chunks - 1) / chunks);   // (even ones: no nearly empty last chunk)
   const dim3 grid((unsigned)((n + chunk - 1) / chunk) << bits, (unsigned)columns);
   hipLaunchKernelGGL((scatter_nd_owner_kernel<T, kMine, kWords, kLayout, kSingle>), grid, dim3(kOwnerThreads), 0, st,
@@ -656,8 +660,10 @@ int launch_rows(const void* updates, void* data, const long long* indices, const
   }
   // Longer chunks find more to merge, shorter ones are sorted sooner, in every workgroup.  4096 updates instead of 2048 from
   // 20000 on (40000 bf16 of 1000 into 131072 rows 80 and 67, distinct indices 83 and 85; 8192 a chunk 69 and 88), 1024 where there are
-  // few (4096 fp32 of 64 into 8000 rows 7.7 and 7.1, 4096 bf16 of 1024 13.7 and 11.2; 3000 fp32 of 4096 27.3 and 31.5).
-  // Two words a lane halve the workgroups that sort the same indices, from 256 words on.
+  // few (4096 fp32 of 64 into 8000 rows 7.7 and 7.1).  Two words a lane halve the workgroups that sort the same indices, from 256 words
+  // on, except with up to 4096 updates, where a word a lane and 2048 a chunk are 7% ahead of two and 1024 over 28 problems
+  // (2295 bf16 of 2824 into 5389 rows 14.5 and 13.3, 2140 fp32 of 366 into 214 (uniform) 8.8 and 6.4, 3873 fp16 of 1048 into 2024 12.6
+  // and 13.3; sorted indices of 40 rows are 14% behind).
   auto owners = [&](auto mine, auto per_lane, auto single) -> int {
     return launch_owner<T, decltype(mine)::value, decltype(per_lane)::value, kLayout, decltype(single)::value>(
         updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
@@ -669,7 +675,7 @@ int launch_rows(const void* updates, void* data, const long long* indices, const
     using Many = std::false_type;
     if (words > 256) {
       if (n >= 20000) return owners(Four{}, Two{}, Many{});
-      return n <= 4096 && n * words <= 8 << 20 ? owners(One{}, Two{}, Many{}) : owners(Two{}, Two{}, Many{});
+      return n <= 4096 ? owners(Two{}, One{}, Many{}) : owners(Two{}, Two{}, Many{});
     }
     if (n >= 20000) return owners(Four{}, One{}, Many{});
     return n <= 8192 ? owners(One{}, One{}, Many{}) : owners(Two{}, One{}, Many{});
