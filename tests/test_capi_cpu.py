@@ -142,6 +142,13 @@ def test_attention_cases_reach_every_workgroup_form():
             assert {lib.tf_flash_attention_rows(b, 256, lkv, 128, causal) for causal in (0, 1)} == {rows}
 
 
+def test_attention_with_few_keys_takes_large_workgroups():
+    # several workgroups a CU that walk few key tiles: 256 rows where 128 took 1.05 to 1.3 times as long
+    lib = _capi.load()
+    for b, lq, lkv in [(869, 214, 8), (58, 1666, 32), (200, 440, 32), (57, 2781, 104), (503, 465, 208), (80, 2291, 280), (59, 2630, 840)]:
+        assert lib.tf_flash_attention_rows(b, lq, lkv, 128, 0) == 256
+
+
 def test_fused_cases_reach_every_streaming_instance():
     from tests.test_gpu_fused_two_gemms import STREAM_CASES
     lib = _capi.load()

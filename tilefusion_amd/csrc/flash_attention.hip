@@ -26,7 +26,11 @@ namespace {
 // they take.  Fitted to 210 problems without a mask and 710 causal ones (4..300 slices, 64..8192 keys); the pick is on
 // average 0.2% and 1% behind the best, and 1.31x and 1.25x ahead of always taking 256 rows.  Small margins (`ahead`)
 // keep 256 rows where the model cannot tell.
-struct SingleCost { double fixed, tile, full, fill, start, mean; };
+//
+// With few keys a further workgroup starts sooner than with many, `few` + `per_tile` us a key tile after the one in front (us, fp16, D = 128, 256 / 128
+// rows: 869 slices of 214 x 8 37.6 / 44.0, 58 of 1666 x 32 20.6 / 26.0, 503 of 465 x 208 65.5 / 77.0, 94 of 936 x 48 19.9 / 20.4; with
+// `start` alone, fitted to many, all four took 128; over 55 problems of 280 to 1150 keys the pick is 0.1% behind the best, 4% before).
+struct SingleCost { double fixed, tile, full, fill, start, mean, few = 1e9, per_tile = 0; };
 struct PairCost { double fixed, tile, fill, start; };
 struct HeadCost { SingleCost plain[3], causal[3]; PairCost pairs[3]; };
 constexpr int kRowChoices[3] = {256, 128, 64};
@@ -40,7 +44,7 @@ constexpr HeadCost kHeadCost[3] = {
      {{7.6, 0.982, 1.280, 0.176, 8.8, 1.440}, {6.2, 0.681, 0.880, 0.160, 6.5, 0.886}, {5.7, 0.643, 0.715, 0.078, 5.1, 0.734}},
      {{0.0, 0.991, 0.178, 13.7}, {1.5, 0.730, 0.061, 8.5}, {1.0, 0.667, 0.0, 7.4}}},
     // 128
-    {{{7.0, 1.269, 1.218, 0.406, 25.6, 0}, {5.8, 0.885, 0.993, 0.309, 7.6, 0}, {5.3, 0.754, 0.802, 0.274, 4.6, 0}},
+    {{{7.0, 1.269, 1.218, 0.406, 25.6, 0, 9.0, 0.95}, {5.8, 0.885, 0.993, 0.309, 7.6, 0, 5.2, 0.15}, {5.3, 0.754, 0.802, 0.274, 4.6, 0}},
      {{8.3, 1.186, 1.636, 0.225, 9.8, 1.883}, {6.5, 0.873, 1.044, 0.125, 8.3, 1.121}, {6.0, 0.690, 0.368, 0.193, 6.4, 0.879}},
      {{7.2, 1.167, 0.536, 8.0}, {3.0, 0.835, 0.225, 8.7}, {1.0, 0.772, 0.0, 8.3}}}};
 
@@ -53,7 +57,7 @@ double expected_single(const SingleCost& c, int64_t batch, int64_t Lq, int64_t L
   auto weight = [&](int64_t i) -> int64_t { return causal ? std::min(all, (i + 1) * rows / 64) : all; };
   double t = (double)weight(q_tiles - 1) * c.tile * (1.0 + c.fill * std::min(1.0, (double)items / 256.0));
   auto share = [&](int64_t j, int64_t i) {
-    if (j > 0) t = std::max(t, (double)((j + 1) * weight(i)) * c.full + (double)j * c.start);
+    if (j > 0) t = std::max(t, (double)((j + 1) * weight(i)) * c.full + (double)j * std::min(c.start, c.few + c.per_tile * (double)weight(i)));
   };
   if (!causal) {
     share(rounds - 1, 0);
