@@ -10,7 +10,8 @@ import torch
 
 import oracle
 from oracle import numerics as N
-from tests.gpu_util import DEV, c_decode
+from tests.gpu_util import DEV, c_decode, stream
+from tilefusion_amd import _capi, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -162,3 +163,42 @@ def test_operands_that_start_anywhere(bh, lkv, d, splits, start, dtype, tol):
     ref = (torch.softmax(scores, -1)[..., None] * v.float()).sum(1)
     o = c_decode(q, k, v, splits)
     assert N.rel_l2(o, ref) <= tol[0] and N.max_abs(o, ref) <= tol[1]
+
+
+# With 256 bytes a slice more than the partials the workgroup that is done last puts a slice together, instead of a second
+# kernel: the same sums in the same order, so the same bits, whatever the workspace held before.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bh,lkv,d,splits", [(1, 30000, 128, 64), (3, 1001, 64, 2), (32, 1999, 64, 64), (127, 2111, 128, 64),
+                                             (128, 1500, 128, 2), (200, 4099, 128, 3), (2, 40000, 64, 257)])
+def test_last_workgroup_merges(bh, lkv, d, splits, dtype):
+    g = torch.Generator(device=DEV).manual_seed(lkv)
+    q, k, v = (torch.randn(*shape, device=DEV, generator=g).to(dtype) for shape in ((bh, d), (bh, lkv, d), (bh, lkv, d)))
+    lib, code = _capi.load(), 2 if dtype == torch.bfloat16 else 1
+    want = c_decode(q, k, v, splits)
+    nbytes = lib.tf_flash_decode_workspace_bytes(bh, d, splits) + 256 * bh
+    o = torch.empty_like(q)
+
+    def run(ws):
+        o.fill_(math.nan)
+        _capi.check(lib.tf_flash_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), code, ws.data_ptr(), nbytes,
+                                        bh, lkv, d, splits, 1.0 / math.sqrt(d), stream()), "tf_flash_decode")
+
+    for held in (0, 255, 1, None):
+        ws = torch.randint(0, 256, (nbytes,), device=DEV, dtype=torch.uint8, generator=g)
+        if held is not None:
+            ws.fill_(held)
+        for _ in range(3):
+            run(ws)
+            assert torch.equal(o, want)
+    assert torch.equal(ops.flash_decode(q.unsqueeze(1), k, v, splits).squeeze(1), want)
+    # replays, with other contents of the workspace and eager calls between them
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        run(ws)
+    for i in range(4):
+        ws.fill_(37 * i)
+        graph.replay()
+        graph.replay()
+        assert torch.equal(o, want)
+        assert torch.equal(ops.flash_decode(q, k, v, splits), want)

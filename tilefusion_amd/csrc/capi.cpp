@@ -1,4 +1,6 @@
 // Error reporting and version of the C ABI (declared in include/tilefusion_c.h).
+#include <atomic>
+#include <chrono>
 #include <cstring>
 
 #include "common.hpp"
@@ -18,6 +20,20 @@ void set_error(const char* fmt, ...) {
 int hip_fail(hipError_t e, const char* what) {
   set_error("HIP error '%s' from %s", hipGetErrorString(e), what);
   return TF_ERR_HIP;
+}
+
+arrivals_t next_arrivals_tag() {
+  // splitmix64 over a count that starts differently in every process: tags do not repeat within 2^48 launches or so, and look like
+  // nothing that a workspace holds (counts or addresses might)
+  static std::atomic<unsigned long long> count{
+      (unsigned long long)std::chrono::system_clock::now().time_since_epoch().count() ^ (unsigned long long)(uintptr_t)&count};
+  for (;;) {
+    unsigned long long x = count.fetch_add(0x9e3779b97f4a7c15ull, std::memory_order_relaxed);
+    x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ull;
+    x = (x ^ (x >> 27)) * 0x94d049bb133111ebull;
+    x = (x ^ (x >> 31)) & ~kArrivalsMask;
+    if (x != 0) return x;   // (zero is what a word without arrivals holds)
+  }
 }
 }  // namespace tfk
 

@@ -93,7 +93,84 @@ TFK_DEVICE void barrier_lds_only() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// ---- results that several workgroups of a launch share -------------------------------------
+// Every workgroup leaves its part in memory and arrives; the one that arrives last puts the parts together.  None waits for
+// another, so nothing has to be resident at the same time.
+//
+// The parts pass the L2s of different XCDs, which are not coherent with each other: they are written through (agent scope) and
+// read past the reader's L2.  Writing back or dropping a whole L2, as release and acquire fences do, costs more than the
+// few KiB that change hands.
+// base: wavefront-uniform; offset in bytes, below 2^31
+template <typename V>
+TFK_DEVICE void store_shared_16B(void* base, unsigned offset, V v) {
+  static_assert(sizeof(V) == 16, "");
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int kRaw32Bit = 0x00020000, kAgent = 16;   // sc1
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, kRaw32Bit);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, v), rsrc, offset, 0, kAgent);
+#endif
+}
+template <typename V>
+TFK_DEVICE V load_shared_16B(const void* base, unsigned offset) {
+  static_assert(sizeof(V) == 16, "");
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int kRaw32Bit = 0x00020000, kAgent = 16;
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, kRaw32Bit);
+  return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset, 0, kAgent));
+#else
+  return V{};
+#endif
+}
+TFK_DEVICE void store_shared(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+TFK_DEVICE float load_shared(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The word in which the workgroups of one result count, out of a workspace that holds anything at first: a tag of 48 bits that no
+// other launch has, and the number of arrivals.  The last to arrive leaves zero behind, which is what the next launch in the same
+// workspace, or the next replay of a captured one, finds and tags with a single operation that nobody waits for.  Anything
+// else that an allocator's block may hold costs the arrivals a second round trip; it would have to equal the tag to
+// be taken for it (2^-48).
+// Atomics on one address, or on one line, are done one after another (~50 ns): a word has 256 bytes to itself, and one workgroup
+// of a result opens it.
+using arrivals_t = unsigned long long;
+constexpr int kArrivalsPitch = 256 / sizeof(arrivals_t);   // words from one result's to the next's
+constexpr arrivals_t kArrivalsMask = 0xffff;   // at most 65535 workgroups a result
+// one lane of one of the workgroups, well ahead of the arrivals
+TFK_DEVICE void open_arrivals(arrivals_t* word, arrivals_t tag) {
+  arrivals_t zero = 0;
+  (void)__hip_atomic_compare_exchange_strong(word, &zero, tag, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// One lane, behind a barrier behind which every wavefront's stores have been acknowledged (wait_vmem_all in front of it): true
+// for the last of `parts` workgroups.
+TFK_DEVICE bool arrive(arrivals_t* word, arrivals_t tag, unsigned parts) {
+  const auto add = [&]() {
+    return __hip_atomic_fetch_add(word, (arrivals_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  arrivals_t old = add();
+  if ((old & ~kArrivalsMask) != tag) {
+    // Counted in something that is no tag: whoever replaces it by the tag counts itself there, the others count again.
+    // (Ends: the word changes only by other arrivals, and once it is tagged it stays so until all have arrived.)
+    arrivals_t seen = old + 1;
+    for (;;) {
+      if (__hip_atomic_compare_exchange_strong(word, &seen, tag | 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        old = tag;
+        break;
+      }
+      if ((seen & ~kArrivalsMask) == tag) {
+        old = add();
+        break;
+      }
+    }
+  }
+  const bool last = (old & kArrivalsMask) + 1 == parts;
+  if (last) __hip_atomic_store(word, (arrivals_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return last;
+}
+
 // ---- host side ---------------------------------------------------------------------------
+// a tag for the arrivals of one launch
+arrivals_t next_arrivals_tag();
 void set_error(const char* fmt, ...);
 int hip_fail(hipError_t e, const char* what);
 

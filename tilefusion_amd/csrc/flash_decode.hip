@@ -14,7 +14,11 @@
 //     two batches of 4 or 6 rows per group are in flight (16 or 24 KiB per wavefront), the next one
 //     requested before the current one is consumed; the partials leave through streaming
 //     stores (ordinary stores in the middle of the read stream cost 7% of its bandwidth);
-//   * combine kernel: grid batch_heads, merges the fp32 partials.
+//   * the partials of a slice are merged by the workgroup of it that is done last, where the workspace has room for a word of
+//     arrivals a slice and fewer than 1024 workgroups run (32 slices of 1999 x 64, bf16: 9.6 us with a second kernel, 6.3 as
+//     this; 9 of 5829 x 128 11.4 and 8.4);
+//   * otherwise by the combine kernel, grid batch_heads: with many workgroups every one holds its place on a CU
+//     until its partials and its arrival are acknowledged (60 slices of 38872 x 64: 95 us, merged in one kernel 112).
 // The kernels are templates of the element type (fp16 / bf16, the reference's 16-bit types,
 // include/kernels/dispatch_macros.hpp:6-23) and of the head dimension (128 / 64).
 // All offsets are 64-bit.
@@ -112,20 +116,86 @@ TFK_DEVICE V load_below(const char* base, unsigned bytes, unsigned offset) {
 #endif
 }
 
-// workspace: o_part [batch_heads][num_splits][D] fp32, then ml_part [batch_heads][num_splits][2].
+// The partials of one slice put together; the first kCombThreads threads of a workgroup, behind which all of it meets at the barrier.  Groups
+// of D / 4 lanes take every kGroups-th split with its loads in flight at once, then the groups are added up in LDS.  (One thread per column
+// that walks the splits one after another is a chain of loads: 9.5 us for 64 splits of 32 slices, 2.4 as here.)
+// kShared: the partials come from other workgroups of the same launch.
+constexpr int kCombThreads = 256;
+template <typename T, int D, bool kShared>
+TFK_DEVICE void combine_slice(const float* o_part, const float* ml_part, T* __restrict__ O, int num_splits) {
+  constexpr int kLanes = D / 4, kGroups = kCombThreads / kLanes, kUnroll = 8;
+  __shared__ float4_t s_o[kGroups][kLanes];
+  __shared__ float s_l[kGroups];
+  const int lane = threadIdx.x % kLanes, grp = threadIdx.x / kLanes;
+  if (threadIdx.x < kCombThreads) {
+    float4_t o[kUnroll];
+    float m[kUnroll], sum[kUnroll];
+    auto load = [&](int s0) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        const int s = min(s0 + u * kGroups, num_splits - 1);
+        if constexpr (kShared) {
+          o[u] = load_shared_16B<float4_t>(o_part, (unsigned)(s * kLanes + lane) * 16u);
+          m[u] = load_shared(ml_part + 2 * s);
+          sum[u] = load_shared(ml_part + 2 * s + 1);
+        } else {
+          o[u] = reinterpret_cast<const float4_t*>(o_part)[s * kLanes + lane];
+          const float2_t x = reinterpret_cast<const float2_t*>(ml_part)[s];
+          m[u] = x[0];
+          sum[u] = x[1];
+        }
+      }
+    };
+    load(grp);   // in flight while the maximum is found
+    float big = -INFINITY;
+    for (int s = threadIdx.x % kWaveSize; s < num_splits; s += kWaveSize)
+      big = fmaxf(big, kShared ? load_shared(ml_part + 2 * s) : ml_part[2 * s]);
+#pragma unroll
+    for (int x = 1; x < kWaveSize; x *= 2) big = fmaxf(big, __shfl_xor(big, x));
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+    for (int s0 = grp; s0 < num_splits; s0 += kGroups * kUnroll) {
+      if (s0 != grp) load(s0);
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        if (s0 + u * kGroups >= num_splits) break;   // (the last split again, which may hold infinities)
+        const float w = __builtin_amdgcn_exp2f(m[u] - big);
+        acc += w * o[u];
+        l += w * sum[u];
+      }
+    }
+    s_o[grp][lane] = acc;
+    if (lane == 0) s_l[grp] = l;
+  }
+  __syncthreads();
+  if (threadIdx.x < D) {
+    float sum = 0.f, total = 0.f;
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+      sum += s_o[g][threadIdx.x / 4][threadIdx.x % 4];
+      total += s_l[g];
+    }
+    O[threadIdx.x] = (T)(sum / total);
+  }
+}
+
+// workspace: o_part [batch_heads][num_splits][D] fp32, then ml_part [batch_heads][num_splits][2], then (kMerged) a word of
+// arrivals a slice.
 // kWhole: one workgroup per slice, which writes O itself (num_splits == 1, chunk == Lkv).
+// kMerged: the workgroup of a slice that is done last puts the parts together; kParts leaves that to a second kernel.
+enum DecodeEnd { kWhole, kMerged, kParts };
 // `chunk` is a multiple of the rows of one load step.
 // kDecWaves wavefronts per workgroup.
-template <typename T, int D, int kDecWaves, bool kWhole>
+template <typename T, int D, int kDecWaves, DecodeEnd kEnd>
 __global__ __launch_bounds__(kDecWaves * kWaveSize) void flash_decode_split_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, T* __restrict__ O,
-    float* __restrict__ o_part, float* __restrict__ ml_part, int64_t Lkv, int num_splits,
-    int64_t chunk, float scale_log2) {
+    float* o_part, float* ml_part, int64_t Lkv, int num_splits,
+    int64_t chunk, float scale_log2, arrivals_t* arrivals, arrivals_t tag) {
   using V8 = typename Vec8<T>::type;
   constexpr int kLanesPerRow = D / 8;                   // 16-byte vectors per row
   constexpr int kRowsPerWave = kWaveSize / kLanesPerRow;  // rows one wavefront load instruction covers
   constexpr int kRowsPerStep = kDecWaves * kRowsPerWave;  // ... and one workgroup load step
-  constexpr int kBatchRows = batch_rows(kDecWaves, kWhole);
+  constexpr int kBatchRows = batch_rows(kDecWaves, kEnd == kWhole);
   __shared__ float s_o[kDecWaves][D];
   __shared__ float s_m[kDecWaves], s_l[kDecWaves];
 
@@ -197,6 +267,7 @@ __global__ __launch_bounds__(kDecWaves * kWaveSize) void flash_decode_split_kern
   };
   V8 k_a[kBatchRows], v_a[kBatchRows], k_b[kBatchRows], v_b[kBatchRows];
   load_batch(k_a, v_a, row_begin);
+  if (kEnd == kMerged && tid == 0 && split == 0) open_arrivals(arrivals + bh * kArrivalsPitch, tag);
   int64_t base = row_begin;
   for (; base + kBatchSpan < row_end; base += 2 * kBatchSpan) {
     load_batch(k_b, v_b, base + kBatchSpan);
@@ -234,76 +305,46 @@ __global__ __launch_bounds__(kDecWaves * kWaveSize) void flash_decode_split_kern
       acc += f * s_o[w][tid];
       l += f * s_l[w];
     }
-    if constexpr (kWhole) {
+    if constexpr (kEnd == kWhole) {
       O[bh * D + tid] = (T)(acc / l);
       return;
     }
     const int64_t idx = bh * num_splits + split;
-    // Streaming stores: an ordinary store of these few hundred bytes per workgroup, issued in
-    // the middle of an 8 GiB read stream, costs 7% of the read bandwidth (6.6 against 7.15
-    // TB/s in a plain two-stream read kernel with and without such a store; 7.05 with this one).
-    __builtin_nontemporal_store(acc, o_part + idx * D + tid);
-    if (tid == 0) {
-      __builtin_nontemporal_store(big, ml_part + idx * 2);
-      __builtin_nontemporal_store(l, ml_part + idx * 2 + 1);
+    if constexpr (kEnd == kMerged) {
+      store_shared(o_part + idx * D + tid, acc);
+      if (tid == 0) {
+        store_shared(ml_part + idx * 2, big);
+        store_shared(ml_part + idx * 2 + 1, l);
+      }
+    } else {
+      // Streaming stores: an ordinary store of these few hundred bytes per workgroup, issued in
+      // the middle of an 8 GiB read stream, costs 7% of the read bandwidth (6.6 against 7.15
+      // TB/s in a plain two-stream read kernel with and without such a store; 7.05 with this one).
+      __builtin_nontemporal_store(acc, o_part + idx * D + tid);
+      if (tid == 0) {
+        __builtin_nontemporal_store(big, ml_part + idx * 2);
+        __builtin_nontemporal_store(l, ml_part + idx * 2 + 1);
+      }
     }
+  }
+  if constexpr (kEnd == kMerged) {
+    __shared__ bool s_last;
+    wait_vmem_all();
+    if constexpr (D > kWaveSize) __syncthreads();   // (otherwise the first wavefront has written all of it)
+    if (tid == 0) s_last = arrive(arrivals + bh * kArrivalsPitch, tag, (unsigned)num_splits);
+    __syncthreads();
+    if (!s_last) return;
+    combine_slice<T, D, true>(o_part + bh * num_splits * D, ml_part + bh * num_splits * 2, O + bh * D, num_splits);
   }
 }
 
-// One workgroup per slice: groups of D / 4 lanes take every kGroups-th split with its loads in flight at
-// once, then the groups are added up in LDS.  (One thread per column that walks the splits one after
-// another is a chain of loads: 9.5 us for 64 splits of 32 slices, 2.4 as here.)
-constexpr int kCombThreads = 256;
+// One workgroup per slice.
 template <typename T, int D>
 __global__ __launch_bounds__(kCombThreads) void flash_decode_combine_kernel(
     const float* __restrict__ o_part, const float* __restrict__ ml_part, T* __restrict__ O,
     int num_splits) {
-  constexpr int kLanes = D / 4, kGroups = kCombThreads / kLanes, kUnroll = 8;
-  __shared__ float4_t s_o[kGroups][kLanes];
-  __shared__ float s_l[kGroups];
   const int64_t bh = blockIdx.x;
-  const int lane = threadIdx.x % kLanes, grp = threadIdx.x / kLanes;
-  const float2_t* ml = reinterpret_cast<const float2_t*>(ml_part) + bh * num_splits;
-  const float4_t* op = reinterpret_cast<const float4_t*>(o_part + bh * num_splits * D) + lane;
-  float4_t o[kUnroll];
-  float2_t m[kUnroll];
-  auto load = [&](int s0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int s = min(s0 + u * kGroups, num_splits - 1);
-      o[u] = op[(int64_t)s * kLanes];
-      m[u] = ml[s];
-    }
-  };
-  load(grp);   // in flight while the maximum is found
-  float big = -INFINITY;
-  for (int s = threadIdx.x % kWaveSize; s < num_splits; s += kWaveSize) big = fmaxf(big, ml[s][0]);
-#pragma unroll
-  for (int x = 1; x < kWaveSize; x *= 2) big = fmaxf(big, __shfl_xor(big, x));
-  float4_t acc = {0.f, 0.f, 0.f, 0.f};
-  float l = 0.f;
-  for (int s0 = grp; s0 < num_splits; s0 += kGroups * kUnroll) {
-    if (s0 != grp) load(s0);
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      if (s0 + u * kGroups >= num_splits) break;   // (the last split again, which may hold infinities)
-      const float w = __builtin_amdgcn_exp2f(m[u][0] - big);
-      acc += w * o[u];
-      l += w * m[u][1];
-    }
-  }
-  s_o[grp][lane] = acc;
-  if (lane == 0) s_l[grp] = l;
-  __syncthreads();
-  if (threadIdx.x < D) {
-    float sum = 0.f, total = 0.f;
-#pragma unroll
-    for (int g = 0; g < kGroups; ++g) {
-      sum += s_o[g][threadIdx.x / 4][threadIdx.x % 4];
-      total += s_l[g];
-    }
-    O[bh * D + threadIdx.x] = (T)(sum / total);
-  }
+  combine_slice<T, D, false>(o_part + bh * num_splits * D, ml_part + bh * num_splits * 2, O + bh * D, num_splits);
 }
 
 }  // namespace
@@ -340,7 +381,7 @@ struct DecodePlan {
   int waves;
 };
 // One workgroup takes in ~45 GB/s when few run, all of them together 6.7 TB/s; the second kernel and its
-// launch cost ~4 us.  Measured (fp16, us, one workgroup per slice / best split): 33 slices of 662 x 64
+// launch, or the arrivals and the merge, cost ~4 or ~2 us.  Measured (fp16, us, one workgroup per slice / best split): 33 slices of 662 x 64
 // 6.5 / 8.1, 964 of 913 x 128 68 / 73, 11 of 825 x 128 10.4 / 8.5, 64 of 8192 x 128 85 / 44.  Slices that the
 // CUs cannot share evenly cost about a third of the unevenness (802 of 2574 x 128: 180 / 165).
 // Where the slices are large and many, one workgroup in each means hundreds of streams, megabytes apart, and a first
@@ -349,6 +390,10 @@ struct DecodePlan {
 // either way (512 of 32768 x 128 1237 / 1235, over ten caches in turn too).  So slices of more than 4 MiB, of
 // more than 2.75 GB together, come in ranges of at most 2 MiB.  (Below neither was ahead at first: 512 of 8192 x 128 375 whole
 // and 384 cut, 512 of 10000 x 128 484 and 491, 200 of 12000 x 128 246 and 242 - then 190 and 196.)
+// Up to 128 slices, of 600 MB together, are cut so that every CU has one workgroup at most: eight wavefronts take in what a
+// CU's share is, more workgroups are a second round and more arrivals (us, 256 workgroups at most / 1024: 24 of 4301 x 128 11.9 /
+// 13.7, 19 of 2620 x 128 8.0 / 10.5, 102 of 1952 x 128 18.9 / 20.9, 66 of 2934 x 64 11.8 / 14.0, 128 of 8192 x 128 84 / 87).  Beyond,
+// long ranges cost a first pass more than they gain (32 of 55533 x 128: first 144-160 us in 4 MiB, 151-181; repeated 139 both).
 // Otherwise the cut aims at 1024 workgroups, and at no more than 256 KiB of keys and values in each: they
 // come in rounds, and the last one fills the chip badly (584 of 16256 x 64: 4 splits 411, 16 364; 136 of
 // 36053 x 64: 8 splits 201, 32 192), but at 32 KiB at least (32 of 1999 x 64: 16 splits 10.2, 64 12.8),
@@ -364,8 +409,11 @@ DecodePlan plan_decode(int64_t batch_heads, int64_t Lkv, int num_splits) {
   const bool shared_evenly = 2.5 + std::max(alone_us, stream_us * uneven) <= 6.5 + stream_us;
   if (num_splits == 1 || (shared_evenly && (slice_bytes <= 4194304.0 || slice_bytes * batch_heads <= 2.75e9))) return whole;
   constexpr int64_t kStep = 8 * (kWaveSize / (D / 8));   // rows of one load step of the larger workgroup
-  const int64_t fill = (1024 + batch_heads - 1) / batch_heads;
-  const int64_t least = shared_evenly ? (int64_t)std::ceil(slice_bytes / 2097152.0) : (int64_t)(slice_bytes / 262144.0) + 1;
+  const bool one_round = batch_heads <= 128 && slice_bytes * batch_heads <= 6e8;
+  const int64_t fill = one_round ? 256 / batch_heads : (1024 + batch_heads - 1) / batch_heads;
+  const int64_t least = one_round       ? 1
+                        : shared_evenly ? (int64_t)std::ceil(slice_bytes / 2097152.0)
+                                        : (int64_t)(slice_bytes / 262144.0) + 1;
   const int64_t most = (int64_t)(slice_bytes / 32768.0) + 1;
   const int64_t want = std::min<int64_t>(num_splits, std::min(std::max(fill, least), most));
   const int64_t chunk = ((Lkv + want - 1) / want + kStep - 1) / kStep * kStep;
@@ -375,49 +423,55 @@ DecodePlan plan_decode(int64_t batch_heads, int64_t Lkv, int num_splits) {
   return splits > 1 ? DecodePlan{(int)splits, chunk, batch_heads * splits < 1024 ? 8 : 4} : whole;
 }
 
-template <typename T, int D, int kDecWaves, bool kWhole>
+template <typename T, int D, int kDecWaves, DecodeEnd kEnd>
 int launch_split(const void* Q, const void* K, const void* V, void* O, float* o_part, float* ml_part,
-                 int64_t batch_heads, int64_t Lkv, DecodePlan plan, double softmax_scale, hipStream_t st) {
+                 int64_t batch_heads, int64_t Lkv, DecodePlan plan, double softmax_scale, hipStream_t st, arrivals_t* arrivals = nullptr) {
   const float scale_log2 = (float)(softmax_scale * 1.4426950408889634);
-  hipLaunchKernelGGL((flash_decode_split_kernel<T, D, kDecWaves, kWhole>), dim3(plan.splits, (unsigned)batch_heads),
+  hipLaunchKernelGGL((flash_decode_split_kernel<T, D, kDecWaves, kEnd>), dim3(plan.splits, (unsigned)batch_heads),
                      dim3(kDecWaves * kWaveSize), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K),
                      static_cast<const T*>(V), static_cast<T*>(O), o_part, ml_part, Lkv, plan.splits, plan.chunk,
-                     scale_log2);
+                     scale_log2, arrivals, kEnd == kMerged ? next_arrivals_tag() : 0);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
 
-// Split kernel and, if the plan cuts, combine kernel on `st`; `partials` holds o_part then ml_part.
+// The kernels on `st`; `partials` holds o_part then ml_part and, where there is `room` (bytes) for them, the words in which the
+// workgroups of a slice arrive, and is at a 16-byte boundary.
 template <typename T, int D>
-int launch_decode_t(const void* Q, const void* K, const void* V, void* O, float* partials,
+int launch_decode_t(const void* Q, const void* K, const void* V, void* O, float* partials, size_t room,
                     int64_t batch_heads, int64_t Lkv, int num_splits, double softmax_scale,
                     hipStream_t st) {
   const DecodePlan plan = plan_decode<D>(batch_heads, Lkv, num_splits);
   if (plan.splits == 1) {
     if (plan.waves == 4)
-      return launch_split<T, D, 4, true>(Q, K, V, O, nullptr, nullptr, batch_heads, Lkv, plan, softmax_scale, st);
-    return launch_split<T, D, 8, true>(Q, K, V, O, nullptr, nullptr, batch_heads, Lkv, plan, softmax_scale, st);
+      return launch_split<T, D, 4, kWhole>(Q, K, V, O, nullptr, nullptr, batch_heads, Lkv, plan, softmax_scale, st);
+    return launch_split<T, D, 8, kWhole>(Q, K, V, O, nullptr, nullptr, batch_heads, Lkv, plan, softmax_scale, st);
   }
   float* o_part = partials;
   float* ml_part = o_part + (size_t)batch_heads * plan.splits * D;
+  const size_t part_floats = (size_t)batch_heads * plan.splits * (D + 2);   // (even: the words behind it are at 8-byte boundaries)
+  if (part_floats * sizeof(float) + (size_t)batch_heads * kArrivalsPitch * sizeof(arrivals_t) <= room && plan.waves == 8) {
+    arrivals_t* arrivals = reinterpret_cast<arrivals_t*>(partials + part_floats);
+    return launch_split<T, D, 8, kMerged>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st, arrivals);
+  }
   const int rc = plan.waves == 8
-      ? launch_split<T, D, 8, false>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st)
-      : launch_split<T, D, 4, false>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st);
+      ? launch_split<T, D, 8, kParts>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st)
+      : launch_split<T, D, 4, kParts>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st);
   if (rc != TF_OK) return rc;
   hipLaunchKernelGGL((flash_decode_combine_kernel<T, D>), dim3((unsigned)batch_heads), dim3(kCombThreads), 0, st,
                      o_part, ml_part, static_cast<T*>(O), plan.splits);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
-int launch_decode(const void* Q, const void* K, const void* V, void* O, float* partials, int dtype,
+int launch_decode(const void* Q, const void* K, const void* V, void* O, float* partials, size_t room, int dtype,
                   int64_t batch_heads, int64_t Lkv, int64_t D, int num_splits, double softmax_scale,
                   hipStream_t st) {
   if (dtype == TF_DTYPE_BF16) {
-    if (D == 128) return launch_decode_t<bf16_t, 128>(Q, K, V, O, partials, batch_heads, Lkv, num_splits, softmax_scale, st);
-    return launch_decode_t<bf16_t, 64>(Q, K, V, O, partials, batch_heads, Lkv, num_splits, softmax_scale, st);
+    if (D == 128) return launch_decode_t<bf16_t, 128>(Q, K, V, O, partials, room, batch_heads, Lkv, num_splits, softmax_scale, st);
+    return launch_decode_t<bf16_t, 64>(Q, K, V, O, partials, room, batch_heads, Lkv, num_splits, softmax_scale, st);
   }
-  if (D == 128) return launch_decode_t<half_t, 128>(Q, K, V, O, partials, batch_heads, Lkv, num_splits, softmax_scale, st);
-  return launch_decode_t<half_t, 64>(Q, K, V, O, partials, batch_heads, Lkv, num_splits, softmax_scale, st);
+  if (D == 128) return launch_decode_t<half_t, 128>(Q, K, V, O, partials, room, batch_heads, Lkv, num_splits, softmax_scale, st);
+  return launch_decode_t<half_t, 64>(Q, K, V, O, partials, room, batch_heads, Lkv, num_splits, softmax_scale, st);
 }
 
 int decode_with_workspace(const char* who, const void* Q, const void* K, const void* V, void* O, int dtype,
@@ -429,7 +483,7 @@ int decode_with_workspace(const char* who, const void* Q, const void* K, const v
   TFK_REQUIRE(workspace_bytes >= need, TF_ERR_INVALID_ARG, "%s: workspace holds %zu bytes, %zu needed", who,
               workspace_bytes, need);
   TFK_REQUIRE(((uintptr_t)workspace & 15) == 0, TF_ERR_INVALID_ARG, "%s: workspace must be 16-byte aligned", who);
-  return launch_decode(Q, K, V, O, static_cast<float*>(workspace), dtype, batch_heads, Lkv, D, num_splits,
+  return launch_decode(Q, K, V, O, static_cast<float*>(workspace), workspace_bytes, dtype, batch_heads, Lkv, D, num_splits,
                        softmax_scale, static_cast<hipStream_t>(stream));
 }
 
@@ -528,6 +582,6 @@ extern "C" int tf_flash_decode_static_f16(const void* Q, const void* K, const vo
   if (int rc = scratch_on_current_device(&partials)) return rc;
   // Nothing has to start at zero: the split kernel writes every (slice, split) partial the
   // combine kernel reads, so whatever an earlier call left in the array is never read.
-  return launch_decode(Q, K, V, O, partials, TF_DTYPE_F16, batch_heads, Lkv, D, num_splits, softmax_scale,
+  return launch_decode(Q, K, V, O, partials, kScratchFloats * sizeof(float), TF_DTYPE_F16, batch_heads, Lkv, D, num_splits, softmax_scale,
                        static_cast<hipStream_t>(stream));
 }

@@ -337,7 +337,8 @@ void flash_decode(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& V,
   TORCH_CHECK(Q.numel() == bh * d && O.numel() == bh * d,
               "flash_decode: Q and O must hold one row of D per (batch, head).");
   TORCH_CHECK(num_splits > 0, "flash_decode: num_splits must be positive.");
-  const size_t bytes = tf_flash_decode_workspace_bytes(bh, d, (int)num_splits);
+  // (256 bytes a slice more than the partials take: with them one kernel does it)
+  const size_t bytes = tf_flash_decode_workspace_bytes(bh, d, (int)num_splits) + 256 * (size_t)bh;
   at::Tensor ws = at::empty({(int64_t)((bytes + 3) / 4)}, Q.options().dtype(at::kFloat));
   check_status(tf_flash_decode(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dtype,
                                ws.data_ptr(), bytes, bh, lkv, d, (int)num_splits, softmax_scale,
