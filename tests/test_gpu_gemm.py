@@ -179,6 +179,31 @@ def test_every_kernel_at_its_edges_is_exact(kernel, m, n, k, dtype):
         assert bool((buf[m * n:] == 7.0).all())                          # nothing behind C is written
 
 
+# Rows that start anywhere in a line (K % 64 != 0, from 328 on): the ring kernels fetch whole lines.  Every place in a line that
+# rows 8 apart can start at (K), first rows at another (operands that start at 16 bytes, not at a line), last tiles that
+# overlap their neighbours by any amount, few and many k-tiles.
+LINES = [(7, 4875, 196, 520), (7, 300, 3476, 528), (7, 3802, 259, 536), (7, 4328, 232, 544), (7, 4432, 228, 552),
+         (7, 1621, 647, 560), (7, 234, 4261, 568), (10, 770, 4610, 328), (10, 773, 4658, 336), (10, 4622, 776, 344),
+         (10, 4659, 771, 352), (10, 776, 4619, 360), (10, 4705, 769, 368), (10, 786, 4615, 376), (11, 1555, 4613, 328),
+         (11, 1539, 4624, 344), (11, 1542, 4633, 352), (11, 1559, 4653, 376), (12, 1159, 4639, 328), (12, 1155, 4609, 344),
+         (12, 1155, 4680, 352), (12, 1157, 4648, 376), (7, 205, 5613, 1904), (10, 2999, 1544, 1032), (12, 3333, 2288, 1944)]
+
+
+@pytest.mark.parametrize("kernel,m,n,k", LINES)
+@pytest.mark.parametrize("start", [0, 8, 40])
+def test_rows_that_start_anywhere_in_a_line(kernel, m, n, k, start):
+    from tilefusion_amd import _capi
+    assert _capi.load().tf_gemm_kernel_index(m, n, k, 0) == kernel
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+
+    def inside(rows, at):   # between numbers that must not count
+        buf = torch.full((rows * k + 128,), float("nan"), device=DEV, dtype=torch.float16)
+        return buf[at:at + rows * k].view(rows, k).copy_(torch.randint(-2, 3, (rows, k), device=DEV, generator=g))
+
+    a, b = inside(m, start), inside(n, 48 - start)
+    assert torch.equal(c_gemm(a, b, torch.float32), a.float() @ b.float().t())   # exact: |sum| <= 4 k < 2^24
+
+
 def test_operands_without_16_byte_alignment():
     g = torch.Generator().manual_seed(5)
     a, b = (torch.randint(-2, 3, (1 + r * 264,), generator=g).half().to(DEV)[1:].view(r, 264) for r in (200, 150))

@@ -112,11 +112,19 @@ TFK_DEVICE float16_t mfma32_t(in8_t<InT> a, in8_t<InT> b, float16_t c) {
 //
 // The same kernel serves smaller tiles (2 x 2 wavefronts of half a tile each way), for grids that 256 x 256
 // tiles would leave CUs idle on: 3333 x 2288 x 1944 takes 45.5 us with 126 tiles of 256 x 256, 36.7 with
-// 216 of 192 x 192 and 36.4 with 252 of 256 x 128; 2999 x 1544 x 1032 27.6 and, with 192 x 128, 18.7 (the bounds-checked kernel that ran
+// 216 of 192 x 192 and 36.4 with 252 of 256 x 128; 2999 x 1544 x 1032 27.6 and, with 192 x 128, 16.0 (the bounds-checked kernel that ran
 // these shapes before: 37.8).  Units then have the size of the larger operand.  128 x 128 tiles have k-steps
 // four times shorter; where a workgroup has its CU to itself their requests run kAhead = 4 tiles
 // ahead (a ring of 2 * kAhead + 1 = 9 units).
-template <int BM_, int BN_, int AHEAD_>
+//
+// K that is no multiple of 64 (kLines): rows start anywhere in a 128-byte line, and k-tiles that start where a row starts
+// would fetch every line twice, for two tiles (8 rows x 128 bytes are 16 lines instead of 8: 0.13 to 0.27 us more a k-tile).
+// So what is fetched are SEGMENTS of whole lines: segment u of a row is its u-th line, and in it k-tile t of the row takes
+// the end of segment t and the front of segment t + 1, by an amount that only depends on the row. Rows 8 apart start at
+// the same place in a line, so a lane's fragments all are shifted alike, and what a lane pays is the choice between
+// the two segments (one v_and and one v_add3 an address). The ring is kept in whole tiles then, kLines of them: two are
+// read, the others in flight. 2999 x 1544 x 1032 18.5 -> 16.0 us (K = 1024: 14.7).
+template <int BM_, int BN_, int AHEAD_, int LINES_ = 0>
 struct Ring64Shape {
   static constexpr int BM = BM_, BN = BN_, BK = 64;
   static constexpr int WAVES_M = 2, WAVES_N = 2;
@@ -129,6 +137,10 @@ struct Ring64Shape {
   static constexpr int kUnits = 2 * kAhead + 1;
   static constexpr int kLoadsA = BM / 8 / kWaves, kLoadsB = BN / 8 / kWaves;   // 1 KiB requests per wavefront and unit
   static constexpr int kLoadsMax = kLoadsA > kLoadsB ? kLoadsA : kLoadsB;
+  static constexpr int kLoads = kLoadsA + kLoadsB;
+  static constexpr int kLines = LINES_;                     // segments in the ring, 0: k-tiles start where rows start
+  static constexpr int kTileBytes = (BM + BN) * kRowBytes;
+  static constexpr int kLdsBytes = kLines ? kLines * kTileBytes : kUnits * kUnitBytes;
   // slot schedule of a k-step (TM slots of TN MFMAs): the TM + TN fragment reads of the next
   // k-step are dealt to the first kReadSlots slots; the scalar bookkeeping runs in the gaps
   // without a read from slot kPrepSlot on
@@ -171,8 +183,10 @@ struct Ring64Shape {
                 "slot schedule: every read and bookkeeping piece needs its own gap");
   // requests in flight behind the barrier in the middle of a tile: A of tile t+kAhead, all of the
   // tiles t+2 .. t+kAhead-1
-  static constexpr int kInFlight = kLoadsA + (kAhead - 2) * (kLoadsA + kLoadsB);
-  static_assert((kAhead - 1) * (kLoadsA + kLoadsB) < 64, "vmcnt is a 6-bit counter");
+  // (kLines: the segments t+3 .. t+kLines-1)
+  static constexpr int kInFlight = kLines ? (kLines - 3) * kLoads : kLoadsA + (kAhead - 2) * kLoads;
+  static_assert((kAhead - 1) * kLoads < 64 && (kLines - 2) * kLoads < 64, "vmcnt is a 6-bit counter");
+  static_assert(kLines == 0 || (kLines >= 3 && free_gaps() >= 8), "two segments are read, one is in flight; a gap for every piece");
   // 128-byte rows: two rows per pass over the banks; chunk ^ (row / 2) % 8 keeps every
   // ds_read_b128 lane pass on 16 different bank groups
   __host__ __device__ static constexpr int swizzle(int row, int c) { return c ^ ((row / 2) % 8); }
@@ -180,7 +194,7 @@ struct Ring64Shape {
 
 __device__ const uint4_t kZeros[1] = {};   // what the chunks in front of a row are fetched from
 
-// M >= BM, N >= BN, and K >= BK: requests past the last k-tile ask for that tile again, which must not
+// M >= BM, N >= BN, and K >= BK (kLines: K > 64 * kLines): requests past the last k-tile ask for that tile again, which must not
 // be the one completed with zeros.
 // InT is half_t or bf16_t: the two differ in the MFMA mnemonic and in the conversion of the
 // result, everything else moves 16-bit elements without looking at them.
@@ -213,13 +227,35 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
   // prologue knows about it.
   const int num_k_tiles = (K + S::BK - 1) / S::BK;
   const int k_pad = num_k_tiles * S::BK - K;
-  const char* a_tile = reinterpret_cast<const char*>(A + (size_t)(m0 + wave * 8 * S::kLoadsA) * K) - 2 * k_pad;
-  const char* b_tile = reinterpret_cast<const char*>(B + (size_t)(n0 + wave * 8 * S::kLoadsB) * K) - 2 * k_pad;
+  // kLines: chunk c of row r, counted from the completed front, is chunk (c + shift(r)) % 8 of segment (c + shift(r)) / 8,
+  // shift(r) = 1 .. 8. In LDS it lies where it would without a shift, so that reads see the same banks.
+  constexpr bool kShift = S::kLines > 0;
+  constexpr int kLead = kShift ? 256 : 0;   // (keeps lane offsets positive: up to 15 chunks in front of a row)
+  const int pad_chunks = k_pad / 8;
+  auto shift_of = [&](const InT* X, int row) __attribute__((always_inline)) {
+    const unsigned in_line = (unsigned)(reinterpret_cast<uintptr_t>(X) >> 4) + (unsigned)row * (unsigned)(K / 8);
+    return (int)((in_line - (unsigned)pad_chunks - 1u) & 7u) + 1;
+  };
+  const int a_shift = shift_of(A, m0 + ld_row), b_shift = shift_of(B, n0 + ld_row);   // of the rows that this lane fetches
+  const char* a_tile = reinterpret_cast<const char*>(A + (size_t)(m0 + wave * 8 * S::kLoadsA) * K) - (kShift ? kLead : 2 * k_pad);
+  const char* b_tile = reinterpret_cast<const char*>(B + (size_t)(n0 + wave * 8 * S::kLoadsB) * K) - (kShift ? kLead : 2 * k_pad);
   unsigned g_off[S::kLoadsMax];
+  unsigned g_off_b[kShift ? S::kLoadsB : 1];
+  // the chunk of a segment that this lane fetches with request n
+  auto segment_chunk = [&](int n, int shift) __attribute__((always_inline)) { return (S::swizzle(ld_row + 8 * n, ld_c) + shift) & 7; };
+  auto segment_off = [&](int n, int shift) __attribute__((always_inline)) {
+    return (unsigned)(ld_row + 8 * n) * (unsigned)K * 2u + (unsigned)(kLead + 16 * (segment_chunk(n, shift) - shift - pad_chunks)) -
+           1024u * (n % 4);
+  };
 #pragma unroll
   for (int n = 0; n < S::kLoadsMax; ++n)
-    g_off[n] = (unsigned)(ld_row + 8 * n) * (unsigned)K * 2u + (unsigned)S::swizzle(ld_row + 8 * n, ld_c) * 16u -
-               1024u * (n % 4);   // the instruction's immediate offset (added to both addresses) gives it back
+    g_off[n] = kShift ? segment_off(n, a_shift)
+                      : (unsigned)(ld_row + 8 * n) * (unsigned)K * 2u + (unsigned)S::swizzle(ld_row + 8 * n, ld_c) * 16u -
+                            1024u * (n % 4);   // the instruction's immediate offset (added to both addresses) gives it back
+  if constexpr (kShift) {
+#pragma unroll
+    for (int n = 0; n < S::kLoadsB; ++n) g_off_b[n] = segment_off(n, b_shift);
+  }
   // LDS -> fragment plan: fragment i of k-step ks: row 16*i + l%16 of the wavefront's rows,
   // logical chunk 4*ks + l/16
   const int fr = lane & 15, fg = lane >> 4;
@@ -250,12 +286,13 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
   // four: the statements do not change it) and cannot use the register for anything else between
   // that write and a request.  The s_nop is the wait state an M0 write needs in front of an
   // LDS-direct load; next to a request at the head of a slot it costs no issue time.
-  auto request = [&](const char* src, unsigned lds_unit, int n) __attribute__((always_inline)) {
+  auto request_at = [&](unsigned off, const char* src, unsigned lds_unit, int n) __attribute__((always_inline)) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%2"
                  :
-                 : "v"(g_off[n]), "s"(src), "n"(1024 * (n % 4)), "{m0}"(lds_unit + (n - n % 4) * 1024)
+                 : "v"(off), "s"(src), "n"(1024 * (n % 4)), "{m0}"(lds_unit + (n - n % 4) * 1024)
                  : "memory");
   };
+  auto request = [&](const char* src, unsigned lds_unit, int n) __attribute__((always_inline)) { request_at(g_off[n], src, lds_unit, n); };
   auto k_src = [&](const char* tile, int t) __attribute__((always_inline)) {
     return tile + (size_t)min(t, num_k_tiles - 1) * S::BK * 2;   // clamped past the end
   };
@@ -315,114 +352,222 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
   constexpr std::integral_constant<int, S::kLoadsA> kOfA{};
   constexpr std::integral_constant<int, S::kLoadsB> kOfB{};
 
-  // prologue: tiles 0 .. kAhead-1 into the first 2 * kAhead units; fragments (0, 0) once
-  // tile 0 is there
-#pragma unroll
-  for (int u = 0; u < 2 * S::kAhead; ++u)
-#pragma unroll
-    for (int n = 0; n < (u % 2 ? S::kLoadsB : S::kLoadsA); ++n) {
-      const char* tile = u % 2 ? b_tile : a_tile;
-      const unsigned unit = (u % 2 ? lds_wave_b : lds_wave_a) + u * S::kUnitBytes;
-      if (u < 2 && k_pad != 0) {
-        const bool in_front = S::swizzle(ld_row + 8 * n, ld_c) * 8 < k_pad;
-        const char* src = tile + (g_off[n] + 1024u * (n % 4));
-        lds_dma_16B(in_front ? reinterpret_cast<const char*>(kZeros) : src, unit + n * 1024);
-      } else {
-        request(k_src(tile, u / 2), unit, n);
-      }
-    }
-  wait_vmem<(S::kAhead - 1) * (S::kLoadsA + S::kLoadsB)>();
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-#pragma unroll
-  for (int f = 0; f < S::TN; ++f)
-    bf[0][f] = *reinterpret_cast<const half8_t*>(smem + S::kUnitBytes + b_rd[0] + f * 16 * S::kRowBytes);
-#pragma unroll
-  for (int i = 0; i < S::TM; ++i)
-    afx[0][i] = *reinterpret_cast<const half8_t*>(smem + a_rd[0] + i * 16 * S::kRowBytes);
-  // drained here, visibly to the compiler, so that the waits it places at the head of the loop
-  // only have to cover the loop's own reads
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  __builtin_amdgcn_sched_barrier(0);
-
-  // Ring bookkeeping, in bytes: oa = LDS offset of the unit holding A of tile t; B of tile t is
-  // one unit further, A of t+1 two, ... (mod kUnits units).  A wavefront alone on its SIMD issues one
-  // instruction every 4 cycles, so a 16-cycle MFMA hides at most three other instructions:
-  // everything an iteration needs (fragment read bases, request destinations and sources) is
-  // therefore computed during the previous k-step in pieces of at most three instructions,
-  // each pinned into its own gap between two MFMAs of the slots that carry no fragment reads.
-  constexpr unsigned kRingBytes = S::kUnits * S::kUnitBytes;
-  auto ring = [](unsigned o) __attribute__((always_inline)) { return o >= kRingBytes ? o - kRingBytes : o; };
-  const unsigned rdbase_a0 = smem_addr + a_rd[0], rdbase_a1 = smem_addr + a_rd[1];
-  const unsigned rdbase_b0 = smem_addr + b_rd[0], rdbase_b1 = smem_addr + b_rd[1];
-  const int last_tile = num_k_tiles - 1;
-  unsigned oa = 0;                                             // A of tile t
-  unsigned oa1 = 2 * S::kUnitBytes, ob1 = 3 * S::kUnitBytes;   // A, B of tile t+1
-  unsigned rd_a1 = rdbase_a1, rd_b1 = rdbase_b1 + S::kUnitBytes;   // reads of (t, k-step 1)
-  unsigned req_a = lds_wave_a + 2 * S::kAhead * S::kUnitBytes;       // A of t+kAhead
-  const char* src_a = k_src(a_tile, S::kAhead);
-  unsigned rd_a0 = 0, rd_b0 = 0, req_b = 0;                        // set during k-step 0
-  const char* src_b = b_tile;
-  int kt = 0;
-#define TFK_PIN_S(x) asm volatile("" : "+s"(x))
-#define TFK_PIN_V(x) asm volatile("" : "+v"(x))
-  // pieces run in the read-free gaps from slot kPrepSlot on of k-step 0 / k-step 1
-  auto prep0 = [&](int step, int t) __attribute__((always_inline)) {
-    __builtin_amdgcn_sched_barrier(0);
-    switch (step) {
-      case 0: TFK_PIN_S(oa); oa1 = ring(oa + 2 * S::kUnitBytes); TFK_PIN_S(oa1); break;
-      case 1: ob1 = ring(oa1 + S::kUnitBytes); TFK_PIN_S(ob1); break;
-      case 2: rd_a0 = rdbase_a0 + oa1; TFK_PIN_V(rd_a0); break;
-      case 3: rd_b0 = rdbase_b0 + ob1; TFK_PIN_V(rd_b0); break;
-      case 4: req_b = lds_wave_b + oa; TFK_PIN_S(req_b); break;
-      case 5: kt = t; TFK_PIN_S(kt); kt = min(kt + S::kAhead, last_tile); TFK_PIN_S(kt); break;
-      case 6: src_b = b_tile + (size_t)(unsigned)(kt * (S::BK * 2)); TFK_PIN_S(src_b); break;
-      default: break;
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto prep1 = [&](int step, int t) __attribute__((always_inline)) {
-    __builtin_amdgcn_sched_barrier(0);
-    switch (step) {
-      case 0: oa = oa1; TFK_PIN_S(oa); rd_a1 = rdbase_a1 + oa; TFK_PIN_V(rd_a1); break;
-      case 1: rd_b1 = rdbase_b1 + ob1; TFK_PIN_V(rd_b1); break;
-      case 2: req_a = ring(oa + 2 * S::kAhead * S::kUnitBytes); TFK_PIN_S(req_a); break;
-      case 3: req_a += lds_wave_a; TFK_PIN_S(req_a); break;
-      case 4: kt = t; TFK_PIN_S(kt); kt = min(kt + S::kAhead + 1, last_tile); TFK_PIN_S(kt); break;
-      case 5: src_a = a_tile + (size_t)(unsigned)(kt * (S::BK * 2)); TFK_PIN_S(src_a); break;
-      default: break;
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  for (int t = 0; t < num_k_tiles; ++t) {
-#pragma unroll
-    for (int i = 0; i < S::TM; ++i) {
-      __builtin_amdgcn_sched_barrier(0);
-      request_slot(i, src_a, req_a, kOfA);
-      slot_pinned(0, i, rd_a1, rd_b1, [&](int j) __attribute__((always_inline)) {
-        prep0(S::kPrep.piece[i * S::TN + j], t);
-      });
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    ring_barrier();
-#pragma unroll
-    for (int i = 0; i < S::TM; ++i) {
-      __builtin_amdgcn_sched_barrier(0);
-      request_slot(i, src_b, req_b, kOfB);
-      slot_pinned(1, i, rd_a0, rd_b0, [&](int j) __attribute__((always_inline)) {
-        prep1(S::kPrep.piece[i * S::TN + j], t);
-      });
-    }
-    // The compiler does not know that the accumulators are written by MFMAs (they are issued
-    // from assembly), so nothing would keep it from reading the youngest results right behind
-    // the loop without the wait states the matrix pipe needs.  The delay therefore sits inside
-    // the last iteration, in front of anything the register allocator may put on the exit
-    // edge.  The iteration count is laundered through an empty asm so that the test is not
-    // recognised as the exit condition and sunk out of the loop.
+  // The compiler does not know that the accumulators are written by MFMAs (they are issued
+  // from assembly), so nothing would keep it from reading the youngest results right behind
+  // the loop without the wait states the matrix pipe needs.  The delay therefore sits inside
+  // the last iteration, in front of anything the register allocator may put on the exit
+  // edge.  The iteration count is laundered through an empty asm so that the test is not
+  // recognised as the exit condition and sunk out of the loop.
+  auto settle_behind_last = [&](int t) __attribute__((always_inline)) {
     int t_seen = t;
     asm volatile("" : "+s"(t_seen));
     if (t_seen + 1 == num_k_tiles) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+  };
+#define TFK_PIN_S(x) asm volatile("" : "+s"(x))
+#define TFK_PIN_V(x) asm volatile("" : "+v"(x))
+  if constexpr (kShift) {
+    // prologue: segments 0 .. kLines-1; the chunks in front of a row, in segments 0 and 1, are zeros
+#pragma unroll
+    for (int u = 0; u < S::kLines; ++u)
+#pragma unroll
+      for (int q = 0; q < S::kLoads; ++q) {
+        const bool of_a = q < S::kLoadsA;
+        const int n = of_a ? q : q - S::kLoadsA;
+        const int shift = of_a ? a_shift : b_shift;
+        const unsigned off = of_a ? g_off[n] : g_off_b[n];
+        const char* tile = (of_a ? a_tile : b_tile) + u * (S::BK * 2);
+        const unsigned unit = (of_a ? lds_wave_a : lds_wave_b + S::BM * S::kRowBytes) + u * S::kTileBytes;
+        if (u < 2) {
+          const bool in_front = 8 * u + segment_chunk(n, shift) - shift < pad_chunks;
+          lds_dma_16B(in_front ? reinterpret_cast<const char*>(kZeros) : tile + (off + 1024u * (n % 4)), unit + n * 1024);
+        } else {
+          request_at(off, tile, unit, n);
+        }
+      }
+    // all ones where this lane's chunk of a k-step lies in the second of the two segments
+    int a_next[2], b_next[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      a_next[ks] = 4 * ks + fg + shift_of(A, m0 + fr) >= 8 ? -1 : 0;
+      b_next[ks] = 4 * ks + fg + shift_of(B, n0 + fr) >= 8 ? -1 : 0;
+    }
+    constexpr unsigned kRingBytes = S::kLines * S::kTileBytes;
+    auto ring = [](unsigned o) __attribute__((always_inline)) { return o >= kRingBytes ? o - kRingBytes : o; };
+    const unsigned rdbase_a0 = smem_addr + a_rd[0], rdbase_a1 = smem_addr + a_rd[1];
+    const unsigned rdbase_b0 = smem_addr + S::BM * S::kRowBytes + b_rd[0], rdbase_b1 = smem_addr + S::BM * S::kRowBytes + b_rd[1];
+    const unsigned lds_b = lds_wave_b + S::BM * S::kRowBytes;
+    wait_vmem<(S::kLines - 2) * S::kLoads>();   // segments 0 and 1 have landed
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    unsigned rd_a0 = rdbase_a0 + (a_next[0] & S::kTileBytes), rd_b0 = rdbase_b0 + (b_next[0] & S::kTileBytes);
+#pragma unroll
+    for (int f = 0; f < S::TN; ++f) bf[0][f] = lds_read_b128(rd_b0 + f * 16 * S::kRowBytes);
+#pragma unroll
+    for (int i = 0; i < S::TM; ++i) afx[0][i] = lds_read_b128(rd_a0 + i * 16 * S::kRowBytes);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_sched_barrier(0);
+    unsigned s0 = 0, s1 = S::kTileBytes, s2 = 0;   // segments t, t+1 and t+2 in the ring
+    unsigned step = S::kTileBytes;                 // from a segment to the next one's
+    unsigned rd_a1 = rdbase_a1 + (a_next[1] & S::kTileBytes), rd_b1 = rdbase_b1 + (b_next[1] & S::kTileBytes);
+    unsigned req_a = 0, req_b = 0;
+    const char *src_a = a_tile, *src_b = b_tile;
+    int kt = 0;
+    // during k-step 0: where the fragments of (t+1, 0) are, and segment t+kLines, which takes the place of segment t in k-step 1
+    auto prep0 = [&](int piece, int t) __attribute__((always_inline)) {
+      __builtin_amdgcn_sched_barrier(0);
+      switch (piece) {
+        case 0: s1 = ring(s0 + S::kTileBytes); TFK_PIN_S(s1); break;
+        case 1: s2 = ring(s1 + S::kTileBytes); TFK_PIN_S(s2); break;
+        case 2: step = s2 - s1; TFK_PIN_S(step); rd_a0 = rdbase_a0 + s1 + (a_next[0] & step); TFK_PIN_V(rd_a0); break;
+        case 3: rd_b0 = rdbase_b0 + s1 + (b_next[0] & step); TFK_PIN_V(rd_b0); break;
+        case 4: req_a = lds_wave_a + s0; TFK_PIN_S(req_a); req_b = lds_b + s0; TFK_PIN_S(req_b); break;
+        case 5: kt = t; TFK_PIN_S(kt); kt = min(kt + S::kLines, num_k_tiles); TFK_PIN_S(kt); break;
+        case 6: src_a = a_tile + (size_t)(unsigned)(kt * (S::BK * 2)); TFK_PIN_S(src_a); break;
+        case 7: src_b = b_tile + (size_t)(unsigned)(kt * (S::BK * 2)); TFK_PIN_S(src_b); break;
+        default: break;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto prep1 = [&](int piece) __attribute__((always_inline)) {
+      __builtin_amdgcn_sched_barrier(0);
+      switch (piece) {
+        case 0: rd_a1 = rdbase_a1 + s1 + (a_next[1] & step); TFK_PIN_V(rd_a1); break;
+        case 1: rd_b1 = rdbase_b1 + s1 + (b_next[1] & step); TFK_PIN_V(rd_b1); break;
+        case 2: s0 = s1; TFK_PIN_S(s0); break;
+        default: break;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int t = 0; t < num_k_tiles; ++t) {
+      // The last segment ends behind the row: what lies there is never read, and not fetched either (the row's last chunk is,
+      // again). Requests from here on ask for no other segment.
+      if (t + S::kLines == num_k_tiles) {
+#pragma unroll
+        for (int n = 0; n < S::kLoadsA; ++n) g_off[n] -= 16u * (unsigned)max(0, segment_chunk(n, a_shift) - (a_shift - 1));
+#pragma unroll
+        for (int n = 0; n < S::kLoadsB; ++n) g_off_b[n] -= 16u * (unsigned)max(0, segment_chunk(n, b_shift) - (b_shift - 1));
+      }
+#pragma unroll
+      for (int i = 0; i < S::TM; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        slot_pinned(0, i, rd_a1, rd_b1, [&](int j) __attribute__((always_inline)) { prep0(S::kPrep.piece[i * S::TN + j], t); });
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      ring_barrier();   // segment t is read out, segment t+2 has landed
+#pragma unroll
+      for (int i = 0; i < S::TM; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < S::kLoads; ++q)
+          if ((q * S::TM) / S::kLoads == i) {
+            if (q < S::kLoadsA) request_at(g_off[q], src_a, req_a, q);
+            else request_at(g_off_b[q - S::kLoadsA], src_b, req_b, q - S::kLoadsA);
+          }
+        slot_pinned(1, i, rd_a0, rd_b0, [&](int j) __attribute__((always_inline)) { prep1(S::kPrep.piece[i * S::TN + j]); });
+      }
+      settle_behind_last(t);
+    }
+  } else {
+    // prologue: tiles 0 .. kAhead-1 into the first 2 * kAhead units; fragments (0, 0) once
+    // tile 0 is there
+#pragma unroll
+    for (int u = 0; u < 2 * S::kAhead; ++u)
+#pragma unroll
+      for (int n = 0; n < (u % 2 ? S::kLoadsB : S::kLoadsA); ++n) {
+        const char* tile = u % 2 ? b_tile : a_tile;
+        const unsigned unit = (u % 2 ? lds_wave_b : lds_wave_a) + u * S::kUnitBytes;
+        if (u < 2 && k_pad != 0) {
+          const bool in_front = S::swizzle(ld_row + 8 * n, ld_c) * 8 < k_pad;
+          const char* src = tile + (g_off[n] + 1024u * (n % 4));
+          lds_dma_16B(in_front ? reinterpret_cast<const char*>(kZeros) : src, unit + n * 1024);
+        } else {
+          request(k_src(tile, u / 2), unit, n);
+        }
+      }
+    wait_vmem<(S::kAhead - 1) * (S::kLoadsA + S::kLoadsB)>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int f = 0; f < S::TN; ++f)
+      bf[0][f] = *reinterpret_cast<const half8_t*>(smem + S::kUnitBytes + b_rd[0] + f * 16 * S::kRowBytes);
+#pragma unroll
+    for (int i = 0; i < S::TM; ++i)
+      afx[0][i] = *reinterpret_cast<const half8_t*>(smem + a_rd[0] + i * 16 * S::kRowBytes);
+    // drained here, visibly to the compiler, so that the waits it places at the head of the loop
+    // only have to cover the loop's own reads
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_sched_barrier(0);
+
+    // Ring bookkeeping, in bytes: oa = LDS offset of the unit holding A of tile t; B of tile t is
+    // one unit further, A of t+1 two, ... (mod kUnits units).  A wavefront alone on its SIMD issues one
+    // instruction every 4 cycles, so a 16-cycle MFMA hides at most three other instructions:
+    // everything an iteration needs (fragment read bases, request destinations and sources) is
+    // therefore computed during the previous k-step in pieces of at most three instructions,
+    // each pinned into its own gap between two MFMAs of the slots that carry no fragment reads.
+    constexpr unsigned kRingBytes = S::kUnits * S::kUnitBytes;
+    auto ring = [](unsigned o) __attribute__((always_inline)) { return o >= kRingBytes ? o - kRingBytes : o; };
+    const unsigned rdbase_a0 = smem_addr + a_rd[0], rdbase_a1 = smem_addr + a_rd[1];
+    const unsigned rdbase_b0 = smem_addr + b_rd[0], rdbase_b1 = smem_addr + b_rd[1];
+    const int last_tile = num_k_tiles - 1;
+    unsigned oa = 0;                                             // A of tile t
+    unsigned oa1 = 2 * S::kUnitBytes, ob1 = 3 * S::kUnitBytes;   // A, B of tile t+1
+    unsigned rd_a1 = rdbase_a1, rd_b1 = rdbase_b1 + S::kUnitBytes;   // reads of (t, k-step 1)
+    unsigned req_a = lds_wave_a + 2 * S::kAhead * S::kUnitBytes;       // A of t+kAhead
+    const char* src_a = k_src(a_tile, S::kAhead);
+    unsigned rd_a0 = 0, rd_b0 = 0, req_b = 0;                        // set during k-step 0
+    const char* src_b = b_tile;
+    int kt = 0;
+    // pieces run in the read-free gaps from slot kPrepSlot on of k-step 0 / k-step 1
+    auto prep0 = [&](int step, int t) __attribute__((always_inline)) {
+      __builtin_amdgcn_sched_barrier(0);
+      switch (step) {
+        case 0: TFK_PIN_S(oa); oa1 = ring(oa + 2 * S::kUnitBytes); TFK_PIN_S(oa1); break;
+        case 1: ob1 = ring(oa1 + S::kUnitBytes); TFK_PIN_S(ob1); break;
+        case 2: rd_a0 = rdbase_a0 + oa1; TFK_PIN_V(rd_a0); break;
+        case 3: rd_b0 = rdbase_b0 + ob1; TFK_PIN_V(rd_b0); break;
+        case 4: req_b = lds_wave_b + oa; TFK_PIN_S(req_b); break;
+        case 5: kt = t; TFK_PIN_S(kt); kt = min(kt + S::kAhead, last_tile); TFK_PIN_S(kt); break;
+        case 6: src_b = b_tile + (size_t)(unsigned)(kt * (S::BK * 2)); TFK_PIN_S(src_b); break;
+        default: break;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto prep1 = [&](int step, int t) __attribute__((always_inline)) {
+      __builtin_amdgcn_sched_barrier(0);
+      switch (step) {
+        case 0: oa = oa1; TFK_PIN_S(oa); rd_a1 = rdbase_a1 + oa; TFK_PIN_V(rd_a1); break;
+        case 1: rd_b1 = rdbase_b1 + ob1; TFK_PIN_V(rd_b1); break;
+        case 2: req_a = ring(oa + 2 * S::kAhead * S::kUnitBytes); TFK_PIN_S(req_a); break;
+        case 3: req_a += lds_wave_a; TFK_PIN_S(req_a); break;
+        case 4: kt = t; TFK_PIN_S(kt); kt = min(kt + S::kAhead + 1, last_tile); TFK_PIN_S(kt); break;
+        case 5: src_a = a_tile + (size_t)(unsigned)(kt * (S::BK * 2)); TFK_PIN_S(src_a); break;
+        default: break;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int t = 0; t < num_k_tiles; ++t) {
+#pragma unroll
+      for (int i = 0; i < S::TM; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        request_slot(i, src_a, req_a, kOfA);
+        slot_pinned(0, i, rd_a1, rd_b1, [&](int j) __attribute__((always_inline)) {
+          prep0(S::kPrep.piece[i * S::TN + j], t);
+        });
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      ring_barrier();
+#pragma unroll
+      for (int i = 0; i < S::TM; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        request_slot(i, src_b, req_b, kOfB);
+        slot_pinned(1, i, rd_a0, rd_b0, [&](int j) __attribute__((always_inline)) {
+          prep1(S::kPrep.piece[i * S::TN + j], t);
+        });
+      }
+      settle_behind_last(t);
+    }
   }
   __builtin_amdgcn_sched_barrier(0);
   wait_vmem_all();  // the clamped tail requests must not outlive the workgroup's LDS
@@ -483,7 +628,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
 template <typename S, typename OutT, typename InT>
 int launch_ring64(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st) {
   auto kern = gemm_ring64_kernel<S, InT, OutT>;
-  constexpr int lds = S::kUnits * S::kUnitBytes;
+  constexpr int lds = S::kLdsBytes;
   static_assert(lds <= kMaxLdsBytes, "ring does not fit in LDS");
   TFK_LDS_OPT_IN(kern, lds);
   const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
@@ -805,12 +950,33 @@ constexpr GemmKernel kGemmKernels[] = {
 };
 constexpr int kNumGemmKernels = sizeof(kGemmKernels) / sizeof(kGemmKernels[0]);
 
-float expected_us(const GemmKernel& g, int64_t tiles, int ktiles, bool unaligned_rows) {
+// Rows that start anywhere in a line: from K = 328 on these ring kernels fetch whole lines (Ring64Shape::kLines), which costs them a
+// segment more at first and saves them 0.13-0.27 us a k-tile. Microseconds as above, fitted to 60 problems (M, N 128-8192, K
+// 328-8192; 4-5% root mean square); picks are 2% behind the best of all kernels on average. us, k-tiles that start where rows
+// start / whole lines: 1500 x 1500 x 3000, 128 x 128 31.0 / 22.6; 700 x 4096 x 4104 40.2 / 30.5; 2999 x 1544 x 1032,
+// 192 x 128 18.5 / 16.0; 3333 x 2288 x 1944, 256 x 128 39.3 / 33.5, 192 x 192 35.3 / 33.6. (The larger tiles leave no room for a third
+// segment, and two workgroups of 128 x 128 none for each other; below K = 328 the further segment costs as much as it saves:
+// 8192 x 1000 x 328 14.0 / 13.5.)
+constexpr int kLinesFrom = 328;
+bool takes_lines(int K) { return K % 64 != 0 && K >= kLinesFrom; }
+struct LinesKernel {
+  int index;                // into kGemmKernels
+  float start, round, step, shared;
+};
+constexpr LinesKernel kLinesKernels[] = {
+    {7, 1.63f, 3.67f, 0.317f, 0.139f},
+    {10, 1.32f, 4.65f, 0.430f, 0.167f},
+    {11, 0.60f, 5.44f, 0.695f, 0.269f},
+    {12, 1.36f, 4.11f, 0.660f, 0.281f},
+};
+
+float expected_us(const GemmKernel& g, int64_t tiles, int ktiles, bool unaligned_rows, const LinesKernel* lines) {
   const int64_t rounds = (tiles + 256 * g.per_cu - 1) / (256 * g.per_cu);
   const float unaligned = unaligned_rows ? g.unaligned : 0.f;
   const float per_cu = tiles / 256.f;
   if (g.ring) {
     const float fill = std::min(1.f, per_cu / (rounds * g.per_cu));
+    if (lines != nullptr) return lines->start + rounds * (lines->round + ktiles * (lines->step + lines->shared * fill));
     return g.start + rounds * g.per_cu * (g.round + ktiles * (g.step + g.shared * fill + unaligned));
   }
   const int chain = (ktiles + g.waves - 1) / g.waves;
@@ -874,7 +1040,11 @@ int pick_gemm_kernel(int M, int N, int K, bool c_is_f32) {
     if (g.ring && (M < g.bm || N < g.bn || K < 64)) continue;   // (what gemm_ring64_kernel asks for)
     const int64_t tiles = (int64_t)((M + g.bm - 1) / g.bm) * ((N + g.bn - 1) / g.bn);
     if (tiles < g.min_tiles || tiles > g.max_tiles) continue;
-    const float us = expected_us(g, tiles, ktiles, K % 64 != 0);
+    const LinesKernel* lines = nullptr;
+    if (takes_lines(K))
+      for (const LinesKernel& l : kLinesKernels)
+        if (l.index == i) lines = &l;
+    const float us = expected_us(g, tiles, ktiles, K % 64 != 0, lines);
     if (us < best_us) {
       best = i;
       best_us = us;
@@ -903,7 +1073,14 @@ int dispatch(const void* A, const void* B, void* C, int M, int N, int K, hipStre
   if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) % 16 != 0 ||
       (K < 64 && (int64_t)M * N >= (int64_t)1 << 35))
     return kLaunchers[kNumGemmKernels](A, B, C, M, N, K, st);
-  return kLaunchers[pick_gemm_kernel(M, N, K, sizeof(OutT) == 4)](A, B, C, M, N, K, st);
+  const int pick = pick_gemm_kernel(M, N, K, sizeof(OutT) == 4);
+  if (takes_lines(K)) {   // (kLinesKernels)
+    if (pick == 7) return launch_ring64<Ring64Shape<128, 128, 2, 5>, OutT, InT>(A, B, C, M, N, K, st);
+    if (pick == 10) return launch_ring64<Ring64Shape<192, 128, 2, 4>, OutT, InT>(A, B, C, M, N, K, st);
+    if (pick == 11) return launch_ring64<Ring64Shape<192, 192, 2, 3>, OutT, InT>(A, B, C, M, N, K, st);
+    if (pick == 12) return launch_ring64<Ring64Shape<256, 128, 2, 3>, OutT, InT>(A, B, C, M, N, K, st);
+  }
+  return kLaunchers[pick](A, B, C, M, N, K, st);
 }
 
 }  // namespace
