@@ -64,7 +64,8 @@ __host__ __device__ constexpr int swz_kt(int row, int c) {
 }
 
 // What a workgroup's number stands for (causal; see the kernel).
-enum : int { kSingle = 0, kPairs = 1, kByXcd = 2 };
+enum : int { kSingle = 0, kPairs = 1, kByXcd = 2, kFolded = 3 };
+constexpr int kCUs = 256;
 
 typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef __fp16 fp16x4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
@@ -260,9 +261,16 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
       qt_of_pass[0] = q_tiles - 1 - p / own;
       bh = xcd + 8 * (p % own);
     } else {
-      if ((int)blockIdx.x >= total_items) return;
-      qt_of_pass[0] = q_tiles - 1 - (int)blockIdx.x / slices;
-      bh = blockIdx.x % slices;
+      const int i = (int)blockIdx.x;
+      if (i >= total_items) return;
+      qt_of_pass[0] = q_tiles - 1 - i / slices;
+      bh = i % slices;
+      if (order == kFolded && i >= kCUs) {
+        // second on their CUs: lightest first
+        const int level = (i - kCUs) / slices;
+        qt_of_pass[0] = level;
+        bh = (i - kCUs) % slices + (level == q_tiles - 1 - kCUs / slices ? kCUs % slices : 0);
+      }
     }
   }
   Q += bh * (size_t)Lq * d_row;
@@ -946,11 +954,12 @@ int launch_w(const AttentionCall& c) {
   // that leaves the XCDs within 4% of each other (bf16, 150 slices of 384 x 384 x 256: 39.4 / 31.4 us).
   const int per_xcd = (c.batch + 7) / 8;
   const bool by_xcd = kCausal && !paired && c.batch % 8 != 0 && 8 * per_xcd * 100 <= c.batch * 104;
+  const bool folded = kCausal && ring_stages(kWavesT, D) == 2 && !paired && !by_xcd && total_items > kCUs && total_items <= 2 * kCUs;
   const dim3 grid(by_xcd ? 8 * per_xcd * q_tiles : 8 * ((total_items + 7) / 8));
   hipLaunchKernelGGL(kern, grid, dim3(kWavesT * 64), lds, c.stream,
                      static_cast<const T*>(c.Q), static_cast<const T*>(c.K),
                      static_cast<const T*>(c.V), static_cast<T*>(c.O), c.Lq, c.Lkv, c.scale_log2,
-                     q_tiles, total_items, paired ? kPairs : by_xcd ? kByXcd : kSingle, c.d, c.part, c.splits, c.chunk);
+                     q_tiles, total_items, paired ? kPairs : by_xcd ? kByXcd : folded ? kFolded : kSingle, c.d, c.part, c.splits, c.chunk);
   TFK_HIP_TRY(hipGetLastError());
   return TF_OK;
 }
