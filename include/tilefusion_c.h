@@ -184,6 +184,10 @@ TF_API int tf_flash_decode(const void* Q, const void* K, const void* V, void* O,
                            int64_t Lkv, int64_t D, int num_splits, double softmax_scale,
                            void* stream);
 
+/* tf_flash_decode where it cuts no slice (tf_flash_decode_plan says 1), which takes no workspace; TF_ERR_UNSUPPORTED where it does. */
+TF_API int tf_flash_decode_uncut(const void* Q, const void* K, const void* V, void* O, int dtype, int64_t batch_heads,
+                                 int64_t Lkv, int64_t D, int num_splits, double softmax_scale, void* stream);
+
 /* tf_flash_decode_f16 without the workspace argument and without any allocation: the per-split
  * partials live in a static device array inside the library (TF_FLASH_DECODE_STATIC_MAX_PARTIALS
  * x (128 + 2) floats = 16.25 MiB, held by every GPU the library runs on until the process ends).

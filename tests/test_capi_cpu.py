@@ -79,6 +79,12 @@ def test_decode_argument_validation_and_workspace():
     assert b"workspace" in lib.tf_last_error()
     assert f(p, p, p, p, p, 1 << 20, 4, 128, 96, 4, 0.1, None) == _capi.TF_ERR_UNSUPPORTED   # 128 and 64 only
     assert f(p, p, p, p, p, 1 << 20, 4, 0, 128, 4, 0.1, None) == _capi.TF_ERR_INVALID_ARG
+    # without a workspace: only what is not cut
+    f = lib.tf_flash_decode_uncut
+    assert f(p, p, p, p, _capi.TF_DTYPE_F16, 8, 4096, 128, 64, 0.1, None) == _capi.TF_ERR_UNSUPPORTED
+    assert f(p, p, p, p, _capi.TF_DTYPE_F32, 8, 64, 128, 64, 0.1, None) == _capi.TF_ERR_UNSUPPORTED
+    assert f(p, p, p, p, _capi.TF_DTYPE_F16, 8, 64, 128, 0, 0.1, None) == _capi.TF_ERR_UNSUPPORTED
+    assert f(p, None, p, p, _capi.TF_DTYPE_F16, 8, 64, 128, 64, 0.1, None) == _capi.TF_ERR_INVALID_ARG
 
 
 # ---- what a call runs, decided on the host ------------------------------------------------------------

@@ -8,6 +8,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <tuple>
 
 #include "tilefusion_c.h"
 
@@ -179,6 +180,23 @@ int hip_fail(hipError_t e, const char* what);
     hipError_t e__ = (expr);                                \
     if (e__ != hipSuccess) return ::tfk::hip_fail(e__, #expr); \
   } while (0)
+
+// Launches `kern`, its arguments converted to the kernel's parameter types.  (The <<<>>> form leaves its configuration with the runtime and
+// takes it back for every launch, and says what went wrong through a second call: 2.5 us a launch in a loop, 2.3 as here.)
+template <typename... P, typename... A>
+int launch_kernel(void (*kern)(P...), dim3 grid, dim3 block, unsigned lds, hipStream_t st, A... args) {
+  static_assert(sizeof...(P) == sizeof...(A), "an argument for every parameter");
+  std::tuple<P...> values(static_cast<P>(args)...);
+  return std::apply(
+      [&](P&... v) -> int {
+        void* pointers[] = {const_cast<void*>(static_cast<const void*>(&v))...};
+        const hipError_t e = hipLaunchKernel(reinterpret_cast<const void*>(kern), grid, block, pointers, lds, st);
+        if (e == hipSuccess) return TF_OK;
+        (void)hipGetLastError();   // (told here, and by no later call)
+        return hip_fail(e, "hipLaunchKernel");
+      },
+      values);
+}
 
 // Opts `kern` in to `lds` bytes of dynamic LDS.  The attribute is per device and sticky, so the
 // runtime call is made once per kernel and device (a bit per device ordinal in a static of the

@@ -961,12 +961,10 @@ int launch_w(const AttentionCall& c) {
   const bool by_xcd = kCausal && !paired && c.batch % 8 != 0 && 8 * per_xcd * 100 <= c.batch * 104;
   const bool folded = kCausal && ring_stages(kWavesT, D) == 2 && !paired && !by_xcd && total_items > kCUs && total_items <= 2 * kCUs;
   const dim3 grid(by_xcd ? 8 * per_xcd * q_tiles : 8 * ((total_items + 7) / 8));
-  hipLaunchKernelGGL(kern, grid, dim3(kWavesT * 64), lds, c.stream,
-                     static_cast<const T*>(c.Q), static_cast<const T*>(c.K),
-                     static_cast<const T*>(c.V), static_cast<T*>(c.O), c.Lq, c.Lkv, c.scale_log2,
-                     q_tiles, total_items, paired ? kPairs : by_xcd ? kByXcd : folded ? kFolded : kSingle, c.d, c.part, c.splits, c.chunk);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(kern, grid, dim3(kWavesT * 64), lds, c.stream,
+                       static_cast<const T*>(c.Q), static_cast<const T*>(c.K),
+                       static_cast<const T*>(c.V), static_cast<T*>(c.O), c.Lq, c.Lkv, c.scale_log2,
+                       q_tiles, total_items, paired ? kPairs : by_xcd ? kByXcd : folded ? kFolded : kSingle, c.d, c.part, c.splits, c.chunk);
 }
 
 template <typename T, int D, bool kKT, bool kVT, bool kCausal, bool kTail>
@@ -994,10 +992,8 @@ int launch_split(const AttentionCall& c) {
                            : launch_w<T, D, D, false, false, false, 4, 1, false, true>(c);
   if (rc != TF_OK) return rc;
   const size_t rows = (size_t)c.batch * c.Lq, threads = rows * (c.d / 8);
-  hipLaunchKernelGGL((merge_parts_kernel<T, D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, c.stream, c.part,
-                     static_cast<T*>(c.O), rows, c.d, c.splits);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(merge_parts_kernel<T, D>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, c.stream, c.part,
+                       static_cast<T*>(c.O), rows, c.d, c.splits);
 }
 template <int D>
 int launch(const AttentionCall& c) {

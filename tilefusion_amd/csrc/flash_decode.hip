@@ -427,12 +427,10 @@ template <typename T, int D, int kDecWaves, DecodeEnd kEnd>
 int launch_split(const void* Q, const void* K, const void* V, void* O, float* o_part, float* ml_part,
                  int64_t batch_heads, int64_t Lkv, DecodePlan plan, double softmax_scale, hipStream_t st, arrivals_t* arrivals = nullptr) {
   const float scale_log2 = (float)(softmax_scale * 1.4426950408889634);
-  hipLaunchKernelGGL((flash_decode_split_kernel<T, D, kDecWaves, kEnd>), dim3(plan.splits, (unsigned)batch_heads),
-                     dim3(kDecWaves * kWaveSize), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K),
-                     static_cast<const T*>(V), static_cast<T*>(O), o_part, ml_part, Lkv, plan.splits, plan.chunk,
-                     scale_log2, arrivals, kEnd == kMerged ? next_arrivals_tag() : 0);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(flash_decode_split_kernel<T, D, kDecWaves, kEnd>, dim3(plan.splits, (unsigned)batch_heads),
+                       dim3(kDecWaves * kWaveSize), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K),
+                       static_cast<const T*>(V), static_cast<T*>(O), o_part, ml_part, Lkv, plan.splits, plan.chunk,
+                       scale_log2, arrivals, kEnd == kMerged ? next_arrivals_tag() : 0);
 }
 
 // The kernels on `st`; `partials` holds o_part then ml_part and, where there is `room` (bytes) for them, the words in which the
@@ -458,10 +456,8 @@ int launch_decode_t(const void* Q, const void* K, const void* V, void* O, float*
       ? launch_split<T, D, 8, kParts>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st)
       : launch_split<T, D, 4, kParts>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st);
   if (rc != TF_OK) return rc;
-  hipLaunchKernelGGL((flash_decode_combine_kernel<T, D>), dim3((unsigned)batch_heads), dim3(kCombThreads), 0, st,
-                     o_part, ml_part, static_cast<T*>(O), plan.splits);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(flash_decode_combine_kernel<T, D>, dim3((unsigned)batch_heads), dim3(kCombThreads), 0, st,
+                       o_part, ml_part, static_cast<T*>(O), plan.splits);
 }
 int launch_decode(const void* Q, const void* K, const void* V, void* O, float* partials, size_t room, int dtype,
                   int64_t batch_heads, int64_t Lkv, int64_t D, int num_splits, double softmax_scale,
@@ -515,6 +511,18 @@ extern "C" int tf_flash_decode(const void* Q, const void* K, const void* V, void
               "tf_flash_decode: dtype must be TF_DTYPE_F16 or TF_DTYPE_BF16");
   return decode_with_workspace("tf_flash_decode", Q, K, V, O, dtype, workspace, workspace_bytes, batch_heads, Lkv, D,
                                num_splits, softmax_scale, stream);
+}
+
+extern "C" int tf_flash_decode_uncut(const void* Q, const void* K, const void* V, void* O, int dtype, int64_t batch_heads,
+                                     int64_t Lkv, int64_t D, int num_splits, double softmax_scale, void* stream) {
+  using namespace tfk;
+  // (no message for what is cut or not taken: tf_flash_decode has one)
+  if (dtype != TF_DTYPE_F16 && dtype != TF_DTYPE_BF16) return TF_ERR_UNSUPPORTED;
+  int waves = 0;
+  if (tf_flash_decode_plan(batch_heads, Lkv, D, num_splits, &waves) != 1) return TF_ERR_UNSUPPORTED;
+  if (int rc = check_decode_args("tf_flash_decode_uncut", Q, K, V, O, batch_heads, Lkv, D, num_splits, softmax_scale)) return rc;
+  return launch_decode(Q, K, V, O, nullptr, 0, dtype, batch_heads, Lkv, D, num_splits, softmax_scale,
+                       static_cast<hipStream_t>(stream));
 }
 
 // ---- the same kernels with the partials in a static device array -------------------

@@ -305,11 +305,9 @@ template <typename T, int TN, int TP, int KC>
 int launch(const void* A, const void* B, const void* C, void* D, int batch, int M, int N, int K,
            int P, hipStream_t st) {
   dim3 grid((M + kRowsPerBlock - 1) / kRowsPerBlock, P / TP, batch);
-  hipLaunchKernelGGL((fused_two_gemms_kernel<T, TN, TP, KC>), grid, dim3(kThreads), 0, st,
-                     static_cast<const T*>(A), static_cast<const T*>(B),
-                     static_cast<const T*>(C), static_cast<T*>(D), M, N, K, P);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(fused_two_gemms_kernel<T, TN, TP, KC>, grid, dim3(kThreads), 0, st,
+                       static_cast<const T*>(A), static_cast<const T*>(B),
+                       static_cast<const T*>(C), static_cast<T*>(D), M, N, K, P);
 }
 
 template <typename T, int TN, int TP>

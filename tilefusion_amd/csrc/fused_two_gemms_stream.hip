@@ -357,20 +357,17 @@ int launch_stream(const FusedCall& c, FusedPlan plan) {
   TFK_LDS_OPT_IN(kern, S::kLds);
   const dim3 grid((unsigned)((c.M + S::kRows - 1) / S::kRows) * (unsigned)plan.parts, 1, c.batch);
   float* w = plan.parts > 1 ? static_cast<float*>(c.workspace) : nullptr;
-  hipLaunchKernelGGL(kern, grid, dim3(kWavesS * 64), S::kLds, c.stream, static_cast<const T*>(c.A),
-                     static_cast<const T*>(c.B), static_cast<const T*>(c.C), static_cast<T*>(c.D), w, c.M, c.N, c.K, c.P,
-                     plan.parts, plan.tiles_per_part);
-  TFK_HIP_TRY(hipGetLastError());
+  if (int rc = launch_kernel(kern, grid, dim3(kWavesS * 64), S::kLds, c.stream, static_cast<const T*>(c.A),
+                       static_cast<const T*>(c.B), static_cast<const T*>(c.C), static_cast<T*>(c.D), w, c.M, c.N, c.K, c.P,
+                       plan.parts, plan.tiles_per_part)) return rc;
   if (plan.parts == 1) return TF_OK;
   const size_t elems = (size_t)c.M * c.P;
   auto sum = plan.parts <= kGroups       ? fused_sum_parts_kernel<T, 1>
              : plan.parts <= 2 * kGroups ? fused_sum_parts_kernel<T, 2>
              : plan.parts <= 4 * kGroups ? fused_sum_parts_kernel<T, 4>
                                          : fused_sum_parts_kernel<T, 8>;
-  hipLaunchKernelGGL(sum, dim3((unsigned)((elems / 4 + 63) / 64), 1, c.batch), dim3(kGroups * 64), 0, c.stream, w,
-                     static_cast<T*>(c.D), plan.parts, elems);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(sum, dim3((unsigned)((elems / 4 + 63) / 64), 1, c.batch), dim3(kGroups * 64), 0, c.stream, w,
+                       static_cast<T*>(c.D), plan.parts, elems);
 }
 template <typename T, int kKS, int kPT>
 int pick_rows(const FusedCall& c, FusedPlan plan) {

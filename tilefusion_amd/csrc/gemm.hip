@@ -632,11 +632,9 @@ int launch_ring64(const void* A, const void* B, void* C, int M, int N, int K, hi
   static_assert(lds <= kMaxLdsBytes, "ring does not fit in LDS");
   TFK_LDS_OPT_IN(kern, lds);
   const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
-  hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(S::kThreads), lds, st,
-                     static_cast<const InT*>(A), static_cast<const InT*>(B),
-                     static_cast<OutT*>(C), M, N, K, tiles_m, tiles_n);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(kern, dim3(tiles_m * tiles_n), dim3(S::kThreads), lds, st,
+                       static_cast<const InT*>(A), static_cast<const InT*>(B),
+                       static_cast<OutT*>(C), M, N, K, tiles_m, tiles_n);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -816,10 +814,8 @@ int launch_split_k(const void* A, const void* B, void* C, int M, int N, int K, h
   static_assert(S::kLdsBytes <= kMaxLdsBytes, "rings do not fit in LDS");
   if constexpr (S::kLdsBytes > 64 * 1024) TFK_LDS_OPT_IN(kern, S::kLdsBytes);
   const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
-  hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(S::kThreads), S::kLdsBytes, st, static_cast<const InT*>(A),
-                     static_cast<const InT*>(B), static_cast<OutT*>(C), M, N, K, tiles_m, tiles_n);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(kern, dim3(tiles_m * tiles_n), dim3(S::kThreads), S::kLdsBytes, st, static_cast<const InT*>(A),
+                       static_cast<const InT*>(B), static_cast<OutT*>(C), M, N, K, tiles_m, tiles_n);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -901,11 +897,9 @@ using ShapeSmall = GemmShape<64, 64, 32, 2, 2>;    // bounds-checked path
 template <typename S, typename OutT, typename InT>
 int launch_guarded(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st) {
   dim3 grid((M + S::BM - 1) / S::BM, (N + S::BN - 1) / S::BN);
-  hipLaunchKernelGGL((gemm_guarded_kernel<S, OutT, InT>), grid, dim3(S::kThreads), 0, st,
-                     static_cast<const InT*>(A), static_cast<const InT*>(B),
-                     static_cast<OutT*>(C), M, N, K);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(gemm_guarded_kernel<S, OutT, InT>, grid, dim3(S::kThreads), 0, st,
+                       static_cast<const InT*>(A), static_cast<const InT*>(B),
+                       static_cast<OutT*>(C), M, N, K);
 }
 
 // ------------------------------------------------------------------------------------------

@@ -581,10 +581,8 @@ int launch_shape(const void* updates, void* data, const long long* indices, cons
   const long long per = (long long)lanes * kWords;
   const dim3 grid((unsigned)std::min<long long>((n + kRows - 1) / kRows, 1 << 20),
                   (unsigned)std::min<long long>((words + per - 1) / per, 1024));
-  hipLaunchKernelGGL((scatter_nd_kernel<T, kThreads, kRows, kWords, kLayout>), grid, dim3(kThreads), 0, st,
-                     static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(scatter_nd_kernel<T, kThreads, kRows, kWords, kLayout>, grid, dim3(kThreads), 0, st,
+                       static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
 }
 
 // As many shares (a power of two, at least two) as bring about 224 workgroups: one a CU.  Twice as many, two a CU, for chunks of
@@ -603,11 +601,9 @@ int launch_owner(const void* updates, void* data, const long long* indices, cons
   if (kMine == 4 && kWords == 2 && bits < 8 && chunks * columns << bits <= 256) ++bits;
   const int chunk = (int)((n + chunks - 1) / chunks);   // (even ones: no nearly empty last chunk)
   const dim3 grid((unsigned)((n + chunk - 1) / chunk) << bits, (unsigned)columns);
-  hipLaunchKernelGGL((scatter_nd_owner_kernel<T, kMine, kWords, kLayout, kSingle>), grid, dim3(kOwnerThreads), 0, st,
-                     static_cast<const T*>(updates), static_cast<T*>(data), indices, numbers, n, k, slice, total, lanes, bits,
-                     chunk);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(scatter_nd_owner_kernel<T, kMine, kWords, kLayout, kSingle>, grid, dim3(kOwnerThreads), 0, st,
+                       static_cast<const T*>(updates), static_cast<T*>(data), indices, numbers, n, k, slice, total, lanes, bits,
+                       chunk);
 }
 
 template <typename T, Layout kLayout, bool kAnyMemory>
@@ -616,10 +612,8 @@ int launch_direct(const void* updates, void* data, const long long* indices, con
   const int per = kScatterThreads / lanes;
   const dim3 grid((unsigned)std::min<long long>((n + per - 1) / per, 1 << 20),
                   (unsigned)std::min<long long>((words + lanes - 1) / lanes, 1024));
-  hipLaunchKernelGGL((scatter_nd_direct_kernel<T, kLayout, kAnyMemory>), grid, dim3(kScatterThreads), 0, st,
-                     static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(scatter_nd_direct_kernel<T, kLayout, kAnyMemory>, grid, dim3(kScatterThreads), 0, st,
+                       static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
 }
 
 // Hardware floating-point atomics are defined for ordinary (coarse-grained) memory of the device that runs the kernel:

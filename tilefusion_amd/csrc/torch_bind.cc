@@ -10,6 +10,9 @@
 // from the right axes for non-square problems, launches go to the current stream instead of
 // the null stream, and errors surface as c10::Error (RuntimeError) instead of exit().
 #include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
@@ -44,6 +47,15 @@ namespace tilefusion {
 namespace {
 
 void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+// Device memory for the length of a call, on the device of `like`: from the allocator that tensors take theirs from, ordered as theirs is
+// by the current stream, without the tensor around it (0.2 us of the calling thread instead of 0.7).
+c10::DataPtr scratch(size_t bytes, const at::Tensor& like) {
+  c10::Allocator* const from = c10::hip::HIPCachingAllocator::get();
+  if (like.get_device() == c10::hip::current_device()) return from->allocate(bytes);
+  const c10::DeviceGuard there(like.device());
+  return from->allocate(bytes);
+}
 
 void check_status(int status, const char* op) {
   TORCH_CHECK(status == TF_OK, "tilefusion::", op, " failed (status ", status, "): ", tf_last_error());
@@ -123,9 +135,9 @@ TILEFUSION_EXPORT void fused_two_gemms(const at::Tensor& A, const at::Tensor& B,
               "batch dimensions must match.");
   // long-N problems are cut along N when the library is handed a workspace for the partial sums
   const size_t ws_bytes = tf_fused_two_gemms_workspace_bytes(dtype, batch, m, n, k, p);
-  at::Tensor ws;
-  if (ws_bytes > 0) ws = at::empty({(int64_t)ws_bytes}, A.options().dtype(at::kByte));
-  void* ws_ptr = ws_bytes > 0 ? ws.data_ptr() : nullptr;
+  c10::DataPtr ws;
+  if (ws_bytes > 0) ws = scratch(ws_bytes, A);
+  void* ws_ptr = ws.get();
   // The plain kernels reduce 32 values of k (and of n, in the second product) per MFMA and write 16
   // columns per base tile.  Shapes the reference accepts with 16-wide base tiles (K or N = 48,
   // ...) run the streaming kernel where K and P are narrow and all are multiples of 8, and are zero-padded here
@@ -193,9 +205,9 @@ void attention_impl(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& 
   if (!causal && !v_transposed && d == dv && (!k_transposed || (lkv % 8 == 0 && (d == 64 || d == 96 || d == 128)))) {
     const int64_t bytes = tf_flash_attention_split_workspace(batch, lq, lkv, d);
     if (bytes > 0) {
-      const at::Tensor room = at::empty({bytes}, Q.options().dtype(at::kByte));
+      const c10::DataPtr room = scratch((size_t)bytes, Q);
       const int status = tf_flash_attention_fwd_split(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dtype, batch, lq,
-                                                      lkv, d, k_transposed ? 1 : 0, softmax_scale, room.data_ptr(),
+                                                      lkv, d, k_transposed ? 1 : 0, softmax_scale, room.get(),
                                                       current_stream());
       if (status != TF_ERR_UNSUPPORTED) {
         check_status(status, op);
@@ -337,11 +349,14 @@ void flash_decode(const at::Tensor& Q, const at::Tensor& K, const at::Tensor& V,
   TORCH_CHECK(Q.numel() == bh * d && O.numel() == bh * d,
               "flash_decode: Q and O must hold one row of D per (batch, head).");
   TORCH_CHECK(num_splits > 0, "flash_decode: num_splits must be positive.");
+  const int status = tf_flash_decode_uncut(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dtype, bh, lkv, d,
+                                           (int)num_splits, softmax_scale, current_stream());
+  if (status == TF_OK) return;
   // (256 bytes a slice more than the partials take: with them one kernel does it)
   const size_t bytes = tf_flash_decode_workspace_bytes(bh, d, (int)num_splits) + 256 * (size_t)bh;
-  at::Tensor ws = at::empty({(int64_t)((bytes + 3) / 4)}, Q.options().dtype(at::kFloat));
+  const c10::DataPtr ws = scratch(bytes, Q);
   check_status(tf_flash_decode(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dtype,
-                               ws.data_ptr(), bytes, bh, lkv, d, (int)num_splits, softmax_scale,
+                               ws.get(), bytes, bh, lkv, d, (int)num_splits, softmax_scale,
                                current_stream()),
                "flash_decode");
 }

@@ -73,8 +73,6 @@ extern "C" int tf_transpose_16bit(const void* in, void* out, int64_t batch, int6
   TFK_REQUIRE(reinterpret_cast<uintptr_t>(in) % 2 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0, TF_ERR_INVALID_ARG,
               "tf_transpose_16bit: out must start at a 16-byte boundary");
   const dim3 grid((unsigned)((cols + kTile - 1) / kTile), (unsigned)((rows + kTile - 1) / kTile), (unsigned)batch);
-  hipLaunchKernelGGL(transpose_kernel, grid, dim3(kTransposeThreads), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const unsigned short*>(in), static_cast<unsigned short*>(out), (int)rows, (int)cols);
-  TFK_HIP_TRY(hipGetLastError());
-  return TF_OK;
+  return launch_kernel(transpose_kernel, grid, dim3(kTransposeThreads), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const unsigned short*>(in), static_cast<unsigned short*>(out), (int)rows, (int)cols);
 }
