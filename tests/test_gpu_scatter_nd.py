@@ -101,6 +101,26 @@ def test_scatter_nd_owners_of_targets(dtype, dims, depth, n, start):
     assert not one[[0, 2]].any()
 
 
+# Wide slices, a word a lane: chunks of 2048 and 4096 updates, up to and beyond the updates, words and workgroups where one takes over.
+# Sums of integers: at most ~1450 updates a target, none or one each way, keep every partial sum below 256 (8 deviations), which all types hold.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("rows,slice_,n", [(900, 1026, 4097), (900, 1024, 8193), (900, 514, 4097), (300, 4226, 4500), (200, 1154, 19999),
+                                           (5000, 1030, 4096)])
+def test_scatter_nd_chunks_of_wide_slices(dtype, rows, slice_, n):
+    from tilefusion_amd.ops import scatter_nd
+    g = torch.Generator().manual_seed(rows + n)
+    data = torch.randint(-2, 3, (rows, slice_), generator=g).to(dtype)
+    idx = (rows * torch.rand(n, generator=g) ** 2).long()
+    idx[5], idx[n - 1] = -1, rows                                 # skipped
+    keep = (idx >= 0) & (idx < rows)
+    upd = torch.randint(-1, 2, (n, slice_), generator=g).to(dtype)
+    want = data.float().index_add(0, idx[keep], upd[keep].float())
+    assert want.abs().max() <= 256
+    dev = data.to(DEV)
+    scatter_nd(dev, idx.unsqueeze(1).to(DEV), upd.to(DEV))
+    assert torch.equal(dev.cpu().float(), want)
+
+
 # Targets with a large part of a chunk's updates: half of them to one row, an eighth to a second and a thirtieth to a third, in
 # chunks of 1024, 2048 and 4096 updates, one and two words a lane, unpaired halves, slices of one element.  All workgroups of a
 # chunk have to agree on who adds what: every update once.

@@ -299,10 +299,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_sgpr(80))) void
 //
 // What bounds it: the atomics where there are many; below ~4 MB the chain of loading indices, sorting (five barriers,
 // an LDS atomic per update in every workgroup), loading updates and the atomics, ~6 us.  us, log-uniform indices, sorted
-// 64 or 128 as they come / hash owners / as here: 8192 bf16 of 1024 into 32000 rows 20.8 / 16.8 / 17.3, 65536 of 1000 into
+// 64 or 128 as they come / hash owners / as here: 8192 bf16 of 1024 into 32000 rows 20.8 / 16.8 / 14.9, 65536 of 1000 into
 // 131072 187 / 90 / 96, 16384 of 4096 into 20000 158 / 74 / 69, 60000 of 40 into 131072 35.9 / 26.6 / 12.8, 49954 fp32 of 622
-// into 77 154 / 60 / 44; all indices distinct: 8192 of 1024 20.1 / 22.5 / 20.6, 32768 fp16 of 512 32.9 / 39.7 / 35.4; half
-// of them one row: 8192 of 1024 20.5 / 34.5 / 21.2, 60000 of 40 23.2 / 74.9 / 18.6; all: 18.7 / 50.3 / 12.2, 25.4 / 136 / 15.7.
+// into 77 154 / 60 / 44; all indices distinct: 8192 of 1024 20.1 / 22.5 / 21.1, 32768 fp16 of 512 32.9 / 39.7 / 35.4; half
+// of them one row: 8192 of 1024 20.5 / 34.5 / 18.2, 60000 of 40 23.2 / 74.9 / 18.6; all: 18.7 / 50.3 / 13.1, 25.4 / 136 / 15.7.
 // Two targets of one slot may lie mixed, which costs them more atomics and nothing else.  kSingle: 16-bit slices of one element.
 constexpr int kOwnerThreads = 1024;
 template <typename T, int kMine, int kWords, Layout kLayout, bool kSingle>
@@ -589,16 +589,26 @@ int launch_shape(const void* updates, void* data, const long long* indices, cons
 // 4096 and two words a lane, which have the most loads to wait for: us, one / two, 20837 fp32 of 2166 into 901 rows 75 / 59, 62413 of 994
 // into 1447 98 / 82, 27577 fp16 of 1990 into 35292 (uniform) 118 / 116; not beyond 512, which the chip does not hold at once (528: 22339 fp16 of 2710
 // 83 / 99), nor with shorter chunks (0-12% behind).
+struct OwnerGrid {
+  long long chunks, columns;
+  int bits;   // of the shares of a chunk
+};
+OwnerGrid owner_grid(long long n, long long words, int lanes, int mine, int per_lane) {
+  OwnerGrid g;
+  g.chunks = (n + mine * kOwnerThreads - 1) / (mine * kOwnerThreads);
+  g.columns = (words + lanes * per_lane - 1) / (lanes * per_lane);
+  g.bits = 1;
+  while (g.bits < 8 && g.chunks * g.columns * 3 << g.bits <= 2 * 224) ++g.bits;
+  if (mine == 4 && per_lane == 2 && g.bits < 8 && g.chunks * g.columns << g.bits <= 256) ++g.bits;
+  return g;
+}
+
 template <typename T, int kMine, int kWords, Layout kLayout, bool kSingle>
 int launch_owner(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
                  long long slice, long long total, int lanes, long long words, hipStream_t st) {
   Strides numbers = s;
   for (int d = 0; d < k; ++d) numbers.stride[d] /= slice;   // the number of a target, not its first element
-  const long long chunks = (n + kMine * kOwnerThreads - 1) / (kMine * kOwnerThreads);
-  const long long columns = (words + lanes * kWords - 1) / (lanes * kWords);
-  int bits = 1;
-  while (bits < 8 && chunks * columns * 3 << bits <= 2 * 224) ++bits;
-  if (kMine == 4 && kWords == 2 && bits < 8 && chunks * columns << bits <= 256) ++bits;
+  const auto [chunks, columns, bits] = owner_grid(n, words, lanes, kMine, kWords);
   const int chunk = (int)((n + chunks - 1) / chunks);   // (even ones: no nearly empty last chunk)
   const dim3 grid((unsigned)((n + chunk - 1) / chunk) << bits, (unsigned)columns);
   return launch_kernel(scatter_nd_owner_kernel<T, kMine, kWords, kLayout, kSingle>, grid, dim3(kOwnerThreads), 0, st,
@@ -654,10 +664,12 @@ int launch_rows(const void* updates, void* data, const long long* indices, const
   }
   // Longer chunks find more to merge, shorter ones are sorted sooner, in every workgroup.  4096 updates instead of 2048 from
   // 20000 on (40000 bf16 of 1000 into 131072 rows 80 and 67, distinct indices 83 and 85; 8192 a chunk 69 and 88), 1024 where there are
-  // few (4096 fp32 of 64 into 8000 rows 7.7 and 7.1).  Two words a lane halve the workgroups that sort the same indices, from 256 words
-  // on, except with up to 4096 updates, where a word a lane and 2048 a chunk are 7% ahead of two and 1024 over 28 problems
-  // (2295 bf16 of 2824 into 5389 rows 14.5 and 13.3, 2140 fp32 of 366 into 214 (uniform) 8.8 and 6.4, 3873 fp16 of 1048 into 2024 12.6
-  // and 13.3; sorted indices of 40 rows are 14% behind).
+  // few (4096 fp32 of 64 into 8000 rows 7.7 and 7.1).  Two words a lane halve the workgroups that sort the same indices, but one
+  // wavefront then waits for twice the loads and atomics: from 20000 updates of more than 256 words on only (31652 fp32 of 2113
+  // into 46286 rows 168 and, a word a lane, 185; 47403 bf16 of 730 into 5971 52.5 and 53.0).  Below, a word a lane and 2048 a
+  // chunk are 10% ahead of two over 48 problems (8192 bf16 of 1024 into 32000 18.2 and 14.9; distinct indices 20.7 and 21.1).  With more than 512 words, where the columns alone
+  // nearly fill the chip, 4096 a chunk find more to merge (9573 fp16 of 1572 into 19695 29.7, 30.3 and 28.8, 5997 fp32 of 835 into 251
+  // 18.4, 18.4 and 15.0), unless that leaves a second workgroup to some CUs (9187 fp32 of 2929 into 4762 63, 60 and 74).
   auto owners = [&](auto mine, auto per_lane, auto single) -> int {
     return launch_owner<T, decltype(mine)::value, decltype(per_lane)::value, kLayout, decltype(single)::value>(
         updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
@@ -669,7 +681,9 @@ int launch_rows(const void* updates, void* data, const long long* indices, const
     using Many = std::false_type;
     if (words > 256) {
       if (n >= 20000) return owners(Four{}, Two{}, Many{});
-      return n <= 4096 ? owners(Two{}, One{}, Many{}) : owners(Two{}, Two{}, Many{});
+      const OwnerGrid g = owner_grid(n, words, lanes, 4, 1);
+      const bool longer = n > 4096 && words > 512 && g.chunks * g.columns << g.bits <= 256;
+      return longer ? owners(Four{}, One{}, Many{}) : owners(Two{}, One{}, Many{});
     }
     if (n >= 20000) return owners(Four{}, One{}, Many{});
     return n <= 8192 ? owners(One{}, One{}, Many{}) : owners(Two{}, One{}, Many{});
