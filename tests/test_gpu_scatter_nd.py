@@ -101,11 +101,11 @@ def test_scatter_nd_owners_of_targets(dtype, dims, depth, n, start):
     assert not one[[0, 2]].any()
 
 
-# Wide slices, a word a lane: chunks of 2048 and 4096 updates, up to and beyond the updates, words and workgroups where one takes over.
+# Wide slices, a word a lane: chunks of 1024, 2048 and 4096 updates, up to and beyond the updates, words and workgroups where one takes over.
 # Sums of integers: at most ~1450 updates a target, none or one each way, keep every partial sum below 256 (8 deviations), which all types hold.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=lambda d: str(d).split(".")[-1])
 @pytest.mark.parametrize("rows,slice_,n", [(900, 1026, 4097), (900, 1024, 8193), (900, 514, 4097), (300, 4226, 4500), (200, 1154, 19999),
-                                           (5000, 1030, 4096)])
+                                           (5000, 1030, 4096), (900, 4226, 400), (900, 6148, 1023), (300, 3090, 1025), (300, 1030, 1281), (900, 514, 2048)])
 def test_scatter_nd_chunks_of_wide_slices(dtype, rows, slice_, n):
     from tilefusion_amd.ops import scatter_nd
     g = torch.Generator().manual_seed(rows + n)

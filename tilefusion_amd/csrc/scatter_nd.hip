@@ -645,13 +645,20 @@ int launch_rows(const void* updates, void* data, const long long* indices, const
     return launch_direct<T, kLayout, true>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   // Times in us with log-uniform indices.  Few updates: no sort (806 of 34 fp32: direct 3.3, 16 of 256 threads' updates
   // sorted 5.6).  From 1024 on contention shows (2048 of 64 bf16 into 64 rows: direct 10.8, sorted 6.3).
-  if (n <= 1024)
-    return launch_direct<T, kLayout, false>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  // Beyond, chunks sorted whole, except: a few 16-bit updates (1489 of 1206 bf16 into 1412 rows: 9.4 sorted by 16, 10.4 by
-  // the chunk; 1894 of 3924 21.8 and 14.6; 1077 fp32 of 26 into 95 5.6 and 6.1, 1469 of 68 into 350 8.1 and 6.9), and what its target
-  // numbers (32 bits) and columns do not hold: 2100 bf16 of 140000 into 300 rows 364 sorted by 64, 527 by 128, all to one row 591 and 2010.
+  // What the target numbers (32 bits) and columns of sorted chunks do not hold: 2100 bf16 of 140000 into 300 rows 364 sorted by 64, 527 by
+  // 128, all to one row 591 and 2010.
   const bool chunks_fit = targets < (1ll << 32) && n < (1ll << 31) && words <= 1024ll * lanes;
-  if ((n <= 2048 && ((sizeof(T) == 2 && n * words < 2 << 20) || !chunks_fit)) || n <= 1280)
+  // Few but wide updates: a chunk of all of them from 1.5 Mi words on, where the atomics are what counts (530 fp16 of 5710 into 39558 rows 10.1
+  // direct and 10.9, 480 of 5668 into 4345 9.9 and 8.7, 598 fp32 of 5672 into 257 19.9 and 12.7, 1242 of 3610 into 1022 25.5 by 16 and 14.9;
+  // uniform indices, which merge less, 882 fp16 of 7196 into 12239 16.7 and 18.1, 884 fp32 of 7770 into 464 32.7 and 20.2), and of 16-bit
+  // ones more than 1280 in any case (1404 of 1228 into 2501 8.8 and 7.7, 1556 of 2002 into 253 11.4 and 8.3; uniform, 1527 of 1914 into 39055
+  // 10.5 and 11.7).
+  const bool wide = kLayout == Layout::kPairs && chunks_fit && words > 256 && (n > 1280 || n * words >= 3 << 19);
+  if (!wide && n <= 1024)
+    return launch_direct<T, kLayout, false>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+  // Beyond, chunks sorted whole, except a few 16-bit updates: 1894 of 3924 21.8 sorted by 16, 14.6 by the chunk; 1077 fp32 of 26 into 95 5.6 and
+  // 6.1, 1469 of 68 into 350 8.1 and 6.9.
+  if (!wide && ((n <= 2048 && ((sizeof(T) == 2 && n * words < 2 << 20) || !chunks_fit)) || n <= 1280))
     return launch_shape<T, 256, 16, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   if (!chunks_fit) {
     // Every target hit at least eight times on average: the deeper sort.  A workgroup of eight wavefronts hides its own
@@ -681,6 +688,8 @@ int launch_rows(const void* updates, void* data, const long long* indices, const
     using Many = std::false_type;
     if (words > 256) {
       if (n >= 20000) return owners(Four{}, Two{}, Many{});
+      // (one chunk, or two of up to 1024 that are sorted sooner: 1872 bf16 of 840 into 856 8.0 and, in one, 9.5, 1556 fp16 of 2002 8.3 and 10.3)
+      if (n <= 1024 || (n > 1280 && n <= 2048 && sizeof(T) == 2 && n * words < 2 << 20)) return owners(One{}, One{}, Many{});
       const OwnerGrid g = owner_grid(n, words, lanes, 4, 1);
       const bool longer = n > 4096 && words > 512 && g.chunks * g.columns << g.bits <= 256;
       return longer ? owners(Four{}, One{}, Many{}) : owners(Two{}, One{}, Many{});
