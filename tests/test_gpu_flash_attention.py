@@ -418,3 +418,17 @@ def test_head_dimension_96_never_reads_the_padding_of_its_lds_rows():
             o = c_attention(q.to(DEV), k.to(DEV), vd.to(DEV), causal, None, vt)
             ok, r, m = N.check_close(o, N.attention_ref(q, k, v, causal=causal))
             assert ok, f"causal={causal} vt={vt}: rel_l2={r:.3e} max_abs={m:.3e}"
+
+
+# Causal tiles end where the queries end: every workgroup size, with queries that fill the first tile but for one wavefront, by one
+# row, by a key tile and not at all.  The rows are those of a call with as many queries as keys, bit for bit: only who computes them differs.
+@pytest.mark.parametrize("rows,b,d", [(64, 3, 64), (64, 3, 128), (128, 130, 64), (256, 300, 128)])
+@pytest.mark.parametrize("cut", [0, 1, 63, 64, 127, 129, 191, 192, 255])
+def test_causal_tiles_end_with_the_queries(rows, b, d, cut):
+    assert cut > 127 or _capi.load().tf_flash_attention_rows(b, 512 - cut, 512, d, 1) == rows
+    q, k, v = (x.to(DEV) for x in _inputs(b, 512, 512, d, rows + d + cut))
+    lq = 512 - cut
+    o = c_attention(q[:, :lq].contiguous(), k, v, True)
+    assert torch.equal(o, c_attention(q, k, v, True)[:, :lq])
+    ok, r, m = N.check_close(o[-1:].cpu(), N.attention_ref(q[-1:, :lq].cpu(), k[-1:].cpu(), v[-1:].cpu(), causal=True))
+    assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"

@@ -292,7 +292,13 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
 
   for (int pass = 0; pass < num_passes; ++pass) {
   const int qt = qt_of_pass[pass];
-  const int q_row0 = qt * kBMq + wave * kRowsPerWave;  // first query row of this wavefront
+  // Causal tiles end where the queries end (up to a multiple of 64), so that the one that is not full is the lightest instead of the
+  // heaviest: up to a tile's keys less for every slice.  (64 slices of 1337 x 1337 x 64 27.0 / 25.8 us, 66 of 1560 x 128 71 / 61, 114 of 704 x
+  // 128 36.0 / 32.6.  Ends at multiples of 16 leave more to the lightest, but then wavefronts of one set meet their masked tiles
+  // at different times: 9 of 1364 x 64, which one workgroup's chain bounds, 14.8 / 15.5.)  The same rows share a wavefront
+  // either way, and their results are the same bits.
+  const int tile_row0 = kCausal ? (Lq + 63) / 64 * 64 - (q_tiles - qt) * kBMq : qt * kBMq;
+  const int q_row0 = tile_row0 + wave * kRowsPerWave;  // first query row of this wavefront
   // this lane's query rows: block qb holds row q_row0 + 16*qb + lr
 
   // The softmax scale (times log2 e) is folded into Q once: Q' = fp16(Q * scale_log2), so the
@@ -303,7 +309,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   V8 qf[kKK][kQB];
 #pragma unroll
   for (int qb = 0; qb < kQB; ++qb) {
-    const int m_ld = min(q_row0 + 16 * qb + lr, Lq - 1);
+    const int m = q_row0 + 16 * qb + lr, m_ld = kCausal ? (int)min((unsigned)m, (unsigned)Lq - 1u) : min(m, Lq - 1);   // (causal: m < 0, too)
 #pragma unroll
     for (int kk = 0; kk < kKK; ++kk) {
       const int col = kk * 32 + lg * 8;
@@ -319,7 +325,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   }
 
   int n_end = Lkv;
-  if (kCausal) n_end = min(Lkv, qt * kBMq + kBMq);
+  if (kCausal) n_end = min(Lkv, tile_row0 + kBMq);
   const int num_tiles = (n_end + kBN - 1) / kBN;
 
   // ---- global -> LDS plan: wavefront instruction i of a tile covers 1 KiB of it ------------
@@ -748,6 +754,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   if (kCausal) {
     n_plain = max(0, min(n_plain, (q_row0 + 1) / kBN));
     n_compute = min(num_tiles, (q_row0 + kRowsPerWave - 1) / kBN + 1);
+    if ((unsigned)q_row0 >= (unsigned)Lq) n_plain = n_compute = 0;   // (all rows in front of the first query or behind the last)
   }
   const int n_fast = min(num_tiles, Lkv / kBN);  // whole tiles of this pass (lean request form)
   if constexpr (kWavesT == 8) {
@@ -896,7 +903,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
         v[1] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)x[1]);
         v[2] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)y[0]);
         v[3] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)y[1]);
-        if (m_row < Lq && (!kTail || 16 * db + 8 * st_seg < dv_row)) *reinterpret_cast<uint4_t*>(o_lane + 16 * db) = v;
+        if (m_row < Lq && (!kCausal || m_row >= 0) && (!kTail || 16 * db + 8 * st_seg < dv_row)) *reinterpret_cast<uint4_t*>(o_lane + 16 * db) = v;
       }
     }
   }
