@@ -432,3 +432,19 @@ def test_causal_tiles_end_with_the_queries(rows, b, d, cut):
     assert torch.equal(o, c_attention(q, k, v, True)[:, :lq])
     ok, r, m = N.check_close(o[-1:].cpu(), N.attention_ref(q[-1:, :lq].cpu(), k[-1:].cpu(), v[-1:].cpu(), causal=True))
     assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
+
+
+# Single causal tiles, two to a CU, the second 256 of them in the opposite order by eights: workgroups below, at and beyond the ends of
+# that range (three tiles of 128 queries a slice), every tile once.
+@pytest.mark.parametrize("bh", [85, 86, 88, 90, 170, 171, 192, 193])
+@pytest.mark.parametrize("d", [64, 56])
+def test_causal_second_round_of_workgroups(bh, d):
+    q, k, v = (x.to(DEV) for x in _inputs(bh, 384, 384, d, bh + d))
+    o = torch.full_like(q, float("nan"))
+    torch.ops.tilefusion.flash_attention_fwd(q, k, v, o, d ** -0.5, True)
+    for i in range(0, bh, 3):
+        alone = torch.empty_like(o[i:i + 1])
+        torch.ops.tilefusion.flash_attention_fwd(q[i:i + 1].contiguous(), k[i:i + 1].contiguous(), v[i:i + 1].contiguous(), alone,
+                                                 d ** -0.5, True)
+        assert torch.equal(o[i:i + 1], alone), i
+    assert not torch.isnan(o).any()

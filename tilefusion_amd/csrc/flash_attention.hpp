@@ -63,6 +63,10 @@ __host__ __device__ constexpr int swz_kt(int row, int c) {
   return c ^ ((((row >> 1) & 1) | ((row >> 2) & 2)) << 1);
 }
 
+// Workgroups of this kernel share a CU in pairs (its LDS and registers hold two).
+__host__ __device__ constexpr bool two_on_cu(int waves, int qb, int D, bool kt) {
+  return ring_stages(waves, D) == 2 || (D == 64 && (waves == 4 || (qb == 1 && !kt)));
+}
 // What a workgroup's number stands for (causal; see the kernel).
 enum : int { kSingle = 0, kPairs = 1, kByXcd = 2, kFolded = 3 };
 constexpr int kCUs = 256;
@@ -191,6 +195,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   constexpr int kBN = key_tile(D);
   constexpr int kStages = ring_stages(kWavesT, D);
   constexpr bool kPairOnCU = kStages == 2;
+  constexpr bool kTwoOnCU = two_on_cu(kWavesT, kQB, D, kKT);
   constexpr int kRowsPerWave = 16 * kQB;  // kQB 16-query blocks per wavefront
   constexpr int kBMq = kWavesT * kRowsPerWave;
   constexpr int DP = lds_pitch(D), DVP = lds_pitch(DV);   // LDS row pitch of the K / natural V tile
@@ -230,9 +235,11 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   //               order (with its L2 locality) is kept.  Where that is done sooner (the
   //               caller tells) and with an odd number of query tiles, one tile per workgroup,
   //               heaviest first over all slices (kSingle) or over those of an XCD (kByXcd).
-  //               Where all of them are on the chip at once, two to a CU (the p-th and the (p + 256)-th, by a probe), the second
-  //               half comes lightest first (kFolded), or the heaviest would share their CUs with ones half as heavy and all
-  //               others wait: 32 slices of 1024 x 1024 x 256 37.2 / 35.9 us, 18 of 1600 51.1 / 48.2, 9 of 3584 x 160 78 / 75.
+  //               Where two share a CU (the p-th and the (p + 256)-th, by a probe) and few are left for a third, the second 256 come
+  //               lightest first (kFolded), or the heaviest would share their CUs with ones half as heavy and all others
+  //               wait: 32 slices of 1024 x 1024 x 256 37.2 / 35.9 us, 18 of 1600 51.1 / 48.2, 9 of 3584 x 160 78 / 75, 33 of 2048 x 64 33.1 /
+  //               30.2, 28 of 2176 x 64 29.7 / 27.8; 77 of D = 64 with 257 to 576 workgroups 0.985. With more than 576 those of the
+  //               third round find the light CUs by themselves.
   int qt_of_pass[2] = {0, 0};
   int num_passes = 1;
   size_t bh;
@@ -264,18 +271,15 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
       qt_of_pass[0] = q_tiles - 1 - p / own;
       bh = xcd + 8 * (p % own);
     } else {
-      const int i = (int)blockIdx.x;
+      int i = (int)blockIdx.x;
       if (i >= total_items) return;
+      if constexpr (kTwoOnCU) {
+        // the second 256 in the opposite order (by eights: a slice's stay on one XCD)
+        const int j = i - kCUs, count = min(total_items - kCUs, kCUs) & ~7;
+        if (order == kFolded && (unsigned)j < (unsigned)count) i = kCUs + (count - 8) - (j & ~7) + (j & 7);
+      }
       qt_of_pass[0] = q_tiles - 1 - i / slices;
       bh = i % slices;
-      if constexpr (kPairOnCU) {
-        if (order == kFolded && i >= kCUs) {
-          // second on their CUs: lightest first
-          const int level = (i - kCUs) / slices;
-          qt_of_pass[0] = level;
-          bh = (i - kCUs) % slices + (level == q_tiles - 1 - kCUs / slices ? kCUs % slices : 0);
-        }
-      }
     }
   }
   Q += bh * (size_t)Lq * d_row;
@@ -966,7 +970,7 @@ int launch_w(const AttentionCall& c) {
   // that leaves the XCDs within 4% of each other (bf16, 150 slices of 384 x 384 x 256: 39.4 / 31.4 us).
   const int per_xcd = (c.batch + 7) / 8;
   const bool by_xcd = kCausal && !paired && c.batch % 8 != 0 && 8 * per_xcd * 100 <= c.batch * 104;
-  const bool folded = kCausal && ring_stages(kWavesT, D) == 2 && !paired && !by_xcd && total_items > kCUs && total_items <= 2 * kCUs;
+  const bool folded = kCausal && two_on_cu(kWavesT, kQB, D, kKT) && !paired && !by_xcd && total_items > kCUs && total_items <= (D == 64 ? kCUs * 9 / 4 : 2 * kCUs);
   const dim3 grid(by_xcd ? 8 * per_xcd * q_tiles : 8 * ((total_items + 7) / 8));
   return launch_kernel(kern, grid, dim3(kWavesT * 64), lds, c.stream,
                        static_cast<const T*>(c.Q), static_cast<const T*>(c.K),
