@@ -204,6 +204,18 @@ def test_rows_that_start_anywhere_in_a_line(kernel, m, n, k, start):
     assert torch.equal(c_gemm(a, b, torch.float32), a.float() @ b.float().t())   # exact: |sum| <= 4 k < 2^24
 
 
+# ... and the tile of 160 rows that takes the place of the pick where that leaves CUs idle or begins another round: an odd number
+# of requests a wavefront and operand.
+BETWEEN = [(3657, 1390, 328), (1895, 2281, 968), (1596, 2453, 464), (1661, 2930, 344), (2975, 1423, 984), (2642, 1847, 480),
+           (2660, 1629, 360), (2501, 1657, 1000), (2315, 2084, 496), (1726, 2728, 376), (2643, 1708, 1016)]
+
+
+@pytest.mark.parametrize("m,n,k", BETWEEN)
+@pytest.mark.parametrize("start", [0, 8, 40])
+def test_tile_of_160_rows(m, n, k, start):
+    test_rows_that_start_anywhere_in_a_line(10, m, n, k, start)
+
+
 def test_operands_without_16_byte_alignment():
     g = torch.Generator().manual_seed(5)
     a, b = (torch.randint(-2, 3, (1 + r * 264,), generator=g).half().to(DEV)[1:].view(r, 264) for r in (200, 150))

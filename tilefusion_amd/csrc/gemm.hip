@@ -178,7 +178,7 @@ struct Ring64Shape {
     }
     return true;
   }
-  static_assert(BM % 64 == 0 && BN % 64 == 0, "whole MFMA tile pairs; even request counts (see the swizzle of g_off)");
+  static_assert(BM % (kLines ? 32 : 64) == 0 && BN % 64 == 0, "whole MFMA tile pairs; even request counts (see the swizzle of g_off)");
   static_assert(reads_fit() && free_gaps() >= 7,
                 "slot schedule: every read and bookkeeping piece needs its own gap");
   // requests in flight behind the barrier in the middle of a tile: A of tile t+kAhead, all of the
@@ -241,20 +241,22 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
   const char* b_tile = reinterpret_cast<const char*>(B + (size_t)(n0 + wave * 8 * S::kLoadsB) * K) - (kShift ? kLead : 2 * k_pad);
   unsigned g_off[S::kLoadsMax];
   unsigned g_off_b[kShift ? S::kLoadsB : 1];
+  // (an odd number of requests: every other wavefront's rows begin in the middle of the swizzle's sixteen)
+  const int a_odd = S::kLoadsA % 2 ? wave & 1 : 0;
   // the chunk of a segment that this lane fetches with request n
   auto segment_chunk = [&](int n, int shift) __attribute__((always_inline)) { return (S::swizzle(ld_row + 8 * n, ld_c) + shift) & 7; };
-  auto segment_off = [&](int n, int shift) __attribute__((always_inline)) {
-    return (unsigned)(ld_row + 8 * n) * (unsigned)K * 2u + (unsigned)(kLead + 16 * (segment_chunk(n, shift) - shift - pad_chunks)) -
+  auto segment_off = [&](int n, int odd, int shift) __attribute__((always_inline)) {
+    return (unsigned)(ld_row + 8 * n) * (unsigned)K * 2u + (unsigned)(kLead + 16 * (segment_chunk(n + odd, shift) - shift - pad_chunks)) -
            1024u * (n % 4);
   };
 #pragma unroll
   for (int n = 0; n < S::kLoadsMax; ++n)
-    g_off[n] = kShift ? segment_off(n, a_shift)
+    g_off[n] = kShift ? segment_off(n, a_odd, a_shift)
                       : (unsigned)(ld_row + 8 * n) * (unsigned)K * 2u + (unsigned)S::swizzle(ld_row + 8 * n, ld_c) * 16u -
                             1024u * (n % 4);   // the instruction's immediate offset (added to both addresses) gives it back
   if constexpr (kShift) {
 #pragma unroll
-    for (int n = 0; n < S::kLoadsB; ++n) g_off_b[n] = segment_off(n, b_shift);
+    for (int n = 0; n < S::kLoadsB; ++n) g_off_b[n] = segment_off(n, 0, b_shift);
   }
   // LDS -> fragment plan: fragment i of k-step ks: row 16*i + l%16 of the wavefront's rows,
   // logical chunk 4*ks + l/16
@@ -378,7 +380,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
         const char* tile = (of_a ? a_tile : b_tile) + u * (S::BK * 2);
         const unsigned unit = (of_a ? lds_wave_a : lds_wave_b + S::BM * S::kRowBytes) + u * S::kTileBytes;
         if (u < 2) {
-          const bool in_front = 8 * u + segment_chunk(n, shift) - shift < pad_chunks;
+          const bool in_front = 8 * u + segment_chunk(of_a ? n + a_odd : n, shift) - shift < pad_chunks;
           lds_dma_16B(in_front ? reinterpret_cast<const char*>(kZeros) : tile + (off + 1024u * (n % 4)), unit + n * 1024);
         } else {
           request_at(off, tile, unit, n);
@@ -444,7 +446,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
       // again). Requests from here on ask for no other segment.
       if (t + S::kLines == num_k_tiles) {
 #pragma unroll
-        for (int n = 0; n < S::kLoadsA; ++n) g_off[n] -= 16u * (unsigned)max(0, segment_chunk(n, a_shift) - (a_shift - 1));
+        for (int n = 0; n < S::kLoadsA; ++n) g_off[n] -= 16u * (unsigned)max(0, segment_chunk(n + a_odd, a_shift) - (a_shift - 1));
 #pragma unroll
         for (int n = 0; n < S::kLoadsB; ++n) g_off_b[n] -= 16u * (unsigned)max(0, segment_chunk(n, b_shift) - (b_shift - 1));
       }
@@ -964,6 +966,13 @@ constexpr LinesKernel kLinesKernels[] = {
     {12, 1.36f, 4.11f, 0.660f, 0.281f},
 };
 
+// A tile of 160 x 128 for whole lines, figures between those of 128 x 128 and 192 x 128, for grids that the one gives a second round and the
+// other leaves CUs idle on (2999 x 1544 x 1032: 208 tiles of 192 rows, 247 of 160). It takes the place of the pick where it is
+// expected to be done sooner: 50 such problems 5% faster (2% slower at most), us, the pick / it: 2999 x 1544 x 1032 17.9 / 16.4, 613 x
+// 7874 x 2040 26.1 / 22.9, 2547 x 1739 x 6712 63.5 / 59.1, fp32 result 66.6 / 61.0.
+constexpr LinesKernel kBetween = {10, 1.45f, 4.15f, 0.373f, 0.153f};
+constexpr int kBetweenRows = 160, kBetweenColumns = 128;
+
 float expected_us(const GemmKernel& g, int64_t tiles, int ktiles, bool unaligned_rows, const LinesKernel* lines) {
   const int64_t rounds = (tiles + 256 * g.per_cu - 1) / (256 * g.per_cu);
   const float unaligned = unaligned_rows ? g.unaligned : 0.f;
@@ -1047,6 +1056,19 @@ int pick_gemm_kernel(int M, int N, int K, bool c_is_f32) {
   return best;
 }
 
+// `pick` with whole lines, and kBetween ahead of it
+bool takes_between(int pick, int M, int N, int K) {
+  if (M < kBetweenRows || N < kBetweenColumns) return false;
+  const GemmKernel& g = kGemmKernels[pick];
+  const int ktiles = (K + 63) / 64;
+  auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  for (const LinesKernel& l : kLinesKernels)
+    if (l.index == pick)
+      return expected_us(kGemmKernels[kBetween.index], tiles(kBetweenRows, kBetweenColumns), ktiles, true, &kBetween) <
+             expected_us(g, tiles(g.bm, g.bn), ktiles, true, &l);
+  return false;
+}
+
 template <typename OutT, typename InT>
 int dispatch(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st) {
   using Launcher = int (*)(const void*, const void*, void*, int, int, int, hipStream_t);
@@ -1069,6 +1091,7 @@ int dispatch(const void* A, const void* B, void* C, int M, int N, int K, hipStre
     return kLaunchers[kNumGemmKernels](A, B, C, M, N, K, st);
   const int pick = pick_gemm_kernel(M, N, K, sizeof(OutT) == 4);
   if (takes_lines(K)) {   // (kLinesKernels)
+    if (takes_between(pick, M, N, K)) return launch_ring64<Ring64Shape<kBetweenRows, kBetweenColumns, 2, 4>, OutT, InT>(A, B, C, M, N, K, st);
     if (pick == 7) return launch_ring64<Ring64Shape<128, 128, 2, 5>, OutT, InT>(A, B, C, M, N, K, st);
     if (pick == 10) return launch_ring64<Ring64Shape<192, 128, 2, 4>, OutT, InT>(A, B, C, M, N, K, st);
     if (pick == 11) return launch_ring64<Ring64Shape<192, 192, 2, 3>, OutT, InT>(A, B, C, M, N, K, st);
