@@ -210,9 +210,18 @@ BETWEEN = [(3657, 1390, 328), (1895, 2281, 968), (1596, 2453, 464), (1661, 2930,
            (2660, 1629, 360), (2501, 1657, 1000), (2315, 2084, 496), (1726, 2728, 376), (2643, 1708, 1016)]
 
 
+
 @pytest.mark.parametrize("m,n,k", BETWEEN)
 @pytest.mark.parametrize("start", [0, 8, 40])
 def test_tile_of_160_rows(m, n, k, start):
+    test_rows_that_start_anywhere_in_a_line(10, m, n, k, start)
+
+
+# ... and with rows that start where lines do.
+@pytest.mark.parametrize("m,n,k", [(2466, 1722, 256), (3003, 1494, 256), (1541, 2582, 448), (861, 5283, 384), (3073, 1373, 1984),
+                                   (4224, 983, 256), (3182, 1397, 1152)])
+@pytest.mark.parametrize("start", [0, 8])
+def test_tile_of_160_rows_of_whole_lines(m, n, k, start):
     test_rows_that_start_anywhere_in_a_line(10, m, n, k, start)
 
 

@@ -178,7 +178,8 @@ struct Ring64Shape {
     }
     return true;
   }
-  static_assert(BM % (kLines ? 32 : 64) == 0 && BN % 64 == 0, "whole MFMA tile pairs; even request counts (see the swizzle of g_off)");
+  static_assert(BM % 32 == 0 && BN % 64 == 0, "whole MFMA tile pairs; an even request count of B (see the swizzle of g_off)");
+  static constexpr bool kOwnOffsetsB = kLines > 0 || kLoadsA % 2 != 0;   // requests of B do not lie as those of A
   static_assert(reads_fit() && free_gaps() >= 7,
                 "slot schedule: every read and bookkeeping piece needs its own gap");
   // requests in flight behind the barrier in the middle of a tile: A of tile t+kAhead, all of the
@@ -240,7 +241,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
   const char* a_tile = reinterpret_cast<const char*>(A + (size_t)(m0 + wave * 8 * S::kLoadsA) * K) - (kShift ? kLead : 2 * k_pad);
   const char* b_tile = reinterpret_cast<const char*>(B + (size_t)(n0 + wave * 8 * S::kLoadsB) * K) - (kShift ? kLead : 2 * k_pad);
   unsigned g_off[S::kLoadsMax];
-  unsigned g_off_b[kShift ? S::kLoadsB : 1];
+  unsigned g_off_b[S::kOwnOffsetsB ? S::kLoadsB : 1];
   // (an odd number of requests: every other wavefront's rows begin in the middle of the swizzle's sixteen)
   const int a_odd = S::kLoadsA % 2 ? wave & 1 : 0;
   // the chunk of a segment that this lane fetches with request n
@@ -249,14 +250,17 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
     return (unsigned)(ld_row + 8 * n) * (unsigned)K * 2u + (unsigned)(kLead + 16 * (segment_chunk(n + odd, shift) - shift - pad_chunks)) -
            1024u * (n % 4);
   };
+  auto tile_off = [&](int n, int odd) __attribute__((always_inline)) {
+    return (unsigned)(ld_row + 8 * n) * (unsigned)K * 2u + (unsigned)S::swizzle(ld_row + 8 * (n + odd), ld_c) * 16u -
+           1024u * (n % 4);   // the instruction's immediate offset (added to both addresses) gives it back
+  };
 #pragma unroll
   for (int n = 0; n < S::kLoadsMax; ++n)
     g_off[n] = kShift ? segment_off(n, a_odd, a_shift)
-                      : (unsigned)(ld_row + 8 * n) * (unsigned)K * 2u + (unsigned)S::swizzle(ld_row + 8 * n, ld_c) * 16u -
-                            1024u * (n % 4);   // the instruction's immediate offset (added to both addresses) gives it back
-  if constexpr (kShift) {
+                      : tile_off(n, a_odd);
+  if constexpr (S::kOwnOffsetsB) {
 #pragma unroll
-    for (int n = 0; n < S::kLoadsB; ++n) g_off_b[n] = segment_off(n, 0, b_shift);
+    for (int n = 0; n < S::kLoadsB; ++n) g_off_b[n] = kShift ? segment_off(n, 0, b_shift) : tile_off(n, 0);
   }
   // LDS -> fragment plan: fragment i of k-step ks: row 16*i + l%16 of the wavefront's rows,
   // logical chunk 4*ks + l/16
@@ -294,7 +298,10 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
                  : "v"(off), "s"(src), "n"(1024 * (n % 4)), "{m0}"(lds_unit + (n - n % 4) * 1024)
                  : "memory");
   };
-  auto request = [&](const char* src, unsigned lds_unit, int n) __attribute__((always_inline)) { request_at(g_off[n], src, lds_unit, n); };
+  auto request = [&](const char* src, unsigned lds_unit, int n, auto of_b) __attribute__((always_inline)) {
+    if constexpr (S::kOwnOffsetsB && decltype(of_b)::value) request_at(g_off_b[n], src, lds_unit, n);
+    else request_at(g_off[n], src, lds_unit, n);
+  };
   auto k_src = [&](const char* tile, int t) __attribute__((always_inline)) {
     return tile + (size_t)min(t, num_k_tiles - 1) * S::BK * 2;   // clamped past the end
   };
@@ -345,11 +352,11 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
     asm volatile("" ::: "memory");
   };
   // the requests of a k-step sit at the heads of its slots, evenly spread
-  auto request_slot = [&](int i, const char* src, unsigned lds_unit, auto loads_c) __attribute__((always_inline)) {
+  auto request_slot = [&](int i, const char* src, unsigned lds_unit, auto loads_c, auto of_b) __attribute__((always_inline)) {
     constexpr int kLoads = decltype(loads_c)::value;
 #pragma unroll
     for (int n = 0; n < kLoads; ++n)
-      if ((n * S::TM) / kLoads == i) request(src, lds_unit, n);
+      if ((n * S::TM) / kLoads == i) request(src, lds_unit, n, of_b);
   };
   constexpr std::integral_constant<int, S::kLoadsA> kOfA{};
   constexpr std::integral_constant<int, S::kLoadsB> kOfB{};
@@ -480,11 +487,12 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
         const char* tile = u % 2 ? b_tile : a_tile;
         const unsigned unit = (u % 2 ? lds_wave_b : lds_wave_a) + u * S::kUnitBytes;
         if (u < 2 && k_pad != 0) {
-          const bool in_front = S::swizzle(ld_row + 8 * n, ld_c) * 8 < k_pad;
-          const char* src = tile + (g_off[n] + 1024u * (n % 4));
+          const bool in_front = S::swizzle(ld_row + 8 * (u % 2 ? n : n + a_odd), ld_c) * 8 < k_pad;
+          const char* src = tile + ((S::kOwnOffsetsB && u % 2 ? g_off_b[n] : g_off[n]) + 1024u * (n % 4));
           lds_dma_16B(in_front ? reinterpret_cast<const char*>(kZeros) : src, unit + n * 1024);
         } else {
-          request(k_src(tile, u / 2), unit, n);
+          if (u % 2) request(k_src(tile, u / 2), unit, n, std::true_type{});
+          else request(k_src(tile, u / 2), unit, n, std::false_type{});
         }
       }
     wait_vmem<(S::kAhead - 1) * (S::kLoadsA + S::kLoadsB)>();
@@ -553,7 +561,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
 #pragma unroll
       for (int i = 0; i < S::TM; ++i) {
         __builtin_amdgcn_sched_barrier(0);
-        request_slot(i, src_a, req_a, kOfA);
+        request_slot(i, src_a, req_a, kOfA, std::false_type{});
         slot_pinned(0, i, rd_a1, rd_b1, [&](int j) __attribute__((always_inline)) {
           prep0(S::kPrep.piece[i * S::TN + j], t);
         });
@@ -563,7 +571,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring64_kernel(
 #pragma unroll
       for (int i = 0; i < S::TM; ++i) {
         __builtin_amdgcn_sched_barrier(0);
-        request_slot(i, src_b, req_b, kOfB);
+        request_slot(i, src_b, req_b, kOfB, std::true_type{});
         slot_pinned(1, i, rd_a0, rd_b0, [&](int j) __attribute__((always_inline)) {
           prep1(S::kPrep.piece[i * S::TN + j], t);
         });
@@ -966,12 +974,14 @@ constexpr LinesKernel kLinesKernels[] = {
     {12, 1.36f, 4.11f, 0.660f, 0.281f},
 };
 
-// A tile of 160 x 128 for whole lines, figures between those of 128 x 128 and 192 x 128, for grids that the one gives a second round and the
+// A tile of 160 x 128, figures between those of 128 x 128 and 192 x 128, for grids that the one gives a second round and the
 // other leaves CUs idle on (2999 x 1544 x 1032: 208 tiles of 192 rows, 247 of 160). It takes the place of the pick where it is
 // expected to be done sooner: 50 such problems 5% faster (2% slower at most), us, the pick / it: 2999 x 1544 x 1032 17.9 / 16.4, 613 x
-// 7874 x 2040 26.1 / 22.9, 2547 x 1739 x 6712 63.5 / 59.1, fp32 result 66.6 / 61.0.
-constexpr LinesKernel kBetween = {10, 1.45f, 4.15f, 0.373f, 0.153f};
+// 7874 x 2040 26.1 / 22.9, 2547 x 1739 x 6712 63.5 / 59.1, fp32 result 66.6 / 61.0. Of K a multiple of 64, from 256 on: 3.5% over 50 (3.5% slower at
+// most): 2466 x 1722 x 256 8.4 / 7.8, 1571 x 3014 x 3008 33.3 / 30.0, 587 x 7483 x 2496 28.3 / 25.8.
+constexpr LinesKernel kBetween = {-1, 1.45f, 4.15f, 0.373f, 0.153f};
 constexpr int kBetweenRows = 160, kBetweenColumns = 128;
+constexpr GemmKernel kBetweenWhole = {kBetweenRows, kBetweenColumns, 1, 1, true, 0.40f, 3.49f, 0.362f, 0.296f, 0.f};
 
 float expected_us(const GemmKernel& g, int64_t tiles, int ktiles, bool unaligned_rows, const LinesKernel* lines) {
   const int64_t rounds = (tiles + 256 * g.per_cu - 1) / (256 * g.per_cu);
@@ -1056,16 +1066,20 @@ int pick_gemm_kernel(int M, int N, int K, bool c_is_f32) {
   return best;
 }
 
-// `pick` with whole lines, and kBetween ahead of it
+// `pick` is a ring kernel with whole lines, or for K that is a multiple of 64, and the tile between is ahead of it
 bool takes_between(int pick, int M, int N, int K) {
   if (M < kBetweenRows || N < kBetweenColumns) return false;
-  const GemmKernel& g = kGemmKernels[pick];
+  const GemmKernel& g = kGemmKernels[pick % kNumGemmKernels];
   const int ktiles = (K + 63) / 64;
   auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  const int64_t between = tiles(kBetweenRows, kBetweenColumns);
+  if (K % 64 == 0)
+    return pick >= 7 && pick <= 12 && K >= 256 &&
+           expected_us(kBetweenWhole, between, ktiles, false, nullptr) < expected_us(g, tiles(g.bm, g.bn), ktiles, false, nullptr);
+  if (!takes_lines(K)) return false;
   for (const LinesKernel& l : kLinesKernels)
     if (l.index == pick)
-      return expected_us(kGemmKernels[kBetween.index], tiles(kBetweenRows, kBetweenColumns), ktiles, true, &kBetween) <
-             expected_us(g, tiles(g.bm, g.bn), ktiles, true, &l);
+      return expected_us(kBetweenWhole, between, ktiles, true, &kBetween) < expected_us(g, tiles(g.bm, g.bn), ktiles, true, &l);
   return false;
 }
 
@@ -1090,8 +1104,11 @@ int dispatch(const void* A, const void* B, void* C, int M, int N, int K, hipStre
       (K < 64 && (int64_t)M * N >= (int64_t)1 << 35))
     return kLaunchers[kNumGemmKernels](A, B, C, M, N, K, st);
   const int pick = pick_gemm_kernel(M, N, K, sizeof(OutT) == 4);
+  if (takes_between(pick, M, N, K)) {
+    if (K % 64 == 0) return launch_ring64<Ring64Shape<kBetweenRows, kBetweenColumns, 2>, OutT, InT>(A, B, C, M, N, K, st);
+    return launch_ring64<Ring64Shape<kBetweenRows, kBetweenColumns, 2, 4>, OutT, InT>(A, B, C, M, N, K, st);
+  }
   if (takes_lines(K)) {   // (kLinesKernels)
-    if (takes_between(pick, M, N, K)) return launch_ring64<Ring64Shape<kBetweenRows, kBetweenColumns, 2, 4>, OutT, InT>(A, B, C, M, N, K, st);
     if (pick == 7) return launch_ring64<Ring64Shape<128, 128, 2, 5>, OutT, InT>(A, B, C, M, N, K, st);
     if (pick == 10) return launch_ring64<Ring64Shape<192, 128, 2, 4>, OutT, InT>(A, B, C, M, N, K, st);
     if (pick == 11) return launch_ring64<Ring64Shape<192, 192, 2, 3>, OutT, InT>(A, B, C, M, N, K, st);
