@@ -202,3 +202,13 @@ def test_last_workgroup_merges(bh, lkv, d, splits, dtype):
         graph.replay()
         assert torch.equal(o, want)
         assert torch.equal(ops.flash_decode(q, k, v, splits), want)
+
+
+def test_output_has_the_strides_of_the_query():
+    # also those of extents of 1, whichever way the wrapper takes
+    k, v = (torch.randn(3, 65, 64, device=DEV, dtype=torch.float16) for _ in range(2))
+    long = torch.randn(3, 10, 64, device=DEV, dtype=torch.float16)
+    for q, key, value in ((long[:1, :1], k[:1], v[:1]), (long[:1, :1].squeeze(1), k[:1], v[:1]), (long[:, 2], k, v),
+                          (long[:, :1].contiguous(), k, v), (long[:1, 3:4], k[:1], v[:1])):
+        out = ops.flash_decode(q, key, value, 4)
+        assert out.shape == q.shape and out.stride() == torch.empty_like(q).stride()

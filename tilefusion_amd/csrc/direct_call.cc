@@ -89,6 +89,16 @@ at::Tensor empty_output(at::IntArrayRef shape, const at::Tensor& like) {
   return at::Tensor(at::detail::empty_cuda(shape, like.scalar_type(), like.device(), c10::nullopt));
 }
 
+// at::empty_like(like), which gives a dense tensor its strides, also the ones that address nothing (of extents of 1).
+at::Tensor empty_output_like(const at::Tensor& like) {
+  int64_t in_order = 1;
+  for (int64_t i = like.dim() - 1; i >= 0; --i) {
+    if (like.stride(i) != in_order) return at::empty_like(like);
+    in_order *= like.size(i);
+  }
+  return empty_output(like.sizes(), like);
+}
+
 bool is_half_type(const at::Tensor& t) { return t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16; }
 
 PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -186,7 +196,7 @@ PyObject* flash_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   at::Tensor out;
   {
     NoGil unlocked;
-    out = q.is_contiguous() ? empty_output(q.sizes(), q) : at::empty_like(q);
+    out = empty_output_like(q);
     op.redispatch(kCuda, q.contiguous(), k.contiguous(), v.contiguous(), out, num_splits, scale);
   }
   return THPVariable_Wrap(out);
