@@ -165,9 +165,11 @@ TF_API int tf_transpose_16bit(const void* in, void* out, int64_t batch, int64_t 
  * kernel 1 writes a partial (o, max, sum) per range in fp32 into `workspace`, kernel 2 merges
  * them with a log-sum-exp weighted sum into O.  `num_splits` is an upper bound: the library takes fewer and
  * longer ranges where that is sooner, or one (then kernel 1 writes O and there is no kernel 2); tf_flash_decode_plan
- * tells.  The workspace always has to hold num_splits partials a slice (tf_flash_decode_workspace_bytes); with 256 bytes a
- * slice more, kernel 1 merges as well where that is sooner (the range of a slice that is done last does it): same bits, one
- * launch.  What the workspace holds before a call does not matter.
+ * tells.  The workspace always has to hold num_splits partials a slice (tf_flash_decode_workspace_bytes).  Where it holds 256
+ * bytes a slice beyond the partials of the ranges that are taken (so it does with 256 bytes a slice beyond num_splits partials, or where
+ * enough fewer ranges are taken) and is ordinary memory of the current device (as tf_scatter_nd has it), kernel 1 merges as well where
+ * that is sooner: the range of a slice that is done last does it, counted by atomics in those bytes.  Same bits, one launch.
+ * What the workspace holds before a call does not matter.
  * Q [batch_heads, D]; K, V [batch_heads, Lkv, D]; O [batch_heads, D]; D must be 128 or 64.
  * All offsets are 64-bit (K alone has 2^31 elements at the benchmark size).
  * No counterpart in the reference (it has no decoding kernel); built on the same online

@@ -3,6 +3,7 @@ against the fp32 CPU oracle.  Tolerance: rel-L2 <= 1e-3, max-abs <= 2e-2.
 The reference has no decoding kernel: the oracle is the closed form, itself pinned by the
 split/combine identity and an independent C loop (tests/test_oracle_numerics.py)."""
 
+import ctypes
 import math
 
 import pytest
@@ -212,3 +213,20 @@ def test_output_has_the_strides_of_the_query():
                           (long[:, :1].contiguous(), k, v), (long[:1, 3:4], k[:1], v[:1])):
         out = ops.flash_decode(q, key, value, 4)
         assert out.shape == q.shape and out.stride() == torch.empty_like(q).stride()
+
+
+def test_workspace_outside_device_memory_holds_partials_only():
+    # whose arrivals are counted by atomics in memory that is ordinary for the device: elsewhere two kernels run, however large it is
+    bh, lkv, d, splits = 3, 1001, 64, 2
+    lib = _capi.load()
+    assert lib.tf_flash_decode_plan(bh, lkv, d, splits, ctypes.byref(ctypes.c_int())) == splits
+    g = torch.Generator(device=DEV).manual_seed(lkv)
+    q, k, v = (torch.randn(*shape, device=DEV, generator=g).half() for shape in ((bh, d), (bh, lkv, d), (bh, lkv, d)))
+    partials = lib.tf_flash_decode_workspace_bytes(bh, d, splits)
+    ws = torch.empty(partials + 4096, dtype=torch.uint8, pin_memory=True).fill_(0xA5)
+    o = torch.empty_like(q)
+    _capi.check(lib.tf_flash_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), 1, ws.data_ptr(), ws.numel(), bh, lkv, d,
+                                    splits, 1.0 / math.sqrt(d), stream()), "tf_flash_decode")
+    torch.cuda.synchronize()
+    assert torch.equal(o, c_decode(q, k, v, splits))
+    assert (ws[partials:] == 0xA5).all() and not (ws[:partials] == 0xA5).all()

@@ -22,6 +22,16 @@ int hip_fail(hipError_t e, const char* what) {
   return TF_ERR_HIP;
 }
 
+bool is_ordinary_device_memory(const void* p) {
+  int device = -1;
+  hipPointerAttribute_t a{};
+  if (hipGetDevice(&device) != hipSuccess || hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();   // not an error of this call
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && !a.isManaged && a.device == device && a.allocationFlags == hipDeviceMallocDefault;
+}
+
 arrivals_t next_arrivals_tag() {
   // splitmix64 over a count that starts differently in every process: tags do not repeat within 2^48 launches or so, and look like
   // nothing that a workspace holds (counts or addresses might)

@@ -174,6 +174,9 @@ TFK_DEVICE bool arrive(arrivals_t* word, arrivals_t tag, unsigned parts) {
 arrivals_t next_arrivals_tag();
 void set_error(const char* fmt, ...);
 int hip_fail(hipError_t e, const char* what);
+// Ordinary (coarse-grained) memory of the current device, for which hardware atomics are defined: on host, managed or fine-grained
+// memory an update may be lost.
+bool is_ordinary_device_memory(const void* p);
 
 #define TFK_HIP_TRY(expr)                                   \
   do {                                                      \

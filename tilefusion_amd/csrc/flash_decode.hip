@@ -434,9 +434,10 @@ int launch_split(const void* Q, const void* K, const void* V, void* O, float* o_
 }
 
 // The kernels on `st`; `partials` holds o_part then ml_part and, where there is `room` (bytes) for them, the words in which the
-// workgroups of a slice arrive, and is at a 16-byte boundary.
+// workgroups of a slice arrive, and is at a 16-byte boundary.  The arrivals are atomics: a caller's workspace elsewhere than in the
+// device's ordinary memory holds partials only.  own: it is the library's, which is.
 template <typename T, int D>
-int launch_decode_t(const void* Q, const void* K, const void* V, void* O, float* partials, size_t room,
+int launch_decode_t(const void* Q, const void* K, const void* V, void* O, float* partials, size_t room, bool own,
                     int64_t batch_heads, int64_t Lkv, int num_splits, double softmax_scale,
                     hipStream_t st) {
   const DecodePlan plan = plan_decode<D>(batch_heads, Lkv, num_splits);
@@ -448,7 +449,8 @@ int launch_decode_t(const void* Q, const void* K, const void* V, void* O, float*
   float* o_part = partials;
   float* ml_part = o_part + (size_t)batch_heads * plan.splits * D;
   const size_t part_floats = (size_t)batch_heads * plan.splits * (D + 2);   // (even: the words behind it are at 8-byte boundaries)
-  if (part_floats * sizeof(float) + (size_t)batch_heads * kArrivalsPitch * sizeof(arrivals_t) <= room && plan.waves == 8) {
+  if (part_floats * sizeof(float) + (size_t)batch_heads * kArrivalsPitch * sizeof(arrivals_t) <= room && plan.waves == 8 &&
+      (own || is_ordinary_device_memory(partials))) {
     arrivals_t* arrivals = reinterpret_cast<arrivals_t*>(partials + part_floats);
     return launch_split<T, D, 8, kMerged>(Q, K, V, O, o_part, ml_part, batch_heads, Lkv, plan, softmax_scale, st, arrivals);
   }
@@ -459,15 +461,15 @@ int launch_decode_t(const void* Q, const void* K, const void* V, void* O, float*
   return launch_kernel(flash_decode_combine_kernel<T, D>, dim3((unsigned)batch_heads), dim3(kCombThreads), 0, st,
                        o_part, ml_part, static_cast<T*>(O), plan.splits);
 }
-int launch_decode(const void* Q, const void* K, const void* V, void* O, float* partials, size_t room, int dtype,
+int launch_decode(const void* Q, const void* K, const void* V, void* O, float* partials, size_t room, bool own, int dtype,
                   int64_t batch_heads, int64_t Lkv, int64_t D, int num_splits, double softmax_scale,
                   hipStream_t st) {
   if (dtype == TF_DTYPE_BF16) {
-    if (D == 128) return launch_decode_t<bf16_t, 128>(Q, K, V, O, partials, room, batch_heads, Lkv, num_splits, softmax_scale, st);
-    return launch_decode_t<bf16_t, 64>(Q, K, V, O, partials, room, batch_heads, Lkv, num_splits, softmax_scale, st);
+    if (D == 128) return launch_decode_t<bf16_t, 128>(Q, K, V, O, partials, room, own, batch_heads, Lkv, num_splits, softmax_scale, st);
+    return launch_decode_t<bf16_t, 64>(Q, K, V, O, partials, room, own, batch_heads, Lkv, num_splits, softmax_scale, st);
   }
-  if (D == 128) return launch_decode_t<half_t, 128>(Q, K, V, O, partials, room, batch_heads, Lkv, num_splits, softmax_scale, st);
-  return launch_decode_t<half_t, 64>(Q, K, V, O, partials, room, batch_heads, Lkv, num_splits, softmax_scale, st);
+  if (D == 128) return launch_decode_t<half_t, 128>(Q, K, V, O, partials, room, own, batch_heads, Lkv, num_splits, softmax_scale, st);
+  return launch_decode_t<half_t, 64>(Q, K, V, O, partials, room, own, batch_heads, Lkv, num_splits, softmax_scale, st);
 }
 
 int decode_with_workspace(const char* who, const void* Q, const void* K, const void* V, void* O, int dtype,
@@ -479,7 +481,7 @@ int decode_with_workspace(const char* who, const void* Q, const void* K, const v
   TFK_REQUIRE(workspace_bytes >= need, TF_ERR_INVALID_ARG, "%s: workspace holds %zu bytes, %zu needed", who,
               workspace_bytes, need);
   TFK_REQUIRE(((uintptr_t)workspace & 15) == 0, TF_ERR_INVALID_ARG, "%s: workspace must be 16-byte aligned", who);
-  return launch_decode(Q, K, V, O, static_cast<float*>(workspace), workspace_bytes, dtype, batch_heads, Lkv, D, num_splits,
+  return launch_decode(Q, K, V, O, static_cast<float*>(workspace), workspace_bytes, false, dtype, batch_heads, Lkv, D, num_splits,
                        softmax_scale, static_cast<hipStream_t>(stream));
 }
 
@@ -521,7 +523,7 @@ extern "C" int tf_flash_decode_uncut(const void* Q, const void* K, const void* V
   int waves = 0;
   if (tf_flash_decode_plan(batch_heads, Lkv, D, num_splits, &waves) != 1) return TF_ERR_UNSUPPORTED;
   if (int rc = check_decode_args("tf_flash_decode_uncut", Q, K, V, O, batch_heads, Lkv, D, num_splits, softmax_scale)) return rc;
-  return launch_decode(Q, K, V, O, nullptr, 0, dtype, batch_heads, Lkv, D, num_splits, softmax_scale,
+  return launch_decode(Q, K, V, O, nullptr, 0, false, dtype, batch_heads, Lkv, D, num_splits, softmax_scale,
                        static_cast<hipStream_t>(stream));
 }
 
@@ -588,8 +590,8 @@ extern "C" int tf_flash_decode_static_f16(const void* Q, const void* K, const vo
               (unsigned long long)TF_FLASH_DECODE_STATIC_MAX_PARTIALS);
   float* partials = nullptr;
   if (int rc = scratch_on_current_device(&partials)) return rc;
-  // Nothing has to start at zero: the split kernel writes every (slice, split) partial the
-  // combine kernel reads, so whatever an earlier call left in the array is never read.
-  return launch_decode(Q, K, V, O, partials, kScratchFloats * sizeof(float), TF_DTYPE_F16, batch_heads, Lkv, D, num_splits, softmax_scale,
-                       static_cast<hipStream_t>(stream));
+  // Nothing has to start at zero: the split kernel writes every (slice, split) partial before it is
+  // read, and a word of arrivals may hold anything (arrivals_t).
+  return launch_decode(Q, K, V, O, partials, kScratchFloats * sizeof(float), true, TF_DTYPE_F16, batch_heads, Lkv, D, num_splits,
+                       softmax_scale, static_cast<hipStream_t>(stream));
 }

@@ -626,21 +626,10 @@ int launch_direct(const void* updates, void* data, const long long* indices, con
                        static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
 }
 
-// Hardware floating-point atomics are defined for ordinary (coarse-grained) memory of the device that runs the kernel:
-// on host, managed or fine-grained memory an update may be lost.
-bool is_ordinary_device_memory(const void* p) {
-  int device = -1;
-  hipPointerAttribute_t a{};
-  if (hipGetDevice(&device) != hipSuccess || hipPointerGetAttributes(&a, p) != hipSuccess) {
-    (void)hipGetLastError();   // not an error of this call
-    return false;
-  }
-  return a.type == hipMemoryTypeDevice && !a.isManaged && a.device == device && a.allocationFlags == hipDeviceMallocDefault;
-}
-
 template <typename T, Layout kLayout>
 int launch_rows(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
                 long long slice, long long targets, int lanes, long long words, hipStream_t st) {
+  // (floating-point atomics may lose an update elsewhere)
   if (!is_ordinary_device_memory(data))
     return launch_direct<T, kLayout, true>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
   // Times in us with log-uniform indices.  Few updates: no sort (806 of 34 fp32: direct 3.3, 16 of 256 threads' updates
