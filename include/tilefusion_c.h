@@ -227,8 +227,9 @@ TF_API int tf_scatter_nd(const void* updates, void* data, const int64_t* indices
                          int index_depth, int dtype, void* stream);
 
 /* What a call would run, decided on the host from the sizes alone; nothing is launched.
- * tf_gemm_kernel_index: position of the kernel in the table kGemmKernels (csrc/gemm.hip), or behind its end for the
- * bounds-checked kernel, with operands at 16-byte boundaries; -1 for sizes that tf_gemm rejects.  tf_flash_decode_plan: ranges per slice (1: not cut), and in
+ * tf_gemm_kernel_index, with operands at 16-byte boundaries: position of the kernel in the table kGemmKernels (csrc/gemm.hip), or behind
+ * its end 0 for the bounds-checked kernel, from 1 on for the whole-line forms of kLinesKernels, then for the tile of 160 x 128, K a
+ * multiple of 64, and its whole-line form; -1 for sizes that tf_gemm rejects.  tf_flash_decode_plan: ranges per slice (1: not cut), and in
  * *wavefronts those of a workgroup; 0 for arguments that tf_flash_decode rejects.  tf_flash_attention_rows:
  * query rows per workgroup of the tuned kernels for D = 64, 96, 128 (0 for other arguments); tf_flash_attention_pairs: 1 where
  * a workgroup of them takes two query tiles of a causal slice; tf_flash_attention_wide_rows: the rows of

@@ -95,10 +95,15 @@ def test_gemm_edge_cases_reach_every_kernel_of_the_table():
         assert [lib.tf_gemm_kernel_index(*mnk, 0) for mnk in problems] == [kernel] * len(problems)
     text = open(os.path.join(ROOT, "tilefusion_amd", "csrc", "gemm.hip")).read()
     table = re.search(r"constexpr GemmKernel kGemmKernels\[\] = \{\n(.*?)\n\};", text, re.S).group(1)
-    assert sorted(EDGES) == list(range(len(table.splitlines()) + 1))   # and the bounds-checked kernel
+    lines = re.search(r"constexpr LinesKernel kLinesKernels\[\] = \{\n(.*?)\n\};", text, re.S).group(1)
+    # the table, the bounds-checked kernel, the tiles that come with whole lines too, both forms of the tile of 160 rows: all that
+    # a call can run
+    assert sorted(EDGES) == list(range(len(table.splitlines()) + 1 + len(lines.splitlines()) + 2))
     assert lib.tf_gemm_kernel_index(0, 64, 64, 0) == -1 and lib.tf_gemm_kernel_index(64, 64, 1 << 22, 0) == -1
     # the grid of the bounds-checked kernel ends at 65535 columns of tiles
     assert lib.tf_gemm_kernel_index(512, 65535 * 64, 8, 1) == 15 and lib.tf_gemm_kernel_index(512, 65535 * 64 + 1, 8, 1) != 15
+    # the split-K kernels' launches end at 2^35 elements of C
+    assert lib.tf_gemm_kernel_index(1 << 25, 1 << 10, 8, 0) == 15
 
 
 def _plan(bh, lkv, d, splits):

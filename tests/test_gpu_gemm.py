@@ -132,7 +132,7 @@ def test_identity_operand():
     assert torch.equal(c, b.T)
 
 
-# Ragged problems for every kernel and tile that the dispatch can pick (for a 16-bit result; position in its table: m, n,
+# Ragged problems for every kernel and tile that the dispatch can pick (for a 16-bit result; its position, see tf_gemm_kernel_index: m, n,
 # k), at the edges where each can go wrong: fewer rows or columns than a tile, a last tile that overlaps its
 # neighbour by all but one row, K that completes its first (ring kernels) or last (split-K kernels)
 # 64-deep k-tile with 8 to 56 zeros, fewer k-tiles than wavefronts.  Small integers: exact in fp32, whatever the
@@ -146,17 +146,23 @@ EDGES = {
     4: [(17, 4561, 72), (257, 513, 328)],                                   # 32 x 32, four
     5: [(6426, 54, 4480), (165, 1765, 7616)],                               # 64 x 32
     6: [(3578, 101, 1000), (1088, 577, 1032), (50, 6432, 5688)],            # 64 x 64
-    7: [(205, 5613, 1904)],                                                 # 128 x 128, requests four tiles ahead
+    7: [(213, 5906, 448), (629, 2005, 448)],                                # 128 x 128, requests four tiles ahead
     8: [(2048, 2048, 136), (2177, 513, 136), (4939, 3091, 80), (1398, 5437, 72), (4929, 1741, 72),
         (4882, 2468, 72)],                                                  # 128 x 128, two ahead
     9: [(5216, 6236, 256)],                                                 # 128 x 128, two per CU
-    10: [(2999, 1544, 1032), (2689, 1409, 136)],                            # 192 x 128
+    10: [(2689, 1409, 136)],                                                # 192 x 128
     11: [(2305, 3265, 136), (1537, 4611, 152)],                             # 192 x 192
-    12: [(3333, 2288, 1944), (6145, 897, 144)],                             # 256 x 128
+    12: [(6145, 897, 144)],                                                 # 256 x 128
     13: [(4097, 2305, 264), (5378, 1537, 144)],                             # 256 x 192
     14: [(4865, 2305, 136), (2305, 4867, 136)],                             # 256 x 256
     15: [(517, 3008, 64), (982, 5472, 72), (4097, 2305, 40), (3301, 2817, 8), (4794, 235, 72),
          (812, 4675, 72)],                                                  # bounds-checked
+    16: [(205, 5613, 1904)],                                                # whole lines: 128 x 128
+    17: [(819, 5552, 352), (2763, 4176, 2184)],                             # 192 x 128
+    18: [(1555, 4613, 328)],                                                # 192 x 192
+    19: [(3333, 2288, 1944)],                                               # 256 x 128
+    20: [(2466, 1722, 256), (861, 5283, 384)],                              # 160 x 128, K a multiple of 64
+    21: [(2999, 1544, 1032), (3657, 1390, 328)],                            # ... whole lines
 }
 
 
@@ -181,27 +187,39 @@ def test_every_kernel_at_its_edges_is_exact(kernel, m, n, k, dtype):
 
 # Rows that start anywhere in a line (K % 64 != 0, from 328 on): the ring kernels fetch whole lines.  Every place in a line that
 # rows 8 apart can start at (K), first rows at another (operands that start at 16 bytes, not at a line), last tiles that
-# overlap their neighbours by any amount, few and many k-tiles.
-LINES = [(7, 4875, 196, 520), (7, 300, 3476, 528), (7, 3802, 259, 536), (7, 4328, 232, 544), (7, 4432, 228, 552),
-         (7, 1621, 647, 560), (7, 234, 4261, 568), (10, 770, 4610, 328), (10, 773, 4658, 336), (10, 4622, 776, 344),
-         (10, 4659, 771, 352), (10, 776, 4619, 360), (10, 4705, 769, 368), (10, 786, 4615, 376), (11, 1555, 4613, 328),
-         (11, 1539, 4624, 344), (11, 1542, 4633, 352), (11, 1559, 4653, 376), (12, 1159, 4639, 328), (12, 1155, 4609, 344),
-         (12, 1155, 4680, 352), (12, 1157, 4648, 376), (7, 205, 5613, 1904), (10, 2999, 1544, 1032), (12, 3333, 2288, 1944)]
+# overlap their neighbours by any amount, few and many k-tiles; every tile that comes with whole lines (the position of
+# what runs, as in EDGES), both operand types, both types of result.
+LINES = [(16, 4875, 196, 520), (16, 300, 3476, 528), (16, 3802, 259, 536), (16, 4328, 232, 544), (16, 4432, 228, 552),
+         (16, 1621, 647, 560), (16, 234, 4261, 568), (21, 770, 4610, 328), (21, 773, 4658, 336), (21, 4622, 776, 344),
+         (21, 4659, 771, 352), (21, 776, 4619, 360), (21, 4705, 769, 368), (21, 786, 4615, 376), (18, 1555, 4613, 328),
+         (18, 1539, 4624, 344), (18, 1542, 4633, 352), (18, 1559, 4653, 376), (19, 1159, 4639, 328), (19, 1155, 4609, 344),
+         (19, 1155, 4680, 352), (19, 1157, 4648, 376), (16, 205, 5613, 1904), (21, 2999, 1544, 1032), (19, 3333, 2288, 1944),
+         (17, 1028, 4632, 328), (17, 969, 4618, 336), (17, 3053, 1579, 344), (17, 3444, 1415, 352), (17, 1937, 2513, 360),
+         (17, 1617, 2985, 368), (17, 1483, 3320, 376), (17, 2763, 4176, 2184)]
 
 
 @pytest.mark.parametrize("kernel,m,n,k", LINES)
 @pytest.mark.parametrize("start", [0, 8, 40])
-def test_rows_that_start_anywhere_in_a_line(kernel, m, n, k, start):
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_rows_that_start_anywhere_in_a_line(kernel, m, n, k, start, dtype):
     from tilefusion_amd import _capi
-    assert _capi.load().tf_gemm_kernel_index(m, n, k, 0) == kernel
+    lib = _capi.load()
+    assert lib.tf_gemm_kernel_index(m, n, k, 0) == lib.tf_gemm_kernel_index(m, n, k, 1) == kernel
     g = torch.Generator(device=DEV).manual_seed(m + n + k)
 
     def inside(rows, at):   # between numbers that must not count
-        buf = torch.full((rows * k + 128,), float("nan"), device=DEV, dtype=torch.float16)
+        buf = torch.full((rows * k + 128,), float("nan"), device=DEV, dtype=dtype)
         return buf[at:at + rows * k].view(rows, k).copy_(torch.randint(-2, 3, (rows, k), device=DEV, generator=g))
 
     a, b = inside(m, start), inside(n, 48 - start)
-    assert torch.equal(c_gemm(a, b, torch.float32), a.float() @ b.float().t())   # exact: |sum| <= 4 k < 2^24
+    ref = a.float() @ b.float().t()                                      # exact: |sum| <= 4 k < 2^24
+    for out_dtype in (torch.float32, dtype):
+        buf = torch.full((m * n + 64,), 7.0, device=DEV, dtype=out_dtype)
+        _capi.check(lib.tf_gemm(a.data_ptr(), b.data_ptr(), buf.data_ptr(), 2 if dtype == torch.bfloat16 else 1,
+                                int(out_dtype == torch.float32), m, n, k, m, n, k, 1, 0,
+                                torch.cuda.current_stream().cuda_stream), "tf_gemm")
+        assert torch.equal(buf[:m * n].view(m, n), ref.to(out_dtype))
+        assert bool((buf[m * n:] == 7.0).all())                          # nothing behind C is written
 
 
 # ... and the tile of 160 rows that takes the place of the pick where that leaves CUs idle or begins another round: an odd number
@@ -210,19 +228,20 @@ BETWEEN = [(3657, 1390, 328), (1895, 2281, 968), (1596, 2453, 464), (1661, 2930,
            (2660, 1629, 360), (2501, 1657, 1000), (2315, 2084, 496), (1726, 2728, 376), (2643, 1708, 1016)]
 
 
-
 @pytest.mark.parametrize("m,n,k", BETWEEN)
 @pytest.mark.parametrize("start", [0, 8, 40])
-def test_tile_of_160_rows(m, n, k, start):
-    test_rows_that_start_anywhere_in_a_line(10, m, n, k, start)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_tile_of_160_rows(m, n, k, start, dtype):
+    test_rows_that_start_anywhere_in_a_line(21, m, n, k, start, dtype)
 
 
 # ... and with rows that start where lines do.
 @pytest.mark.parametrize("m,n,k", [(2466, 1722, 256), (3003, 1494, 256), (1541, 2582, 448), (861, 5283, 384), (3073, 1373, 1984),
                                    (4224, 983, 256), (3182, 1397, 1152)])
 @pytest.mark.parametrize("start", [0, 8])
-def test_tile_of_160_rows_of_whole_lines(m, n, k, start):
-    test_rows_that_start_anywhere_in_a_line(10, m, n, k, start)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_tile_of_160_rows_of_whole_lines(m, n, k, start, dtype):
+    test_rows_that_start_anywhere_in_a_line(20, m, n, k, start, dtype)
 
 
 def test_operands_without_16_byte_alignment():

@@ -1042,7 +1042,38 @@ int pick_short_k_kernel(int M, int N, int K, bool c_is_f32) {
   return best;
 }
 
+// What runs in place of `pick`, a kernel of the table: the tile between where it is ahead of a ring kernel of its kind, the same tile with whole
+// lines where rows start anywhere in one. Their positions are those behind the bounds-checked kernel's.
+constexpr int kLinesAt = kNumGemmKernels + 1, kBetweenWholeAt = kLinesAt + sizeof(kLinesKernels) / sizeof(kLinesKernels[0]),
+              kBetweenLinesAt = kBetweenWholeAt + 1, kNumGemmLaunchers = kBetweenLinesAt + 1;
+int stand_in(int pick, int M, int N, int K) {
+  const bool lines = takes_lines(K);
+  int at = pick;
+  const LinesKernel* of_pick = nullptr;
+  if (lines) {
+    for (const LinesKernel& l : kLinesKernels)
+      if (l.index == pick) {
+        of_pick = &l;
+        at = kLinesAt + (int)(&l - kLinesKernels);
+      }
+    if (of_pick == nullptr) return pick;
+  } else if (K % 64 != 0 || K < 256 || pick < 7 || pick > 12) {
+    return pick;
+  }
+  if (M < kBetweenRows || N < kBetweenColumns) return at;
+  const GemmKernel& g = kGemmKernels[pick];
+  const int ktiles = (K + 63) / 64;
+  auto expected = [&](const GemmKernel& k, const LinesKernel* l) {
+    return expected_us(k, (int64_t)((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn), ktiles, lines, l);
+  };
+  if (expected(kBetweenWhole, lines ? &kBetween : nullptr) < expected(g, of_pick)) return lines ? kBetweenLinesAt : kBetweenWholeAt;
+  return at;
+}
+
+// The kernel of a call whose operands start at 16-byte boundaries: a position in the launchers of dispatch().
 int pick_gemm_kernel(int M, int N, int K, bool c_is_f32) {
+  // (2^35 elements of C with a K below the ring kernels' are more threads than a launch of the split-K kernels may have)
+  if (K < 64 && (int64_t)M * N >= (int64_t)1 << 35) return kNumGemmKernels;
   if (K <= (c_is_f32 ? 128 : 120) && (int64_t)((M + 63) / 64) * ((N + 63) / 64) >= 96) return pick_short_k_kernel(M, N, K, c_is_f32);
   int best = 0;
   float best_us = INFINITY;
@@ -1063,24 +1094,7 @@ int pick_gemm_kernel(int M, int N, int K, bool c_is_f32) {
       best_us = us;
     }
   }
-  return best;
-}
-
-// `pick` is a ring kernel with whole lines, or for K that is a multiple of 64, and the tile between is ahead of it
-bool takes_between(int pick, int M, int N, int K) {
-  if (M < kBetweenRows || N < kBetweenColumns) return false;
-  const GemmKernel& g = kGemmKernels[pick % kNumGemmKernels];
-  const int ktiles = (K + 63) / 64;
-  auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  const int64_t between = tiles(kBetweenRows, kBetweenColumns);
-  if (K % 64 == 0)
-    return pick >= 7 && pick <= 12 && K >= 256 &&
-           expected_us(kBetweenWhole, between, ktiles, false, nullptr) < expected_us(g, tiles(g.bm, g.bn), ktiles, false, nullptr);
-  if (!takes_lines(K)) return false;
-  for (const LinesKernel& l : kLinesKernels)
-    if (l.index == pick)
-      return expected_us(kBetweenWhole, between, ktiles, true, &kBetween) < expected_us(g, tiles(g.bm, g.bn), ktiles, true, &l);
-  return false;
+  return stand_in(best, M, N, K);
 }
 
 template <typename OutT, typename InT>
@@ -1096,25 +1110,17 @@ int dispatch(const void* A, const void* B, void* C, int M, int N, int K, hipStre
       launch_ring64<Ring64Shape<192, 192, 2>, OutT, InT>, launch_ring64<Ring64Shape<256, 128, 2>, OutT, InT>,
       launch_ring64<Ring64Shape<256, 192, 2>, OutT, InT>, launch_ring64<Ring64Shape<256, 256, 2>, OutT, InT>,
       launch_guarded<ShapeSmall, OutT, InT>,
+      launch_ring64<Ring64Shape<128, 128, 2, 5>, OutT, InT>, launch_ring64<Ring64Shape<192, 128, 2, 4>, OutT, InT>,
+      launch_ring64<Ring64Shape<192, 192, 2, 3>, OutT, InT>, launch_ring64<Ring64Shape<256, 128, 2, 3>, OutT, InT>,
+      launch_ring64<Ring64Shape<kBetweenRows, kBetweenColumns, 2>, OutT, InT>,
+      launch_ring64<Ring64Shape<kBetweenRows, kBetweenColumns, 2, 4>, OutT, InT>,
   };
-  static_assert(sizeof(kLaunchers) / sizeof(kLaunchers[0]) == kNumGemmKernels + 1, "one launcher per row of kGemmKernels");
-  // LDS-direct requests take 16 bytes at a 16-byte boundary.  (2^35 elements of C with a K below the ring
-  // kernels' are more threads than a launch of the split-K kernels may have.)
-  if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) % 16 != 0 ||
-      (K < 64 && (int64_t)M * N >= (int64_t)1 << 35))
+  static_assert(sizeof(kLaunchers) / sizeof(kLaunchers[0]) == kNumGemmLaunchers,
+                "a launcher per row of kGemmKernels, the bounds-checked kernel, one per row of kLinesKernels, the two of 160 rows");
+  // LDS-direct requests take 16 bytes at a 16-byte boundary.
+  if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) % 16 != 0)
     return kLaunchers[kNumGemmKernels](A, B, C, M, N, K, st);
-  const int pick = pick_gemm_kernel(M, N, K, sizeof(OutT) == 4);
-  if (takes_between(pick, M, N, K)) {
-    if (K % 64 == 0) return launch_ring64<Ring64Shape<kBetweenRows, kBetweenColumns, 2>, OutT, InT>(A, B, C, M, N, K, st);
-    return launch_ring64<Ring64Shape<kBetweenRows, kBetweenColumns, 2, 4>, OutT, InT>(A, B, C, M, N, K, st);
-  }
-  if (takes_lines(K)) {   // (kLinesKernels)
-    if (pick == 7) return launch_ring64<Ring64Shape<128, 128, 2, 5>, OutT, InT>(A, B, C, M, N, K, st);
-    if (pick == 10) return launch_ring64<Ring64Shape<192, 128, 2, 4>, OutT, InT>(A, B, C, M, N, K, st);
-    if (pick == 11) return launch_ring64<Ring64Shape<192, 192, 2, 3>, OutT, InT>(A, B, C, M, N, K, st);
-    if (pick == 12) return launch_ring64<Ring64Shape<256, 128, 2, 3>, OutT, InT>(A, B, C, M, N, K, st);
-  }
-  return kLaunchers[pick](A, B, C, M, N, K, st);
+  return kLaunchers[pick_gemm_kernel(M, N, K, sizeof(OutT) == 4)](A, B, C, M, N, K, st);
 }
 
 }  // namespace
