@@ -102,6 +102,8 @@ def test_gemm_edge_cases_reach_every_kernel_of_the_table():
     assert lib.tf_gemm_kernel_index(0, 64, 64, 0) == -1 and lib.tf_gemm_kernel_index(64, 64, 1 << 22, 0) == -1
     # the grid of the bounds-checked kernel ends at 65535 columns of tiles
     assert lib.tf_gemm_kernel_index(512, 65535 * 64, 8, 1) == 15 and lib.tf_gemm_kernel_index(512, 65535 * 64 + 1, 8, 1) != 15
+    # the tile of 160 rows stands in for those of 128 columns, not for the larger ones
+    assert [lib.tf_gemm_kernel_index(*mnk, 0) for mnk in ((5288, 4630, 1768), (6509, 3887, 1848), (2388, 6435, 1312))] == [18, 18, 19]
     # the split-K kernels' launches end at 2^35 elements of C
     assert lib.tf_gemm_kernel_index(1 << 25, 1 << 10, 8, 0) == 15
 

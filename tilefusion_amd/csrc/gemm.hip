@@ -975,10 +975,12 @@ constexpr LinesKernel kLinesKernels[] = {
 };
 
 // A tile of 160 x 128, figures between those of 128 x 128 and 192 x 128, for grids that the one gives a second round and the
-// other leaves CUs idle on (2999 x 1544 x 1032: 208 tiles of 192 rows, 247 of 160). It takes the place of the pick where it is
-// expected to be done sooner: 50 such problems 5% faster (2% slower at most), us, the pick / it: 2999 x 1544 x 1032 17.9 / 16.4, 613 x
-// 7874 x 2040 26.1 / 22.9, 2547 x 1739 x 6712 63.5 / 59.1, fp32 result 66.6 / 61.0. Of K a multiple of 64, from 256 on: 3.5% over 50 (3.5% slower at
-// most): 2466 x 1722 x 256 8.4 / 7.8, 1571 x 3014 x 3008 33.3 / 30.0, 587 x 7483 x 2496 28.3 / 25.8.
+// other leaves CUs idle on (2999 x 1544 x 1032: 208 tiles of 192 rows, 247 of 160). It takes the place of one of these two where it is
+// expected to be done sooner. us, the pick / it, of one run each: 2999 x 1544 x 1032 17.9 / 16.4, 613 x 7874 x 2040 26.1 / 22.9, 2547 x
+// 1739 x 6712 63.5 / 59.1; 56 such problems take 0.923 of the time (1.00 at most). Of K a multiple of 64, from 256 on: 0.961 over 119
+// (1.02 at most): 2466 x 1722 x 256 8.4 / 7.8, 1571 x 3014 x 3008 33.3 / 30.0, 587 x 7483 x 2496 28.3 / 25.8. Not in place of the larger
+// tiles: whole lines of 192 x 192, which the model would have it replace now and then, are ahead of it by 5% on average (10% at most)
+// over 52 problems (5288 x 4630 x 1768, fp32 result, 94.8 / 104.4).
 constexpr LinesKernel kBetween = {-1, 1.45f, 4.15f, 0.373f, 0.153f};
 constexpr int kBetweenRows = 160, kBetweenColumns = 128;
 constexpr GemmKernel kBetweenWhole = {kBetweenRows, kBetweenColumns, 1, 1, true, 0.40f, 3.49f, 0.362f, 0.296f, 0.f};
@@ -1057,9 +1059,10 @@ int stand_in(int pick, int M, int N, int K) {
         at = kLinesAt + (int)(&l - kLinesKernels);
       }
     if (of_pick == nullptr) return pick;
-  } else if (K % 64 != 0 || K < 256 || pick < 7 || pick > 12) {
+  } else if (K % 64 != 0 || K < 256 || pick < 7) {
     return pick;
   }
+  if (pick > 10) return at;   // (tiles that are larger both ways)
   if (M < kBetweenRows || N < kBetweenColumns) return at;
   const GemmKernel& g = kGemmKernels[pick];
   const int ktiles = (K + 63) / 64;
