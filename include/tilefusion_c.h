@@ -234,12 +234,15 @@ TF_API int tf_scatter_nd(const void* updates, void* data, const int64_t* indices
  * query rows per workgroup of the tuned kernels for D = 64, 96, 128 (0 for other arguments); tf_flash_attention_pairs: 1 where
  * a workgroup of them takes two query tiles of a causal slice; tf_flash_attention_wide_rows: the rows of
  * tf_flash_attention_fwd_wide, twice that for pairs.  tf_fused_two_gemms_rows: rows per workgroup (64 or 128) where a problem, handed
- * `workspace_bytes`, runs the streaming kernel with operands at 16-byte boundaries, otherwise 0. */
+ * `workspace_bytes`, runs the streaming kernel with operands at 16-byte boundaries, otherwise 0.  tf_scatter_nd_plan, `data` in ordinary memory of the
+ * current device, it and 16-bit updates at 4-byte boundaries: updates that are sorted together (0: each goes straight to memory), and in
+ * *words_a_lane the 32-bit words of an update that a lane adds; -1 for other arguments. */
 TF_API int tf_gemm_kernel_index(int64_t M, int64_t N, int64_t K, int c_is_f32);
 TF_API int tf_flash_decode_plan(int64_t batch_heads, int64_t Lkv, int64_t D, int num_splits, int* wavefronts);
 TF_API int tf_flash_attention_rows(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D, int causal);
 TF_API int tf_flash_attention_pairs(int64_t batch, int64_t Lq, int64_t Lkv, int64_t D, int causal);
 TF_API int tf_flash_attention_wide_rows(int64_t batch, int64_t Lq, int causal);
+TF_API int tf_scatter_nd_plan(int64_t num_index_rows, int64_t targets, int64_t slice, int dtype, int* words_a_lane);
 TF_API int tf_fused_two_gemms_rows(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t P, size_t workspace_bytes);
 
 /* Run-time compilation of kernels written against the tile headers (tilefusion_amd/include),

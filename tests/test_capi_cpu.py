@@ -132,6 +132,32 @@ def test_decode_plan():
         assert 1 <= n <= splits and waves in (4, 8)  # the workspace holds `splits` partials a slice
 
 
+def _scatter_plan(n, targets, slice_, dtype):
+    lane = ctypes.c_int(0)
+    return _capi.load().tf_scatter_nd_plan(n, targets, slice_, dtype, ctypes.byref(lane)), lane.value
+
+
+def test_scatter_plan():
+    from tests.test_gpu_scatter_nd import FEW_WIDE
+    for dtype, elems in ((0, 1), (1, 2), (2, 2)):
+        for rows, words, n, chunk in FEW_WIDE:
+            fewer = 0 if n <= 1024 else 16
+            assert _scatter_plan(n, rows, words * elems, dtype) == ((1024 if n <= 1024 else 2048) if chunk else fewer, 1)
+        # distinct targets are possible: a sort would be in the way
+        for n, rows, words in ((407, 3872, 5048), (1000, 2732, 2248), (88, 2892, 32224), (560, 588, 3977)):
+            assert _scatter_plan(n, rows, words * elems, dtype) == (0, 1)
+        # a word a lane where that is a workgroup on every CU, with eight to a chunk or more
+        for n, words, lane in ((4096, 2000, 1), (4097, 257, 1), (8192, 512, 1), (8193, 512, 2), (8192, 513, 2), (11264, 300, 1), (12886, 491, 2),
+                               (9604, 696, 2), (5032, 581, 2), (19999, 2000, 2)):
+            assert _scatter_plan(n, 32000, words * elems, dtype) == (2048, lane)
+        assert _scatter_plan(20000, 32000, 512 * elems, dtype) == (4096, 2)
+        assert [_scatter_plan(n, 32000, 100 * elems, dtype)[0] for n in (1024, 1280, 8192, 8193, 20000)] == [0, 16, 1024, 2048, 4096]
+    # 16-bit updates of less than 2 Mi words are sorted by 16 up to 2048
+    assert _scatter_plan(1791, 3285, 632, 0) == (2048, 1) and _scatter_plan(1791, 3285, 1264, 2) == (16, 1)
+    assert _scatter_plan(2100, 300, 140000, 2) == (64, 1) and _scatter_plan(2401, 300, 140000, 2) == (128, 2)
+    assert _scatter_plan(0, 64, 64, 0)[0] == -1 and _scatter_plan(64, 64, 64, 3)[0] == -1
+
+
 def test_wide_attention_cases_reach_both_workgroup_sizes():
     import tests.test_gpu_ops as t
     marks = t.test_flash_attention_wide_heads.pytestmark

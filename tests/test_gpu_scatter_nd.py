@@ -101,7 +101,8 @@ def test_scatter_nd_owners_of_targets(dtype, dims, depth, n, start):
     assert not one[[0, 2]].any()
 
 
-# Wide slices, a word a lane: chunks of 1024, 2048 and 4096 updates, up to and beyond the updates, words and workgroups where one takes over.
+# Wide slices: each update for itself, sorted by 16, by 1024 and 2048 a chunk with a word or two a lane, around the numbers of updates, words
+# and workgroups where one takes over.
 # Sums of integers: at most ~1450 updates a target, none or one each way, keep every partial sum below 256 (8 deviations), which all types hold.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=lambda d: str(d).split(".")[-1])
 @pytest.mark.parametrize("rows,slice_,n", [(900, 1026, 4097), (900, 1024, 8193), (900, 514, 4097), (300, 4226, 4500), (200, 1154, 19999),
@@ -119,6 +120,30 @@ def test_scatter_nd_chunks_of_wide_slices(dtype, rows, slice_, n):
     dev = data.to(DEV)
     scatter_nd(dev, idx.unsqueeze(1).to(DEV), upd.to(DEV))
     assert torch.equal(dev.cpu().float(), want)
+
+
+# Few but wide updates in one chunk, from the fewest on: rows x 32-bit words of a slice x updates, and what test_capi_cpu.py's plan says of
+# them (1: a chunk of all, two of up to 1280; 0: one of the forms for fewer updates).
+FEW_WIDE = [(60, 12290, 128, 1), (60, 12290, 127, 0), (64, 12288, 128, 1), (65, 12290, 128, 0), (3, 7500, 300, 1), (300, 65536, 256, 1),
+            (300, 65535, 256, 0), (2000, 16384, 1024, 1), (512, 3070, 1025, 1), (640, 2458, 1280, 1), (640, 2457, 1280, 0),
+            (641, 2458, 1280, 0), (20, 24580, 131, 1)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("rows,words,n,chunk", FEW_WIDE)
+def test_scatter_nd_few_but_wide_updates(dtype, rows, words, n, chunk):
+    g = torch.Generator(device=DEV).manual_seed(rows + n)
+    slice_ = words * (4 // dtype.itemsize)
+    data = torch.randint(-2, 3, (rows, slice_), device=DEV, generator=g).to(dtype)
+    idx = (rows * torch.rand(n, device=DEV, generator=g) ** 2).long()
+    idx[5], idx[n - 1], idx[n // 2] = -1, rows, rows - 1          # two of them skipped
+    upd = torch.randint(-1, 2, (n, slice_), device=DEV, generator=g).to(dtype)
+    keep = (idx >= 0) & (idx < rows)
+    want = data.cpu().float().index_add_(0, idx[keep].cpu(), upd[keep].cpu().float())
+    assert want.abs().max() <= 256                                # exact in every type, whatever the order
+    from tilefusion_amd.ops import scatter_nd
+    scatter_nd(data, idx.unsqueeze(1), upd)
+    assert torch.equal(data.cpu().float(), want)
 
 
 # Targets with a large part of a chunk's updates: half of them to one row, an eighth to a second and a thirtieth to a third, in

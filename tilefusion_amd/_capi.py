@@ -45,6 +45,7 @@ SIGNATURES = {
     "tf_flash_attention_rows": (_i, [_i64, _i64, _i64, _i64, _i]),
     "tf_flash_attention_pairs": (_i, [_i64, _i64, _i64, _i64, _i]),
     "tf_flash_attention_wide_rows": (_i, [_i64, _i64, _i]),
+    "tf_scatter_nd_plan": (_i, [_i64, _i64, _i64, _i, ctypes.POINTER(_i)]),
     "tf_fused_two_gemms_rows": (_i, [_i64, _i64, _i64, _i64, _i64, _sz]),
     "tf_jit_compile": (_i, [ctypes.c_char_p, ctypes.c_char_p, ctypes.POINTER(ctypes.c_char_p), _i,
                             ctypes.POINTER(ctypes.c_char_p), _i, ctypes.POINTER(_vp)]),

@@ -626,68 +626,99 @@ int launch_direct(const void* updates, void* data, const long long* indices, con
                        static_cast<const T*>(updates), static_cast<T*>(data), indices, s, n, k, slice, total, lanes);
 }
 
+// What a call whose `data` is ordinary memory runs.  chunk: updates that are sorted together, 0: none, each goes straight to memory.
+// owners: by the owners' kernel, otherwise (chunk > 0) by workgroups of `threads`.  per_lane: words of an update that a lane has.
+struct ScatterPlan {
+  int chunk, threads, per_lane;
+  bool owners;
+};
+
+// Times in us, log-uniform indices where no others are named.  The host does not see the indices: a form is taken only where none of
+// log-uniform, uniform, distinct, evenly repeated and sorted ones, all of them one row or half of them, loses more than 6% by it.
+ScatterPlan plan_scatter(int elem_bytes, Layout layout, long long n, long long targets, long long words, int lanes) {
+  auto owners = [](int mine, int per_lane) { return ScatterPlan{mine * kOwnerThreads, kOwnerThreads, per_lane, true}; };
+  const bool pairs = layout == Layout::kPairs;
+  // What the target numbers (32 bits) and columns of sorted chunks do not hold: 2100 bf16 of 140000 into 300 rows 364 sorted by 64, 527 by
+  // 128, all to one row 591 and 2010.
+  const bool chunks_fit = targets < (1ll << 32) && n < (1ll << 31) && words <= 1024ll * lanes;
+  // Few but wide updates, where the atomics are what counts: sorted by the chunk where targets repeat twice on average, from 1.5 Mi words on
+  // (3 Mi in place of the sorted 16 below), and from 16 Mi on, where the sort is little beside the rest. The time of the other form / so: 214
+  // fp32 of 12266 into 67 rows 16.5 / 10.0, 598 of 5653 into 73 21.9 / 12.6, uniform 19.0 / 10.2, 1138 fp16 of 12030 into 266 32.2 / 20.1; 836
+  // fp16 of 41838 into 894 84 / 42, distinct 76 / 74. Over 109 problems 0.51, distinct 0.89, 1.02 at most in any order. Not elsewhere: 407 bf16
+  // of 10096 into 3872 12.0 / 10.7, but distinct 10.6 / 12.6; fewer than 128 updates 40 fp32 of 45341 into 3502 9.5 / 19.1.
+  const bool few_wide = pairs && chunks_fit && words > 256 && n >= 128 && n <= 1280 &&
+                        (n * words >= 16 << 20 || (n / 2 >= targets && n * words >= (n > 1024 ? 3 << 20 : 3 << 19)));
+  if (few_wide) return owners(n <= 1024 ? 1 : 2, 1);
+  // Few updates: no sort (806 of 34 fp32: direct 3.3, 16 of 256 threads' updates sorted 5.6).  From 1024 on contention shows (2048 of 64
+  // bf16 into 64 rows: direct 10.8, sorted 6.3).
+  if (n <= 1024) return {0, kScatterThreads, 1, false};
+  // Beyond, chunks sorted whole, except a few 16-bit updates: 1894 of 3924 21.8 sorted by 16, 14.6 by the chunk; 1077 fp32 of 26 into 95 5.6 and
+  // 6.1, 1469 of 68 into 350 8.1 and 6.9.  (Wide 16-bit ones of less than 2 Mi words: 1791 bf16 of 1264 into 3285 10.0 and 8.1, but
+  // distinct 8.1 and 9.4, sorted indices 8.1 and 10.2.)
+  if ((n <= 2048 && ((elem_bytes == 2 && n * words < 2 << 20) || !chunks_fit)) || n <= 1280) return {16, 256, 1, false};
+  if (!chunks_fit) {
+    // Every target hit at least eight times on average: the deeper sort.  A workgroup of eight wavefronts hides its own
+    // latencies where there are few of them, enough of four do it better.
+    if (n / 8 >= targets) return {128, 1024, 2, false};
+    return {64, (n / 64) * ((words + lanes - 1) / lanes) < 1024 ? 512 : 256, 1, false};
+  }
+  if (!pairs) return owners(2, 1);
+  // Longer chunks find more to merge, shorter ones are sorted sooner, in every workgroup.  4096 updates instead of 2048 from
+  // 20000 on (40000 bf16 of 1000 into 131072 rows 80 and 67, distinct indices 83 and 85; 8192 a chunk 69 and 88), 1024 where there are
+  // few (4096 fp32 of 64 into 8000 rows 7.7 and 7.1).
+  if (words <= 256) return owners(n >= 20000 ? 4 : n > 8192 ? 2 : 1, 1);
+  // Two words a lane halve the workgroups that sort the same indices, but one wavefront then waits for twice the loads and atomics.  So a word
+  // a lane up to 4096 updates (3873 fp16 of 1048 into 2024 12.6 and 13.3 with two), and up to 512 words where that is a workgroup on every CU and
+  // eight or more to a chunk: 8192 bf16 of 1024 into 32000 18.2 with two and 14.9, distinct 20.7 and 21.1; over 19 problems 0.81 of the
+  // time, uniform 0.92, distinct 0.94, all of them one row 0.81, half of them 0.78, sorted 0.95, 1.06 at most in any order. Elsewhere it
+  // loses where rows repeat: 9604 fp32 of 696 into 2760 21.9 and 19.0, all one row 15.5 and 18.6, sorted 21.1 and 24.3. (4096 a
+  // chunk and a word a lane: 5032 fp16 of 1162 into 890 14.6 and 14.3, all one row 11.8 and 17.0.)
+  if (n >= 20000) return owners(4, 2);
+  const OwnerGrid g = owner_grid(n, words, lanes, 2, 1);
+  const long long all = g.chunks * g.columns << g.bits;
+  return owners(2, n <= 4096 || (words <= 512 && g.bits >= 3 && all >= 224 && all <= 256) ? 1 : 2);
+}
+
 template <typename T, Layout kLayout>
 int launch_rows(const void* updates, void* data, const long long* indices, const Strides& s, long long n, int k,
                 long long slice, long long targets, int lanes, long long words, hipStream_t st) {
   // (floating-point atomics may lose an update elsewhere)
   if (!is_ordinary_device_memory(data))
     return launch_direct<T, kLayout, true>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  // Times in us with log-uniform indices.  Few updates: no sort (806 of 34 fp32: direct 3.3, 16 of 256 threads' updates
-  // sorted 5.6).  From 1024 on contention shows (2048 of 64 bf16 into 64 rows: direct 10.8, sorted 6.3).
-  // What the target numbers (32 bits) and columns of sorted chunks do not hold: 2100 bf16 of 140000 into 300 rows 364 sorted by 64, 527 by
-  // 128, all to one row 591 and 2010.
-  const bool chunks_fit = targets < (1ll << 32) && n < (1ll << 31) && words <= 1024ll * lanes;
-  // Few but wide updates: a chunk of all of them from 1.5 Mi words on, where the atomics are what counts (530 fp16 of 5710 into 39558 rows 10.1
-  // direct and 10.9, 480 of 5668 into 4345 9.9 and 8.7, 598 fp32 of 5672 into 257 19.9 and 12.7, 1242 of 3610 into 1022 25.5 by 16 and 14.9;
-  // uniform indices, which merge less, 882 fp16 of 7196 into 12239 16.7 and 18.1, 884 fp32 of 7770 into 464 32.7 and 20.2), and of 16-bit
-  // ones more than 1280 in any case (1404 of 1228 into 2501 8.8 and 7.7, 1556 of 2002 into 253 11.4 and 8.3; uniform, 1527 of 1914 into 39055
-  // 10.5 and 11.7).
-  const bool wide = kLayout == Layout::kPairs && chunks_fit && words > 256 && (n > 1280 || n * words >= 3 << 19);
-  if (!wide && n <= 1024)
-    return launch_direct<T, kLayout, false>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  // Beyond, chunks sorted whole, except a few 16-bit updates: 1894 of 3924 21.8 sorted by 16, 14.6 by the chunk; 1077 fp32 of 26 into 95 5.6 and
-  // 6.1, 1469 of 68 into 350 8.1 and 6.9.
-  if (!wide && ((n <= 2048 && ((sizeof(T) == 2 && n * words < 2 << 20) || !chunks_fit)) || n <= 1280))
-    return launch_shape<T, 256, 16, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  if (!chunks_fit) {
-    // Every target hit at least eight times on average: the deeper sort.  A workgroup of eight wavefronts hides its own
-    // latencies where there are few of them, enough of four do it better.
-    if (n / 8 >= targets)
-      return launch_shape<T, 1024, 128, 2, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-    if ((n / 64) * ((words + lanes - 1) / lanes) < 1024)
-      return launch_shape<T, 512, 64, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-    return launch_shape<T, 256, 64, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  }
-  // Longer chunks find more to merge, shorter ones are sorted sooner, in every workgroup.  4096 updates instead of 2048 from
-  // 20000 on (40000 bf16 of 1000 into 131072 rows 80 and 67, distinct indices 83 and 85; 8192 a chunk 69 and 88), 1024 where there are
-  // few (4096 fp32 of 64 into 8000 rows 7.7 and 7.1).  Two words a lane halve the workgroups that sort the same indices, but one
-  // wavefront then waits for twice the loads and atomics: from 20000 updates of more than 256 words on only (31652 fp32 of 2113
-  // into 46286 rows 168 and, a word a lane, 185; 47403 bf16 of 730 into 5971 52.5 and 53.0).  Below, a word a lane and 2048 a
-  // chunk are 10% ahead of two over 48 problems (8192 bf16 of 1024 into 32000 18.2 and 14.9; distinct indices 20.7 and 21.1).  With more than 512 words, where the columns alone
-  // nearly fill the chip, 4096 a chunk find more to merge (9573 fp16 of 1572 into 19695 29.7, 30.3 and 28.8, 5997 fp32 of 835 into 251
-  // 18.4, 18.4 and 15.0), unless that leaves a second workgroup to some CUs (9187 fp32 of 2929 into 4762 63, 60 and 74).
-  auto owners = [&](auto mine, auto per_lane, auto single) -> int {
-    return launch_owner<T, decltype(mine)::value, decltype(per_lane)::value, kLayout, decltype(single)::value>(
-        updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
-  };
-  using One = std::integral_constant<int, 1>;
-  using Two = std::integral_constant<int, 2>;
-  if constexpr (kLayout == Layout::kPairs) {
-    using Four = std::integral_constant<int, 4>;
-    using Many = std::false_type;
-    if (words > 256) {
-      if (n >= 20000) return owners(Four{}, Two{}, Many{});
-      // (one chunk, or two of up to 1024 that are sorted sooner: 1872 bf16 of 840 into 856 8.0 and, in one, 9.5, 1556 fp16 of 2002 8.3 and 10.3)
-      if (n <= 1024 || (n > 1280 && n <= 2048 && sizeof(T) == 2 && n * words < 2 << 20)) return owners(One{}, One{}, Many{});
-      const OwnerGrid g = owner_grid(n, words, lanes, 4, 1);
-      const bool longer = n > 4096 && words > 512 && g.chunks * g.columns << g.bits <= 256;
-      return longer ? owners(Four{}, One{}, Many{}) : owners(Two{}, One{}, Many{});
+  const ScatterPlan plan = plan_scatter(sizeof(T), kLayout, n, targets, words, lanes);
+  if (plan.owners) {
+    auto owners = [&](auto mine, auto per_lane, auto single) -> int {
+      return launch_owner<T, decltype(mine)::value, decltype(per_lane)::value, kLayout, decltype(single)::value>(
+          updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+    };
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    if constexpr (kLayout == Layout::kPairs) {
+      using Four = std::integral_constant<int, 4>;
+      using Many = std::false_type;
+      if (plan.chunk == kOwnerThreads) return owners(One{}, One{}, Many{});
+      if (plan.chunk == 2 * kOwnerThreads) return plan.per_lane == 1 ? owners(Two{}, One{}, Many{}) : owners(Two{}, Two{}, Many{});
+      return plan.per_lane == 1 ? owners(Four{}, One{}, Many{}) : owners(Four{}, Two{}, Many{});
+    } else {
+      return slice == 1 ? owners(Two{}, One{}, std::true_type{}) : owners(Two{}, One{}, std::false_type{});
     }
-    if (n >= 20000) return owners(Four{}, One{}, Many{});
-    return n <= 8192 ? owners(One{}, One{}, Many{}) : owners(Two{}, One{}, Many{});
-  } else {
-    return slice == 1 ? owners(Two{}, One{}, std::true_type{}) : owners(Two{}, One{}, std::false_type{});
   }
+  if (plan.chunk == 16)
+    return launch_shape<T, 256, 16, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+  if (plan.chunk == 64 && plan.threads == 512)
+    return launch_shape<T, 512, 64, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+  if (plan.chunk == 64)
+    return launch_shape<T, 256, 64, 1, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+  if (plan.chunk == 128)
+    return launch_shape<T, 1024, 128, 2, kLayout>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+  return launch_direct<T, kLayout, false>(updates, data, indices, s, n, k, slice, slice * targets, lanes, words, st);
+}
+
+// Lanes that share an update of `words` words.
+int lanes_of(long long words) {
+  int lanes = 1;
+  while (lanes < kWaveSize && lanes < words) lanes *= 2;
+  return lanes;
 }
 
 template <typename T>
@@ -698,8 +729,7 @@ int launch(const void* updates, void* data, const long long* indices, const Stri
   const bool pairs = kElems == 1 || (slice % 2 == 0 && reinterpret_cast<size_t>(updates) % 4 == 0 &&
                                      reinterpret_cast<size_t>(data) % 4 == 0);
   const long long words = (slice + kElems - 1 + (pairs ? 0 : 1)) / kElems;
-  int lanes = 1;
-  while (lanes < kWaveSize && lanes < words) lanes *= 2;
+  const int lanes = lanes_of(words);
   if constexpr (kElems == 2) {
     const size_t first = reinterpret_cast<size_t>(data), behind = first + (size_t)(slice * targets) * sizeof(T);
     if (!pairs && (first % 4 != 0 || behind % 4 != 0))
@@ -741,4 +771,15 @@ extern "C" int tf_scatter_nd(const void* updates, void* data, const int64_t* ind
   if (dtype == 0) return launch<float>(updates, data, idx, s, num_index_rows, index_depth, slice, targets, st);
   if (dtype == 1) return launch<half_t>(updates, data, idx, s, num_index_rows, index_depth, slice, targets, st);
   return launch<bf16_t>(updates, data, idx, s, num_index_rows, index_depth, slice, targets, st);
+}
+
+extern "C" int tf_scatter_nd_plan(int64_t num_index_rows, int64_t targets, int64_t slice, int dtype, int* words_a_lane) {
+  using namespace tfk;
+  if (num_index_rows <= 0 || targets <= 0 || slice <= 0 || dtype < 0 || dtype > 2 || !words_a_lane) return -1;
+  const bool split = dtype != 0 && slice % 2 != 0;
+  const long long words = dtype == 0 ? slice : (slice + 1 + (split ? 1 : 0)) / 2;
+  const ScatterPlan plan = plan_scatter(dtype == 0 ? 4 : 2, split ? Layout::kSplit : Layout::kPairs, num_index_rows, targets, words,
+                                        lanes_of(words));
+  *words_a_lane = plan.per_lane;
+  return plan.chunk;
 }
