@@ -420,7 +420,7 @@ def test_head_dimension_96_never_reads_the_padding_of_its_lds_rows():
             assert ok, f"causal={causal} vt={vt}: rel_l2={r:.3e} max_abs={m:.3e}"
 
 
-# Causal tiles end where the queries end: every workgroup size, with queries that fill the first tile but for one wavefront, by one
+# Causal tiles end where the queries end where CUs get several: every workgroup size, with queries that fill the first tile but for one wavefront, by one
 # row, by a key tile and not at all.  The rows are those of a call with as many queries as keys, bit for bit: only who computes them differs.
 @pytest.mark.parametrize("rows,b,d", [(64, 3, 64), (64, 3, 128), (128, 130, 64), (256, 300, 128)])
 @pytest.mark.parametrize("cut", [0, 1, 63, 64, 127, 129, 191, 192, 255])
@@ -431,6 +431,22 @@ def test_causal_tiles_end_with_the_queries(rows, b, d, cut):
     o = c_attention(q[:, :lq].contiguous(), k, v, True)
     assert torch.equal(o, c_attention(q, k, v, True)[:, :lq])
     ok, r, m = N.check_close(o[-1:].cpu(), N.attention_ref(q[-1:, :lq].cpu(), k[-1:].cpu(), v[-1:].cpu(), causal=True))
+    assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
+
+
+# Single causal tiles for no more than the CUs begin at the first query, up to 8 of a slice: (rows, slices, queries, D) with a last tile that is not
+# full, up to 256 workgroups and 8 tiles and beyond.  The rows are those of a slice alone, bit for bit.
+@pytest.mark.parametrize("rows,b,l,d", [(256, 95, 320, 128), (256, 101, 352, 128), (256, 128, 300, 128), (256, 42, 1290, 96), (128, 60, 311, 96),
+                                        (128, 98, 176, 128), (128, 115, 174, 64), (128, 33, 827, 128), (128, 29, 949, 96),
+                                        (128, 24, 1192, 128), (64, 129, 300, 128)])
+def test_causal_tiles_of_one_round_begin_with_the_queries(rows, b, l, d):
+    assert _capi.load().tf_flash_attention_rows(b, l, l, d, 1) == rows and not _capi.load().tf_flash_attention_pairs(b, l, l, d, 1)
+    q, k, v = (x.to(DEV) for x in _inputs(b, l, l, d, rows + l))
+    o = c_attention(q, k, v, True)
+    for i in (0, b // 2, b - 1):
+        assert torch.equal(o[i:i + 1], c_attention(q[i:i + 1], k[i:i + 1], v[i:i + 1], True)), i
+    assert not torch.isnan(o).any()
+    ok, r, m = N.check_close(o[-1:].cpu(), N.attention_ref(q[-1:].cpu(), k[-1:].cpu(), v[-1:].cpu(), causal=True))
     assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
 
 

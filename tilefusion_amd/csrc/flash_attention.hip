@@ -53,7 +53,7 @@ constexpr double kSplitMergeUs = 3.5, kSplitBytesPerUs = 2e6;
 double expected_single(const SingleCost& c, int64_t batch, int64_t Lq, int64_t Lkv, bool causal, int rows) {
   const int64_t q_tiles = (Lq + rows - 1) / rows, items = q_tiles * batch, rounds = (items + 255) / 256;
   const int64_t all = (Lkv + 63) / 64;   // key tiles of a slice
-  // key tiles of query tile i, all of them counted as full (fitted so; the kernel leaves a rest to the lightest)
+  // key tiles of query tile i, all of them counted as full (fitted so; where CUs get several the kernel leaves a rest to the lightest)
   auto weight = [&](int64_t i) -> int64_t { return causal ? std::min(all, (i + 1) * rows / 64) : all; };
   double t = (double)weight(q_tiles - 1) * c.tile * (1.0 + c.fill * std::min(1.0, (double)items / 256.0));
   auto share = [&](int64_t j, int64_t i) {

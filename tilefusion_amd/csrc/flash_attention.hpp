@@ -187,7 +187,7 @@ TFK_DEVICE SplitWeight<T> split_weight(float p) {
 template <typename T, int D, int DV, bool kKT, bool kVT, bool kCausal, int kWavesT, int kQB, bool kTail, bool kSplit>
 __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1) void flash_attention_fwd_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
-    T* __restrict__ O, int Lq, int Lkv, float scale_log2, int q_tiles, int total_items, int order, int d, float* __restrict__ part, int splits, int chunk) {
+    T* __restrict__ O, int Lq, int Lkv, float scale_log2, int q_tiles, int total_items, int order, int d, int end, float* __restrict__ part, int splits, int chunk) {
   using V2 = typename Vec<T>::v2;
   using V4 = typename Vec<T>::v4;
   using V8 = typename Vec<T>::v8;
@@ -296,12 +296,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
 
   for (int pass = 0; pass < num_passes; ++pass) {
   const int qt = qt_of_pass[pass];
-  // Causal tiles end where the queries end (up to a multiple of 64), so that the one that is not full is the lightest instead of the
-  // heaviest: up to a tile's keys less for every slice.  (64 slices of 1337 x 1337 x 64 27.0 / 25.8 us, 66 of 1560 x 128 71 / 61, 114 of 704 x
-  // 128 36.0 / 32.6.  Ends at multiples of 16 leave more to the lightest, but then wavefronts of one set meet their masked tiles
-  // at different times: 9 of 1364 x 64, which one workgroup's chain bounds, 14.8 / 15.5.)  The same rows share a wavefront
-  // either way, and their results are the same bits.
-  const int tile_row0 = kCausal ? (Lq + 63) / 64 * 64 - (q_tiles - qt) * kBMq : qt * kBMq;
+  const int tile_row0 = kCausal ? 64 * end - (q_tiles - qt) * kBMq : qt * kBMq;   // (causal: below 0 where the caller says so)
   const int q_row0 = tile_row0 + wave * kRowsPerWave;  // first query row of this wavefront
   // this lane's query rows: block qb holds row q_row0 + 16*qb + lr
 
@@ -971,11 +966,20 @@ int launch_w(const AttentionCall& c) {
   const int per_xcd = (c.batch + 7) / 8;
   const bool by_xcd = kCausal && !paired && c.batch % 8 != 0 && 8 * per_xcd * 100 <= c.batch * 104;
   const bool folded = kCausal && two_on_cu(kWavesT, kQB, D, kKT) && !paired && !by_xcd && total_items > kCUs && total_items <= (D == 64 ? kCUs * 9 / 4 : 2 * kCUs);
+  // Where causal tiles end, in 64 rows: where the queries end where CUs get several, so that the tile that is not full is the lightest instead of
+  // the heaviest: up to a tile's keys less for every slice.  (64 slices of 1337 x 1337 x 64 27.0 / 25.8 us, 66 of 1560 x 128 71 / 61, 114 of 704 x
+  // 128 36.0 / 32.6.  Ends at multiples of 16 leave more to the lightest, but then wavefronts of one set meet their masked tiles
+  // at different times: 9 of 1364 x 64, which one workgroup's chain bounds, 14.8 / 15.5.)  Rows in front of the first query are none then.
+  // With single tiles for no more than the CUs the heaviest is what counts, and it is done sooner if it is the one that is not full: 95 of
+  // 320 x 128 16.2 / 14.6, 0.94 of the time over 114 problems of up to 8 tiles a slice, 1.015 at most; longer slices are 2% behind so (6
+  // of 10 to 32 tiles, 8 of 3992 x 96 50.8 / 53.3).  The same rows share a wavefront either way, and their results are the same bits.
+  const bool from_front = !paired && total_items <= kCUs && q_tiles <= 8;
+  const int end = from_front ? q_tiles * (bm / 64) : (c.Lq + 63) / 64;
   const dim3 grid(by_xcd ? 8 * per_xcd * q_tiles : 8 * ((total_items + 7) / 8));
   return launch_kernel(kern, grid, dim3(kWavesT * 64), lds, c.stream,
                        static_cast<const T*>(c.Q), static_cast<const T*>(c.K),
                        static_cast<const T*>(c.V), static_cast<T*>(c.O), c.Lq, c.Lkv, c.scale_log2,
-                       q_tiles, total_items, paired ? kPairs : by_xcd ? kByXcd : folded ? kFolded : kSingle, c.d, c.part, c.splits, c.chunk);
+                       q_tiles, total_items, paired ? kPairs : by_xcd ? kByXcd : folded ? kFolded : kSingle, c.d, end, c.part, c.splits, c.chunk);
 }
 
 template <typename T, int D, bool kKT, bool kVT, bool kCausal, bool kTail>
