@@ -103,7 +103,9 @@ def test_gemm_edge_cases_reach_every_kernel_of_the_table():
     # the grid of the bounds-checked kernel ends at 65535 columns of tiles
     assert lib.tf_gemm_kernel_index(512, 65535 * 64, 8, 1) == 15 and lib.tf_gemm_kernel_index(512, 65535 * 64 + 1, 8, 1) != 15
     # the tile of 160 rows stands in for those of 128 columns, not for the larger ones
-    assert [lib.tf_gemm_kernel_index(*mnk, 0) for mnk in ((5288, 4630, 1768), (6509, 3887, 1848), (2388, 6435, 1312))] == [18, 18, 19]
+    assert [lib.tf_gemm_kernel_index(*mnk, 0) for mnk in ((2060, 7341, 816), (2073, 7409, 848), (2316, 6408, 904))] == [18, 18, 19]
+    # nor do whole lines for 256 x 192 and 256 x 256
+    assert [lib.tf_gemm_kernel_index(*mnk, 0) for mnk in ((5530, 3814, 1184), (7918, 1536, 1952), (7568, 5021, 1424))] == [13, 13, 14]
     # the split-K kernels' launches end at 2^35 elements of C
     assert lib.tf_gemm_kernel_index(1 << 25, 1 << 10, 8, 0) == 15
 

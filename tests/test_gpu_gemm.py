@@ -158,7 +158,7 @@ EDGES = {
     15: [(517, 3008, 64), (982, 5472, 72), (4097, 2305, 40), (3301, 2817, 8), (4794, 235, 72),
          (812, 4675, 72)],                                                  # bounds-checked
     16: [(205, 5613, 1904)],                                                # whole lines: 128 x 128
-    17: [(819, 5552, 352), (2763, 4176, 2184)],                             # 192 x 128
+    17: [(819, 5552, 352), (2944, 2016, 1056)],                             # 192 x 128
     18: [(1555, 4613, 328)],                                                # 192 x 192
     19: [(3333, 2288, 1944)],                                               # 256 x 128
     20: [(2466, 1722, 256), (861, 5283, 384)],                              # 160 x 128, K a multiple of 64
@@ -195,7 +195,7 @@ LINES = [(16, 4875, 196, 520), (16, 300, 3476, 528), (16, 3802, 259, 536), (16, 
          (18, 1539, 4624, 344), (18, 1542, 4633, 352), (18, 1559, 4653, 376), (19, 1159, 4639, 328), (19, 1155, 4609, 344),
          (19, 1155, 4680, 352), (19, 1157, 4648, 376), (16, 205, 5613, 1904), (21, 2999, 1544, 1032), (19, 3333, 2288, 1944),
          (17, 1028, 4632, 328), (17, 969, 4618, 336), (17, 3053, 1579, 344), (17, 3444, 1415, 352), (17, 1937, 2513, 360),
-         (17, 1617, 2985, 368), (17, 1483, 3320, 376), (17, 2763, 4176, 2184)]
+         (17, 1617, 2985, 368), (17, 1483, 3320, 376), (17, 2944, 2016, 1056)]
 
 
 @pytest.mark.parametrize("kernel,m,n,k", LINES)

@@ -1078,8 +1078,8 @@ int pick_gemm_kernel(int M, int N, int K, bool c_is_f32) {
   // (2^35 elements of C with a K below the ring kernels' are more threads than a launch of the split-K kernels may have)
   if (K < 64 && (int64_t)M * N >= (int64_t)1 << 35) return kNumGemmKernels;
   if (K <= (c_is_f32 ? 128 : 120) && (int64_t)((M + 63) / 64) * ((N + 63) / 64) >= 96) return pick_short_k_kernel(M, N, K, c_is_f32);
-  int best = 0;
-  float best_us = INFINITY;
+  int best = 0, best_plain = 0;
+  float best_us = INFINITY, best_plain_us = INFINITY;
   const int ktiles = (K + 63) / 64;
 #pragma unroll   // the divisions are by constants then
   for (int i = 0; i < kNumGemmKernels; ++i) {
@@ -1087,16 +1087,24 @@ int pick_gemm_kernel(int M, int N, int K, bool c_is_f32) {
     if (g.ring && (M < g.bm || N < g.bn || K < 64)) continue;   // (what gemm_ring64_kernel asks for)
     const int64_t tiles = (int64_t)((M + g.bm - 1) / g.bm) * ((N + g.bn - 1) / g.bn);
     if (tiles < g.min_tiles || tiles > g.max_tiles) continue;
-    const LinesKernel* lines = nullptr;
+    const float plain_us = expected_us(g, tiles, ktiles, K % 64 != 0, nullptr);
+    float us = plain_us;
     if (takes_lines(K))
       for (const LinesKernel& l : kLinesKernels)
-        if (l.index == i) lines = &l;
-    const float us = expected_us(g, tiles, ktiles, K % 64 != 0, lines);
+        if (l.index == i) us = expected_us(g, tiles, ktiles, true, &l);
     if (us < best_us) {
       best = i;
       best_us = us;
     }
+    if (plain_us < best_plain_us) {
+      best_plain = i;
+      best_plain_us = plain_us;
+    }
   }
+  // Where tiles of 256 x 192 or 256 x 256 would be picked if there were no whole lines they are: the two fits do not compare well there
+  // (us, those / the whole-line tile that is expected to be ahead: 5530 x 3814 x 1184 55.0 / 68.5, 7568 x 5021 x 1424 113 / 135, 3727 x 6430 x
+  // 1256 66 / 76; 80 such problems 1.077 of the time with whole lines, those tiles 0.3% behind the best of all).
+  if (best_plain == 13 || best_plain == 14) return best_plain;
   return stand_in(best, M, N, K);
 }
 
