@@ -107,6 +107,20 @@ def test_c5_full_size():
         assert (o.float() - c_decode(q, k, v, splits).float()).abs().max() < 1e-3
 
 
+# Not cut: one kernel that leaves the workspace alone.
+@pytest.mark.parametrize("bh,lkv,d,splits", [(127, 2111, 128, 64), (128, 1500, 128, 2), (200, 4099, 128, 3), (520, 63, 64, 3)])
+def test_uncut_slices_take_no_workspace(bh, lkv, d, splits):
+    lib, waves = _capi.load(), ctypes.c_int()
+    assert lib.tf_flash_decode_plan(bh, lkv, d, splits, ctypes.byref(waves)) == 1
+    g = torch.Generator(device=DEV).manual_seed(lkv)
+    q, k, v = (torch.randn(*shape, device=DEV, generator=g).half() for shape in ((bh, d), (bh, lkv, d), (bh, lkv, d)))
+    ws = torch.full((lib.tf_flash_decode_workspace_bytes(bh, d, splits) + 256 * bh,), 0xA5, device=DEV, dtype=torch.uint8)
+    o = torch.empty_like(q)
+    _capi.check(lib.tf_flash_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), 1, ws.data_ptr(), ws.numel(), bh, lkv, d,
+                                    splits, 1.0 / math.sqrt(d), stream()), "tf_flash_decode")
+    assert (ws == 0xA5).all() and torch.equal(o, ops.flash_decode(q, k, v, splits))
+
+
 # The cut is the library's: one workgroup of 8 or (from 512 slices on) 4 wavefronts per slice and no
 # partials, or up to num_splits ranges reduced by workgroups of 8 (fewer than 1024 of them) or 4
 # wavefronts; slices of more than 4 MiB, 2.75 GB together, come in ranges of 2 MiB in any case.  Lengths around the
@@ -166,23 +180,40 @@ def test_operands_that_start_anywhere(bh, lkv, d, splits, start, dtype, tol):
     assert N.rel_l2(o, ref) <= tol[0] and N.max_abs(o, ref) <= tol[1]
 
 
-# With 256 bytes a slice more than the partials the workgroup that is done last puts a slice together, instead of a second
-# kernel: the same sums in the same order, so the same bits, whatever the workspace held before.
+# Where the workspace has 256 bytes a slice beyond the partials of the ranges taken, the workgroup that is done last puts a slice together,
+# instead of a second kernel: the same sums in the same order, so the same bits, whatever the workspace held before.  Two and many
+# ranges, more than one turn of the loop that merges them (64 at D = 128, 128 at 64), up to 1023 workgroups.  The two kernels it is
+# compared with are those that a workspace outside the device's memory gets.
+MERGED = [(1, 30000, 128, 64), (3, 1001, 64, 2), (32, 1999, 64, 64), (1, 31360, 128, 70), (1, 38400, 64, 150), (100, 8192, 128, 2),
+          (127, 8192, 64, 2), (341, 8192, 64, 3), (2, 40000, 64, 257)]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("bh,lkv,d,splits", [(1, 30000, 128, 64), (3, 1001, 64, 2), (32, 1999, 64, 64), (127, 2111, 128, 64),
-                                             (128, 1500, 128, 2), (200, 4099, 128, 3), (2, 40000, 64, 257)])
+@pytest.mark.parametrize("bh,lkv,d,splits", MERGED)
 def test_last_workgroup_merges(bh, lkv, d, splits, dtype):
     g = torch.Generator(device=DEV).manual_seed(lkv)
     q, k, v = (torch.randn(*shape, device=DEV, generator=g).to(dtype) for shape in ((bh, d), (bh, lkv, d), (bh, lkv, d)))
     lib, code = _capi.load(), 2 if dtype == torch.bfloat16 else 1
-    want = c_decode(q, k, v, splits)
-    nbytes = lib.tf_flash_decode_workspace_bytes(bh, d, splits) + 256 * bh
+    partials = lib.tf_flash_decode_workspace_bytes(bh, d, splits)
+    nbytes = partials + 256 * bh
     o = torch.empty_like(q)
 
     def run(ws):
         o.fill_(math.nan)
-        _capi.check(lib.tf_flash_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), code, ws.data_ptr(), nbytes,
+        _capi.check(lib.tf_flash_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), code, ws.data_ptr(), ws.numel(),
                                         bh, lkv, d, splits, 1.0 / math.sqrt(d), stream()), "tf_flash_decode")
+
+    host = torch.empty(partials, dtype=torch.uint8, pin_memory=True)
+    run(host)
+    torch.cuda.synchronize()
+    want = o.clone()
+    assert torch.equal(c_decode(q, k, v, splits), want) and not torch.isnan(want).any()
+    # it does merge: the last to arrive leaves a zero behind
+    ranges = lib.tf_flash_decode_plan(bh, lkv, d, splits, ctypes.byref(ctypes.c_int()))
+    ws = torch.full((nbytes,), 0xA5, device=DEV, dtype=torch.uint8)
+    run(ws)
+    words = ws[lib.tf_flash_decode_workspace_bytes(bh, d, ranges):][:256 * bh].view(bh, 256)
+    assert not words[:, :8].any() and (words[:, 8:] == 0xA5).all()
 
     for held in (0, 255, 1, None):
         ws = torch.randint(0, 256, (nbytes,), device=DEV, dtype=torch.uint8, generator=g)
