@@ -121,6 +121,14 @@ def test_decode_cases_reach_every_way_to_cut():
     assert ways == {(cut, waves, d) for cut in (False, True) for waves in (4, 8) for d in (64, 128)}
 
 
+def test_decode_cases_that_are_merged_by_the_last_workgroup():
+    from tests.test_gpu_flash_decode import MERGED
+    plans = [(_plan(*c), c) for c in MERGED]
+    assert all(n > 1 and waves == 8 for (n, waves), _ in plans)
+    assert {d for (n, _), (_, _, d, _) in plans if n > 8192 // d} == {64, 128}   # a second turn of the merging loop
+    assert max(bh * n for (n, _), (bh, _, _, _) in plans) == 1023
+
+
 def test_decode_plan():
     assert _plan(512, 32768, 128, 64) == (8, 4)      # ranges of 2 MiB
     assert _plan(512, 32768, 128, 3) == (3, 4)       # the caller's limit
@@ -167,6 +175,15 @@ def test_wide_attention_cases_reach_both_workgroup_sizes():
     lib = _capi.load()
     assert {(lib.tf_flash_attention_wide_rows(bh, lq, int(causal)), causal) for bh, lq, _, causal in cases} == {
         (rows, causal) for rows in (64, 128) for causal in (False, True)}
+
+
+def test_attention_cases_of_a_second_round_reorder_workgroups():
+    from tests.test_gpu_flash_attention import BY_XCD, FOLDED
+    # (a slice's tiles stay on one XCD by their numbers, or where the XCDs get within 4% of the same number of slices)
+    for cases, by_xcd in ((FOLDED, False), (BY_XCD, True)):
+        assert {bh % 8 != 0 and (bh + 7) // 8 * 8 * 100 <= bh * 104 for _, bh, _, _ in cases} == {by_xcd}
+    counts = {(d > 128, (l + rows - 1) // rows * bh) for rows, bh, l, d in FOLDED}
+    assert {n for wide, n in counts if not wide} >= {264, 267, 291, 507, 576, 600} and {n for wide, n in counts if wide} >= {272, 450, 504, 512, 528}
 
 
 def test_attention_cases_reach_every_workgroup_form():

@@ -450,15 +450,26 @@ def test_causal_tiles_of_one_round_begin_with_the_queries(rows, b, l, d):
     assert ok, f"rel_l2={r:.3e} max_abs={m:.3e}"
 
 
-# Single causal tiles, two to a CU, the second 256 of them in the opposite order by eights: workgroups below, at and beyond the ends of
-# that range (three tiles of 128 queries a slice), every tile once.
-@pytest.mark.parametrize("bh", [85, 86, 88, 90, 170, 171, 192, 193])
-@pytest.mark.parametrize("d", [64, 56])
-def test_causal_second_round_of_workgroups(bh, d):
-    q, k, v = (x.to(DEV) for x in _inputs(bh, 384, 384, d, bh + d))
+# Single causal tiles where two share a CU (rows, slices, queries, D): the second 256 workgroups come in the opposite order, by eights, up to 576 of
+# them at D = 64 and 512 of wide heads; just beyond 256, where less than two eights are reordered, between, at the ends and beyond.
+FOLDED = [(128, 88, 384, 64), (128, 89, 384, 64), (128, 90, 384, 64), (128, 97, 384, 64), (128, 121, 384, 56), (128, 169, 384, 64), (128, 176, 384, 56),
+          (128, 192, 384, 64), (128, 192, 384, 56), (128, 200, 384, 64), (64, 32, 1024, 256), (64, 18, 1600, 256), (64, 9, 3584, 160), (64, 17, 1024, 192),
+          (64, 33, 1024, 256)]
+# ... and where a slice's stay on one XCD instead, or 64 rows are picked.
+BY_XCD = [(128, 85, 384, 64), (64, 86, 384, 64), (128, 170, 384, 64), (128, 171, 384, 56), (128, 193, 384, 64)]
+
+
+@pytest.mark.parametrize("rows,bh,l,d", FOLDED + BY_XCD)
+def test_causal_second_round_of_workgroups(rows, bh, l, d):
+    lib = _capi.load()
+    if d > 128:
+        assert lib.tf_flash_attention_wide_rows(bh, l, 1) == rows
+    else:
+        assert lib.tf_flash_attention_rows(bh, l, l, 64, 1) == rows and lib.tf_flash_attention_pairs(bh, l, l, 64, 1) == 0
+    q, k, v = (x.to(DEV) for x in _inputs(bh, l, l, d, bh + d))
     o = torch.full_like(q, float("nan"))
     torch.ops.tilefusion.flash_attention_fwd(q, k, v, o, d ** -0.5, True)
-    for i in range(0, bh, 3):
+    for i in range(0, bh, 3):   # every tile of a slice once, as alone
         alone = torch.empty_like(o[i:i + 1])
         torch.ops.tilefusion.flash_attention_fwd(q[i:i + 1].contiguous(), k[i:i + 1].contiguous(), v[i:i + 1].contiguous(), alone,
                                                  d ** -0.5, True)
