@@ -33,8 +33,9 @@ bool is_ordinary_device_memory(const void* p) {
 }
 
 arrivals_t next_arrivals_tag() {
-  // splitmix64 over a count that starts differently in every process: tags do not repeat within 2^48 launches or so, and look like
-  // nothing that a workspace holds (counts or addresses might)
+  // splitmix64 over a count that starts differently in every process, 48 bits of it: tags look like nothing that a workspace holds (counts or
+  // addresses might).  Two launches may have the same one (to be expected within some 2^24 of them); nothing rests on it, as no launch
+  // leaves its tag behind.
   static std::atomic<unsigned long long> count{
       (unsigned long long)std::chrono::system_clock::now().time_since_epoch().count() ^ (unsigned long long)(uintptr_t)&count};
   for (;;) {

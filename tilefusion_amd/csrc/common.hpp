@@ -103,19 +103,10 @@ TFK_DEVICE void barrier_lds_only() {
 // few KiB that change hands.
 // base: wavefront-uniform; offset in bytes, below 2^31
 template <typename V>
-TFK_DEVICE void store_shared_16B(void* base, unsigned offset, V v) {
-  static_assert(sizeof(V) == 16, "");
-#if defined(__HIP_DEVICE_COMPILE__)
-  constexpr int kRaw32Bit = 0x00020000, kAgent = 16;   // sc1
-  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, kRaw32Bit);
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, v), rsrc, offset, 0, kAgent);
-#endif
-}
-template <typename V>
 TFK_DEVICE V load_shared_16B(const void* base, unsigned offset) {
   static_assert(sizeof(V) == 16, "");
 #if defined(__HIP_DEVICE_COMPILE__)
-  constexpr int kRaw32Bit = 0x00020000, kAgent = 16;
+  constexpr int kRaw32Bit = 0x00020000, kAgent = 16;   // sc1
   const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, kRaw32Bit);
   return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset, 0, kAgent));
 #else
@@ -127,11 +118,11 @@ TFK_DEVICE float load_shared(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The word in which the workgroups of one result count, out of a workspace that holds anything at first: a tag of 48 bits that no
-// other launch has, and the number of arrivals.  The last to arrive leaves zero behind, which is what the next launch in the same
-// workspace, or the next replay of a captured one, finds and tags with a single operation that nobody waits for.  Anything
-// else that an allocator's block may hold costs the arrivals a second round trip; it would have to equal the tag to
-// be taken for it (2^-48).
+// The word in which the workgroups of one result count, out of a workspace that holds anything at first: a tag of 48 bits that is
+// drawn for the launch (a captured one has it in every replay), and the number of arrivals.  The last to arrive leaves zero behind, so that what
+// the next launch in the same workspace, or the next replay, finds is zero whatever its tag is, and it is tagged with a single
+// operation that nobody waits for.  Anything else that an allocator's block may hold costs the arrivals a second round trip;
+// it would have to equal the tag to be taken for it (2^-48).
 // Atomics on one address, or on one line, are done one after another (~50 ns): a word has 256 bytes to itself, and one workgroup
 // of a result opens it.
 using arrivals_t = unsigned long long;
@@ -170,7 +161,7 @@ TFK_DEVICE bool arrive(arrivals_t* word, arrivals_t tag, unsigned parts) {
 }
 
 // ---- host side ---------------------------------------------------------------------------
-// a tag for the arrivals of one launch
+// a tag for the arrivals of one launch: not zero, the count's bits clear
 arrivals_t next_arrivals_tag();
 void set_error(const char* fmt, ...);
 int hip_fail(hipError_t e, const char* what);

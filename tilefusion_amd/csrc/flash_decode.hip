@@ -396,8 +396,8 @@ struct DecodePlan {
 // long ranges cost a first pass more than they gain (32 of 55533 x 128: first 144-160 us in 4 MiB, 151-181; repeated 139 both).
 // Otherwise the cut aims at 1024 workgroups, and at no more than 256 KiB of keys and values in each: they
 // come in rounds, and the last one fills the chip badly (584 of 16256 x 64: 4 splits 411, 16 364; 136 of
-// 36053 x 64: 8 splits 201, 32 192), but at 32 KiB at least (32 of 1999 x 64: 16 splits 10.2, 64 12.8),
-// all within the caller's num_splits.
+// 36053 x 64: 8 splits 201, 32 192).  In any case 32 KiB at least (with the second kernel, 32 of 1999 x 64: 16 splits 10.2,
+// 64 12.8; for few slices, 3 of 1001 x 64, it is what limits the cut), all within the caller's num_splits.
 template <int D>
 DecodePlan plan_decode(int64_t batch_heads, int64_t Lkv, int num_splits) {
   const double slice_bytes = 4.0 * D * Lkv, stream_us = slice_bytes * batch_heads / 6.7e6, alone_us = slice_bytes / 45e3;

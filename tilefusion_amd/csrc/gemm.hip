@@ -112,8 +112,8 @@ TFK_DEVICE float16_t mfma32_t(in8_t<InT> a, in8_t<InT> b, float16_t c) {
 //
 // The same kernel serves smaller tiles (2 x 2 wavefronts of half a tile each way), for grids that 256 x 256
 // tiles would leave CUs idle on: 3333 x 2288 x 1944 takes 45.5 us with 126 tiles of 256 x 256, 36.7 with
-// 216 of 192 x 192 and 36.4 with 252 of 256 x 128; 2999 x 1544 x 1032 27.6 and, with 192 x 128, 16.0 (the bounds-checked kernel that ran
-// these shapes before: 37.8).  Units then have the size of the larger operand.  128 x 128 tiles have k-steps
+// 216 of 192 x 192 and 36.4 with 252 of 256 x 128; 2999 x 1544 x 1032 27.6 and, with 192 x 128, 18.7 (the bounds-checked kernel that ran
+// these shapes before: 37.8; whole lines, below, 17.3, and with 160 x 128 16.6).  Units then have the size of the larger operand.  128 x 128 tiles have k-steps
 // four times shorter; where a workgroup has its CU to itself their requests run kAhead = 4 tiles
 // ahead (a ring of 2 * kAhead + 1 = 9 units).
 //
@@ -123,7 +123,7 @@ TFK_DEVICE float16_t mfma32_t(in8_t<InT> a, in8_t<InT> b, float16_t c) {
 // the end of segment t and the front of segment t + 1, by an amount that only depends on the row. Rows 8 apart start at
 // the same place in a line, so a lane's fragments all are shifted alike, and what a lane pays is the choice between
 // the two segments (one v_and and one v_add3 an address). The ring is kept in whole tiles then, kLines of them: two are
-// read, the others in flight. 2999 x 1544 x 1032 18.5 -> 16.0 us (K = 1024: 14.7).
+// read, the others in flight. 2999 x 1544 x 1032 18.7 -> 17.3 us (K = 1024: 14.7).
 template <int BM_, int BN_, int AHEAD_, int LINES_ = 0>
 struct Ring64Shape {
   static constexpr int BM = BM_, BN = BN_, BK = 64;
@@ -958,7 +958,7 @@ constexpr int kNumGemmKernels = sizeof(kGemmKernels) / sizeof(kGemmKernels[0]);
 // segment more at first and saves them 0.13-0.27 us a k-tile. Microseconds as above, fitted to 60 problems (M, N 128-8192, K
 // 328-8192; 4-5% root mean square); picks are 2% behind the best of all kernels on average. us, k-tiles that start where rows
 // start / whole lines: 1500 x 1500 x 3000, 128 x 128 31.0 / 22.6; 700 x 4096 x 4104 40.2 / 30.5; 2999 x 1544 x 1032,
-// 192 x 128 18.5 / 16.0; 3333 x 2288 x 1944, 256 x 128 39.3 / 33.5, 192 x 192 35.3 / 33.6. (The larger tiles leave no room for a third
+// 192 x 128 18.7 / 17.3; 3333 x 2288 x 1944, 256 x 128 39.3 / 33.5, 192 x 192 35.3 / 33.6. (The larger tiles leave no room for a third
 // segment, and two workgroups of 128 x 128 none for each other; below K = 328 the further segment costs as much as it saves:
 // 8192 x 1000 x 328 14.0 / 13.5.)
 constexpr int kLinesFrom = 328;
@@ -976,7 +976,7 @@ constexpr LinesKernel kLinesKernels[] = {
 
 // A tile of 160 x 128, figures between those of 128 x 128 and 192 x 128, for grids that the one gives a second round and the
 // other leaves CUs idle on (2999 x 1544 x 1032: 208 tiles of 192 rows, 247 of 160). It takes the place of one of these two where it is
-// expected to be done sooner. us, the pick / it, of one run each: 2999 x 1544 x 1032 17.9 / 16.4, 613 x 7874 x 2040 26.1 / 22.9, 2547 x
+// expected to be done sooner. us, the pick / it, of one run each: 2999 x 1544 x 1032 17.3 / 16.6, 613 x 7874 x 2040 26.1 / 22.9, 2547 x
 // 1739 x 6712 63.5 / 59.1; 56 such problems take 0.923 of the time (1.00 at most). Of K a multiple of 64, from 256 on: 0.961 over 119
 // (1.02 at most): 2466 x 1722 x 256 8.4 / 7.8, 1571 x 3014 x 3008 33.3 / 30.0, 587 x 7483 x 2496 28.3 / 25.8. Not in place of the larger
 // tiles: whole lines of 192 x 192, which the model would have it replace now and then, are ahead of it by 5% on average (10% at most)
