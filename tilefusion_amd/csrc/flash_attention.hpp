@@ -199,6 +199,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   constexpr int kRowsPerWave = 16 * kQB;  // kQB 16-query blocks per wavefront
   constexpr int kBMq = kWavesT * kRowsPerWave;
   constexpr int DP = lds_pitch(D), DVP = lds_pitch(DV);   // LDS row pitch of the K / natural V tile
+  constexpr bool kEnds = kCausal && kBMq > 64;   // (tiles of 64 rows end where the queries end as they are)
   static_assert(!kKT || !kWide, "K^T tiles are 64 keys wide");
   static_assert(!kTail || (D == DV && !kWide && !kKT && !kVT), "");
   static_assert(!kSplit || (!kCausal && !kVT && kWavesT == 4 && kQB == 1), "");
@@ -296,7 +297,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
 
   for (int pass = 0; pass < num_passes; ++pass) {
   const int qt = qt_of_pass[pass];
-  const int tile_row0 = kCausal ? 64 * end - (q_tiles - qt) * kBMq : qt * kBMq;   // (causal: below 0 where the caller says so)
+  const int tile_row0 = kEnds ? 64 * end - (q_tiles - qt) * kBMq : qt * kBMq;   // (below 0 where the caller says so)
   const int q_row0 = tile_row0 + wave * kRowsPerWave;  // first query row of this wavefront
   // this lane's query rows: block qb holds row q_row0 + 16*qb + lr
 
@@ -308,7 +309,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
   V8 qf[kKK][kQB];
 #pragma unroll
   for (int qb = 0; qb < kQB; ++qb) {
-    const int m = q_row0 + 16 * qb + lr, m_ld = kCausal ? (int)min((unsigned)m, (unsigned)Lq - 1u) : min(m, Lq - 1);   // (causal: m < 0, too)
+    const int m = q_row0 + 16 * qb + lr, m_ld = kEnds ? (int)min((unsigned)m, (unsigned)Lq - 1u) : min(m, Lq - 1);   // (m < 0, too)
 #pragma unroll
     for (int kk = 0; kk < kKK; ++kk) {
       const int col = kk * 32 + lg * 8;
@@ -902,7 +903,7 @@ __global__ __launch_bounds__(kWavesT * 64, ring_stages(kWavesT, D) == 2 ? 2 : 1)
         v[1] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)x[1]);
         v[2] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)y[0]);
         v[3] = (unsigned)__builtin_amdgcn_ds_bpermute(4 * src_lane, (int)y[1]);
-        if (m_row < Lq && (!kCausal || m_row >= 0) && (!kTail || 16 * db + 8 * st_seg < dv_row)) *reinterpret_cast<uint4_t*>(o_lane + 16 * db) = v;
+        if (m_row < Lq && (!kEnds || m_row >= 0) && (!kTail || 16 * db + 8 * st_seg < dv_row)) *reinterpret_cast<uint4_t*>(o_lane + 16 * db) = v;
       }
     }
   }
